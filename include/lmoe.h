@@ -140,6 +140,12 @@ typedef struct lmoe_args {
    * counterpart in fla's signature. */
   lmoe_tensor q_raw, k_raw;
   float qk_eps;
+  /* optional fp32 buffers of lmoe_split_floats(a, op, 0 / 1) numbers for sequences cut along T (few (sequence, head)
+   * pairs: the sequential passes then run over segments of the sequences at once): seg_p is written by *_fwd and read
+   * by *_bwd, seg_ws is workspace of one call.  NULL: not cut.  A cut changes results by rounding only.  No counterpart
+   * in fla, which runs one program per (sequence, head, block of the state) whatever their number. */
+  float* seg_p;
+  float* seg_ws;
 } lmoe_args;
 
 /* Library version (major*10000 + minor*100 + patch). */
@@ -156,6 +162,10 @@ const char* lmoe_last_error(void);
  * in the reference; the ops are reached from the files named below). */
 int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B, int32_t T, int32_t H, int32_t K,
                              int32_t V, int32_t NT);
+
+/* Numbers (fp32) seg_p (part 0) and seg_ws (part 1) of this call need; 0 for both where the call is not cut.  Reads
+ * dtype, B, T, H, K, V, N, NT and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op / part. */
+int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part);
 
 /* chunk_simple_gla: S_t = e^{g_t} S_{t-1} + k_t^T v_t, o_t = scale q_t S_t, g scalar per
  * token-head (gate = SCALAR) or absent (gate = NONE).

@@ -98,6 +98,14 @@ int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B,
   return bytes;
 }
 
+int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part) {
+  const char* nm = "lmoe_split_floats";
+  if (!a) return fail(-1, "%s: null argument block", nm);
+  if (op != LMOE_OP_SIMPLE_GLA && op != LMOE_OP_GLA && op != LMOE_OP_GATED_DELTA_RULE) return fail(-21, "%s: unknown op %d", nm, op);
+  if (part != 0 && part != 1) return fail(-22, "%s: part must be 0 (seg_p) or 1 (seg_ws)", nm);
+  return lmoe::split_floats(*a, op, part);
+}
+
 int lmoe_chunk_simple_gla_fwd(const lmoe_args* a, void* stream) {
   const char* op = "lmoe_chunk_simple_gla_fwd";
   if (int r = check_common(a, op)) return r;

@@ -2,25 +2,59 @@
 #include "lmoe_launch.hpp"
 #include "lmoe_gdn_state.hpp"
 #include "lmoe_gdn_state_reg.hpp"
+#include "lmoe_gdn_split.hpp"
 
 namespace lmoe {
 
 // Width of the V-slice a work-group carries: the narrow slice gives more work-groups (a problem
 // with few (sequence, head) pairs must still reach every CU); with enough pairs the wide slice
 // halves the number of times k, w, q, P are read and stores whole 128-byte lines of o, v_new.
+// (V = 256: not cut; 12 waves of a fine segment's work-group would leave each too few registers for its columns)
+Split gdn_split_plan(const lmoe_args& a) { return a.V <= 128 ? plan_split(a, a.V / 32) : Split{}; }
 template <typename T, int V> inline bool wide_slices(const lmoe_args& a) {
   constexpr int BW = GdnStateCfg<T>::BV_WIDE;
   return BW <= V && BW != GdnStateCfg<T>::BV && (int64_t)a.N * a.H * (V / BW) >= cu_count();
 }
+// How the sequences of a call are cut: not at all without a workspace for it.
+inline Split gdn_split(const lmoe_args& a, bool bwd) {
+  Split sp = {};
+  if (!a.seg_ws || ((bwd || a.hs) && !a.seg_p)) return sp;
+  sp = gdn_split_plan(a);
+  if (!sp.len1) return sp;
+  const int64_t n1 = (int64_t)sp.n1 * a.H, n3 = (int64_t)sp.n3 * a.H;
+  sp.Q = a.seg_ws;
+  sp.S = sp.Q + n1 * a.K * a.V;
+  sp.P = (bf16*)(sp.S + n3 * a.K * a.V);
+  sp.D = (float*)(sp.P + n1 * a.K * a.K);
+  if (bwd || a.hs) {
+    sp.PT = (bf16*)a.seg_p;
+    sp.DT = (float*)(sp.PT + n1 * a.K * a.K);
+  }
+  return sp;
+}
+template <int K, int V> void combine(const lmoe_args& a, const Split& sp, bool bwd, hipStream_t st) {
+  const dim3 grid((a.N * a.H + 7) / 8 * 8 * (V / 16)), block(2 * K);
+  if (bwd) hipLaunchKernelGGL((k_split_combine<K, true>), grid, block, 0, st, a, sp);
+  else hipLaunchKernelGGL((k_split_combine<K, false>), grid, block, 0, st, a, sp);
+}
 template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, hipStream_t st) {
-  const int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
+  int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
   // w formed on the chip from Tinv where Tinv is there and LDS has room for a second k tile
   constexpr bool CAN_WT = sizeof(T) == 2;
   const bool wt = CAN_WT && a.tinv != nullptr;
   if constexpr (CAN_WT && BV == 32) {
     if (wt) {       // 2-byte elements with Tinv: the state stays in registers (lmoe_gdn_state_reg.hpp)
-      if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, (long long*)nullptr, -1);
-      else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, (long long*)nullptr, -1);
+      Split sp = {};
+      if constexpr (V <= 128) {
+        sp = gdn_split(a, false);
+        if (sp.len1) {
+          hipLaunchKernelGGL((k_gdn_seg_fwd<K, V>), dim3(sp.n1 * a.H), dim3(SEG_FWD_THREADS), 0, st, a, sp);
+          combine<K, V>(a, sp, false, st);
+          grid = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
+        }
+      }
+      if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
+      else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
       return;
     }
   }
@@ -36,8 +70,17 @@ template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, 
   }
 }
 template <typename T, int K, int V, int BV> void launch_bwd(const lmoe_args& a, hipStream_t st) {
-  const int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
-  hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV>), dim3(grid), dim3(3 * NTHR), 0, st, a);
+  int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
+  Split sp = {};
+  if constexpr (sizeof(T) == 2 && BV == 32 && V <= 128) {
+    sp = gdn_split(a, true);
+    if (sp.len1) {
+      hipLaunchKernelGGL((k_gdn_seg_bwd<K, V>), dim3(sp.n1 * a.H), dim3(SEG_BWD_THREADS), 0, st, a, sp);
+      combine<K, V>(a, sp, true, st);
+      grid = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
+    }
+  }
+  hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
 }
 template <typename T, int K, int V> struct GdnStateFwd {
   static void run(const lmoe_args& a, hipStream_t st) {
@@ -62,8 +105,14 @@ bool launch_gdn_state_fwd_trace(const lmoe_args& a, long long* tr, int work_grou
   if (a.dtype != LMOE_BF16 || a.K != 128 || a.V != 128 || !a.tinv || !a.hs) return false;
   const int grid = ((a.N * a.H + 7) / 8) * 8 * (128 / 32);
   if (work_group < 0 || work_group >= grid) return false;
-  hipLaunchKernelGGL((k_gdn_state_fwd_reg<128, 128, true, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, tr, work_group);
+  hipLaunchKernelGGL((k_gdn_state_fwd_reg<128, 128, true, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, Split{}, tr, work_group);
   return true;
+}
+int64_t split_floats(const lmoe_args& a, int op, int part) {
+  if (op != LMOE_OP_GATED_DELTA_RULE) return 0;
+  const Split sp = gdn_split_plan(a);
+  const int64_t trans = (int64_t)sp.n1 * a.H * (a.K * a.K / 2 + 1);      // a 2-byte matrix and a decay per fine segment
+  return part == 0 ? trans : (int64_t)(sp.n1 + sp.n3) * a.H * a.K * a.V + trans;
 }
 void launch_gdn_state_bwd(const lmoe_args& a, hipStream_t st) { dispatch_gdn<GdnStateBwd>(a, st); }
 

@@ -25,7 +25,7 @@
 //     get ids congruent mod 8, i.e. run on the same XCD and share k, w, q, P through its L2.
 #pragma once
 #include <type_traits>
-#include "lmoe_seq.hpp"
+#include "lmoe_split.hpp"
 
 namespace lmoe {
 
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd(const lmoe_args a) {
 //                      fragments of (k beta e^{b})^T | B3 | dS -= (k beta e^{b})^T dZ
 // ------------------------------------------------------------------------- //
 template <typename T, int K, int V, int BV>
-__global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a) {
+__global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16, KS = K / 32;
   constexpr int LPF = GdnStateCfg<T>::LPF;
@@ -437,9 +437,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a) {
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = vsl * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  if (pair >= (sp.len3 ? sp.n3 : a.N) * a.H) return;
+  const int v0 = vsl * BV, h = pair % a.H;
+  const PassItem item = pass_item(a, sp, pair / a.H);
+  if (item.n < 0) return;
+  const int n = item.n;
+  const SeqInfo sq = item.sq;
   const int l = lane_id();
   const int team = threadIdx.x / NTHR;
   if (sq.nchunks == 0) {
@@ -592,8 +595,8 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a) {
   const float scale = a.scale;
   f32x4 dS[MB][NB];
   acc_zero(dS);
-  if (a.dht) {
-    const float* p = a.dht + ((int64_t)n * a.H + h) * K * V;
+  if (a.dht || !item.last) {
+    const float* p = item.last ? a.dht + ((int64_t)n * a.H + h) * K * V : sp.S + (int64_t)pair * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)
 #pragma unroll
@@ -690,7 +693,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a) {
     }
   }
   lds_barrier();
-  if (a.dh0) {
+  if (a.dh0 && item.first) {
     float* p = a.dh0 + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)

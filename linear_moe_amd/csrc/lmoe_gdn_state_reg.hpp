@@ -31,6 +31,7 @@
 #pragma once
 #include <type_traits>
 #include "lmoe_gdn_state.hpp"
+#include "lmoe_split.hpp"
 
 namespace lmoe {
 
@@ -54,7 +55,7 @@ __device__ __forceinline__ bf16x8 load_frag_t_state(const bf16* tile, int ld, in
 // (frag_of_blocks, lmoe_common.hpp: two accumulator blocks -> the 8 contraction elements of an operand)
 
 template <int K, int V, bool SAVE, bool TRACE = false>
-__global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args a, long long* tr, int traced_wg) {
+__global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   typedef bf16 T;
   constexpr int BV = 32;
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
@@ -89,9 +90,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = vsl * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  if (pair >= (sp.len3 ? sp.n3 : a.N) * a.H) return;
+  const int v0 = vsl * BV, h = pair % a.H;
+  const PassItem item = pass_item(a, sp, pair / a.H);
+  if (item.n < 0) return;
+  const int n = item.n;
+  const SeqInfo sq = item.sq;
   const int l = lane_id();
   const int team = threadIdx.x / NTHR;
   if (sq.nchunks == 0) {
@@ -384,8 +388,8 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
   f32x4 S[KT];
 #pragma unroll
   for (int mi = 0; mi < KT; ++mi) S[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (a.h0) {
-    const float* h0 = a.h0 + ((int64_t)n * a.H + h) * K * V;
+  if (a.h0 || !item.first) {
+    const float* h0 = item.first ? a.h0 + ((int64_t)n * a.H + h) * K * V : sp.S + (int64_t)pair * K * V;
 #pragma unroll
     for (int mi = 0; mi < KT; ++mi)
 #pragma unroll
@@ -520,7 +524,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
     if (wv == 0) TR(0, c, 4);
   }
   lds_barrier();                                                                         // results of the last chunk
-  if (a.ht) {
+  if (a.ht && item.last) {
     float* ht = a.ht + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < KT; ++mi)

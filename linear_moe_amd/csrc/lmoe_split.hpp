@@ -1,0 +1,153 @@
+// Sequences cut along T for the sequential passes: when there are too few (sequence, head) pairs for the 256 CUs, a
+// pass over the chunks of a pair leaves most of the GPU idle (16 pairs x 4 V slices = 64 work-groups) and takes as
+// long as its chain of chunks.  A sequence is then cut into segments:
+//   1. every FINE segment (len1 chunks) is run from a zero state, all at once, for the state alone (no output): its
+//      own contribution Q and, for the delta rule, the matrix P that carries an initial state to its end;
+//   2. the segments of a pair are combined in order, S <- P S + Q (one small product per fine segment), which leaves
+//      the initial state of every COARSE segment (len3 = a multiple of len1 chunks) in memory;
+//   3. the ordinary pass runs over the coarse segments as if each were a sequence of its own.
+// Backward likewise from the end, with P transposed.  Cuts lie on chunk boundaries and never show outside: every
+// per-chunk buffer keeps its place.
+#pragma once
+#include "lmoe_seq.hpp"
+
+namespace lmoe {
+
+// What the kernels need to know; len1 = 0: not cut.
+struct Split {
+  int32_t len1;          // chunks per fine segment
+  int32_t len3;          // chunks per coarse segment (a multiple of len1)
+  int32_t n1, n3;        // segments of all sequences (packed input: upper bounds; a segment beyond the true count ends at once)
+  bf16 *P, *PT;          // [n1][H][K][K]  transitions of the fine segments less their decay (delta rule), in operand order, and
+                         // the same transposed (kept for the backward; NULL in a call that keeps nothing)
+  float *D, *DT;         // [n1][H]        decays of the fine segments (beside P, PT)
+  float* Q;              // [n1][H][K][V]  their contributions
+  float* S;              // [n3][H][K][V]  state (gradient) a coarse segment starts from
+};
+
+// Sequences of fewer chunks gain nothing (three kernels in place of one).  Longer ones than 32 768 tokens are left whole
+// although they would gain: there a sequence gives the same bits alone and inside a large packed batch, whose other
+// sequences fill the CUs (tests/test_gpu_large.py holds the ops to it).
+constexpr int SPLIT_MIN_CHUNKS = 24, SPLIT_MAX_CHUNKS = 512;
+
+__host__ __device__ inline int seg_count(int nchunks, int len) { return (nchunks + len - 1) / len; }
+
+struct SegInfo {
+  int n;          // sequence (-1: no such segment)
+  int j;          // segment inside the sequence
+  int nseg;       // segments of the sequence
+};
+
+// Segment number s (segments of all sequences in order) -> sequence and place inside it.  Packed input: every lane
+// counts the segments of one sequence, a scan over the wave gives the first segment of each (64 sequences a round).
+// All lanes of the wave must be active.
+__device__ __forceinline__ SegInfo seg_find(const lmoe_args& a, int len, int s) {
+  SegInfo r;
+  if (!a.cu_seqlens) {
+    r.nseg = seg_count((a.T + CH - 1) / CH, len);
+    r.n = s / r.nseg;
+    r.j = s % r.nseg;
+    if (r.n >= a.N) r.n = -1;
+    return r;
+  }
+  const int l = lane_id();
+  int base = 0;
+  for (int n0 = 0; n0 < a.N; n0 += 64) {
+    const int n = n0 + l;
+    const int cnt = n < a.N ? seg_count(a.seq_chunk0[n + 1] - a.seq_chunk0[n], len) : 0;
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(incl, d, 64);
+      if (l >= d) incl += y;
+    }
+    const int total = __shfl(incl, 63, 64);
+    if (s < base + total) {
+      const unsigned long long m = __ballot(s < base + incl);
+      const int w = __ffsll(m) - 1;                    // the first sequence whose segments reach past s
+      r.n = __builtin_amdgcn_readfirstlane(n0 + w);
+      r.nseg = __builtin_amdgcn_readlane(cnt, w);
+      r.j = s - base - (__builtin_amdgcn_readlane(incl, w) - r.nseg);
+      r.j = __builtin_amdgcn_readfirstlane(r.j);
+      return r;
+    }
+    base += total;
+  }
+  r.n = -1; r.j = 0; r.nseg = 0;
+  return r;
+}
+// number of the first segment of sequence n
+__device__ __forceinline__ int seg_base(const lmoe_args& a, int len, int n) {
+  if (!a.cu_seqlens) return n * seg_count((a.T + CH - 1) / CH, len);
+  const int l = lane_id();
+  int sum = 0;
+  for (int m = l; m < n; m += 64) sum += seg_count(a.seq_chunk0[m + 1] - a.seq_chunk0[m], len);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+// chunks [j len, (j + 1) len) of a sequence as a sequence of their own
+__device__ __forceinline__ SeqInfo seg_cut(SeqInfo s, int j, int len) {
+  s.tok0 += j * len * CH;
+  s.len = min(s.len - j * len * CH, len * CH);
+  s.chunk0 += j * len;
+  s.nchunks = (s.len + CH - 1) / CH;
+  return s;
+}
+
+// What a sequential pass works on: sequence number i of the call in the order of seq_at, or coarse segment number i.
+struct PassItem {
+  SeqInfo sq;
+  int n;                 // sequence (-1: nothing to do)
+  bool first, last;      // the item holds the first / the last chunk of its sequence
+};
+__device__ __forceinline__ PassItem pass_item(const lmoe_args& a, const Split& sp, int i) {
+  PassItem p;
+  if (sp.len3 == 0) {
+    p.n = seq_at(a, i);
+    p.sq = seq_info(a, p.n);
+    p.first = p.last = true;
+    return p;
+  }
+  const SegInfo g = seg_find(a, sp.len3, i);
+  p.n = g.n;
+  p.first = g.j == 0;
+  p.last = g.j == g.nseg - 1;
+  if (g.n >= 0) p.sq = seg_cut(seq_info(a, g.n), g.j, sp.len3);
+  return p;
+}
+// How a call is cut (pointers left open), or len1 = 0.  `slices` = work-groups of the ordinary pass per (sequence, head),
+// which hold a CU each; the work-groups of step 1 carry all columns and hold a CU each too.  Chosen by what the three steps
+// were measured to take (us, K = V = 128, delta rule; half of it per chunk at K = V = 64):
+//   ordinary pass   1.7 per chunk up to 64 work-groups, 2.1 beyond, 2.2 on a full GPU
+//   step 1          7 + 3.3 per chunk        step 2   4 + 0.65 per fine segment       step 3   1 + 2.2 per chunk
+// e.g. 16 heads, one sequence: 47 chunks 83 -> 56, 256 chunks 433 -> 213 (forward), 381 -> 215 (backward).
+inline Split plan_split(const lmoe_args& a, int slices) {
+  Split s = {};
+  if (a.dtype != LMOE_BF16 || a.N < 1 || a.T < 1) return s;
+  const int cus = cu_count(), slots = cus / (a.H * slices);       // coarse segments that fill the CUs, all sequences together
+  // at least three coarse segments each: with two, the longest sequence that gained (256 chunks, 32 pairs) took 0.8 of
+  // the time, most 0.9 and more
+  if (slots < 3 * a.N) return s;
+  const bool packed = a.cu_seqlens != nullptr;                    // (the lengths are not known here: as if they were equal)
+  const int nch = packed ? (a.NT + a.N - 1) / a.N : (a.T + CH - 1) / CH;
+  if (nch < SPLIT_MIN_CHUNKS || a.NT > a.N * SPLIT_MAX_CHUNKS) return s;
+  const float w = (a.K + a.V) / 256.f;
+  float best = 0.9f * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
+  // packed: sum over the sequences of ceil(chunks / len3) <= NT / len3 + N segments
+  const int rmax = packed && a.N > 1 ? (slots - a.N) / a.N : slots / a.N;
+  for (int r = 3; r <= rmax && r <= 32; ++r)
+    for (int f = 1; f <= 4; ++f) {
+      const int len3 = seg_count(nch, r), len1 = seg_count(len3, f), nf = seg_count(nch, len1);
+      const int rounds = seg_count(a.N * a.H * nf, cus);
+      const float t = 12.f + 3.3f * w * len1 * rounds + 0.65f * w * (nf - f) + 2.2f * w * (len1 * f);
+      if (t < best) { best = t; s.len1 = len1; s.len3 = len1 * f; }
+    }
+  if (!s.len1) return s;
+  s.n1 = packed ? a.NT / s.len1 + a.N : a.N * seg_count(nch, s.len1);
+  s.n3 = packed ? a.NT / s.len3 + a.N : a.N * seg_count(nch, s.len3);
+  return s;
+}
+inline int pass_items(const lmoe_args& a, const Split& sp) { return sp.len3 ? sp.n3 : a.N; }
+
+}  // namespace lmoe

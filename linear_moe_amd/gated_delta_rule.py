@@ -87,12 +87,27 @@ class GDNCall:
             raise ValueError("v_act exists for bfloat16")
         a.v_act = int(bool(v_act))
         ctx.v_act = bool(v_act)
+        seg_p = self._cut(lib, a, dev, save)
         _lib.check(lib.lmoe_chunk_gated_delta_rule_fwd(C.byref(a), stream_ptr()), "chunk_gated_delta_rule forward")
-        ctx.saved = (q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew)
-        ctx.fwd_args, ctx.fwd_keep = a, ((o, ht, w, u) if self.keep else None)
+        ctx.saved = (q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew, seg_p)
+        ctx.fwd_args, ctx.fwd_keep = a, ((o, ht, w, u, seg_p, self.seg_ws) if self.keep else None)
         ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, dims, head_first, scale
         ctx.has_h0 = initial_state is not None
+        self.seg_ws = None
         return o, ht
+
+    def _cut(self, lib, a, dev, save=False, seg_p=None):
+        """The buffers of a call whose sequences are cut along T (``lmoe_args.seg_ws``; ``seg_p``, which a call that
+        saves hands to its backward), or none."""
+        self.seg_ws = None
+        n = lib.lmoe_split_floats(C.byref(a), self.OP, 1)
+        if n <= 0:
+            return None
+        if save:
+            seg_p = torch.empty(lib.lmoe_split_floats(C.byref(a), self.OP, 0), dtype=torch.float32, device=dev)
+        self.seg_ws = torch.empty(n, dtype=torch.float32, device=dev)
+        a.seg_p, a.seg_ws = ptr(seg_p), self.seg_ws.data_ptr()
+        return seg_p
 
     def backward(self, do, dht, dv_out=None, dq_out=None, dk_out=None, qk_raw=None, qk_eps=1e-6):
         """dv_out, dq_out, dk_out: where the gradients go (tensors of the shapes of v, q, k, any strides the kernels
@@ -101,7 +116,7 @@ class GDNCall:
         dk are returned with respect to them."""
         ctx = self
         lib = _lib.load()
-        q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew = ctx.saved
+        q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew, seg_p = ctx.saved
         plan, dims, head_first = ctx.plan, ctx.dims, ctx.head_first
         B, T, H, K, V = dims
         do = _aligned(do)
@@ -143,9 +158,12 @@ class GDNCall:
         dvnew = torch.empty_like(vnew)
         a.dhs = dhs.data_ptr()
         a.dvnew.ptr = dvnew.data_ptr()
+        if seg_p is not None:
+            self._cut(lib, a, dev, seg_p=seg_p)
         _lib.check(lib.lmoe_chunk_gated_delta_rule_bwd(C.byref(a), stream_ptr()), "chunk_gated_delta_rule backward")
         ctx.bwd_args = a
-        ctx.bwd_keep = (do, dht, dq, dk, dv, dg, dbeta, dh0, dhs, dvnew, qk_raw) if self.keep else None
+        ctx.bwd_keep = (do, dht, dq, dk, dv, dg, dbeta, dh0, dhs, dvnew, qk_raw, self.seg_ws) if self.keep else None
+        self.seg_ws = None
         dg = None if g is None else dg.to(g.dtype)
         return dq, dk, dv, dg, dbeta.to(beta.dtype), dh0
 
