@@ -334,6 +334,27 @@ int lmoe_mom_combine(const void* src, const int32_t* idx, const void* w, void* o
 int lmoe_mom_rowdot(const void* src, const int32_t* idx, const void* g, void* dw, int64_t ntok, int32_t topk, int32_t D,
                     int32_t dtype, void* stream);
 
+/* The backward of combine in one pass over g and y: dy[row_of[t][k]] = w[t][k] * g[t], dw[t][k] = <g[t], y[row_of[t][k]]>
+ * (0 for row_of < 0); rows of dy that belong to no choice (src_choice < 0) are set to zero.  y, dy: [nrows][D]. */
+int lmoe_mom_combine_bwd(const void* y, const int32_t* row_of, const int32_t* src_choice, const void* w, const void* g,
+                         void* dy, void* dw, int64_t ntok, int64_t nrows, int32_t topk, int32_t D, int32_t dtype,
+                         void* stream);
+/* Routing tables on the device (`transform`'s sort, mom_linear_attention.py:28-66).  sel: the memory index of every
+ * choice, [B][per_row] with per_row = S * topk, int64 (is64) or int32; E memories; cap: tokens kept per (memory, batch
+ * row), the last ones, -1 = all.  counts: scratch of lmoe_mom_plan_ints() int32 (0: sizes the kernels do not take).
+ * Results: cu [E * B + 1], max_len [1], mem_offsets [E + 1], src_token and src_choice [B * per_row] (rows past
+ * cu[E * B] hold -1), row_of [B * per_row] (-1: dropped). */
+int64_t lmoe_mom_plan_ints(int32_t B, int32_t per_row, int32_t E);
+int lmoe_mom_plan(const void* sel, int32_t is64, int32_t B, int32_t per_row, int32_t topk, int32_t E, int32_t cap,
+                  int32_t* counts, int32_t* cu, int64_t* max_len, int64_t* mem_offsets, int32_t* src_token,
+                  int32_t* src_choice, int32_t* row_of, void* stream);
+
+/* Chunk tables of packed input from N + 1 offsets on the device (int64 with is64, else int32; N <= 4096): what
+ * lmoe_args.cu_seqlens, chunk_map ([nt_max][2]), seq_chunk0 ([N + 1]), nt_dev ([1]) and seq_order ([N], longest first;
+ * may be null) point to.  nt_max: an upper bound of the chunk count; rows of chunk_map past the count name sequence N. */
+int lmoe_seq_tables(const void* offsets, int32_t is64, int32_t N, int32_t nt_max, int32_t* cu, int32_t* chunk_map,
+                    int32_t* seq_chunk0, int32_t* nt_dev, int32_t* seq_order, void* stream);
+
 /* Launch ONE kernel of an op's pipeline (profiling support: lets a harness time each kernel
  * with events on its own stream).  `a` must be the fully populated argument block of the
  * op's fwd (stages 0-2, 7) or bwd (stages 3-5) entry point, with the intermediates of the

@@ -19,6 +19,9 @@ from ._lib import Args, Tensor4, CHUNK
 _DT = {torch.bfloat16: _lib.LMOE_BF16, torch.float32: _lib.LMOE_F32}
 
 
+SEQ_TABLES_MAX = 4096      # sequences that lmoe_seq_tables takes
+
+
 def _check_inputs(q, k, v, head_first: bool, cu_seqlens, wide_v: bool = False) -> Tuple[int, int, int, int, int]:
     """wide_v: the op also has kernels for K = 128 with V = 256 (the gated delta rule)."""
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
@@ -150,7 +153,7 @@ class SeqPlan:
     the device tables the kernels index with.  Build through ``seq_plan`` (cached).
 
     Offsets on the host (a CPU ``cu_seqlens``) are validated and give exact tables.  Offsets on the device are never
-    read back: the tables are built there by a handful of small device operations, sized for the upper bound
+    read back: the tables are built there (by one kernel; above 4096 sequences by tensor operations), sized for the upper bound
     ``NT <= ceil(T / 64) + N`` of the chunk count (every sequence ends in at most one partial chunk), with the true
     count in ``nt_dev`` for the kernels; nothing synchronises with the host, so the build can run inside a HIP
     graph capture and a replay follows the offsets the buffer holds at that time.  Device offsets are trusted
@@ -197,6 +200,20 @@ class SeqPlan:
         dev = cu_seqlens.device
         N = cu_seqlens.numel() - 1
         nt_max = (T + CHUNK - 1) // CHUNK + N
+        if N <= SEQ_TABLES_MAX and cu_seqlens.is_cuda and dev.index == torch.cuda.current_device():
+            offs = cu_seqlens.detach()
+            if offs.dtype not in (torch.int32, torch.int64):
+                offs = offs.to(torch.int64)
+            offs = offs.contiguous()
+            self.N, self.NT = N, nt_max
+            tables = torch.empty(2 * nt_max + 3 * N + 3, dtype=torch.int32, device=dev)
+            cmap, self.cu, self.seq_chunk0, self.nt_dev, order = tables.split([2 * nt_max, N + 1, N + 1, 1, N])
+            self.chunk_map = cmap.view(nt_max, 2)
+            self.seq_order = order if N > 1 else None
+            _lib.check(_lib.load().lmoe_seq_tables(
+                offs.data_ptr(), int(offs.dtype == torch.int64), N, nt_max, self.cu.data_ptr(), self.chunk_map.data_ptr(),
+                self.seq_chunk0.data_ptr(), self.nt_dev.data_ptr(), ptr(self.seq_order), stream_ptr()), "chunk tables")
+            return
         cu = cu_seqlens.detach().to(torch.int64)
         nch = (cu[1:] - cu[:-1] + (CHUNK - 1)) // CHUNK                        # chunks per sequence
         c0 = torch.cat([cu.new_zeros(1), torch.cumsum(nch, 0)])                 # [N + 1] first chunk of every sequence

@@ -59,6 +59,7 @@ ENTRY_POINTS = (
     "lmoe_hgrn2_gate_fwd", "lmoe_hgrn2_gate_bwd", "lmoe_quad_featmap_features", "lmoe_quad_featmap_fwd",
     "lmoe_quad_featmap_bwd",
     "lmoe_fused_recurrent_fwd", "lmoe_trace_gdn_state_fwd", "lmoe_trace_simple_gla_fwd", "lmoe_mom_gather", "lmoe_mom_combine", "lmoe_mom_rowdot",
+    "lmoe_mom_combine_bwd", "lmoe_mom_plan_ints", "lmoe_mom_plan", "lmoe_seq_tables",
 )
 
 _lib = None
@@ -145,6 +146,14 @@ def load() -> C.CDLL:
     for fn in (lib.lmoe_mom_combine, lib.lmoe_mom_rowdot):
         fn.argtypes = [C.c_void_p] * 4 + [C.c_int64, C.c_int32, C.c_int32, C.c_int32, C.c_void_p]
         fn.restype = C.c_int
+    lib.lmoe_mom_combine_bwd.argtypes = [C.c_void_p] * 7 + [C.c_int64] * 2 + [C.c_int32] * 3 + [C.c_void_p]
+    lib.lmoe_mom_combine_bwd.restype = C.c_int
+    lib.lmoe_mom_plan_ints.argtypes = [C.c_int32] * 3
+    lib.lmoe_mom_plan_ints.restype = C.c_int64
+    lib.lmoe_mom_plan.argtypes = [C.c_void_p] + [C.c_int32] * 6 + [C.c_void_p] * 8
+    lib.lmoe_mom_plan.restype = C.c_int
+    lib.lmoe_seq_tables.argtypes = [C.c_void_p] + [C.c_int32] * 3 + [C.c_void_p] * 6
+    lib.lmoe_seq_tables.restype = C.c_int
     lib.lmoe_split_floats.argtypes = [C.POINTER(Args), C.c_int32, C.c_int32]
     lib.lmoe_split_floats.restype = C.c_int64
     lib.lmoe_workspace_bytes.argtypes = [C.c_int32] * 9

@@ -433,6 +433,41 @@ int lmoe_mom_rowdot(const void* src, const int32_t* idx, const void* g, void* dw
   return launched(nm);
 }
 
+int lmoe_mom_combine_bwd(const void* y, const int32_t* row_of, const int32_t* src_choice, const void* w, const void* g,
+                         void* dy, void* dw, int64_t ntok, int64_t nrows, int32_t topk, int32_t D, int32_t dtype, void* stream) {
+  const char* nm = "lmoe_mom_combine_bwd";
+  if (int r = check_mom(nm, y, row_of, dy, ntok, D, dtype)) return r;
+  if (!src_choice || !w || !dw) return fail(-1, "%s: null pointer", nm);
+  if (!g || ((uintptr_t)g & 15)) return fail(-1, "%s: g must be a 16-byte aligned pointer", nm);
+  if (topk <= 0) return fail(-4, "%s: topk must be positive", nm);
+  if (nrows < 0) return fail(-4, "%s: negative row count", nm);
+  if (ntok == 0) return 0;
+  lmoe::launch_mom_combine_bwd(dtype, y, row_of, src_choice, w, g, dy, dw, ntok, nrows, topk, D, (hipStream_t)stream);
+  return launched(nm);
+}
+int64_t lmoe_mom_plan_ints(int32_t B, int32_t per_row, int32_t E) { return lmoe::mom_plan_ints(B, per_row, E); }
+int lmoe_mom_plan(const void* sel, int32_t is64, int32_t B, int32_t per_row, int32_t topk, int32_t E, int32_t cap,
+                  int32_t* counts, int32_t* cu, int64_t* max_len, int64_t* mem_offsets, int32_t* src_token,
+                  int32_t* src_choice, int32_t* row_of, void* stream) {
+  const char* nm = "lmoe_mom_plan";
+  if (!sel || !counts || !cu || !max_len || !mem_offsets || !src_token || !src_choice || !row_of)
+    return fail(-1, "%s: null pointer", nm);
+  if (topk <= 0 || per_row % topk) return fail(-4, "%s: topk must be positive and divide the choices of a row", nm);
+  if (lmoe::mom_plan_ints(B, per_row, E) == 0) return fail(-3, "%s: sizes unsupported (lmoe_mom_plan_ints returns 0)", nm);
+  lmoe::launch_mom_plan(sel, is64, B, per_row, topk, E, cap, counts, cu, max_len, mem_offsets, src_token, src_choice, row_of,
+                        (hipStream_t)stream);
+  return launched(nm);
+}
+int lmoe_seq_tables(const void* offsets, int32_t is64, int32_t N, int32_t nt_max, int32_t* cu, int32_t* chunk_map,
+                    int32_t* seq_chunk0, int32_t* nt_dev, int32_t* seq_order, void* stream) {
+  const char* nm = "lmoe_seq_tables";
+  if (!offsets || !cu || !chunk_map || !seq_chunk0 || !nt_dev) return fail(-1, "%s: null pointer", nm);
+  if (N <= 0 || N > lmoe::SEQ_TABLES_MAX) return fail(-3, "%s: N = %d outside 1..%d", nm, N, lmoe::SEQ_TABLES_MAX);
+  if (nt_max < 0) return fail(-4, "%s: negative chunk count", nm);
+  lmoe::launch_seq_tables(offsets, is64, N, nt_max, cu, chunk_map, seq_chunk0, nt_dev, seq_order, (hipStream_t)stream);
+  return launched(nm);
+}
+
 static int check_gates(const char* nm, int64_t rows, int32_t H, int32_t dtype) {
   if (dtype != LMOE_BF16 && dtype != LMOE_F32) return fail(-2, "%s: dtype must be LMOE_BF16 or LMOE_F32", nm);
   if (H <= 0 || H > 256) return fail(-3, "%s: H = %d outside 1..256", nm, H);

@@ -104,6 +104,18 @@ void launch_mom_combine(int dtype, const void* src, const int32_t* idx, const vo
                         int D, hipStream_t st);
 void launch_mom_rowdot(int dtype, const void* src, const int32_t* idx, const void* g, void* dw, int64_t ntok, int topk,
                        int D, hipStream_t st);
+// the backward of combine: dy = w * g per packed row, dw = <g, y> per choice
+void launch_mom_combine_bwd(int dtype, const void* y, const int32_t* row_of, const int32_t* src_choice, const void* w,
+                            const void* g, void* dy, void* dw, int64_t ntok, int64_t nrows, int topk, int D, hipStream_t st);
+// chunk tables of packed input from offsets on the device (N <= SEQ_TABLES_MAX; seq_order may be null)
+constexpr int SEQ_TABLES_MAX = 4096;
+void launch_seq_tables(const void* offs, int is64, int N, int nt_max, int32_t* cu, int32_t* chunk_map, int32_t* seq_chunk0,
+                       int32_t* nt_dev, int32_t* seq_order, hipStream_t st);
+// routing tables; mom_plan_ints: int32 numbers of `counts`, 0 where launch_mom_plan does not take the sizes
+int64_t mom_plan_ints(int64_t B, int64_t per_row, int64_t E);
+void launch_mom_plan(const void* sel, int is64, int B, int per_row, int topk, int E, int cap, int32_t* counts, int32_t* cu,
+                     int64_t* max_len, int64_t* mem_offsets, int32_t* src_token, int32_t* src_choice, int32_t* row_of,
+                     hipStream_t st);
 // token-by-token forward (decoding); delta = the (gated) delta rule
 void launch_recurrent(const lmoe_args& a, bool delta, hipStream_t st);
 void launch_selftest(int dtype, int kd, const void* A, const void* B, float* C, float* G, hipStream_t st);

@@ -57,8 +57,9 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
     """Index tables for ``selected_memories`` [B, S, topk] (as ``torch.topk`` returns them,
     mom_linear_attention.py:288).  ``capacity``: the reference's capacity factor; ``None`` keeps every token.
 
-    Built by device operations only (stable sort by (memory, batch row), counts, prefix sums, scatters), as the
-    reference builds its tables on the device (mom_linear_attention.py:28-66).  Without a capacity nothing is read
+    Built on the device (a stable counting sort by (memory, batch row) in three launches; what its kernels do not take
+    -- more than 1024 memories, or more than 8192 counts of a memory in 2048 choices of a batch row --
+    by tensor operations), as the reference builds its tables (mom_linear_attention.py:28-66).  Without a capacity nothing is read
     back to the host: every routed token is kept, ``T_total = B * S * topk`` is known up front, and pack -> op ->
     combine can run inside a HIP graph capture with the plan in it.  With a capacity the number of surviving rows is
     the one device-to-host read of the call.  ``check`` validates the memory indices (two more reads)."""
@@ -66,10 +67,44 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
         raise ValueError("selected_memories must be [B, S, topk]")
     B, S, topk = selected_memories.shape
     dev = selected_memories.device
-    sel = selected_memories.reshape(-1).to(torch.int64)                        # flat (b, t, k)
+    sel = selected_memories.reshape(-1)                                        # flat (b, t, k)
     if check and sel.numel() and (int(sel.min()) < 0 or int(sel.max()) >= num_memories):
         raise ValueError("selected_memories out of range")
     n = sel.numel()
+    if sel.is_cuda and sel.device.index == torch.cuda.current_device() and n < 2 ** 31:
+        plan = _plan_native(sel, B, S, topk, num_memories, capacity)
+        if plan is not None:
+            return plan
+    return _plan_by_sorting(sel.to(torch.int64), B, S, topk, num_memories, capacity)
+
+
+def _plan_native(sel, B, S, topk, num_memories, capacity):
+    """The plan from the library's kernels, or None for sizes they do not take."""
+    lib = _lib.load()
+    n, dev = sel.numel(), sel.device
+    ints = lib.lmoe_mom_plan_ints(B, S * topk, num_memories)
+    if ints == 0:
+        return None
+    if sel.dtype not in (torch.int32, torch.int64):
+        sel = sel.to(torch.int64)
+    seqs = num_memories * B
+    wide = torch.empty(num_memories + 2, dtype=torch.int64, device=dev)
+    counts, cu, src_token, src_choice, row_of = (torch.empty(k, dtype=torch.int32, device=dev)
+                                                 for k in (ints, seqs + 1, n, n, n))
+    cap = -1 if capacity is None else max(0, min(math.ceil(S * capacity), 2 ** 31 - 1))
+    _lib.check(lib.lmoe_mom_plan(sel.data_ptr(), int(sel.dtype == torch.int64), B, S * topk, topk, num_memories, cap,
+                                 counts.data_ptr(), cu.data_ptr(), wide.data_ptr(), wide.data_ptr() + 8,
+                                 src_token.data_ptr(), src_choice.data_ptr(), row_of.data_ptr(), stream_ptr()), "mom_plan")
+    T_total = n
+    if capacity is not None:
+        T_total = int(cu[-1])                                                  # (the one read: how many survive)
+        src_token, src_choice = src_token[:T_total], src_choice[:T_total]
+    return MomPlan(B, S, topk, num_memories, T_total, src_token, src_choice, row_of.view(B * S, topk), cu, wide[0],
+                   wide[1:])
+
+
+def _plan_by_sorting(sel, B, S, topk, num_memories, capacity):
+    dev, n = sel.device, sel.numel()
     flat = torch.arange(n, device=dev)
     b_of = flat // (S * topk)
     key = sel * B + b_of                                                       # memory-major sequences
@@ -158,13 +193,10 @@ class _Combine(torch.autograd.Function):
         D = y2.shape[1]
         g = dout.reshape(plan.B * plan.S, D).contiguous()
         # dy[row] = w[choice(row)] * dout[token(row)];  dw[t][k] = <dout[t], y[row_of[t][k]]>
-        scale = w2.reshape(-1)[plan.src_choice.long()].contiguous()
-        dy = torch.empty_like(y2)
-        _lib.check(lib.lmoe_mom_gather(g.data_ptr(), plan.src_token.data_ptr(), scale.data_ptr(), dy.data_ptr(),
-                                       plan.T_total, D, _dt(y2), stream_ptr()), "mom_combine backward")
-        dw = torch.empty_like(w2)
-        _lib.check(lib.lmoe_mom_rowdot(y2.data_ptr(), plan.row_of.data_ptr(), g.data_ptr(), dw.data_ptr(),
-                                       plan.B * plan.S, plan.topk, D, _dt(y2), stream_ptr()), "mom_combine backward")
+        dy, dw = torch.empty_like(y2), torch.empty_like(w2)
+        _lib.check(lib.lmoe_mom_combine_bwd(y2.data_ptr(), plan.row_of.data_ptr(), plan.src_choice.data_ptr(),
+                                            w2.data_ptr(), g.data_ptr(), dy.data_ptr(), dw.data_ptr(), plan.B * plan.S,
+                                            plan.T_total, plan.topk, D, _dt(y2), stream_ptr()), "mom_combine backward")
         return dy.view(ctx.yshape), dw.view(ctx.wshape).to(ctx.wdtype), None
 
 
