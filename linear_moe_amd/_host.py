@@ -115,6 +115,8 @@ def no_tokens(q, k, v, head_first: bool, cu_seqlens, initial_state, output_final
     """The call without any token (T = 0, or a batch of zero rows): nothing to launch.  Returns None when there
     are tokens, else ``(o, final_state)``: an empty o and the initial state handed through (so that its gradient
     is the gradient of the final state), zeros without one."""
+    if q.numel() and v.numel():
+        return None                                    # (the op checks its arguments)
     B, T, H, K, V = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v)
     if B * T > 0:
         return None
@@ -132,18 +134,15 @@ def _desc(x: Optional[torch.Tensor], head_first: bool) -> Tensor4:
     """Stride descriptor of a [B,H,T,(D)] or [B,T,H,(D)] tensor."""
     if x is None:
         return Tensor4(None, 0, 0, 0)
-    if head_first:
-        sb, sh, st = x.stride(0), x.stride(1), x.stride(2)
-    else:
-        sb, st, sh = x.stride(0), x.stride(1), x.stride(2)
-    return Tensor4(x.data_ptr(), sb, st, sh)
+    s = x.stride()
+    return Tensor4(x.data_ptr(), s[0], s[2], s[1]) if head_first else Tensor4(x.data_ptr(), s[0], s[1], s[2])
 
 
 def _aligned(x: torch.Tensor) -> torch.Tensor:
     """Return x (or a contiguous copy) such that rows are 16-byte aligned and last dim contiguous."""
     if x.dim() == 4:
-        vec = 16 // x.element_size()
-        ok = x.stride(3) == 1 and x.data_ptr() % 16 == 0 and all(x.stride(i) % vec == 0 for i in range(3))
+        s = x.stride()
+        ok = s[3] == 1 and x.data_ptr() % 16 == 0 and (s[0] | s[1] | s[2]) % (16 // x.element_size()) == 0
         return x if ok else x.contiguous()
     return x
 
@@ -289,7 +288,8 @@ def _state_check(x: Optional[torch.Tensor], N, H, K, V, name: str) -> Optional[t
 
 def base_args(q, k, v, head_first: bool, scale: Optional[float], plan: SeqPlan, dims) -> Args:
     B, T, H, K, V = dims
-    if not (q.device == k.device == v.device) or q.device.index != torch.cuda.current_device():
+    dev = q.device
+    if not (dev == k.device == v.device) or dev.index != torch._C._cuda_getDevice():
         # (the kernels go to the current stream of the current device: one process per GPU, as the launchers run it)
         raise RuntimeError(f"q, k, v must live on the current device cuda:{torch.cuda.current_device()}, got "
                            f"{q.device}, {k.device}, {v.device}")
@@ -330,8 +330,10 @@ def unstash(ctx, call):
     return t[ctx.n_stashed:]
 
 
-def stream_ptr() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+def stream_ptr() -> int:
+    """The current stream of the current device, as the library takes it.  (The raw handle: building the stream object
+    of ``torch.cuda.current_stream()`` for it takes longer than all the other arguments of a small call.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def ptr(x: Optional[torch.Tensor]):

@@ -55,8 +55,10 @@ class _GdnGates(torch.autograd.Function):
         dgc = (torch.zeros_like(ac, dtype=torch.float32) if dg is None else dg.float().contiguous())
         dbc = (torch.zeros_like(bc) if dbeta is None else dbeta.to(bc.dtype).contiguous())
         da, db = torch.empty_like(ac), torch.empty_like(bc)
-        dpar = torch.zeros(2, H, dtype=torch.float32, device=ac.device)
-        if rows:
+        if rows == 0:
+            dpar = torch.zeros(2, H, dtype=torch.float32, device=ac.device)
+        else:
+            dpar = torch.empty(2, H, dtype=torch.float32, device=ac.device)
             part = torch.empty(lib.lmoe_gdn_gates_partials(rows, H), 2, H, dtype=torch.float32, device=ac.device)
             _lib.check(lib.lmoe_gdn_gates_bwd(ac.data_ptr(), bc.data_ptr(), Af.data_ptr(), Bf.data_ptr(), dgc.data_ptr(),
                                               dbc.data_ptr(), da.data_ptr(), db.data_ptr(), part.data_ptr(),
