@@ -18,15 +18,15 @@ enum Stage {
   ST_GLA_INTRA_FWD = 7 // chunk_gla: intra-chunk attention matrix        (chunk-parallel)
 };
 
-// F<T, K, V>::run(a, st) for the runtime (dtype, K, V) of the problem
-template <template <typename, int, int> class F>
-inline void dispatch(const lmoe_args& a, hipStream_t st) {
+// F<T, K, V>::run(a, more ..., st) for the runtime (dtype, K, V) of the problem
+template <template <typename, int, int> class F, typename... More>
+inline void dispatch(const lmoe_args& a, hipStream_t st, const More&... more) {
   typedef __bf16 bf16_t;
 #define LMOE_KV(T)                                                   \
-  if (a.K == 64 && a.V == 64) F<T, 64, 64>::run(a, st);              \
-  else if (a.K == 64 && a.V == 128) F<T, 64, 128>::run(a, st);       \
-  else if (a.K == 128 && a.V == 64) F<T, 128, 64>::run(a, st);       \
-  else F<T, 128, 128>::run(a, st);
+  if (a.K == 64 && a.V == 64) F<T, 64, 64>::run(a, more..., st);              \
+  else if (a.K == 64 && a.V == 128) F<T, 64, 128>::run(a, more..., st);       \
+  else if (a.K == 128 && a.V == 64) F<T, 128, 64>::run(a, more..., st);       \
+  else F<T, 128, 128>::run(a, more..., st);
   if (a.dtype == LMOE_BF16) { LMOE_KV(bf16_t) } else { LMOE_KV(float) }
 #undef LMOE_KV
 }
@@ -46,6 +46,10 @@ inline void dispatch_gdn(const lmoe_args& a, hipStream_t st) {
 }
 
 void launch_state_fwd(const lmoe_args& a, hipStream_t st);        // chunk_simple_gla
+// what the segments of a call cut along T add to the state (chunk_simple_gla), and how it is cut
+struct Split;
+Split launch_scalar_seg(const lmoe_args& a, bool bwd, hipStream_t st);
+int64_t scalar_split_floats(const lmoe_args& a);                  // fp32 numbers of lmoe_args.seg_ws, as split_floats
 // traced forward pass of chunk_simple_gla (bf16, K = V = 128, forward-only): false when the problem is not of that shape
 bool launch_state_fwd_trace(const lmoe_args& a, long long* tr, int work_group, hipStream_t st);
 void launch_gdn_state_fwd(const lmoe_args& a, hipStream_t st);    // gated delta rule

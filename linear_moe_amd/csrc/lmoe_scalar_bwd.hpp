@@ -116,7 +116,7 @@ __global__ __launch_bounds__(NTHR) void k_bwd_dv(const lmoe_args a) {
 // V slice (the other slices carry zeros).
 constexpr int NORM_SLOT_COLS = 32;
 template <typename T, int K, int V, int BV, int NORM = 0>
-__global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a) {
+__global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
   static_assert(!NORM || sizeof(T) == 2, "the normalised pass exists for 2-byte elements");
@@ -133,9 +133,12 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a) {
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = vsl * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
+  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  const int v0 = vsl * BV, h = pair % a.H;
+  const PassItem item = CUT ? pass_item(a, sp, pair / a.H) : pass_item(a, Split{}, pair / a.H);
+  const int n = item.n;
+  const SeqInfo sq = item.sq;
   const int l = lane_id();
   const int team = threadIdx.x / NTHR;      // 0: consumers, 1: loaders
   const bool producer = team == 1;
@@ -288,6 +291,16 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a) {
   f32x4 dz[NORM ? MB : 1];                  // NORM: gradient of the column of ones (the same sum in every column)
 #pragma unroll
   for (int mi = 0; mi < (NORM ? MB : 1); ++mi) dz[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (CUT && !item.last) {
+    const int nch = (a.T + CH - 1) / CH, nfs = seg_count(nch, sp.len1);
+    const int nf = nfs - (sq.chunk0 - n * nch + sp.len3) / sp.len1;        // fine segments behind
+    const int64_t o = (int64_t)((n + 1) * nfs - 1) * a.H + h;              // the last one
+    seg_prefix<K, V>(dS, sp.Q + (o * V + v0 + acc_col(0)) * K + krow0 + acc_row(0, 0), sp.D + o, a.H, nf, -1);
+    // (dz is carried as partial sums of the V slices: the first one takes what the segments behind add)
+    if constexpr (NORM != 0) {
+      if (vsl == 0) seg_prefix_z<K>(dz, sp.Z + o * K + krow0 + acc_row(0, 0), a.H, nf, -1);
+    }
+  }
   lds_barrier();                                     // P0
   for (int it = 0; it < sq.nchunks; ++it) {
     const int c = sq.nchunks - 1 - it;
@@ -345,7 +358,7 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a) {
       lds_barrier();                                                                     // B4
     }
   }
-  if (a.dh0) {
+  if (a.dh0 && item.first) {
     float* p = a.dh0 + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)

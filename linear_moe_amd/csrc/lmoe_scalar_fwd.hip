@@ -1,6 +1,6 @@
 // Instantiation and launch of the forward kernel of chunk_simple_gla, plus the toolkit self-test.
 #include "lmoe_launch.hpp"
-#include "lmoe_scalar_fwd.hpp"
+#include "lmoe_scalar_split.hpp"
 
 namespace lmoe {
 
@@ -9,16 +9,61 @@ template <typename T, int V> struct FwdTiles {
   static constexpr int BVS = sizeof(T) == 4 ? 16 : 32;
 };
 
+// How the sequences of a call are cut along T: not at all without a workspace for it.
+inline Split scalar_split(const lmoe_args& a) {
+  Split sp = {};
+  if (!a.seg_ws) return sp;
+  sp = plan_split_scalar(a);
+  if (!sp.len1) return sp;
+  const int64_t n1 = (int64_t)sp.n1 * a.H;
+  sp.Q = a.seg_ws;
+  sp.Z = sp.Q + n1 * a.K * a.V;
+  sp.D = sp.Z + n1 * a.K;
+  return sp;
+}
+int64_t scalar_split_floats(const lmoe_args& a) {
+  const Split sp = plan_split_scalar(a);
+  return (int64_t)sp.n1 * a.H * (a.K * a.V + a.K + 1);
+}
+// what the fine segments add (forward: but for those of the last coarse segment; backward: of the first)
+template <bool BWD> struct ScalarSeg {
+  template <typename T, int K, int V> struct F {
+    template <int NORM> static void go(const lmoe_args& a, const Split& sp, hipStream_t st) {
+      constexpr int BV = sizeof(T) == 4 ? 32 : V;
+      const int n = sp.n1 / a.N, f = sp.len3 / sp.len1, r = sp.n3 / a.N;
+      const int seg0 = BWD ? f : 0, nsegs = BWD ? n - f : (r - 1) * f;
+      hipLaunchKernelGGL((k_scalar_seg_state<T, K, V, BV, BWD, NORM>), dim3(a.N * nsegs * a.H * (V / BV)), dim3(NTHR), 0, st,
+                         a, sp, seg0, nsegs);
+    }
+    static void run(const lmoe_args& a, const Split& sp, hipStream_t st) {
+      if constexpr (sizeof(T) == 2) {
+        if (a.normalize && !BWD) return go<1>(a, sp, st);
+        if (a.normalize == 1) return go<1>(a, sp, st);
+        if (a.normalize == 2) return go<2>(a, sp, st);
+      }
+      go<0>(a, sp, st);
+    }
+  };
+};
+Split launch_scalar_seg(const lmoe_args& a, bool bwd, hipStream_t st) {
+  const Split sp = scalar_split(a);
+  if (sp.len1) {
+    if (bwd) dispatch<ScalarSeg<true>::F>(a, st, sp);
+    else dispatch<ScalarSeg<false>::F>(a, st, sp);
+  }
+  return sp;
+}
+
 // the pass for 2-byte elements on V slices of BV columns: saving or forward-only, plain or with the normalised output
-template <typename T, int K, int V, int BV> void launch_fwd_b(const lmoe_args& a, hipStream_t st) {
-  const dim3 grid(((a.N * a.H + 7) / 8) * 8 * (V / BV)), block(3 * NTHR);
+template <typename T, int K, int V, int BV> void launch_fwd_b(const lmoe_args& a, const Split& sp, hipStream_t st) {
+  const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BV)), block(3 * NTHR);
   long long* const no_trace = nullptr;
   if (a.normalize) {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, true>), grid, block, 0, st, a, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, true>), grid, block, 0, st, a, no_trace, -1);
+    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, true>), grid, block, 0, st, a, sp, no_trace, -1);
+    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, true>), grid, block, 0, st, a, sp, no_trace, -1);
   } else {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true>), grid, block, 0, st, a, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false>), grid, block, 0, st, a, no_trace, -1);
+    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true>), grid, block, 0, st, a, sp, no_trace, -1);
+    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false>), grid, block, 0, st, a, sp, no_trace, -1);
   }
 }
 template <typename T, int K, int V> struct StateFwd {
@@ -30,15 +75,16 @@ template <typename T, int K, int V> struct StateFwd {
       // depend on the width (a state element and an output element are the same sums in either split)
       if constexpr (V >= 64) {
         if ((int64_t)a.N * a.H * (V / 64) >= cu_count()) {
-          launch_fwd_b<T, K, V, 64>(a, st);
+          launch_fwd_b<T, K, V, 64>(a, Split{}, st);
           return;
         }
       }
-      launch_fwd_b<T, K, V, BV>(a, st);
+      launch_fwd_b<T, K, V, BV>(a, launch_scalar_seg(a, false, st), st);
     } else {
-      const int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
-      if (a.hs) hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, true>), dim3(grid), dim3(3 * NTHR), 0, st, a);
-      else hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, false>), dim3(grid), dim3(3 * NTHR), 0, st, a);
+      const Split sp = launch_scalar_seg(a, false, st);
+      const int grid = ((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BV);
+      if (a.hs) hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+      else hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
     }
   }
 };
@@ -49,7 +95,7 @@ bool launch_state_fwd_trace(const lmoe_args& a, long long* tr, int work_group, h
   constexpr int BV = FwdTiles<bf16, 128>::BVS;
   const int grid = ((a.N * a.H + 7) / 8) * 8 * (128 / BV);
   if (work_group < 0 || work_group >= grid) return false;
-  hipLaunchKernelGGL((k_state_fwd_b<bf16, 128, 128, BV, false, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, tr, work_group);
+  hipLaunchKernelGGL((k_state_fwd_b<bf16, 128, 128, BV, false, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, Split{}, tr, work_group);
   return true;
 }
 // C = A B^T (64 x 64, contraction along the tile columns) and G = A^T B (KD x KD, contraction

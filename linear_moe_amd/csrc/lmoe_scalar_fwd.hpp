@@ -3,7 +3,7 @@
 //   o = scale [ e^{b_i} q_i S + ((q k^T) . Gamma) v ],   S' = e^{b_C} S + (k . e^{b_C - b})^T v,
 //   Gamma_ij = e^{b_i - b_j} [i >= j].
 #pragma once
-#include "lmoe_seq.hpp"
+#include "lmoe_split.hpp"
 
 namespace lmoe {
 
@@ -36,7 +36,7 @@ template <typename T> __device__ __forceinline__ void scale_frag(typename ET<T>:
 //   All teams meet at the same barriers; three waves per SIMD hide each other's latencies.
 // ------------------------------------------------------------------------- //
 template <typename T, int K, int V, int BV, bool SAVE>
-__global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a) {
+__global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a, const Split sp) {
   static_assert(sizeof(T) == 4, "fp32 elements; 2-byte elements: k_state_fwd_b");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
@@ -52,9 +52,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a) {
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = vsl * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
+  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  const int v0 = vsl * BV, h = pair % a.H;
+  const PassItem item = CUT ? pass_item(a, sp, pair / a.H) : pass_item(a, Split{}, pair / a.H);
+  const int n = item.n;
+  const SeqInfo sq = item.sq;
   const int l = lane_id();
   const int team = threadIdx.x / NTHR;
   if (sq.nchunks == 0) {
@@ -196,6 +199,11 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a) {
         for (int i = 0; i < 4; ++i)
           S[mi][ni][i] = h0[(int64_t)(krow0 + acc_row(mi, i)) * V + v0 + acc_col(ni)];
   }
+  if (CUT && !item.first) {
+    const int nf = (sq.chunk0 - n * ((a.T + CH - 1) / CH)) / sp.len1;      // fine segments in front
+    const int64_t o = (int64_t)n * seg_count((a.T + CH - 1) / CH, sp.len1) * a.H + h;
+    seg_prefix<K, V>(S, sp.Q + (o * V + v0 + acc_col(0)) * K + krow0 + acc_row(0, 0), sp.D + o, a.H, nf, 1);
+  }
   for (int c = 0; c < sq.nchunks; ++c) {
     constexpr int cur = 0;
     // S (state at chunk start) -> LDS as S^T
@@ -237,7 +245,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a) {
     lds_barrier();                                                                       // B2
     lds_barrier();                                                                       // B3
   }
-  if (a.ht) {
+  if (a.ht && item.last) {
     float* ht = a.ht + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)
@@ -280,7 +288,7 @@ constexpr int SFWD_TRACE_CHUNKS = 24, SFWD_TRACE_MARKS = 8, SFWD_TRACE_SLOTS = 3
 // keys of the chunks before, fp32 in LDS and, for the backward, in zs) and formed by every V slice for itself:
 // consumers z += k^T 1, output team q z and the row sums of P as two more products against a fragment of ones.
 template <typename T, int K, int V, int BV, bool SAVE, bool TRACE = false, bool NORM = false>
-__global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, long long* tr, int traced_wg) {
+__global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   static_assert(sizeof(T) == 2, "2-byte elements");
   static_assert(!(NORM && TRACE), "the traced instance is the plain pass");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
@@ -320,9 +328,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, lon
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = vsl * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
+  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  const int v0 = vsl * BV, h = pair % a.H;
+  const PassItem item = CUT ? pass_item(a, sp, pair / a.H) : pass_item(a, Split{}, pair / a.H);
+  const int n = item.n;
+  const SeqInfo sq = item.sq;
   const int l = lane_id();
   // (wave-uniform by construction; said to the compiler, so that the branches on it are scalar branches: a matrix
   // instruction runs whatever the lane mask, and a short masked region is not jumped over)
@@ -629,6 +640,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, lon
   f32x4 Sz[NORM ? MB : 1];                  // NORM: the column of ones (every column of the tile holds the same sum)
 #pragma unroll
   for (int mi = 0; mi < (NORM ? MB : 1); ++mi) Sz[mi] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (CUT && !item.first) {
+    const int nf = (sq.chunk0 - n * ((a.T + CH - 1) / CH)) / sp.len1;      // fine segments in front
+    const int64_t o = (int64_t)n * seg_count((a.T + CH - 1) / CH, sp.len1) * a.H + h;
+    seg_prefix<K, V>(S, sp.Q + (o * V + v0 + acc_col(0)) * K + krow0 + acc_row(0, 0), sp.D + o, a.H, nf, 1);
+    if constexpr (NORM) seg_prefix_z<K>(Sz, sp.Z + o * K + krow0 + acc_row(0, 0), a.H, nf, 1);
+  }
   auto copy_state = [&](int c) {            // S at the start of chunk c -> LDS as S^T
     const int buf = c & 1;
 #pragma unroll
@@ -709,7 +726,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, lon
     if (wv == 0) TR(0, c, 3);
   }
   if (wv == 0) trace_out(0);
-  if (a.ht) {
+  if (a.ht && item.last) {
     float* ht = a.ht + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)

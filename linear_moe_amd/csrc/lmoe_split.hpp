@@ -23,6 +23,7 @@ struct Split {
   float *D, *DT;         // [n1][H]        decays of the fine segments (beside P, PT)
   float* Q;              // [n1][H][K][V]  their contributions
   float* S;              // [n3][H][K][V]  state (gradient) a coarse segment starts from
+  float* Z;              // [n1][H][K]     contributions to the normaliser's column (chunk_simple_gla)
 };
 
 // Sequences of fewer chunks gain nothing (three kernels in place of one).  Longer ones than 32 768 tokens are left whole
@@ -44,9 +45,10 @@ struct SegInfo {
 __device__ __forceinline__ SegInfo seg_find(const lmoe_args& a, int len, int s) {
   SegInfo r;
   if (!a.cu_seqlens) {
-    r.nseg = seg_count((a.T + CH - 1) / CH, len);
-    r.n = s / r.nseg;
-    r.j = s % r.nseg;
+    // (uniform, said to the compiler: what derives from it stays in scalar registers)
+    r.nseg = __builtin_amdgcn_readfirstlane(seg_count((a.T + CH - 1) / CH, len));
+    r.n = __builtin_amdgcn_readfirstlane(s / r.nseg);
+    r.j = s - r.n * r.nseg;
     if (r.n >= a.N) r.n = -1;
     return r;
   }
@@ -113,7 +115,13 @@ __device__ __forceinline__ PassItem pass_item(const lmoe_args& a, const Split& s
   p.n = g.n;
   p.first = g.j == 0;
   p.last = g.j == g.nseg - 1;
-  if (g.n >= 0) p.sq = seg_cut(seq_info(a, g.n), g.j, sp.len3);
+  if (g.n >= 0) {
+    p.sq = seg_cut(seq_info(a, g.n), g.j, sp.len3);
+    p.sq.tok0 = __builtin_amdgcn_readfirstlane(p.sq.tok0);
+    p.sq.len = __builtin_amdgcn_readfirstlane(p.sq.len);
+    p.sq.chunk0 = __builtin_amdgcn_readfirstlane(p.sq.chunk0);
+    p.sq.nchunks = __builtin_amdgcn_readfirstlane(p.sq.nchunks);
+  }
   return p;
 }
 // How a call is cut (pointers left open), or len1 = 0.  `slices` = work-groups of the ordinary pass per (sequence, head),
@@ -148,6 +156,74 @@ inline Split plan_split(const lmoe_args& a, int slices) {
   s.n3 = packed ? a.NT / s.len3 + a.N : a.N * seg_count(nch, s.len3);
   return s;
 }
-inline int pass_items(const lmoe_args& a, const Split& sp) { return sp.len3 ? sp.n3 : a.N; }
+// The same for chunk_simple_gla, whose transitions are numbers: step 2 is a few loads at the start of the pass
+// (seg_prefix), and a cut pays from a handful of chunks on.  Dense input only (the places of packed sequences are not
+// known here).  Measured, us per chunk of the ordinary pass (V slices of 32, 4-byte elements 16): K = V = 64 0.88,
+// 128 1.3; 4-byte elements 3.9, 6.0 (whatever the number of work-groups, up to one per CU).  us per call, not cut -> cut:
+// forward K = V = 128, T = 4096, 16 pairs 82 -> 52, 4 pairs 80 -> 34; K = V = 64, T = 8192, 8 pairs 113 -> 32; 4-byte
+// elements K = V = 64, 4 pairs, T = 512 33.8 -> 13.6 (kernels alone), T = 2048 124 -> 28; with the normaliser, forward +
+// backward, K = V = 128, T = 8192, 8 pairs 383 -> 172.  64 pairs at K = V = 128 fill the CUs: never cut.
+inline Split plan_split_scalar(const lmoe_args& a) {
+  Split s = {};
+  if (a.N < 1 || a.T < 1 || a.cu_seqlens) return s;
+  const bool f4 = a.dtype != LMOE_BF16;
+  const int cus = cu_count(), nch = (a.T + CH - 1) / CH, pairs = a.N * a.H;
+  if (!f4 && (int64_t)pairs * (a.V / 64) >= cus) return s;        // the pass takes wide slices there and fills the CUs
+  // (2-byte elements: short and very long sequences give the same bits alone and in a batch that fills the CUs)
+  if (nch < (f4 ? 3 : 8) || nch > SPLIT_MAX_CHUNKS) return s;
+  const float w = (a.K + a.V) / 256.f;
+  const float c3 = f4 ? 1.9f + 4.1f * w : 0.45f + 0.85f * w, c1 = f4 ? 1.f + 2.f * w : 0.3f + 0.6f * w;
+  const int64_t wg3 = (int64_t)pairs * (a.V / (f4 ? 16 : 32)), wg1 = (int64_t)pairs * (f4 ? a.V / 32 : 1);
+  auto rounds = [](int64_t n, int64_t per) { return (float)((n + per - 1) / per); };
+  float best = 0.9f * rounds(wg3, cus) * nch * c3;
+  for (int r = 2; r <= 32 && r <= nch; ++r) {
+    const int len3 = seg_count(nch, r);
+    if (seg_count(nch, len3) != r) continue;
+    for (int f = 1; f <= 4; ++f) {
+      if (len3 % f) continue;
+      const int len1 = len3 / f, nf = seg_count(nch, len1);
+      // step 1 two work-groups to a CU; a fine segment at the start of the pass 0.15
+      const float t = 8.f + c1 * len1 * rounds(wg1 * (r - 1) * f, 2 * cus) + 0.15f * (r - 1) * f + c3 * len3 * rounds(wg3 * r, cus);
+      if (t < best) { best = t; s.len1 = len1; s.len3 = len3; s.n1 = a.N * nf; s.n3 = a.N * r; }
+    }
+  }
+  return s;
+}
+// S <- D S + Q over the n fine segments in front of a coarse one, in order (step = -1: behind it, from the last on).
+// q, d: Q (its column v0 + lane % 16, row krow0 + 4 (lane / 16)) and D of the first; four segments' loads at a time.
+template <int K, int V, int MB, int NB>
+__device__ __forceinline__ void seg_prefix(f32x4 (&S)[MB][NB], const float* q, const float* d, int H, int n, int step) {
+  const int64_t qs = (int64_t)step * H * V * K, ds = (int64_t)step * H;
+  for (int i0 = 0; i0 < n; i0 += 4) {
+    f32x4 x[4][MB][NB];
+    float dec[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = min(i0 + u, n - 1);
+      dec[u] = d[i * ds];
+#pragma unroll
+      for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+        for (int ni = 0; ni < NB; ++ni) x[u][mi][ni] = *(const f32x4*)(q + i * qs + 16 * ni * K + 16 * mi);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + u < n) {
+#pragma unroll
+        for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+          for (int ni = 0; ni < NB; ++ni) S[mi][ni] = S[mi][ni] * dec[u] + x[u][mi][ni];
+      }
+    }
+  }
+}
+// the same for the column of the normaliser (no decay: ungated calls)
+template <int K, int MB> __device__ __forceinline__ void seg_prefix_z(f32x4 (&z)[MB], const float* p, int H, int n, int step) {
+  const int64_t zs = (int64_t)step * H * K;
+  for (int i = 0; i < n; ++i)
+#pragma unroll
+    for (int mi = 0; mi < MB; ++mi) z[mi] += *(const f32x4*)(p + i * zs + 16 * mi);
+}
+__host__ __device__ inline int pass_items(const lmoe_args& a, const Split& sp) { return sp.len3 ? sp.n3 : a.N; }
 
 }  // namespace lmoe

@@ -1,4 +1,4 @@
-"""Sequences cut along T for the sequential passes (few (sequence, head) pairs, bfloat16): outputs, final state and all
+"""Sequences cut along T for the sequential passes (few (sequence, head) pairs): outputs, final state and all
 gradients against the token recurrence in float64, at the edges of the cut -- a last segment of one token, of whole
 chunks, of a partial chunk; states in and out; packed sequences of very unequal length, some empty, some of one
 segment."""
@@ -12,18 +12,18 @@ from tests.util import TOL, gen, max_abs_rel, oracle_grads
 pytestmark = pytest.mark.gpu
 
 
-def is_cut(op, B, T, H, K, V, N=None):
+def is_cut(op, B, T, H, K, V, N=None, dtype=torch.bfloat16):
     """Whether the library cuts a call of these sizes (NT as the host layer counts it for offsets on the device)."""
     import ctypes as C
     from linear_moe_amd import _lib
     a = _lib.Args()
-    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N = _lib.LMOE_BF16, B, T, H, K, V, N or B
+    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N = _lib.LMOE_BF16 if dtype == torch.bfloat16 else _lib.LMOE_F32, B, T, H, K, V, N or B
     a.NT = B * ((T + 63) // 64) + (N if N else 0)
     a.cu_seqlens = 16 if N else None               # (only asked whether it is there)
     return _lib.load().lmoe_split_floats(C.byref(a), op, 1) > 0
 
 
-def check(fn_ref, fn, ins, do, dht, cuda):
+def check(fn_ref, fn, ins, do, dht, cuda, dtype=torch.bfloat16):
     ref_o, ref_ht, ref = oracle_grads(fn_ref, ins, do, dht)
     dev = {n: x.to(cuda).requires_grad_(True) for n, x in ins.items()}
     o, ht = fn(**dev)
@@ -31,7 +31,7 @@ def check(fn_ref, fn, ins, do, dht, cuda):
     with torch.no_grad():                          # the forward-only instance
         of, hf = fn(**dev)
     torch.cuda.synchronize()
-    tol = TOL[torch.bfloat16]
+    tol = TOL[dtype]
     for x in (o, of):
         assert max_abs_rel(x.detach().cpu(), ref_o) < tol
     for x in (ht, hf):
@@ -63,3 +63,47 @@ def test_gated_delta_rule_cut_along_t(cuda, B, T, H, K, V, lens):
     check(lambda q, k, v, g, beta, h0: naive.naive_recurrent_gated_delta_rule(q, k, v, g, beta, None, h0, True, cu, False),
           lambda q, k, v, g, beta, h0: chunk_gated_delta_rule(q, k, v, g, beta, None, h0, True, cud, False),
           ins, do, dht, cuda)
+
+
+@pytest.mark.parametrize("dtype,B,T,H,K,V", [
+    (torch.bfloat16, 1, 1281, 2, 128, 128),        # last chunk, and last segment, of one token
+    (torch.bfloat16, 2, 1536, 1, 64, 64),          # whole chunks
+    (torch.bfloat16, 1, 1500, 3, 64, 128),
+    (torch.bfloat16, 2, 3000, 2, 128, 64),
+    (torch.float32, 1, 321, 2, 64, 64),
+    (torch.float32, 1, 512, 4, 64, 64),
+    (torch.float32, 2, 1000, 1, 128, 128),
+    (torch.float32, 1, 700, 3, 128, 64),
+])
+@pytest.mark.parametrize("gated", [True, False])
+def test_simple_gla_cut_along_t(cuda, dtype, B, T, H, K, V, gated):
+    from linear_moe_amd import chunk_simple_gla
+    assert is_cut(0, B, T, H, K, V, dtype=dtype)
+    ins = dict(q=gen(7100, B, T, H, K).to(dtype), k=(gen(7101, B, T, H, K) * K ** -0.5).to(dtype),
+               v=gen(7102, B, T, H, V).to(dtype), h0=gen(7105, B, H, K, V) * 0.3)
+    if gated:
+        ins["g"] = -F.softplus(gen(7103, B, T, H)) * 0.003
+    do, dht = gen(7106, B, T, H, V).to(dtype), gen(7107, B, H, K, V)
+    check(lambda q, k, v, h0, g=None: naive.naive_recurrent_simple_gla(q, k, v, g, None, h0, True, None, False),
+          lambda q, k, v, h0, g=None: chunk_simple_gla(q, k, v, g, None, h0, True, None, False),
+          ins, do, dht, cuda, dtype)
+
+
+@pytest.mark.parametrize("B,T,H,K,V", [(1, 1281, 2, 128, 128), (2, 1500, 1, 64, 64), (1, 2000, 2, 64, 128),
+                                       (1, 1500, 2, 256, 64)])      # two key blocks: the divisor formed outside
+def test_normalised_linear_attention_cut_along_t(cuda, B, T, H, K, V):
+    """The normaliser's column goes through the cut beside the state, forward and backward."""
+    from linear_moe_amd import chunk_linear_attn
+    assert is_cut(0, B, T, H, min(K, 128), V)
+    rows = lambda seed: torch.rand(B, H, T, K, generator=torch.Generator().manual_seed(seed)).bfloat16()
+    ins = dict(q=rows(7200), k=rows(7201), v=gen(7202, B, H, T, V).bfloat16())
+    do = gen(7206, B, H, T, V).bfloat16()
+    leaves = {n: x.double().requires_grad_(True) for n, x in ins.items()}
+    ref, _ = naive.naive_linear_attn(*leaves.values(), normalize=True)
+    refs = torch.autograd.grad((ref * do.double()).sum(), list(leaves.values()))
+    dev = {n: x.to(cuda).requires_grad_(True) for n, x in ins.items()}
+    o, _ = chunk_linear_attn(*dev.values(), normalize=True)
+    grads = torch.autograd.grad(o, list(dev.values()), do.to(cuda))
+    torch.cuda.synchronize()
+    for x, r in zip((o.detach(),) + grads, (ref.detach(),) + refs):
+        assert max_abs_rel(x.cpu(), r) < TOL[torch.bfloat16]
