@@ -401,7 +401,8 @@ int lmoe_trace_simple_gla_fwd(const lmoe_args* a, int64_t* trace, int32_t work_g
 /* Token-by-token forward of an op (op = LMOE_OP_*; the delta rule without a gate: gate = LMOE_GATE_NONE):
  * the state stays in registers, nothing is saved for a backward.  For decoding (T = 1 with h0 / ht) and
  * short sequences.  Uses q, k, v, g, beta, h0, scale, cu_seqlens (+ seq_chunk0, chunk_map as for the chunk
- * entry points) -> o, ht.  Stands where the reference selects fla's fused_recurrent_* callables
+ * entry points) -> o, ht.  The delta rule with qk_eps > 0: the rows of q and k are L2-normalised as they are read, qk_eps
+ * inside the root.  Stands where the reference selects fla's fused_recurrent_* callables
  * (la_mode = 'fused_recurrent': linear_moe/sequence_modeling/gated_deltanet/gated_deltanet.py:72-73,
  * gla/gla.py:58-59, deltanet/deltanet.py:81-82, basic_linear_attention/basic_linear_attention.py:99-100). */
 int lmoe_fused_recurrent_fwd(const lmoe_args* a, int32_t op, void* stream);

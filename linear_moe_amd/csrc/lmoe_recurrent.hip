@@ -22,6 +22,9 @@ namespace lmoe {
 constexpr int RBV = 32;     // V columns per work-group
 constexpr int RTB = 16;     // tokens staged per block
 
+// Delta rule with lmoe_args.qk_eps > 0: the rows of q and k are divided by sqrt(sum of squares + qk_eps) as they are
+// read (use_qk_l2norm_in_kernel), in fp32 and not rounded in between: one decoded token then is one launch in place of
+// three (K = V = 128, 16 heads, one sequence: 41 -> 22 us with the host work of two more calls).
 __device__ __forceinline__ float group8_sum(float x) {
   x += __shfl_xor(x, 1, 64);
   x += __shfl_xor(x, 2, 64);
@@ -60,6 +63,28 @@ __global__ __launch_bounds__(NTHR) void k_recurrent_fwd(const lmoe_args a) {
         s_g[tt][kk] = __expf(load_scalar(a.g.ptr, a.g_dtype, row_off(a.g, sq.b, sq.tok0 + t0 + tt, h) + kk));
     }
     __syncthreads();
+    if constexpr (DELTA) {
+      if (a.qk_eps > 0.f) {                 // sixteen neighbouring lanes per token
+        const int tt = threadIdx.x >> 4, l16 = threadIdx.x & 15;
+        float ssq = 0.f, ssk = 0.f;
+        if (tt < nt) {
+#pragma unroll
+          for (int kk = 0; kk < K; kk += 16) {
+            ssq += s_q[tt][kk + l16] * s_q[tt][kk + l16];
+            ssk += s_k[tt][kk + l16] * s_k[tt][kk + l16];
+          }
+        }
+        const float rq = 1.f / sqrtf(group_sum<16>(ssq) + a.qk_eps), rk = 1.f / sqrtf(group_sum<16>(ssk) + a.qk_eps);
+        if (tt < nt) {
+#pragma unroll
+          for (int kk = 0; kk < K; kk += 16) {
+            s_q[tt][kk + l16] *= rq;
+            s_k[tt][kk + l16] *= rk;
+          }
+        }
+        __syncthreads();
+      }
+    }
     for (int tt = 0; tt < nt; ++tt) {
       const int tok = sq.tok0 + t0 + tt;
       const float vt = ET<T>::to_f(((const T*)a.v.ptr)[row_off(a.v, sq.b, tok, h) + vcol]);
@@ -145,6 +170,20 @@ __global__ __launch_bounds__(NTHR) void k_recurrent_step(const lmoe_args a) {
     for (int j = 0; j < KR; ++j) {
       qv[j] = ET<T>::to_f(qp[kg + 32 * j]);
       kv[j] = ET<T>::to_f(kp[kg + 32 * j]);
+    }
+    if constexpr (DELTA) {
+      if (a.qk_eps > 0.f) {                 // every wave forms the norms for itself: no barrier, the row is in the L1
+        float ssq = 0.f, ssk = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < K; kk += 64) {
+          const float x = ET<T>::to_f(qp[kk + (threadIdx.x & 63)]), y = ET<T>::to_f(kp[kk + (threadIdx.x & 63)]);
+          ssq += x * x;
+          ssk += y * y;
+        }
+        const float rq = 1.f / sqrtf(wave_sum(ssq) + a.qk_eps), rk = 1.f / sqrtf(wave_sum(ssk) + a.qk_eps);
+#pragma unroll
+        for (int j = 0; j < KR; ++j) { qv[j] *= rq; kv[j] *= rk; }
+      }
     }
     const typename ET<T>::vec4 vraw = *(const typename ET<T>::vec4*)((const T*)a.v.ptr + row_off(a.v, sq.b, tok, h) + vcol);
     f32x4 vt;

@@ -19,7 +19,6 @@ from ._host import seq_plan, _aligned, _check_inputs, _desc, _state_check, base_
 from .delta_rule import chunk_delta_rule
 from .gated_delta_rule import chunk_gated_delta_rule
 from .gla import chunk_gla
-from .l2norm import l2_norm
 from .simple_gla import chunk_simple_gla
 
 _OP_SIMPLE, _OP_GLA, _OP_GDN = 0, 1, 2
@@ -33,7 +32,8 @@ def _sdt(x: torch.Tensor) -> int:
     return _lib.LMOE_F32 if x.dtype == torch.float32 else _lib.LMOE_BF16
 
 
-def _recurrent(op, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first):
+def _recurrent(op, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first, qk_eps=0.0):
+    """qk_eps > 0 (delta rule): q and k are L2-normalised by the kernel, qk_eps inside the root."""
     lib = _lib.load()
     dims = _check_inputs(q, k, v, head_first, cu_seqlens)
     B, T, H, K, V = dims
@@ -69,7 +69,7 @@ def _recurrent(op, q, k, v, g, beta, scale, initial_state, output_final_state, c
     a.h0 = ptr(h0)
     o = torch.empty_like(v)
     ht = torch.empty(plan.N, H, K, V, dtype=torch.float32, device=q.device) if output_final_state else None
-    a.o, a.ht = _desc(o, head_first), ptr(ht)
+    a.o, a.ht, a.qk_eps = _desc(o, head_first), ptr(ht), qk_eps
     _lib.check(lib.lmoe_fused_recurrent_fwd(C.byref(a), op, stream_ptr()), "fused_recurrent forward")
     return o, ht
 
@@ -97,9 +97,8 @@ def fused_recurrent_gated_delta_rule(q, k, v, g, beta, scale: Optional[float] = 
     if _needs_grad(q, k, v, g, beta, initial_state):
         return chunk_gated_delta_rule(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                                       head_first, use_qk_l2norm_in_kernel)
-    if use_qk_l2norm_in_kernel:
-        q, k = l2_norm(q.detach()), l2_norm(k.detach())
-    return _recurrent(_OP_GDN, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first)
+    return _recurrent(_OP_GDN, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first,
+                      1e-6 if use_qk_l2norm_in_kernel else 0.0)
 
 
 def fused_recurrent_delta_rule(q, k, v, beta, scale: Optional[float] = None, initial_state=None,

@@ -41,6 +41,29 @@ def test_recurrent_gated_delta_rule(cuda, dtype, shape, gated):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("head_first", [True, False])
+def test_recurrent_gated_delta_rule_normalises_q_and_k(cuda, dtype, shape, head_first):
+    """use_qk_l2norm_in_kernel: rows of any length, one of zeros (the epsilon alone) among them."""
+    from linear_moe_amd import fused_recurrent_gated_delta_rule
+    B, T, H, K, V = shape
+    _, _, v, g, beta = gdn_inputs(2300 + T, B, T, H, K, V, dtype, False, True)
+    q, k = (3 * gen(2305, B, T, H, K)).to(dtype), (0.2 * gen(2306, B, T, H, K)).to(dtype)
+    q[0, 0, 0] = 0
+    k[0, -1, -1] = 0
+    h0 = 0.3 * gen(2307, B, H, K, V)
+    ref_o, ref_ht = naive.naive_recurrent_gated_delta_rule(naive.naive_l2_norm(q), naive.naive_l2_norm(k), v, g, beta, None,
+                                                           h0, True, None, False)
+    d = lambda x: (x.transpose(1, 2) if head_first else x).to(cuda)       # (head first: strided views)
+    o, ht = fused_recurrent_gated_delta_rule(d(q), d(k), d(v), d(g), d(beta), initial_state=h0.to(cuda),
+                                             output_final_state=True, head_first=head_first, use_qk_l2norm_in_kernel=True)
+    torch.cuda.synchronize()
+    o = o.transpose(1, 2) if head_first else o
+    assert max_abs_rel(o.cpu(), ref_o) < TOL[dtype]
+    assert max_abs_rel(ht.cpu(), ref_ht) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("gate", ["none", "scalar", "vector"])
 def test_recurrent_simple_gla_and_gla(cuda, dtype, shape, gate):
     from linear_moe_amd import fused_recurrent_gla, fused_recurrent_simple_gla
