@@ -411,29 +411,29 @@ template <typename T, int D> struct RowFrags {
 };
 
 // ------------------------------------------------------------------------- //
-// cooperative global <-> LDS tile movement (all 256 threads)
+// cooperative global <-> LDS tile movement (NT = 256 threads unless said otherwise)
 //   a tile is ROWS x COLS elements, source rows `row_stride` elements apart;
 //   rows >= nvalid read as zero / are not written.
 // ------------------------------------------------------------------------- //
-template <typename T, int ROWS, int COLS> struct TileIO {
+template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
   static constexpr int VEC = ET<T>::VEC;
   static constexpr int VPR = COLS / VEC;                 // vectors per row
   static constexpr int NVEC = ROWS * VPR;                // vectors in the tile
-  static constexpr int PASSES = (NVEC + NTHR - 1) / NTHR;
+  static constexpr int PASSES = (NVEC + NT - 1) / NT;
   typedef typename ET<T>::vec vec;
   struct Regs { vec v[PASSES]; };
 
-  // thread index inside a team of 256: work-groups of 512 threads use two teams (waves 0-3 and
-  // 4-7) that each move whole tiles
-  static __device__ __forceinline__ void coords(int p, int& row, int& col, int tid = threadIdx.x & (NTHR - 1)) {
-    const int idx = p * NTHR + tid;
+  // thread index inside a team of NT: work-groups of 512 threads use two teams of 256 (waves 0-3 and
+  // 4-7) that each move whole tiles, or one of 512
+  static __device__ __forceinline__ void coords(int p, int& row, int& col, int tid = threadIdx.x & (NT - 1)) {
+    const int idx = p * NT + tid;
     row = idx / VPR; col = (idx % VPR) * VEC;
   }
   // Branch-free loads: rows >= nvalid (nvalid >= 1) re-read the last valid row, so that no load
   // sits behind a branch and the compiler can count outstanding loads exactly (prefetches stay in
   // flight across barriers).  mask() then zeroes the rows >= nvalid; software-pipelined kernels
   // call load_nomask() when they issue a prefetch and mask() when they consume it.
-  static __device__ __forceinline__ void load_nomask(Regs& r, const T* __restrict__ src, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void load_nomask(Regs& r, const T* __restrict__ src, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     const int last = (nvalid < ROWS ? nvalid : ROWS) - 1;
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
@@ -442,7 +442,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
       r.v[p] = *(const vec*)(src + (int64_t)row * row_stride + col);
     }
   }
-  static __device__ __forceinline__ void mask(Regs& r, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void mask(Regs& r, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     if (nvalid >= ROWS) return;                 // uniform: full tiles (the common case) skip it
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -460,7 +460,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
     mask(r, nvalid);
   }
   // tile[row][col] = x
-  static __device__ __forceinline__ void store_lds(const Regs& r, T* tile, int ld, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void store_lds(const Regs& r, T* tile, int ld, int tid = threadIdx.x & (NT - 1)) {
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col, tid);
@@ -468,7 +468,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
     }
   }
   // tile[row][col] = x * rs[row]
-  static __device__ __forceinline__ void store_lds_scaled(const Regs& r, T* tile, int ld, const float* rs, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void store_lds_scaled(const Regs& r, T* tile, int ld, const float* rs, int tid = threadIdx.x & (NT - 1)) {
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col, tid);
@@ -533,7 +533,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
   }
   // registers <- tile[row][col]  /  global[row][col] <- registers (rows < nvalid): the two halves of
   // lds_to_global for callers that must leave the tile before the stores are issued
-  static __device__ __forceinline__ void load_lds(Regs& r, const T* tile, int ld, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void load_lds(Regs& r, const T* tile, int ld, int tid = threadIdx.x & (NT - 1)) {
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col, tid);
@@ -550,7 +550,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
     else *p = x;
   }
   template <bool STREAM = false>
-  static __device__ __forceinline__ void store_global(const Regs& r, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void store_global(const Regs& r, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col, tid);
@@ -561,7 +561,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
   // and rewrites row nvalid - 1, i.e. stores the same bytes to the same address as the thread that
   // owns that row.  No store sits behind a branch, so the compiler can count outstanding memory
   // operations exactly and the caller's prefetches stay in flight across the stores.
-  static __device__ __forceinline__ void load_lds_clamped(Regs& r, const T* tile, int ld, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void load_lds_clamped(Regs& r, const T* tile, int ld, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     const int last = (nvalid < ROWS ? nvalid : ROWS) - 1;
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
@@ -571,7 +571,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
     }
   }
   template <bool STREAM = false>
-  static __device__ __forceinline__ void store_global_clamped(const Regs& r, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void store_global_clamped(const Regs& r, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     const int last = (nvalid < ROWS ? nvalid : ROWS) - 1;
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
@@ -582,7 +582,7 @@ template <typename T, int ROWS, int COLS> struct TileIO {
   }
   // global[row][col] = tile[row][col]
   template <bool STREAM = false>
-  static __device__ __forceinline__ void lds_to_global(const T* tile, int ld, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NTHR - 1)) {
+  static __device__ __forceinline__ void lds_to_global(const T* tile, int ld, T* __restrict__ dst, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
 #pragma unroll
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col, tid);

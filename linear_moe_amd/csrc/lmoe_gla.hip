@@ -57,7 +57,7 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
     case ST_DV:
       hipLaunchKernelGGL((k_gla_bwd_dv<T, GT, K, V, Tl::BVO>), dim3(a.NT, a.H, V / Tl::BVO), block, 0, st, a); break;
     case ST_DQK:
-      hipLaunchKernelGGL((k_gla_bwd_dqkg<T, GT, K, V, Tl::BVH>), dim3(a.NT, a.H), block, 0, st, a); break;
+      hipLaunchKernelGGL((k_gla_bwd_dqkg<T, GT, K, V, Tl::BVH>), dim3(a.NT, a.H), dim3(2 * NTHR), 0, st, a); break;
     default: break;
   }
 }

@@ -18,6 +18,7 @@
 // sub-chunks the decay factors through the cumulative gate at the sub-chunk boundary, which turns
 // those parts into products of scaled tiles on MFMA, like every other product here.
 #pragma once
+#include <type_traits>
 #include "lmoe_seq.hpp"
 
 namespace lmoe {
@@ -42,23 +43,23 @@ template <int N> __device__ __forceinline__ void load_f32_group(const float* p, 
 }
 
 // g tile of the chunk -> fp32 LDS tile s_b[64][LDB] holding the inclusive cumsum over tokens.
-// The scan: a thread takes one channel over a segment of 64 K / 256 tokens (its values in registers, so the
+// The scan: a thread takes one channel over a segment of 64 K / NT tokens (its values in registers, so the
 // LDS reads are independent of each other), the segment totals go through a small LDS array, and every thread
-// adds the totals of the segments before its own.  All 256 threads; ends with a barrier (the barriers order
+// adds the totals of the segments before its own.  All NT threads; ends with a barrier (the barriers order
 // LDS traffic only: loads a caller keeps in flight stay in flight).
-template <typename GT, int K>
+template <typename GT, int K, int NT = NTHR>
 struct GlaGate {
-  typedef TileIO<GT, CH, K> IOG;
+  typedef TileIO<GT, CH, K, NT> IOG;
   typedef typename IOG::Regs Regs;
   static __device__ __forceinline__ void issue(Regs& rg, const lmoe_args& a, int b, int tok, int len, int h) {
     IOG::load_nomask(rg, row_ptr<GT>(a.g, b, tok, h), a.g.st, len);
   }
-  // tot: NTHR floats of LDS for the segment totals
+  // tot: NT floats of LDS for the segment totals
   template <int LDB>
   // mult: factor applied to the stored cumsum (1, or TEXP_PRESCALE<T> for kernels that only form exponentials of it)
   static __device__ __forceinline__ void finish(Regs& rg, int len, float* s_b, float* s_tot, float mult = 1.0f) {
-    constexpr int NSEG = NTHR / K, SEG = CH / NSEG;
-    static_assert(NTHR % K == 0 && CH % NSEG == 0, "one channel and one token segment per thread");
+    constexpr int NSEG = NT / K, SEG = CH / NSEG;
+    static_assert(NT % K == 0 && CH % NSEG == 0, "one channel and one token segment per thread");
     IOG::mask(rg, len);
     IOG::store_lds_f32(rg, s_b, LDB);
     lds_barrier();
@@ -79,7 +80,7 @@ struct GlaGate {
   }
   template <int LDB>
   static __device__ __forceinline__ void finish(Regs& rg, int len, float* s_b) {
-    __shared__ float s_tot[NTHR];
+    __shared__ float s_tot[NT];
     finish<LDB>(rg, len, s_b, s_tot);
   }
 };
@@ -883,14 +884,16 @@ __global__ __launch_bounds__(NTHR) void k_gla_bwd_dv(const lmoe_args a) {
 }
 
 // ------------------------------------------------------------------------- //
-// dq, dk, dg (2-byte elements: dv as well), grid = (NT, H)
+// dq, dk, dg (2-byte elements: dv as well), grid = (NT, H), 512 threads: wave w forms rows 16 (w % 4) .. of every product and
+// of its columns the half w / 4.  The kernel is a chain of short phases on LDS tiles (76 KB at K = 64, 135 KB at K = 128:
+// two, one work-groups per CU), so what hides its latencies is the number of waves per work-group.
 // ------------------------------------------------------------------------- //
 template <typename T, typename GT, int K, int V, int BVH>
-__global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 && sizeof(T) == 2) ? 2 : 1))) void k_gla_bwd_dqkg(const lmoe_args a) {
+__global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 && sizeof(T) == 2) ? 4 : 2))) void k_gla_bwd_dqkg(const lmoe_args a) {
   // (LDB: rows of the fp32 gate tile start on 16-byte boundaries, and the rows 4 apart that the lanes of an accumulator
   // column read fall into different banks)
   constexpr int LDV = BVH + LPAD, LDB = K + 4, LDP = CH + 1;
-  constexpr int NBK = K / 16;
+  constexpr int NW = 2 * NTHR, NBK = K / 16, NBH = NBK / 2;
   // phase A (element type T): do, v, S, dS' slices.  phase B (fp32): dA, q, k, b tiles
   constexpr int A_DO = 0, A_V = A_DO + CH * LDV, A_H = A_V + CH * LDV, A_DH = A_H + K * LDV, A_END0 = A_DH + K * LDV;
   // 2-byte elements: dv is formed here as well, from the do and dS' slices that phase A stages anyway and two more
@@ -922,12 +925,13 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   const int cid = blockIdx.x, h = blockIdx.y;
   if (cid >= num_chunks(a)) return;          // launch sized by an upper bound of the chunk count
   const ChunkInfo ci = chunk_info(a, cid);
-  const int wv = wave_id(), l = lane_id();
-  typedef TileIO<T, CH, BVH> IOV;
-  typedef TileIO<T, K, BVH> IOH;
-  typedef TileIO<T, CH, K> IOK;
+  const int wv = wave_id() & 3, hf = wave_id() >> 2, l = lane_id();
+  typedef TileIO<T, CH, BVH, NW> IOV;
+  typedef TileIO<T, K, BVH, NW> IOH;
+  typedef TileIO<T, CH, K, NW> IOK;
+  typedef GlaGate<GT, K, NW> GG;
 
-  f32x4 dP[1][4], dqi[1][NBK], dkd[1][NBK];
+  f32x4 dP[1][2], dqi[1][NBH], dkd[1][NBH];
   acc_zero(dP); acc_zero(dqi); acc_zero(dkd);
   float hdh[IOH::PASSES];
 #pragma unroll
@@ -938,7 +942,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   struct Slice { typename IOV::Regs rd, rv; typename IOH::Regs rh, rdh; };
   Slice sl[2];
   typename IOK::Regs rq, rk;
-  typename GlaGate<GT, K>::Regs rg;
+  typename GG::Regs rg;
   auto issue_slice = [&](Slice& x, int vv) {
     IOV::load_nomask(x.rd, row_ptr<T>(a.d_o, ci.b, ci.tok, h) + vv, a.d_o.st, ci.len);
     IOV::load_nomask(x.rv, row_ptr<T>(a.v, ci.b, ci.tok, h) + vv, a.v.st, ci.len);
@@ -946,7 +950,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
     IOH::load_nomask(x.rdh, (const T*)a.dhs + ((int64_t)cid * a.H + h) * K * V + vv, V, K);
   };
   issue_slice(sl[0], 0);
-  typedef TileIO<T, CH, CH> IOA;
+  typedef TileIO<T, CH, CH, NW> IOA;
   typename IOK::Regs rke;
   typename IOA::Regs ram;
   if constexpr (DV) {
@@ -956,7 +960,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   auto issue_qkg = [&]() {
     IOK::load_nomask(rq, row_ptr<T>(a.q, ci.b, ci.tok, h), a.q.st, ci.len);
     IOK::load_nomask(rk, row_ptr<T>(a.k, ci.b, ci.tok, h), a.k.st, ci.len);
-    GlaGate<GT, K>::issue(rg, a, ci.b, ci.tok, ci.len, h);
+    GG::issue(rg, a, ci.b, ci.tok, ci.len, h);
   };
   // with two slices everything is requested at the start (a load of this kernel takes 5 to 9 thousand cycles to
   // arrive, the work on a slice 1500); with more, q, k, g go out with the last slice
@@ -983,20 +987,20 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
       }
     }
     lds_barrier();      // LDS-only barriers: the loads requested above stay in flight
-    gemm_nt<T, 1, 4, true>(dP, smT + A_DO, LDV, 16 * wv, smT + A_V, LDV, 0, 0, BVH);
-    gemm_nt<T, 1, NBK, true>(dqi, smT + A_DO, LDV, 16 * wv, smT + A_H, LDV, 0, 0, BVH);
-    gemm_nt<T, 1, NBK, true>(dkd, smT + A_V, LDV, 16 * wv, smT + A_DH, LDV, 0, 0, BVH);
+    gemm_nt<T, 1, 2, true>(dP, smT + A_DO, LDV, 16 * wv, smT + A_V, LDV, 32 * hf, 0, BVH);
+    gemm_nt<T, 1, NBH, true>(dqi, smT + A_DO, LDV, 16 * wv, smT + A_H, LDV, hf * (K / 2), 0, BVH);
+    gemm_nt<T, 1, NBH, true>(dkd, smT + A_V, LDV, 16 * wv, smT + A_DH, LDV, hf * (K / 2), 0, BVH);
     if constexpr (DV) {
       // dv^T of the slice = scale do^T A + dS'^T (k e^{b_C - b})^T, the products and the rounding of k_gla_bwd_dv
       // (same operands, same order): a lane holds four consecutive V columns of one token, 8-byte stores
-      constexpr int NBV = BVH / 16;
+      constexpr int NBV = BVH / 32;
       f32x4 dv[NBV][1], dv2[NBV][1];
       acc_zero(dv); acc_zero(dv2);
-      gemm<T, NBV, 1, true, false>(dv2, smT + A_DH, LDV, 0, smT + A_KE, LDK, 16 * wv, 0, K);
-      gemm<T, NBV, 1, true, true>(dv, smT + A_DO, LDV, 0, smT + A_AM, LDC, 16 * wv, 0, CH);
+      gemm<T, NBV, 1, true, false>(dv2, smT + A_DH, LDV, hf * (BVH / 2), smT + A_KE, LDK, 16 * wv, 0, K);
+      gemm<T, NBV, 1, true, true>(dv, smT + A_DO, LDV, hf * (BVH / 2), smT + A_AM, LDC, 16 * wv, 0, CH);
       const int r = 16 * wv + (l & 15);
       if (r < ci.len) {
-        T* dd = row_ptr<T>(a.dv, ci.b, ci.tok + r, h) + si * BVH + 4 * (l >> 4);
+        T* dd = row_ptr<T>(a.dv, ci.b, ci.tok + r, h) + si * BVH + hf * (BVH / 2) + 4 * (l >> 4);
 #pragma unroll
         for (int ni = 0; ni < NBV; ++ni) {
           typename ET<T>::vec4 y;
@@ -1023,15 +1027,15 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   float* sBw = SUB ? smF + S_B / 4 : smF + B_B;
   {
 #pragma unroll
-    for (int nj = 0; nj < 4; ++nj) {
+    for (int nj = 0; nj < 2; ++nj) {
       f32x4 p;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wv + 4 * (l >> 4) + i, cc = 16 * nj + (l & 15);
+        const int r = 16 * wv + 4 * (l >> 4) + i, cc = 32 * hf + 16 * nj + (l & 15);
         p[i] = (r >= cc) ? a.scale * dP[0][nj][i] : 0.f;
         if constexpr (!SUB) smF[B_DP + r * LDP + cc] = p[i];
       }
-      if constexpr (SUB) acc_to_lds<T>(p, tDA, LDC, 16 * wv, 16 * nj);
+      if constexpr (SUB) acc_to_lds<T>(p, tDA, LDC, 16 * wv, 32 * hf + 16 * nj);
     }
     IOK::mask(rq, ci.len);
     IOK::mask(rk, ci.len);
@@ -1043,7 +1047,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
       IOK::store_lds_f32(rk, smF + B_K, LDB);
     }
   }
-  GlaGate<GT, K>::template finish<LDB>(rg, ci.len, sBw);   // barriers inside
+  GG::template finish<LDB>(rg, ci.len, sBw);   // barriers inside
   const float* sB = sBw;
   // dA, q, k of the pairwise loops and the epilogue, from whichever tiles this layout keeps
   auto Pm = [&](int r, int j) { if constexpr (SUB) return ET<T>::to_f(tDA[r * LDC + j]); else return smF[B_DP + r * LDP + j]; };
@@ -1058,7 +1062,7 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   // Two rounds over one stacked LDS tile: sub-chunks {0, 3}, then {1, 2} (contraction ranges in multiples of 32
   // tokens: k~ of sub-chunk 0 / 1 / 2 / 3 holds 32 / 32 / 64 / 64 rows, q~ 64 / 64 / 32 / 32).
   int unsafe = 0;
-  f32x4 dqo[1][NBK], dko[1][NBK];
+  f32x4 dqo[1][NBH], dko[1][NBH];
   acc_zero(dqo); acc_zero(dko);
   if constexpr (SUB) {
     __shared__ int s_unsafe;
@@ -1081,58 +1085,56 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
       constexpr int SEGROW[4] = {0, 32, 96, 160};                       // k~(wa) 32 | k~(wb) 64 | q~(wa) 64 | q~(wb) 32
       constexpr int VEC = ET<T>::VEC;
       typedef typename ET<T>::vec vec;
-      // A thread keeps its 16-byte column group c0 and takes one stacked row out of every RPI: the segment of a row
-      // is then known at compile time, the gate row that a whole segment shares (its reference) is read once, and
-      // every gate value arrives in 16-byte reads
-      constexpr int PPR = K / VEC, RPI = NTHR / PPR, NIT = 192 / RPI;
+      // The first four waves scale the k~ rows, the other four the q~ rows (96 each).  A thread keeps its 16-byte column
+      // group c0 and takes one row out of every RPI: the segment of a row is then known at compile time, the gate row
+      // that a whole segment shares (its reference) is read once, and every gate value arrives in 16-byte reads
+      constexpr int PPR = K / VEC, RPI = NTHR / PPR, NIT = 96 / RPI;
       static_assert(32 % RPI == 0 && NTHR % PPR == 0, "segment boundaries fall between the passes");
-      const int c0 = (threadIdx.x % PPR) * VEC, rin = threadIdx.x / PPR;
+      const int tid = threadIdx.x & (NTHR - 1), c0 = (tid % PPR) * VEC, rin = tid / PPR;
       auto gate_row = [&](int row, float (&b)[VEC]) { load_f32_group(sB + row * LDB + c0, b); };
-      float ref[4][VEC];                                                // k~: b_{16 w - 1} (0 for w = 0); q~: b_{16 w + 15}
+      auto scale_rows = [&](auto is_q) {
+        constexpr bool Q = decltype(is_q)::value;
+        constexpr int FIRST = Q ? 64 : 32;                              // rows of the first of the two segments
+        float ref[2][VEC];                                              // k~: b_{16 w - 1} (0 for w = 0); q~: b_{16 w + 15}
 #pragma unroll
-      for (int sg = 0; sg < 4; ++sg) {
-        const int w = (sg & 1) ? wb : wa;
-        if (sg < 2 && w == 0) {
+        for (int sg = 0; sg < 2; ++sg) {
+          const int w = sg ? wb : wa;
+          if (!Q && w == 0) {
 #pragma unroll
-          for (int e = 0; e < VEC; ++e) ref[sg][e] = 0.f;
-        } else {
-          gate_row(sg < 2 ? 16 * w - 1 : 16 * w + 15, ref[sg]);
+            for (int e = 0; e < VEC; ++e) ref[sg][e] = 0.f;
+          } else {
+            gate_row(Q ? 16 * w + 15 : 16 * w - 1, ref[sg]);
+          }
         }
-      }
 #pragma unroll
-      for (int it = 0; it < NIT; ++it) {
-        const int sr0 = it * RPI, sg = sr0 < 32 ? 0 : sr0 < 96 ? 1 : sr0 < 160 ? 2 : 3;   // known after unrolling
-        const int sr = sr0 + rin;
-        const int w = (sg & 1) ? wb : wa;
-        const bool own_ok = !((unsafe >> w) & 1);
-        // token of this row and whether the row is in use
-        int tok;
-        bool use;
-        if (sg < 2) {
-          tok = sr - SEGROW[sg];
-          use = tok < 16 * w + 16 && (tok < 16 * w || own_ok);          // k_j e^{ref_w - b_j}
-        } else {
-          tok = (w < 2 ? 0 : 32) + sr - SEGROW[sg];
-          use = tok >= 16 * w && (tok >= 16 * w + 16 || own_ok);        // q_i e^{b_i - ref'_w}
-        }
-        vec o = ET<T>::zero();
-        if (use) {
-          const vec x = *(const vec*)((sg < 2 ? tK : tQ) + tok * LDK + c0);
-          float bt[VEC];
-          gate_row(tok, bt);
+        for (int it = 0; it < NIT; ++it) {
+          const int sr0 = it * RPI, sg = sr0 < FIRST ? 0 : 1;           // known after unrolling
+          const int sr = sr0 + rin, w = sg ? wb : wa;
+          const bool own_ok = !((unsafe >> w) & 1);
+          // token of this row and whether the row is in use: q_i e^{b_i - ref'_w} | k_j e^{ref_w - b_j}
+          const int tok = (Q && w >= 2 ? 32 : 0) + sr - (sg ? FIRST : 0);
+          const bool use = Q ? tok >= 16 * w && (tok >= 16 * w + 16 || own_ok) : tok < 16 * w + 16 && (tok < 16 * w || own_ok);
+          vec o = ET<T>::zero();
+          if (use) {
+            const vec x = *(const vec*)((Q ? tQ : tK) + tok * LDK + c0);
+            float bt[VEC];
+            gate_row(tok, bt);
 #pragma unroll
-          for (int e = 0; e < VEC; ++e)
-            o[e] = ET<T>::from_f(ET<T>::to_f(x[e]) * texp<T>(sg < 2 ? ref[sg][e] - bt[e] : bt[e] - ref[sg][e]));
+            for (int e = 0; e < VEC; ++e)
+              o[e] = ET<T>::from_f(ET<T>::to_f(x[e]) * texp<T>(Q ? bt[e] - ref[sg][e] : ref[sg][e] - bt[e]));
+          }
+          *(vec*)(tKT + ((Q ? 96 : 0) + sr) * LDK + c0) = o;
         }
-        *(vec*)(tKT + sr * LDK + c0) = o;
-      }
+      };
+      if (hf == 0) scale_rows(std::false_type{});
+      else scale_rows(std::true_type{});
       __syncthreads();
       if (wv == wa || wv == wb) {
         const int sg = wv == wa ? 0 : 1;
         const int nk = wv < 2 ? 32 : 64;                                // tokens j < nk
-        gemm<T, 1, NBK, false, true>(dqo, tDA, LDC, 16 * wv, tKT + SEGROW[sg] * LDK, LDK, 0, 0, nk);
+        gemm<T, 1, NBH, false, true>(dqo, tDA, LDC, 16 * wv, tKT + SEGROW[sg] * LDK, LDK, hf * (K / 2), 0, nk);
         const int i0 = wv < 2 ? 0 : 32;                                 // tokens i >= i0
-        gemm<T, 1, NBK, true, true>(dko, tDA, LDC, 16 * wv, tKT + (SEGROW[2 + sg] - i0) * LDK, LDK, 0, i0, CH);
+        gemm<T, 1, NBH, true, true>(dko, tDA, LDC, 16 * wv, tKT + (SEGROW[2 + sg] - i0) * LDK, LDK, hf * (K / 2), i0, CH);
       }
       __syncthreads();
     }
@@ -1140,29 +1142,31 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   const int jlo = SUB ? 16 * wv : 0, ihi = SUB ? 16 * wv + 16 : CH;   // range of the pairwise loops
   T* dqd = row_ptr<T>(a.dq, ci.b, ci.tok, h);
   T* dkd_g = row_ptr<T>(a.dk, ci.b, ci.tok, h);
-  float kkp[NBK];                      // per column: sum over this lane's rows of (dk_d . k_d)
-  float dbv[NBK][4];
-  static_assert(NBK % 4 == 0, "column tiles are taken four at a time");
+  const int ch = hf * (K / 2) + (l & 15);   // first column of this lane
+  constexpr int NG = NBH < 4 ? NBH : 4;
+  float kkp[NBH];                      // per column: sum over this lane's rows of (dk_d . k_d)
+  float dbv[NBH][4];
+  static_assert(NBH % NG == 0, "column tiles are taken NG at a time");
 #pragma unroll
-  for (int nh = 0; nh < NBK; nh += 4) {
-    // Diagonal block of this wave's sub-chunk, for four column tiles at a time.  One pass over the 16 tokens
+  for (int nh = 0; nh < NBH; nh += NG) {
+    // Diagonal block of this wave's sub-chunk, for NG column tiles at a time.  One pass over the 16 tokens
     // j of the sub-chunk serves both sums: dA is lower triangular (zero above the diagonal), so
     //   sq[r] += dA(r, j) k_j e,   sk[r] += dA(j, r) q_j e,   e = e^{-|b_r - b_j|}
     // (b decreases along the chunk: the exponent wanted is b_r - b_j for j <= r and b_j - b_r for j >= r;
     // where it is not, the dA factor is zero).  k_j, q_j, b_j are read once per token and column and serve
-    // the lane's four rows; the dA values are read once per token and serve the four column tiles.
-    float sqv[4][4], skv[4][4], brv[4][4];
+    // the lane's four rows; the dA values are read once per token and serve the NG column tiles.
+    float sqv[NG][4], skv[NG][4], brv[NG][4];
 #pragma unroll
-    for (int n4 = 0; n4 < 4; ++n4)
+    for (int n4 = 0; n4 < NG; ++n4)
 #pragma unroll
       for (int i = 0; i < 4; ++i) sqv[n4][i] = skv[n4][i] = 0.f;
     if (SUB && ((unsafe >> wv) & 1)) {
 #pragma unroll
-      for (int n4 = 0; n4 < 4; ++n4)
+      for (int n4 = 0; n4 < NG; ++n4)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           sqv[n4][i] = skv[n4][i] = 0.f;
-          brv[n4][i] = sB[(16 * wv + 4 * (l >> 4) + i) * LDB + 16 * (nh + n4) + (l & 15)] * TEXP_PRESCALE<T>;
+          brv[n4][i] = sB[(16 * wv + 4 * (l >> 4) + i) * LDB + 16 * (nh + n4) + ch] * TEXP_PRESCALE<T>;
         }
       for (int jj = 0; jj < 16; ++jj) {
         const int j = 16 * wv + jj;
@@ -1174,8 +1178,8 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
           pk[i] = Pm(j, r);
         }
 #pragma unroll
-        for (int n4 = 0; n4 < 4; ++n4) {
-          const int cc = 16 * (nh + n4) + (l & 15);
+        for (int n4 = 0; n4 < NG; ++n4) {
+          const int cc = 16 * (nh + n4) + ch;
           const float kj = Km(j, cc), qj = Qm(j, cc), bj = sB[j * LDB + cc] * TEXP_PRESCALE<T>;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -1187,9 +1191,9 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
       }
     }
 #pragma unroll
-    for (int n4 = 0; n4 < 4; ++n4) {
+    for (int n4 = 0; n4 < NG; ++n4) {
       const int ni = nh + n4;
-      const int cc = 16 * ni + (l & 15);
+      const int cc = 16 * ni + ch;
       const float bC = sB[63 * LDB + cc];
       // Two exponentials per element, e^{b_r - ref_w} and e^{ref'_w - b_r} (both exponents <= 0); the other two
       // factors of a row follow from them through one factor per column: e^{b_r} = e^{ref_w} e^{b_r - ref_w},
@@ -1242,18 +1246,18 @@ __global__ __launch_bounds__(NTHR) __attribute__((amdgpu_waves_per_eu((K <= 64 &
   }
   float* sDB = SUB ? (float*)tKT : smF + B_Q;
 #pragma unroll
-  for (int ni = 0; ni < NBK; ++ni)
+  for (int ni = 0; ni < NBH; ++ni)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int r = 16 * wv + 4 * (l >> 4) + i, cc = 16 * ni + (l & 15);
+      const int r = 16 * wv + 4 * (l >> 4) + i, cc = 16 * ni + ch;
       sDB[r * LDB + cc] = dbv[ni][i];
     }
   __syncthreads();
   // dg = reverse cumsum of db over the tokens (+ the last-row term): a thread takes one channel over a segment
   // of tokens, the segment totals go through LDS (rows past the end of a partial chunk have zero db)
   {
-    constexpr int NSEG = NTHR / K, SEG = CH / NSEG;
-    __shared__ float s_seg[NTHR];
+    constexpr int NSEG = NW / K, SEG = CH / NSEG;
+    __shared__ float s_seg[NW];
     const int cc = threadIdx.x % K, sg = threadIdx.x / K;
     float v[SEG];
 #pragma unroll
