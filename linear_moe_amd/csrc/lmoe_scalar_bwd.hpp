@@ -136,7 +136,7 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const
   constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
   if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = CUT ? pass_item(a, sp, pair / a.H) : pass_item(a, Split{}, pair / a.H);
+  const PassItem item = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();

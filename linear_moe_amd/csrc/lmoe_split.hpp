@@ -124,6 +124,18 @@ __device__ __forceinline__ PassItem pass_item(const lmoe_args& a, const Split& s
   }
   return p;
 }
+// the same where only dense input is ever cut
+__device__ __forceinline__ PassItem pass_item_dense(const lmoe_args& a, const Split& sp, int i) {
+  PassItem p;
+  const bool cut = sp.len3 != 0;
+  const int nseg = cut ? seg_count((a.T + CH - 1) / CH, sp.len3) : 1, m = __builtin_amdgcn_readfirstlane(i / nseg), j = i - m * nseg;
+  p.n = cut ? m : seq_at(a, m);
+  p.sq = seq_info(a, p.n);
+  if (cut) p.sq = seg_cut(p.sq, j, sp.len3);
+  p.first = j == 0;
+  p.last = j == nseg - 1;
+  return p;
+}
 // How a call is cut (pointers left open), or len1 = 0.  `slices` = work-groups of the ordinary pass per (sequence, head),
 // which hold a CU each; the work-groups of step 1 carry all columns and hold a CU each too.  Chosen by what the three steps
 // were measured to take (us, K = V = 128, delta rule; half of it per chunk at K = V = 64):
@@ -156,6 +168,37 @@ inline Split plan_split(const lmoe_args& a, int slices) {
   s.n3 = packed ? a.NT / s.len3 + a.N : a.N * seg_count(nch, s.len3);
   return s;
 }
+// The cut of a dense call whose step 2 is a few loads at the start of the pass.  c3 us per chunk of the ordinary pass, b3
+// more where every CU runs one, wg3 its work-groups; c1, wg1 the same of step 1, per fine segment.  A work-group of the
+// pass takes 2.5 to start, and `pre` per fine segment it starts from: work-groups in several rounds pay that every time.
+// Without these two terms 16 pairs of 49 chunks (K = V = 128, retention) were cut into 25 (1600 work-groups of two chunks,
+// 82 us for the pass that takes 64 in one piece), 28 pairs of 110 chunks into 16 (123 against 138).
+inline Split plan_cut(const lmoe_args& a, float c3, float b3, float c1, float pre, int64_t wg3, int64_t wg1) {
+  Split s = {};
+  const int cus = cu_count(), nch = (a.T + CH - 1) / CH;
+  const float w = (a.K + a.V) / 256.f;
+  auto rounds = [](int64_t n, int64_t per) { return (float)((n + per - 1) / per); };
+  auto pass = [&](int64_t wg, int chunks) {             // (the last round may leave CUs idle)
+    const int64_t full = wg / cus, rest = wg % cus;
+    return 2.5f * rounds(wg, cus) + chunks * (full * (c3 + b3) + (rest ? c3 + b3 * rest / cus : 0.f));
+  };
+  float best = 0.9f * pass(wg3, nch);
+  for (int r = 2; r <= 32 && r <= nch; ++r) {
+    const int len3 = seg_count(nch, r);
+    if (seg_count(nch, len3) != r) continue;
+    for (int f = 1; f <= 4; ++f) {
+      if (len3 % f) continue;
+      const int len1 = len3 / f, nf = seg_count(nch, len1);
+      const int64_t segs = wg1 * (r - 1) * f;
+      // step 1: two work-groups to a CU, and what they write; the pass: the last segment starts from all, the average
+      // one from half of them
+      const float t = 8.f + c1 * len1 * rounds(segs, 2 * cus) + 0.015f * w * segs + pass(wg3 * r, len3) +
+                      pre * (r - 1) * f * fmaxf(1.f, 0.5f * rounds(wg3 * r, cus));
+      if (t < best) { best = t; s.len1 = len1; s.len3 = len3; s.n1 = a.N * nf; s.n3 = a.N * r; }
+    }
+  }
+  return s;
+}
 // The same for chunk_simple_gla, whose transitions are numbers: step 2 is a few loads at the start of the pass
 // (seg_prefix), and a cut pays from a handful of chunks on.  Dense input only (the places of packed sequences are not
 // known here).  Measured, us per chunk of the ordinary pass (V slices of 32, 4-byte elements 16): K = V = 64 0.88,
@@ -164,30 +207,21 @@ inline Split plan_split(const lmoe_args& a, int slices) {
 // elements K = V = 64, 4 pairs, T = 512 33.8 -> 13.6 (kernels alone), T = 2048 124 -> 28; with the normaliser, forward +
 // backward, K = V = 128, T = 8192, 8 pairs 383 -> 172.  64 pairs at K = V = 128 fill the CUs: never cut.
 inline Split plan_split_scalar(const lmoe_args& a) {
-  Split s = {};
+  const Split s = {};
   if (a.N < 1 || a.T < 1 || a.cu_seqlens) return s;
   const bool f4 = a.dtype != LMOE_BF16;
   const int cus = cu_count(), nch = (a.T + CH - 1) / CH, pairs = a.N * a.H;
   if (!f4 && (int64_t)pairs * (a.V / 64) >= cus) return s;        // the pass takes wide slices there and fills the CUs
-  // (2-byte elements: short and very long sequences give the same bits alone and in a batch that fills the CUs)
-  if (nch < (f4 ? 3 : 8) || nch > SPLIT_MAX_CHUNKS) return s;
+  // (2-byte elements: up to 16 chunks a cut saves 5 us at most; those and very long sequences are left whole and give the
+  // same bits alone and in a batch that fills the CUs)
+  if (nch < (f4 ? 3 : 17) || nch > SPLIT_MAX_CHUNKS) return s;
   const float w = (a.K + a.V) / 256.f;
+  const int64_t wg3 = (int64_t)pairs * (a.V / (f4 ? 16 : 32));
+  // (the passes of a normalised call ask for more per chunk: 128 work-groups of K = 64, V = 128 in two took 270 -> 297 for
+  // forward and backward together, 384 of K = V = 128 759 -> 857)
+  if (!f4 && a.normalize && 2 * wg3 >= cus) return s;
   const float c3 = f4 ? 1.9f + 4.1f * w : 0.45f + 0.85f * w, c1 = f4 ? 1.f + 2.f * w : 0.3f + 0.6f * w;
-  const int64_t wg3 = (int64_t)pairs * (a.V / (f4 ? 16 : 32)), wg1 = (int64_t)pairs * (f4 ? a.V / 32 : 1);
-  auto rounds = [](int64_t n, int64_t per) { return (float)((n + per - 1) / per); };
-  float best = 0.9f * rounds(wg3, cus) * nch * c3;
-  for (int r = 2; r <= 32 && r <= nch; ++r) {
-    const int len3 = seg_count(nch, r);
-    if (seg_count(nch, len3) != r) continue;
-    for (int f = 1; f <= 4; ++f) {
-      if (len3 % f) continue;
-      const int len1 = len3 / f, nf = seg_count(nch, len1);
-      // step 1 two work-groups to a CU; a fine segment at the start of the pass 0.15
-      const float t = 8.f + c1 * len1 * rounds(wg1 * (r - 1) * f, 2 * cus) + 0.15f * (r - 1) * f + c3 * len3 * rounds(wg3 * r, cus);
-      if (t < best) { best = t; s.len1 = len1; s.len3 = len3; s.n1 = a.N * nf; s.n3 = a.N * r; }
-    }
-  }
-  return s;
+  return plan_cut(a, c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
 }
 // S <- D S + Q over the n fine segments in front of a coarse one, in order (step = -1: behind it, from the last on).
 // q, d: Q (its column v0 + lane % 16, row krow0 + 4 (lane / 16)) and D of the first; four segments' loads at a time.
