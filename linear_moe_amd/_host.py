@@ -286,6 +286,16 @@ def _state_check(x: Optional[torch.Tensor], N, H, K, V, name: str) -> Optional[t
     return x.detach().to(torch.float32).contiguous()
 
 
+def cut_workspace(lib, a: Args, op: int, device):
+    """The workspace of a call whose sequences are cut along T (``lmoe_args.seg_ws``), or None."""
+    n = lib.lmoe_split_floats(C.byref(a), op, 1)
+    if n <= 0:
+        return None
+    ws = torch.empty(n, dtype=torch.float32, device=device)
+    a.seg_ws = ws.data_ptr()
+    return ws
+
+
 def base_args(q, k, v, head_first: bool, scale: Optional[float], plan: SeqPlan, dims) -> Args:
     B, T, H, K, V = dims
     dev = q.device

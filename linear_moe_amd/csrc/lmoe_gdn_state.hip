@@ -110,6 +110,7 @@ bool launch_gdn_state_fwd_trace(const lmoe_args& a, long long* tr, int work_grou
 }
 int64_t split_floats(const lmoe_args& a, int op, int part) {
   if (op == LMOE_OP_SIMPLE_GLA && part == 1) return scalar_split_floats(a);
+  if (op == LMOE_OP_GLA && part == 1) return gla_split_floats(a);
   if (op != LMOE_OP_GATED_DELTA_RULE) return 0;
   const Split sp = gdn_split_plan(a);
   const int64_t trans = (int64_t)sp.n1 * a.H * (a.K * a.K / 2 + 1);      // a 2-byte matrix and a decay per fine segment

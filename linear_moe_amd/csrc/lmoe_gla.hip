@@ -1,6 +1,6 @@
 // Instantiation and launch of the chunk_gla kernels.
 #include "lmoe_launch.hpp"
-#include "lmoe_gla.hpp"
+#include "lmoe_gla_split.hpp"
 
 namespace lmoe {
 
@@ -14,6 +14,27 @@ template <typename T, int V> struct GlaTiles {
   static constexpr int BVH = sizeof(T) == 4 ? 32 : 64;                // V-slice loop of dq/dk/dg
 };
 
+// How the sequences of a call are cut along T: not at all without a workspace for it.
+static Split gla_split(const lmoe_args& a) {
+  Split sp = {};
+  if (!a.seg_ws) return sp;
+  sp = plan_split_gla(a);
+  sp.Q = a.seg_ws;
+  sp.D = sp.Q + (int64_t)sp.n1 * a.H * a.K * a.V;
+  return sp;
+}
+int64_t gla_split_floats(const lmoe_args& a) { return (int64_t)plan_split_gla(a).n1 * a.H * (a.K * a.V + a.K); }
+// what the fine segments add (forward: but for those of the last coarse segment; backward: of the first)
+template <typename T, int K, int V, bool BWD> static Split launch_gla_seg(const lmoe_args& a, hipStream_t st) {
+  const Split sp = gla_split(a);
+  if (sp.len1) {
+    const int n = sp.n1 / a.N, f = sp.len3 / sp.len1, r = sp.n3 / a.N;
+    const int seg0 = BWD ? f : 0, nsegs = BWD ? n - f : (r - 1) * f;
+    hipLaunchKernelGGL((k_gla_seg_state<T, K, V, BWD>), dim3(a.N * nsegs * a.H), dim3(NTHR), 0, st, a, sp, seg0, nsegs);
+  }
+  return sp;
+}
+
 template <typename T, typename GT, int K, int V>
 static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
   typedef GlaTiles<T, V> Tl;
@@ -26,23 +47,24 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
       if constexpr (sizeof(T) == 2) {
         // 2-byte elements: the pass that holds the state also forms the output (k_gla_fwd_fused); hs == NULL: nothing
         // saved
-        const int pairs8 = (a.N * a.H + 7) / 8 * 8;
+        const Split sp = wide ? Split{} : launch_gla_seg<T, K, V, false>(a, st);
+        const int pairs8 = (pass_items(a, sp) * a.H + 7) / 8 * 8;
         if constexpr (Tl::BVS_WIDE != Tl::BVS) {
           // (the saving instance of a wide slice at K = 128 has no registers left for the copy of the state beside the
           // loaders' three register sets: saving calls keep the narrow slice there)
           if (wide && (K == 64 || !a.hs)) {
             if constexpr (K == 64) {
               if (a.hs) {
-                hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS_WIDE, true>), dim3(pairs8 * (V / Tl::BVS_WIDE)), dim3(3 * NTHR), 0, st, a);
+                hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS_WIDE, true>), dim3(pairs8 * (V / Tl::BVS_WIDE)), dim3(3 * NTHR), 0, st, a, sp);
                 break;
               }
             }
-            hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS_WIDE, false>), dim3(pairs8 * (V / Tl::BVS_WIDE)), dim3(3 * NTHR), 0, st, a);
+            hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS_WIDE, false>), dim3(pairs8 * (V / Tl::BVS_WIDE)), dim3(3 * NTHR), 0, st, a, sp);
             break;
           }
         }
-        if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a);
-        else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a);
+        if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
+        else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
         break;
       }
       if (wide) hipLaunchKernelGGL((k_gla_state_fwd<T, GT, K, V, Tl::BVS_WIDE>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS_WIDE)), block, 0, st, a);
@@ -50,10 +72,16 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
       break;
     case ST_OUT_FWD:
       hipLaunchKernelGGL((k_gla_out_fwd<T, GT, K, V, Tl::BVO>), dim3(a.NT, a.H, V / Tl::BVO), block, 0, st, a); break;
-    case ST_STATE_BWD:
-      if (wide) hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS_WIDE>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS_WIDE)), block, 0, st, a);
-      else hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a);
+    case ST_STATE_BWD: {
+      if (wide) {
+        hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS_WIDE>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS_WIDE)), block, 0, st, a, Split{});
+        break;
+      }
+      Split sp = {};
+      if constexpr (sizeof(T) == 2) sp = launch_gla_seg<T, K, V, true>(a, st);
+      hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS>), dim3((pass_items(a, sp) * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a, sp);
       break;
+    }
     case ST_DV:
       hipLaunchKernelGGL((k_gla_bwd_dv<T, GT, K, V, Tl::BVO>), dim3(a.NT, a.H, V / Tl::BVO), block, 0, st, a); break;
     case ST_DQK:

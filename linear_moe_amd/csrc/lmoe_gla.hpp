@@ -19,7 +19,7 @@
 // those parts into products of scaled tiles on MFMA, like every other product here.
 #pragma once
 #include <type_traits>
-#include "lmoe_seq.hpp"
+#include "lmoe_split.hpp"
 
 namespace lmoe {
 
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_fwd(const lmoe_args a) {
 // window before (see k_state_fwd_b).
 // ------------------------------------------------------------------------- //
 template <typename T, int K, int V, int BV, bool SAVE>
-__global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a) {
+__global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a, const Split sp) {
   static_assert(sizeof(T) == 2, "2-byte elements");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16, KS = K / 32, CS = CH / 32;
@@ -425,9 +425,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a) {
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = (jj % NVS) * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  constexpr bool CUT = BV < 64;      // wide slices fill the CUs: never cut along T
+  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  const int v0 = (jj % NVS) * BV, h = pair % a.H;
+  const PassItem part = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const int n = part.n;
+  const SeqInfo sq = part.sq;
   const int l = lane_id();
   // (wave-uniform by construction; said to the compiler, so that the branches on it are scalar branches: a matrix
   // instruction runs whatever the lane mask, and a short masked region is not jumped over)
@@ -603,6 +606,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[mi][ni][i] = h0[(int64_t)(krow0 + acc_row(mi, i)) * V + v0 + acc_col(ni)];
   }
+  if (CUT && !part.first) {
+    const int nch = (a.T + CH - 1) / CH;
+    const int64_t o = (int64_t)n * seg_count(nch, sp.len1) * a.H + h;      // the first of the fine segments in front
+    seg_prefix_rows<K, V>(S, sp.Q + (o * V + v0 + acc_col(0)) * K + krow0 + acc_row(0, 0), sp.D + o * K + krow0 + acc_row(0, 0),
+                          a.H, (sq.chunk0 - n * nch) / sp.len1, 1);
+  }
   auto copy_state = [&](int buf) {          // S -> LDS as S^T
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)
@@ -645,7 +654,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a) {
       preread(c + 1);
     }
   }
-  if (a.ht) {
+  if (a.ht && part.last) {
     float* ht = a.ht + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)
@@ -722,7 +731,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_out_fwd(const lmoe_args a) {
 // reverse state pass, 1-D grid (XCD-aware, see k_gla_state_fwd)
 // ------------------------------------------------------------------------- //
 template <typename T, typename GT, int K, int V, int BV>
-__global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a) {
+__global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
   __shared__ __attribute__((aligned(16))) T s_q[CH * LDK];     // q e^{b}             [64][K]
@@ -733,9 +742,12 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a) {
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int pair = (jj / NVS) * 8 + xcd;
-  if (pair >= a.N * a.H) return;
-  const int v0 = (jj % NVS) * BV, h = pair % a.H, n = seq_at(a, pair / a.H);
-  const SeqInfo sq = seq_info(a, n);
+  constexpr bool CUT = sizeof(T) == 2 && BV < 64;      // wide slices fill the CUs: never cut along T
+  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  const int v0 = (jj % NVS) * BV, h = pair % a.H;
+  const PassItem part = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const int n = part.n;
+  const SeqInfo sq = part.sq;
   const int wv = wave_id();
   const int krow0 = wv * (K / 4);
   f32x4 dS[MB][NB];
@@ -748,6 +760,13 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a) {
       for (int ni = 0; ni < NB; ++ni)
 #pragma unroll
         for (int i = 0; i < 4; ++i) dS[mi][ni][i] = p[(int64_t)(krow0 + acc_row(mi, i)) * V + v0 + acc_col(ni)];
+  }
+  if (CUT && !part.last) {
+    const int nch = (a.T + CH - 1) / CH, nfs = seg_count(nch, sp.len1);
+    const int nf = nfs - (sq.chunk0 - n * nch + sp.len3) / sp.len1;        // fine segments behind
+    const int64_t o = (int64_t)((n + 1) * nfs - 1) * a.H + h;              // the last one
+    seg_prefix_rows<K, V>(dS, sp.Q + (o * V + v0 + acc_col(0)) * K + krow0 + acc_row(0, 0), sp.D + o * K + krow0 + acc_row(0, 0),
+                          a.H, nf, -1);
   }
   typedef TileIO<T, CH, K> IOK;
   typedef TileIO<T, CH, BV> IOV;
@@ -814,7 +833,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a) {
       lds_barrier();
     }
   }
-  if (a.dh0) {
+  if (a.dh0 && part.first) {
     float* p = a.dh0 + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi)

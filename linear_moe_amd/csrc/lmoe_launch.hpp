@@ -50,6 +50,7 @@ void launch_state_fwd(const lmoe_args& a, hipStream_t st);        // chunk_simpl
 struct Split;
 Split launch_scalar_seg(const lmoe_args& a, bool bwd, hipStream_t st);
 int64_t scalar_split_floats(const lmoe_args& a);                  // fp32 numbers of lmoe_args.seg_ws, as split_floats
+int64_t gla_split_floats(const lmoe_args& a);                     // the same for chunk_gla
 // traced forward pass of chunk_simple_gla (bf16, K = V = 128, forward-only): false when the problem is not of that shape
 bool launch_state_fwd_trace(const lmoe_args& a, long long* tr, int work_group, hipStream_t st);
 void launch_gdn_state_fwd(const lmoe_args& a, hipStream_t st);    // gated delta rule

@@ -20,7 +20,7 @@ struct Split {
   int32_t n1, n3;        // segments of all sequences (packed input: upper bounds; a segment beyond the true count ends at once)
   bf16 *P, *PT;          // [n1][H][K][K]  transitions of the fine segments less their decay (delta rule), in operand order, and
                          // the same transposed (kept for the backward; NULL in a call that keeps nothing)
-  float *D, *DT;         // [n1][H]        decays of the fine segments (beside P, PT)
+  float *D, *DT;         // [n1][H]        decays of the fine segments (beside P, PT); chunk_gla: [n1][H][K]
   float* Q;              // [n1][H][K][V]  their contributions
   float* S;              // [n3][H][K][V]  state (gradient) a coarse segment starts from
   float* Z;              // [n1][H][K]     contributions to the normaliser's column (chunk_simple_gla)
@@ -223,6 +223,19 @@ inline Split plan_split_scalar(const lmoe_args& a) {
   const float c3 = f4 ? 1.9f + 4.1f * w : 0.45f + 0.85f * w, c1 = f4 ? 1.f + 2.f * w : 0.3f + 0.6f * w;
   return plan_cut(a, c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
 }
+// The same for chunk_gla (2-byte elements, dense; a transition is one decay per state row).  The pass fetches q, k and the
+// intra-chunk matrix once per V slice of 32, so a chunk costs more the more CUs run one.  Measured, us per chunk with 64, 128,
+// 256 work-groups: K = V = 64 0.8-1.0, 1.2, 1.6, K = V = 128 1.0, 1.2-1.7, 1.8-2.2; step 1 6-9 + 1.3 per chunk (128).
+// us of pass + step 1, not cut -> cut: forward K = V = 128, T = 4096, 16 pairs 64 -> 40, T = 8192, 4 pairs 120 -> 41; K = 64,
+// V = 128, T = 8192, 8 pairs 89 -> 33 (backward 65 -> 34).  32 pairs, T = 2048, K = V = 128 in two would take 39 -> 54: not cut.
+inline Split plan_split_gla(const lmoe_args& a) {
+  if (a.N < 1 || a.T < 1 || a.cu_seqlens || a.dtype != LMOE_BF16) return Split{};
+  const int nch = (a.T + CH - 1) / CH, pairs = a.N * a.H;
+  // wide slices fill the CUs; short and very long sequences are left whole, as above
+  if ((int64_t)pairs * (a.V / 64) >= cu_count() || nch < 17 || nch > SPLIT_MAX_CHUNKS) return Split{};
+  const float w = (a.K + a.V) / 256.f;
+  return plan_cut(a, 0.35f + 0.4f * w, 0.6f + 0.4f * w, 0.4f + 0.8f * w, 0.5f * w, (int64_t)pairs * (a.V / 32), pairs);
+}
 // S <- D S + Q over the n fine segments in front of a coarse one, in order (step = -1: behind it, from the last on).
 // q, d: Q (its column v0 + lane % 16, row krow0 + 4 (lane / 16)) and D of the first; four segments' loads at a time.
 template <int K, int V, int MB, int NB>
@@ -257,6 +270,33 @@ template <int K, int MB> __device__ __forceinline__ void seg_prefix_z(f32x4 (&z)
   for (int i = 0; i < n; ++i)
 #pragma unroll
     for (int mi = 0; mi < MB; ++mi) z[mi] += *(const f32x4*)(p + i * zs + 16 * mi);
+}
+// chunk_gla: a decay per state row (d: D at row krow0 + 4 (lane / 16) of the first segment)
+template <int K, int V, int MB, int NB>
+__device__ __forceinline__ void seg_prefix_rows(f32x4 (&S)[MB][NB], const float* q, const float* d, int H, int n, int step) {
+  const int64_t qs = (int64_t)step * H * V * K, ds = (int64_t)step * H * K;
+  for (int i0 = 0; i0 < n; i0 += 4) {
+    f32x4 x[4][MB][NB], dec[4][MB];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = min(i0 + u, n - 1);
+#pragma unroll
+      for (int mi = 0; mi < MB; ++mi) {
+        dec[u][mi] = *(const f32x4*)(d + i * ds + 16 * mi);
+#pragma unroll
+        for (int ni = 0; ni < NB; ++ni) x[u][mi][ni] = *(const f32x4*)(q + i * qs + 16 * ni * K + 16 * mi);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i0 + u < n) {
+#pragma unroll
+        for (int mi = 0; mi < MB; ++mi)
+#pragma unroll
+          for (int ni = 0; ni < NB; ++ni) S[mi][ni] = S[mi][ni] * dec[u][mi] + x[u][mi][ni];
+      }
+    }
+  }
 }
 __host__ __device__ inline int pass_items(const lmoe_args& a, const Split& sp) { return sp.len3 ? sp.n3 : a.N; }
 

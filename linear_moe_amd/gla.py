@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    no_tokens, ptr, stash, stream_ptr, unstash)
+                    cut_workspace, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class GLACall:
@@ -60,9 +60,10 @@ class GLACall:
         gdec = torch.empty(max(plan.NT, 1), H, K, dtype=torch.float32, device=dev)
         a.o, a.ht, a.hs, a.amat = _desc(o, head_first), ptr(ht), ptr(hs), amat.data_ptr()
         a.qe, a.ke, a.gcum = qe.data_ptr(), ke.data_ptr(), gdec.data_ptr()
+        seg_ws = cut_workspace(lib, a, self.OP, dev)
         _lib.check(lib.lmoe_chunk_gla_fwd(C.byref(a), stream_ptr()), "chunk_gla forward")
         self.saved = (q, k, v, g, h0, hs, amat, qe, ke, gdec)
-        self.fwd_args, self.fwd_keep = a, ((o, ht) if self.keep else None)
+        self.fwd_args, self.fwd_keep = a, ((o, ht, seg_ws) if self.keep else None)
         self.plan, self.dims, self.head_first, self.scale = plan, dims, head_first, scale
         self.has_h0 = initial_state is not None
         return o, ht
@@ -87,9 +88,10 @@ class GLACall:
         a.dh0 = ptr(dh0)
         dhs = torch.empty_like(hs)
         a.dhs = dhs.data_ptr()
+        seg_ws = cut_workspace(lib, a, self.OP, q.device)
         _lib.check(lib.lmoe_chunk_gla_bwd(C.byref(a), stream_ptr()), "chunk_gla backward")
         self.bwd_args = a
-        self.bwd_keep = (do, dht, dq, dk, dv, dg, dh0, dhs) if self.keep else None
+        self.bwd_keep = (do, dht, dq, dk, dv, dg, dh0, dhs, seg_ws) if self.keep else None
         return dq, dk, dv, dg, dh0
 
 

@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    no_tokens, ptr, stash, stream_ptr, unstash)
+                    cut_workspace, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class SimpleGLACall:
@@ -69,7 +69,7 @@ class SimpleGLACall:
             den = torch.empty((B, H, T) if head_first else (B, T, H), dtype=torch.float32, device=q.device)
             zs = torch.empty(max(plan.NT, 1), H, K, dtype=torch.float32, device=q.device) if save else None
             a.normalize, a.norm_eps, a.den, a.zs = (2 if emit_den else 1), norm_eps, _desc(den, head_first), ptr(zs)
-        seg_ws = self._cut(lib, a, q.device)
+        seg_ws = cut_workspace(lib, a, self.OP, q.device)
         _lib.check(lib.lmoe_chunk_simple_gla_fwd(C.byref(a), stream_ptr()), "chunk_simple_gla forward")
         # (emit_den: den belongs to the caller, the backward does not read it)
         ctx.saved = (q, k, v, g, h0, hs, None if emit_den else den, zs)
@@ -79,15 +79,6 @@ class SimpleGLACall:
         ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, dims, head_first, scale
         ctx.has_h0 = initial_state is not None
         return o, ht
-
-    def _cut(self, lib, a, dev):
-        """The workspace of a call whose sequences are cut along T (``lmoe_args.seg_ws``), or None."""
-        n = lib.lmoe_split_floats(C.byref(a), self.OP, 1)
-        if n <= 0:
-            return None
-        ws = torch.empty(n, dtype=torch.float32, device=dev)
-        a.seg_ws = ws.data_ptr()
-        return ws
 
     def backward(self, do, dht, o=None, dden=None):
         """o: the output of the forward call, for a call with norm_eps (handed in by the caller, who holds it: this
@@ -131,7 +122,7 @@ class SimpleGLACall:
             else:
                 o = _aligned(o)
                 a.normalize, a.den, a.o = 1, _desc(den, head_first), _desc(o, head_first)
-        seg_ws = self._cut(lib, a, q.device)
+        seg_ws = cut_workspace(lib, a, self.OP, q.device)
         _lib.check(lib.lmoe_chunk_simple_gla_bwd(C.byref(a), stream_ptr()), "chunk_simple_gla backward")
         ctx.bwd_args = a
         ctx.bwd_keep = (do, dht, dq, dk, dv, dg, dh0, dhs, norm_ws, o, dden, seg_ws) if self.keep else None

@@ -89,6 +89,27 @@ def test_simple_gla_cut_along_t(cuda, dtype, B, T, H, K, V, gated):
           ins, do, dht, cuda, dtype)
 
 
+@pytest.mark.parametrize("B,T,H,K,V", [
+    (1, 2049, 2, 128, 128),                        # last chunk, and last segment, of one token
+    (2, 2304, 1, 64, 64),                          # whole chunks
+    (1, 2400, 2, 64, 128),
+    (2, 3000, 2, 128, 64),
+])
+@pytest.mark.parametrize("head_first", [True, False])
+def test_gla_cut_along_t(cuda, B, T, H, K, V, head_first):
+    from linear_moe_amd import chunk_gla
+    assert is_cut(1, B, T, H, K, V)
+    tr = lambda x: x.transpose(1, 2) if head_first else x
+    ins = dict(q=gen(7300, B, T, H, K).bfloat16(), k=(gen(7301, B, T, H, K) * K ** -0.5).bfloat16(),
+               v=gen(7302, B, T, H, V).bfloat16(), g=F.logsigmoid(gen(7303, B, T, H, K)) * 0.01, h0=gen(7305, B, H, K, V) * 0.3)
+    do, dht = gen(7306, B, T, H, V).bfloat16(), gen(7307, B, H, K, V)
+
+    def ours(q, k, v, g, h0):
+        o, ht = chunk_gla(tr(q), tr(k), tr(v), tr(g), None, h0, True, None, head_first)
+        return tr(o), ht
+    check(lambda q, k, v, g, h0: naive.naive_recurrent_gla(q, k, v, g, None, h0, True, None, False), ours, ins, do, dht, cuda)
+
+
 @pytest.mark.parametrize("B,T,H,K,V", [(1, 1281, 2, 128, 128), (2, 1500, 1, 64, 64), (1, 2000, 2, 64, 128),
                                        (1, 1500, 2, 256, 64)])      # two key blocks: the divisor formed outside
 def test_normalised_linear_attention_cut_along_t(cuda, B, T, H, K, V):
