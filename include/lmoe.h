@@ -93,7 +93,7 @@ typedef struct lmoe_args {
   /* backward outputs */
   lmoe_tensor dq, dk, dv; /* same shapes as q,k,v, element type = dtype                */
   lmoe_tensor dg;      /* shape of g; fp32, except chunk_gla: element type of g (g_dtype) */
-  lmoe_tensor dbeta;   /* fp32, shape of beta                                          */
+  lmoe_tensor dbeta;   /* shape of beta; fp32, or bf16 with dbeta_bf16                 */
   float* dh0;          /* [N,H,K,V] fp32 or NULL                                       */
   /* backward workspace (caller-allocated, element type = dtype) */
   void* dhs;           /* gradient w.r.t. the state at the END of every chunk, laid out as hs */
@@ -146,6 +146,7 @@ typedef struct lmoe_args {
    * in fla, which runs one program per (sequence, head, block of the state) whatever their number. */
   float* seg_p;
   float* seg_ws;
+  int32_t dbeta_bf16;  /* element type of dbeta: 0 fp32, 1 bf16 (rounded once, on its way to memory) */
 } lmoe_args;
 
 /* Library version (major*10000 + minor*100 + patch). */

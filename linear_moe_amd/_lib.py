@@ -43,7 +43,7 @@ class Args(C.Structure):
         ("normalize", C.c_int32), ("norm_eps", C.c_float), ("den", Tensor4), ("zs", C.c_void_p),
         ("norm_ws", C.c_void_p), ("v_act", C.c_int32), ("dden", Tensor4),
         ("q_raw", Tensor4), ("k_raw", Tensor4), ("qk_eps", C.c_float),
-        ("seg_p", C.c_void_p), ("seg_ws", C.c_void_p),
+        ("seg_p", C.c_void_p), ("seg_ws", C.c_void_p), ("dbeta_bf16", C.c_int32),
     ]
 
 

@@ -583,7 +583,10 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
       const int j = fresh_index(threadIdx.x) & 63;
       float x = 0.f;
       if (j < ci.len) {
-        ((float*)a.dbeta.ptr)[row_off(a.dbeta, ci.b, ci.tok + j, h)] = s_dbeta[0][j] + s_dbeta[1][j] + s_dbv[j];
+        const float y = s_dbeta[0][j] + s_dbeta[1][j] + s_dbv[j];
+        const int64_t at = row_off(a.dbeta, ci.b, ci.tok + j, h);
+        if (a.dbeta_bf16) ((bf16*)a.dbeta.ptr)[at] = (bf16)y;
+        else ((float*)a.dbeta.ptr)[at] = y;
         x = s_db[0][j] + s_db[1][j];
         // last-row term; rows past the end of a partial chunk carry zero q, k, so the term may sit
         // on the last valid row without changing the reverse cumulative sum

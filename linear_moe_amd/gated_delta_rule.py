@@ -150,7 +150,9 @@ class GDNCall:
                     raise ValueError("qk_raw: the shapes and dtype of q, k, 16-byte aligned rows, a contiguous last dimension")
             a.q_raw, a.k_raw, a.qk_eps = _desc(q_raw, head_first), _desc(k_raw, head_first), float(qk_eps)
         dg = torch.empty(beta.shape, dtype=torch.float32, device=dev)
-        dbeta = torch.empty(beta.shape, dtype=torch.float32, device=dev)
+        # (rounded to the type of beta by the kernel that forms it: a conversion pass cost a launch)
+        dbeta = torch.empty(beta.shape, dtype=torch.bfloat16 if beta.dtype == torch.bfloat16 else torch.float32, device=dev)
+        a.dbeta_bf16 = int(dbeta.dtype == torch.bfloat16)
         a.dg, a.dbeta = _desc(dg, head_first), _desc(dbeta, head_first)
         dh0 = torch.empty_like(h0) if ctx.has_h0 else None
         a.dh0 = ptr(dh0)
