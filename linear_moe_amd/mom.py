@@ -87,6 +87,7 @@ def _plan_native(sel, B, S, topk, num_memories, capacity):
         return None
     if sel.dtype not in (torch.int32, torch.int64):
         sel = sel.to(torch.int64)
+    sel = sel.contiguous()                             # (a flattened slice or expanded tensor keeps its stride)
     seqs = num_memories * B
     wide = torch.empty(num_memories + 2, dtype=torch.int64, device=dev)
     counts, cu, src_token, src_choice, row_of = (torch.empty(k, dtype=torch.int32, device=dev)

@@ -45,6 +45,22 @@ def test_routing_tables(cuda, B, S, topk, E, capacity):
             assert x.dtype == y.dtype and torch.equal(x.cpu(), y), name
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_routing_tables_of_views(cuda, dtype):
+    """Choices that flatten to a view with a stride: one column of wider choices, one choice for all tokens."""
+    from linear_moe_amd.mom import _plan_by_sorting, mom_plan
+    B, S, E = 2, 300, 4
+    sel = torch.topk(torch.rand(B, S, E, generator=torch.Generator().manual_seed(8)), 2, dim=-1).indices.to(dtype)
+    wide = sel.to(cuda)
+    for s, x in ((sel[:1, :, :1], wide[:1, :, :1]), (sel[..., 1:], wide[..., 1:]),
+                 (sel[:1, :1, :1].expand(B, S, 1), wide[:1, :1, :1].expand(B, S, 1)),
+                 (sel.transpose(0, 1), wide.transpose(0, 1))):
+        b, t, k = s.shape
+        ref, got = _plan_by_sorting(s.reshape(-1).long(), b, t, k, E, None), mom_plan(x, E)
+        for name in ("src_token", "src_choice", "row_of", "cu_seqlens", "mem_offsets_dev", "max_len_dev"):
+            assert torch.equal(getattr(got, name).cpu(), getattr(ref, name)), name
+
+
 def test_memories_out_of_range_are_dropped(cuda):
     from linear_moe_amd.mom import mom_combine, mom_pack, mom_plan
     sel = torch.tensor([[[0, 9], [-1, 1], [1, 0]]]).to(cuda)
