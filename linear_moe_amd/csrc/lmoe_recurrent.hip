@@ -24,7 +24,7 @@ constexpr int RTB = 16;     // tokens staged per block
 
 // Delta rule with lmoe_args.qk_eps > 0: the rows of q and k are divided by sqrt(sum of squares + qk_eps) as they are
 // read (use_qk_l2norm_in_kernel), in fp32 and not rounded in between: one decoded token then is one launch in place of
-// three (K = V = 128, 16 heads, one sequence: 41 -> 22 us with the host work of two more calls).
+// three (K = V = 128, 16 heads, one sequence: 49 -> 19 us with the host work of two more calls).
 __device__ __forceinline__ float group8_sum(float x) {
   x += __shfl_xor(x, 1, 64);
   x += __shfl_xor(x, 2, 64);
