@@ -165,7 +165,8 @@ int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B,
                              int32_t V, int32_t NT);
 
 /* Numbers (fp32) seg_p (part 0) and seg_ws (part 1) of this call need; 0 for both where the call is not cut.  Reads
- * dtype, B, T, H, K, V, N, NT, normalize and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op / part. */
+ * dtype, B, T, H, K, V, N, NT, normalize and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op or
+ * part and for sizes the op itself refuses. */
 int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part);
 
 /* chunk_simple_gla: S_t = e^{g_t} S_{t-1} + k_t^T v_t, o_t = scale q_t S_t, g scalar per

@@ -20,17 +20,16 @@ int fail(int code, const char* fmt, ...) {
 }
 
 // wide_v: the op has instances for K = 128, V = 256 (the gated delta rule)
-int check_common(const lmoe_args* a, const char* op, bool wide_v = false) {
+int check_shape(const lmoe_args* a, const char* op, bool wide_v) {
   if (!a) return fail(-1, "%s: null argument block", op);
   if (a->dtype != LMOE_BF16 && a->dtype != LMOE_F32) return fail(-2, "%s: dtype must be LMOE_BF16 or LMOE_F32", op);
   if (!((a->K == 64 || a->K == 128) && (a->V == 64 || a->V == 128)) && !(wide_v && a->K == 128 && a->V == 256))
     return fail(-3, "%s: head dims K=%d V=%d unsupported (K, V must be 64 or 128%s)", op, a->K, a->V,
                 wide_v ? "; or K = 128 with V = 256" : "");
   if (a->B < 0 || a->T < 0 || a->H <= 0 || a->N < 0 || a->NT < 0) return fail(-4, "%s: negative dimension", op);
-  if (a->cu_seqlens && (a->B != 1 || !a->chunk_map || !a->seq_chunk0))
-    return fail(-5, "%s: packed input needs B == 1, chunk_map and seq_chunk0", op);
-  if (!a->cu_seqlens && a->N != a->B) return fail(-6, "%s: dense input needs N == B", op);
-  if (!a->q.ptr || !a->k.ptr || !a->v.ptr) return fail(-7, "%s: q, k, v must not be null", op);
+  return 0;
+}
+int check_counts(const lmoe_args* a, const char* op) {
   if (a->H > 65535 || a->N > 65535) return fail(-8, "%s: H and N must be <= 65535", op);
   // The kernels derive every address from these numbers: a chunk count that does not belong to B and T would send
   // them past the end of the inputs, rows that are not 16-byte aligned break their 16-byte accesses.
@@ -41,6 +40,15 @@ int check_common(const lmoe_args* a, const char* op, bool wide_v = false) {
   if (a->cu_seqlens && (int64_t)a->NT > per_row + a->N)
     return fail(-4, "%s: packed input of T=%d, N=%d has at most %lld chunks, NT=%d given", op, a->T, a->N,
                 (long long)(per_row + a->N), a->NT);
+  return 0;
+}
+int check_common(const lmoe_args* a, const char* op, bool wide_v = false) {
+  if (int r = check_shape(a, op, wide_v)) return r;
+  if (a->cu_seqlens && (a->B != 1 || !a->chunk_map || !a->seq_chunk0))
+    return fail(-5, "%s: packed input needs B == 1, chunk_map and seq_chunk0", op);
+  if (!a->cu_seqlens && a->N != a->B) return fail(-6, "%s: dense input needs N == B", op);
+  if (!a->q.ptr || !a->k.ptr || !a->v.ptr) return fail(-7, "%s: q, k, v must not be null", op);
+  if (int r = check_counts(a, op)) return r;
   const int64_t vec = a->dtype == LMOE_BF16 ? 8 : 4;            // elements per 16 bytes
   const lmoe_tensor* rows[] = {&a->q, &a->k, &a->v, &a->o, &a->d_o, &a->dq, &a->dk, &a->dv, &a->q_raw, &a->k_raw};
   for (const lmoe_tensor* t : rows)
@@ -103,6 +111,11 @@ int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part) {
   if (!a) return fail(-1, "%s: null argument block", nm);
   if (op != LMOE_OP_SIMPLE_GLA && op != LMOE_OP_GLA && op != LMOE_OP_GATED_DELTA_RULE) return fail(-21, "%s: unknown op %d", nm, op);
   if (part != 0 && part != 1) return fail(-22, "%s: part must be 0 (seg_p) or 1 (seg_ws)", nm);
+  // (asked before the op itself has seen the block: the rule divides by what these refuse)
+  if (int r = check_shape(a, nm, op == LMOE_OP_GATED_DELTA_RULE)) return r;
+  if (a->cu_seqlens && a->B != 1) return fail(-5, "%s: packed input needs B == 1", nm);
+  if (!a->cu_seqlens && a->N != a->B) return fail(-6, "%s: dense input needs N == B", nm);
+  if (int r = check_counts(a, nm)) return r;
   return lmoe::split_floats(*a, op, part);
 }
 

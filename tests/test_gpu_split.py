@@ -128,3 +128,15 @@ def test_normalised_linear_attention_cut_along_t(cuda, B, T, H, K, V):
     torch.cuda.synchronize()
     for x, r in zip((o.detach(),) + grads, (ref.detach(),) + refs):
         assert max_abs_rel(x.cpu(), r) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_calls_without_heads_are_refused(cuda, dtype):
+    """The rule of the cut sees a call before the op's checks do; the call still ends in the op's error."""
+    from linear_moe_amd import chunk_gated_delta_rule, chunk_gla, chunk_simple_gla
+    x, s = torch.empty(1, 3000, 0, 64, device=cuda, dtype=dtype), torch.empty(1, 3000, 0, device=cuda)
+    for fn in (lambda: chunk_gated_delta_rule(x, x, x, s, s.to(dtype), head_first=False),
+               lambda: chunk_simple_gla(x, x, x, s, head_first=False),
+               lambda: chunk_gla(x, x, x, x.float(), head_first=False)):
+        with pytest.raises(ValueError, match="dimension"):
+            fn()

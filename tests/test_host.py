@@ -130,6 +130,34 @@ def test_chunk_count_and_row_alignment_are_checked_before_any_launch():
     assert lib.lmoe_chunk_simple_gla_bwd(C.byref(f32), None) == -11                     # (passes on to the next check)
 
 
+def test_the_cut_along_t_refuses_the_sizes_the_op_refuses():
+    """lmoe_split_floats is asked before the op's own checks have run: no heads, head dimensions without an instance and
+    counts that do not fit each other get the op's error code, nothing is computed from them."""
+    from linear_moe_amd import _lib
+    lib = _lib.load()
+    fake = 0x1000                                  # never dereferenced: every call below is refused
+
+    def args(**kw):
+        a = _lib.Args()
+        a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_BF16, 1, 3000, 2, 128, 128, 1, 47
+        for n in ("q", "k", "v", "o", "g", "beta"):
+            setattr(a, n, _lib.Tensor4(fake, 3000 * 256, 256, 128))
+        for n, x in kw.items():
+            setattr(a, n, x)
+        return a
+
+    assert all(lib.lmoe_split_floats(C.byref(args()), op, 1) > 0 for op in (0, 1, 2))
+    packed = dict(cu_seqlens=fake, chunk_map=fake, seq_chunk0=fake)
+    bad = [dict(H=0), dict(H=-1), dict(V=16), dict(V=0), dict(K=0), dict(K=48), dict(dtype=7), dict(T=-1), dict(N=2),
+           dict(H=70000), dict(NT=48), dict(NT=-1), dict(B=2, **packed), dict(NT=49, **packed)]
+    for op, name in enumerate(("simple_gla", "gla", "gated_delta_rule")):
+        for kw in bad:
+            rc = getattr(lib, f"lmoe_chunk_{name}_fwd")(C.byref(args(**kw)), None)
+            assert rc < 0, (name, kw)
+            assert [lib.lmoe_split_floats(C.byref(args(**kw)), op, part) for part in (0, 1)] == [rc, rc], (name, kw)
+    assert lib.lmoe_split_floats(C.byref(args()), 3, 1) == -21 and lib.lmoe_split_floats(C.byref(args()), 2, 2) == -22
+
+
 def test_options_outside_flas_signature_are_validated_before_any_launch():
     """V = 256 belongs to the gated delta rule alone (2-byte calls then need tinv); normalize belongs to ungated 2-byte
     calls of chunk_simple_gla and names the buffers it needs; v_act needs 2-byte elements and tinv.  Calls without
