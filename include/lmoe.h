@@ -166,8 +166,11 @@ int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B,
 
 /* Numbers (fp32) seg_p (part 0) and seg_ws (part 1) of this call need; 0 for both where the call is not cut.  Reads
  * dtype, B, T, H, K, V, N, NT, normalize and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op or
- * part and for sizes the op itself refuses. */
+ * part and for sizes the op itself refuses.  What is cut depends on T, N, H, K, V, the type, normalize and whether the input
+ * is packed, not on where the offsets of packed input lie. */
 int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part);
+/* How the same call is cut: chunks per segment of the state-only step and of the ordinary pass (a multiple of it); 0, 0: whole. */
+int lmoe_split_lengths(const lmoe_args* a, int32_t op, int32_t* fine, int32_t* coarse);
 
 /* chunk_simple_gla: S_t = e^{g_t} S_{t-1} + k_t^T v_t, o_t = scale q_t S_t, g scalar per
  * token-head (gate = SCALAR) or absent (gate = NONE).

@@ -52,7 +52,7 @@ ENTRY_POINTS = (
     "lmoe_chunk_simple_gla_fwd", "lmoe_chunk_simple_gla_bwd",
     "lmoe_chunk_gla_fwd", "lmoe_chunk_gla_bwd",
     "lmoe_chunk_gated_delta_rule_fwd", "lmoe_chunk_gated_delta_rule_bwd",
-    "lmoe_launch_stage", "lmoe_selftest_gemm", "lmoe_workspace_bytes", "lmoe_split_floats", "lmoe_l2norm_fwd", "lmoe_l2norm_bwd",
+    "lmoe_launch_stage", "lmoe_selftest_gemm", "lmoe_workspace_bytes", "lmoe_split_floats", "lmoe_split_lengths", "lmoe_l2norm_fwd", "lmoe_l2norm_bwd",
     "lmoe_silu_l2norm_fwd", "lmoe_silu_l2norm_bwd", "lmoe_gdn_qkv_prologue_fwd", "lmoe_gdn_qkv_prologue_bwd",
     "lmoe_swish_gate_relayout_fwd", "lmoe_swish_gate_relayout_bwd", "lmoe_rmsnorm_partials", "lmoe_rmsnorm_fwd", "lmoe_rmsnorm_bwd", "lmoe_rmsnorm_bwd_noalloc",
     "lmoe_gdn_gates_partials", "lmoe_gdn_gates_fwd", "lmoe_gdn_gates_bwd", "lmoe_gla_gate_fwd", "lmoe_gla_gate_bwd",
@@ -156,6 +156,8 @@ def load() -> C.CDLL:
     lib.lmoe_seq_tables.restype = C.c_int
     lib.lmoe_split_floats.argtypes = [C.POINTER(Args), C.c_int32, C.c_int32]
     lib.lmoe_split_floats.restype = C.c_int64
+    lib.lmoe_split_lengths.argtypes = [C.POINTER(Args), C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
+    lib.lmoe_split_lengths.restype = C.c_int
     lib.lmoe_workspace_bytes.argtypes = [C.c_int32] * 9
     lib.lmoe_workspace_bytes.restype = C.c_int64
     _lib = lib

@@ -106,17 +106,27 @@ int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B,
   return bytes;
 }
 
-int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part) {
-  const char* nm = "lmoe_split_floats";
+// (asked before the op itself has seen the block: the rule divides by what these checks refuse)
+static int check_split(const char* nm, const lmoe_args* a, int32_t op) {
   if (!a) return fail(-1, "%s: null argument block", nm);
   if (op != LMOE_OP_SIMPLE_GLA && op != LMOE_OP_GLA && op != LMOE_OP_GATED_DELTA_RULE) return fail(-21, "%s: unknown op %d", nm, op);
-  if (part != 0 && part != 1) return fail(-22, "%s: part must be 0 (seg_p) or 1 (seg_ws)", nm);
-  // (asked before the op itself has seen the block: the rule divides by what these refuse)
   if (int r = check_shape(a, nm, op == LMOE_OP_GATED_DELTA_RULE)) return r;
   if (a->cu_seqlens && a->B != 1) return fail(-5, "%s: packed input needs B == 1", nm);
   if (!a->cu_seqlens && a->N != a->B) return fail(-6, "%s: dense input needs N == B", nm);
-  if (int r = check_counts(a, nm)) return r;
+  return check_counts(a, nm);
+}
+int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part) {
+  const char* nm = "lmoe_split_floats";
+  if (int r = check_split(nm, a, op)) return r;
+  if (part != 0 && part != 1) return fail(-22, "%s: part must be 0 (seg_p) or 1 (seg_ws)", nm);
   return lmoe::split_floats(*a, op, part);
+}
+int lmoe_split_lengths(const lmoe_args* a, int32_t op, int32_t* fine, int32_t* coarse) {
+  const char* nm = "lmoe_split_lengths";
+  if (int r = check_split(nm, a, op)) return r;
+  if (!fine || !coarse) return fail(-1, "%s: null pointer", nm);
+  lmoe::split_lengths(*a, op, fine, coarse);
+  return 0;
 }
 
 int lmoe_chunk_simple_gla_fwd(const lmoe_args* a, void* stream) {

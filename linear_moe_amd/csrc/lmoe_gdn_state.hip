@@ -108,6 +108,11 @@ bool launch_gdn_state_fwd_trace(const lmoe_args& a, long long* tr, int work_grou
   hipLaunchKernelGGL((k_gdn_state_fwd_reg<128, 128, true, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, Split{}, tr, work_group);
   return true;
 }
+void split_lengths(const lmoe_args& a, int op, int32_t* fine, int32_t* coarse) {
+  const Split sp = op == LMOE_OP_SIMPLE_GLA ? plan_split_scalar(a) : op == LMOE_OP_GLA ? plan_split_gla(a) : gdn_split_plan(a);
+  *fine = sp.len1;
+  *coarse = sp.len3;
+}
 int64_t split_floats(const lmoe_args& a, int op, int part) {
   if (op == LMOE_OP_SIMPLE_GLA && part == 1) return scalar_split_floats(a);
   if (op == LMOE_OP_GLA && part == 1) return gla_split_floats(a);

@@ -57,6 +57,7 @@ void launch_gdn_state_fwd(const lmoe_args& a, hipStream_t st);    // gated delta
 void launch_gdn_state_bwd(const lmoe_args& a, hipStream_t st);
 // fp32 numbers of lmoe_args.seg_p (part 0) / seg_ws (part 1); 0: the call is not cut along T
 int64_t split_floats(const lmoe_args& a, int op, int part);
+void split_lengths(const lmoe_args& a, int op, int32_t* fine, int32_t* coarse);      // chunks per segment, 0: not cut
 // traced forward pass (bf16, K = V = 128, Tinv and hs given): false when the problem is not of that shape
 bool launch_gdn_state_fwd_trace(const lmoe_args& a, long long* tr, int work_group, hipStream_t st);
 void launch_gdn_wy_fwd(const lmoe_args& a, hipStream_t st);

@@ -149,9 +149,11 @@ inline Split plan_split(const lmoe_args& a, int slices) {
   // at least three coarse segments each: with two, the longest sequence that gained (256 chunks, 32 pairs) took 0.8 of
   // the time, most 0.9 and more
   if (slots < 3 * a.N) return s;
-  const bool packed = a.cu_seqlens != nullptr;                    // (the lengths are not known here: as if they were equal)
-  const int nch = packed ? (a.NT + a.N - 1) / a.N : (a.T + CH - 1) / CH;
-  if (nch < SPLIT_MIN_CHUNKS || a.NT > a.N * SPLIT_MAX_CHUNKS) return s;
+  // Packed: the lengths are not known here, as if they were equal.  T and N alone decide: NT is the chunk count where the
+  // offsets lie on the host and a bound where they lie on the device, and a batch gives the same bits either way.
+  const bool packed = a.cu_seqlens != nullptr;
+  const int nch = seg_count(seg_count(a.T, CH), packed ? a.N : 1);
+  if (nch < SPLIT_MIN_CHUNKS || nch > SPLIT_MAX_CHUNKS) return s;
   const float w = (a.K + a.V) / 256.f;
   float best = 0.9f * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
   // packed: sum over the sequences of ceil(chunks / len3) <= NT / len3 + N segments

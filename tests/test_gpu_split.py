@@ -65,6 +65,26 @@ def test_gated_delta_rule_cut_along_t(cuda, B, T, H, K, V, lens):
           ins, do, dht, cuda)
 
 
+@pytest.mark.parametrize("lens,H", [([4096], 4), ([1472], 2), ([5000, 0, 1000, 1000], 2), ([2100, 1996], 4)])
+def test_offsets_on_the_device_are_cut_as_those_on_the_host(cuda, lens, H):
+    """Where cu_seqlens lies does not show: the same bits, outputs, states and every gradient."""
+    from linear_moe_amd import chunk_gated_delta_rule
+    T, N, D = sum(lens), len(lens), 128
+    x = [F.normalize(gen(7400, 1, T, H, D), dim=-1).bfloat16(), F.normalize(gen(7401, 1, T, H, D), dim=-1).bfloat16(),
+         gen(7402, 1, T, H, D).bfloat16(), -F.softplus(gen(7403, 1, T, H)) * 0.01, torch.sigmoid(gen(7404, 1, T, H)).bfloat16()]
+    x = [t.to(cuda).requires_grad_(True) for t in x]
+    h0 = gen(7405, N, H, D, D).to(cuda).requires_grad_(True)
+    do, dht = gen(7406, 1, T, H, D).bfloat16().to(cuda), gen(7407, N, H, D, D).to(cuda)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    outs = []
+    for offs in (cu, cu.to(cuda)):
+        o, ht = chunk_gated_delta_rule(*x, None, h0, True, offs, False)
+        outs.append((o.detach(), ht.detach()) + torch.autograd.grad([o, ht], x + [h0], [do, dht]))
+    torch.cuda.synchronize()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,B,T,H,K,V", [
     (torch.bfloat16, 1, 1281, 2, 128, 128),        # last chunk, and last segment, of one token
     (torch.bfloat16, 2, 1536, 1, 64, 64),          # whole chunks

@@ -158,6 +158,41 @@ def test_the_cut_along_t_refuses_the_sizes_the_op_refuses():
     assert lib.lmoe_split_floats(C.byref(args()), 3, 1) == -21 and lib.lmoe_split_floats(C.byref(args()), 2, 2) == -22
 
 
+def test_the_cut_along_t_of_packed_input_follows_from_t_and_n():
+    """NT is the chunk count where the offsets lie on the host and a bound of it where they lie on the device: the batch
+    is cut the same way.  One packed sequence is cut as a dense one of its length."""
+    from linear_moe_amd import _lib
+    lib = _lib.load()
+
+    def lengths(T, H, D, N, NT, packed=True):
+        a = _lib.Args()
+        a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_BF16, 1, T, H, D, D, N, NT
+        a.cu_seqlens = 0x1000 if packed else None  # (only asked whether it is there)
+        fine, coarse = C.c_int32(), C.c_int32()
+        assert lib.lmoe_split_lengths(C.byref(a), 2, C.byref(fine), C.byref(coarse)) == 0
+        parts = [lib.lmoe_split_floats(C.byref(a), 2, part) for part in (0, 1)]
+        assert [p > 0 for p in parts] == [fine.value > 0] * 2
+        return fine.value, coarse.value
+
+    cut = 0
+    for T in (1472, 1473, 1537, 3001, 4096, 5000, 8192, 20001, 32768, 32769, 65536):
+        for N in (1, 2, 3, 5):
+            for H in (1, 2, 4, 16):
+                for D in (64, 128):
+                    ch = -(-T // 64)
+                    got = {lengths(T, H, D, N, nt) for nt in range(ch, ch + N + 1)}
+                    if N == 1:
+                        got.add(lengths(T, H, D, 1, ch, packed=False))
+                    assert len(got) == 1, (T, N, H, D, got)
+                    cut += got != {(0, 0)}
+    assert cut > 100
+    a = _lib.Args()
+    assert lib.lmoe_split_lengths(None, 2, None, None) == -1
+    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_BF16, 1, 64, 1, 64, 64, 1, 1
+    assert lib.lmoe_split_lengths(C.byref(a), 2, None, None) == -1
+    assert lib.lmoe_split_lengths(C.byref(a), 3, None, None) == -21
+
+
 def test_options_outside_flas_signature_are_validated_before_any_launch():
     """V = 256 belongs to the gated delta rule alone (2-byte calls then need tinv); normalize belongs to ungated 2-byte
     calls of chunk_simple_gla and names the buffers it needs; v_act needs 2-byte elements and tinv.  Calls without
