@@ -38,23 +38,25 @@ template <int K, int V> void combine(const lmoe_args& a, const Split& sp, bool b
   else hipLaunchKernelGGL((k_split_combine<K, false>), grid, block, 0, st, a, sp);
 }
 template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, hipStream_t st) {
-  int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
+  const int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
   // w formed on the chip from Tinv where Tinv is there and LDS has room for a second k tile
   constexpr bool CAN_WT = sizeof(T) == 2;
   const bool wt = CAN_WT && a.tinv != nullptr;
   if constexpr (CAN_WT && BV == 32) {
     if (wt) {       // 2-byte elements with Tinv: the state stays in registers (lmoe_gdn_state_reg.hpp)
-      Split sp = {};
       if constexpr (V <= 128) {
-        sp = gdn_split(a, false);
+        const Split sp = gdn_split(a, false);
         if (sp.len1) {
           hipLaunchKernelGGL((k_gdn_seg_fwd<K, V>), dim3(sp.n1 * a.H), dim3(SEG_FWD_THREADS), 0, st, a, sp);
           combine<K, V>(a, sp, false, st);
-          grid = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
+          const int items = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
+          if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true, false, true>), dim3(items), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
+          else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false, false, true>), dim3(items), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
+          return;
         }
       }
-      if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
-      else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
+      if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, Split{}, (long long*)nullptr, -1);
+      else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, Split{}, (long long*)nullptr, -1);
       return;
     }
   }
@@ -70,17 +72,16 @@ template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, 
   }
 }
 template <typename T, int K, int V, int BV> void launch_bwd(const lmoe_args& a, hipStream_t st) {
-  int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
-  Split sp = {};
   if constexpr (sizeof(T) == 2 && BV == 32 && V <= 128) {
-    sp = gdn_split(a, true);
+    const Split sp = gdn_split(a, true);
     if (sp.len1) {
       hipLaunchKernelGGL((k_gdn_seg_bwd<K, V>), dim3(sp.n1 * a.H), dim3(SEG_BWD_THREADS), 0, st, a, sp);
       combine<K, V>(a, sp, true, st);
-      grid = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
+      hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV, true>), dim3(((sp.n3 * a.H + 7) / 8) * 8 * (V / BV)), dim3(3 * NTHR), 0, st, a, sp);
+      return;
     }
   }
-  hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+  hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV>), dim3(((a.N * a.H + 7) / 8) * 8 * (V / BV)), dim3(3 * NTHR), 0, st, a, Split{});
 }
 template <typename T, int K, int V> struct GdnStateFwd {
   static void run(const lmoe_args& a, hipStream_t st) {

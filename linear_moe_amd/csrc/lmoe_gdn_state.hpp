@@ -414,7 +414,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd(const lmoe_args a) {
 //   consumers, chunk c: dS' -> LDS | B1 | k dS', P^T do, dv_new -> LDS | B2 | dS = e^{b_C} dS + q^T (..);
 //                      fragments of (k beta e^{b})^T | B3 | dS -= (k beta e^{b})^T dZ
 // ------------------------------------------------------------------------- //
-template <typename T, int K, int V, int BV>
+template <typename T, int K, int V, int BV, bool CUT = false>
 __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16, KS = K / 32;
@@ -437,10 +437,10 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a, c
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= (sp.len3 ? sp.n3 : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = pass_item(a, sp, pair / a.H);
-  if (item.n < 0) return;
+  const PassItem item = pass_item<CUT>(a, sp, pair / a.H);
+  if (CUT && item.n < 0) return;
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();

@@ -54,7 +54,7 @@ __device__ __forceinline__ bf16x8 load_frag_t_state(const bf16* tile, int ld, in
 }
 // (frag_of_blocks, lmoe_common.hpp: two accumulator blocks -> the 8 contraction elements of an operand)
 
-template <int K, int V, bool SAVE, bool TRACE = false>
+template <int K, int V, bool SAVE, bool TRACE = false, bool CUT = false>
 __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   typedef bf16 T;
   constexpr int BV = 32;
@@ -90,10 +90,10 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  if (pair >= (sp.len3 ? sp.n3 : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = pass_item(a, sp, pair / a.H);
-  if (item.n < 0) return;
+  const PassItem item = pass_item<CUT>(a, sp, pair / a.H);
+  if (CUT && item.n < 0) return;
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();

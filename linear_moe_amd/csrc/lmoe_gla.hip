@@ -63,6 +63,11 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
             break;
           }
         }
+        if (sp.len1) {
+          if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, true, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
+          else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
+          break;
+        }
         if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
         else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
         break;
@@ -77,9 +82,14 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
         hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS_WIDE>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS_WIDE)), block, 0, st, a, Split{});
         break;
       }
-      Split sp = {};
-      if constexpr (sizeof(T) == 2) sp = launch_gla_seg<T, K, V, true>(a, st);
-      hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS>), dim3((pass_items(a, sp) * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a, sp);
+      if constexpr (sizeof(T) == 2) {
+        const Split sp = launch_gla_seg<T, K, V, true>(a, st);
+        if (sp.len1) {
+          hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS, true>), dim3((sp.n3 * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a, sp);
+          break;
+        }
+      }
+      hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS>), dim3((a.N * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a, Split{});
       break;
     }
     case ST_DV:

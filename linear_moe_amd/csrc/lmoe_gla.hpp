@@ -411,7 +411,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_fwd(const lmoe_args a) {
 // Two buffers of every tile: what a window reads of a chunk's own operands was read into registers at the end of the
 // window before (see k_state_fwd_b).
 // ------------------------------------------------------------------------- //
-template <typename T, int K, int V, int BV, bool SAVE>
+template <typename T, int K, int V, int BV, bool SAVE, bool CUT = false>
 __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a, const Split sp) {
   static_assert(sizeof(T) == 2, "2-byte elements");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
@@ -425,10 +425,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a, c
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int pair = (jj / NVS) * 8 + xcd;
-  constexpr bool CUT = BV < 64;      // wide slices fill the CUs: never cut along T
-  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = (jj % NVS) * BV, h = pair % a.H;
-  const PassItem part = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const PassItem part = pass_item_dense<CUT>(a, sp, pair / a.H);
   const int n = part.n;
   const SeqInfo sq = part.sq;
   const int l = lane_id();
@@ -730,7 +729,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_out_fwd(const lmoe_args a) {
 // ------------------------------------------------------------------------- //
 // reverse state pass, 1-D grid (XCD-aware, see k_gla_state_fwd)
 // ------------------------------------------------------------------------- //
-template <typename T, typename GT, int K, int V, int BV>
+template <typename T, typename GT, int K, int V, int BV, bool CUT = false>
 __global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
@@ -742,10 +741,9 @@ __global__ __launch_bounds__(NTHR) void k_gla_state_bwd(const lmoe_args a, const
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int pair = (jj / NVS) * 8 + xcd;
-  constexpr bool CUT = sizeof(T) == 2 && BV < 64;      // wide slices fill the CUs: never cut along T
-  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = (jj % NVS) * BV, h = pair % a.H;
-  const PassItem part = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const PassItem part = pass_item_dense<CUT>(a, sp, pair / a.H);
   const int n = part.n;
   const SeqInfo sq = part.sq;
   const int wv = wave_id();

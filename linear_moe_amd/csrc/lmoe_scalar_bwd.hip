@@ -26,24 +26,26 @@ template <typename T, int K, int V> struct StateBwd {
     // element is the same sum over the tokens in either split
     constexpr int BW = (sizeof(T) == 2 && V >= 64) ? 64 : BV;
     if (BW != BV && (int64_t)a.N * a.H * (V / BW) >= cu_count()) {
-      launch<BW>(a, Split{}, st);
+      launch<BW, false>(a, Split{}, st);
       return;
     }
-    launch<BV>(a, launch_scalar_seg(a, true, st), st);
+    const Split sp = launch_scalar_seg(a, true, st);
+    if (sp.len1) launch<BV, true>(a, sp, st);
+    else launch<BV, false>(a, sp, st);
   }
-  template <int BVX> static void launch(const lmoe_args& a, const Split& sp, hipStream_t st) {
+  template <int BVX, bool CUT> static void launch(const lmoe_args& a, const Split& sp, hipStream_t st) {
     const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BVX)), block(2 * NTHR);
     if constexpr (sizeof(T) == 2) {        // the pass behind the normalised output exists for 2-byte elements
       if (a.normalize == 1) {
-        hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 1>), grid, block, 0, st, a, sp);
+        hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 1, CUT>), grid, block, 0, st, a, sp);
         return;
       }
       if (a.normalize == 2) {
-        hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 2>), grid, block, 0, st, a, sp);
+        hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 2, CUT>), grid, block, 0, st, a, sp);
         return;
       }
     }
-    hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX>), grid, block, 0, st, a, sp);
+    hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 0, CUT>), grid, block, 0, st, a, sp);
   }
 };
 template <typename T, int K, int V> struct BwdDqk {

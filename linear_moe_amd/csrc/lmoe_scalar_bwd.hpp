@@ -115,7 +115,7 @@ __global__ __launch_bounds__(NTHR) void k_bwd_dv(const lmoe_args a) {
 // before it divides): d_o is the gradient of o as it stands and dden comes in as a tensor; it enters once, in the first
 // V slice (the other slices carry zeros).
 constexpr int NORM_SLOT_COLS = 32;
-template <typename T, int K, int V, int BV, int NORM = 0>
+template <typename T, int K, int V, int BV, int NORM = 0, bool CUT = false>
 __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
@@ -133,10 +133,9 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
-  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const PassItem item = pass_item_dense<CUT>(a, sp, pair / a.H);
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();

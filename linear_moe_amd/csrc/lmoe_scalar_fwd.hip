@@ -55,15 +55,15 @@ Split launch_scalar_seg(const lmoe_args& a, bool bwd, hipStream_t st) {
 }
 
 // the pass for 2-byte elements on V slices of BV columns: saving or forward-only, plain or with the normalised output
-template <typename T, int K, int V, int BV> void launch_fwd_b(const lmoe_args& a, const Split& sp, hipStream_t st) {
+template <typename T, int K, int V, int BV, bool CUT> void launch_fwd_b(const lmoe_args& a, const Split& sp, hipStream_t st) {
   const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BV)), block(3 * NTHR);
   long long* const no_trace = nullptr;
   if (a.normalize) {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, true>), grid, block, 0, st, a, sp, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, true>), grid, block, 0, st, a, sp, no_trace, -1);
+    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, true, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
+    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, true, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
   } else {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true>), grid, block, 0, st, a, sp, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false>), grid, block, 0, st, a, sp, no_trace, -1);
+    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, false, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
+    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, false, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
   }
 }
 template <typename T, int K, int V> struct StateFwd {
@@ -75,16 +75,23 @@ template <typename T, int K, int V> struct StateFwd {
       // depend on the width (a state element and an output element are the same sums in either split)
       if constexpr (V >= 64) {
         if ((int64_t)a.N * a.H * (V / 64) >= cu_count()) {
-          launch_fwd_b<T, K, V, 64>(a, Split{}, st);
+          launch_fwd_b<T, K, V, 64, false>(a, Split{}, st);
           return;
         }
       }
-      launch_fwd_b<T, K, V, BV>(a, launch_scalar_seg(a, false, st), st);
+      const Split sp = launch_scalar_seg(a, false, st);
+      if (sp.len1) launch_fwd_b<T, K, V, BV, true>(a, sp, st);
+      else launch_fwd_b<T, K, V, BV, false>(a, sp, st);
     } else {
       const Split sp = launch_scalar_seg(a, false, st);
       const int grid = ((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BV);
-      if (a.hs) hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
-      else hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+      if (sp.len1) {
+        if (a.hs) hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, true, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+        else hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, false, true>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+      } else {
+        if (a.hs) hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, true, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+        else hipLaunchKernelGGL((k_state_fwd<T, K, V, BV, false, false>), dim3(grid), dim3(3 * NTHR), 0, st, a, sp);
+      }
     }
   }
 };

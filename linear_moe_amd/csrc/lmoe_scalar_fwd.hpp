@@ -35,7 +35,7 @@ template <typename T> __device__ __forceinline__ void scale_frag(typename ET<T>:
 //     P = (q k^T) . Gamma (through a wave-private LDS strip) and P v; the rows are stored after B2.
 //   All teams meet at the same barriers; three waves per SIMD hide each other's latencies.
 // ------------------------------------------------------------------------- //
-template <typename T, int K, int V, int BV, bool SAVE>
+template <typename T, int K, int V, int BV, bool SAVE, bool CUT>
 __global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a, const Split sp) {
   static_assert(sizeof(T) == 4, "fp32 elements; 2-byte elements: k_state_fwd_b");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
@@ -52,10 +52,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd(const lmoe_args a, const
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
-  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const PassItem item = pass_item_dense<CUT>(a, sp, pair / a.H);
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();
@@ -287,9 +286,10 @@ constexpr int SFWD_TRACE_CHUNKS = 24, SFWD_TRACE_MARKS = 8, SFWD_TRACE_SLOTS = 3
 // op with one more value column of ones, carried beside the state as one more accumulator column (z = the sum of the
 // keys of the chunks before, fp32 in LDS and, for the backward, in zs) and formed by every V slice for itself:
 // consumers z += k^T 1, output team q z and the row sums of P as two more products against a fragment of ones.
-template <typename T, int K, int V, int BV, bool SAVE, bool TRACE = false, bool NORM = false>
+template <typename T, int K, int V, int BV, bool SAVE, bool TRACE = false, bool NORM = false, bool CUT = false>
 __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   static_assert(sizeof(T) == 2, "2-byte elements");
+  static_assert(!CUT || BV < 64, "wide slices fill the CUs: never cut along T");
   static_assert(!(NORM && TRACE), "the traced instance is the plain pass");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16, KS = K / 32, CS = CH / 32;
@@ -328,10 +328,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
   constexpr int NVS = V / BV;
   const int xcd = blockIdx.x & 7, jj = blockIdx.x >> 3;
   const int vsl = jj % NVS, pair = (jj / NVS) * 8 + xcd;
-  constexpr bool CUT = sizeof(T) == 4 || BV < 64;      // wide slices fill the CUs: never cut along T
-  if (pair >= (CUT ? pass_items(a, sp) : a.N) * a.H) return;
+  if (pair >= (CUT ? sp.n3 : a.N) * a.H) return;
   const int v0 = vsl * BV, h = pair % a.H;
-  const PassItem item = CUT ? pass_item_dense(a, sp, pair / a.H) : pass_item_dense(a, Split{}, pair / a.H);
+  const PassItem item = pass_item_dense<CUT>(a, sp, pair / a.H);
   const int n = item.n;
   const SeqInfo sq = item.sq;
   const int l = lane_id();
