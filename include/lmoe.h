@@ -142,7 +142,7 @@ typedef struct lmoe_args {
   float qk_eps;
   /* optional fp32 buffers of lmoe_split_floats(a, op, 0 / 1) numbers for sequences cut along T (few (sequence, head)
    * pairs: the sequential passes then run over segments of the sequences at once): seg_p is written by *_fwd and read
-   * by *_bwd, seg_ws is workspace of one call.  NULL: not cut.  A cut changes results by rounding only.  No counterpart
+   * by *_bwd, seg_ws is workspace of one call; both 16-byte aligned.  NULL: not cut.  A cut changes results by rounding only.  No counterpart
    * in fla, which runs one program per (sequence, head, block of the state) whatever their number. */
   float* seg_p;
   float* seg_ws;

@@ -54,6 +54,7 @@ int check_common(const lmoe_args* a, const char* op, bool wide_v = false) {
   for (const lmoe_tensor* t : rows)
     if (t->ptr && (((uintptr_t)t->ptr & 15) || t->sb % vec || t->st % vec || t->sh % vec))
       return fail(-9, "%s: q, k, v, o and their gradients need 16-byte aligned rows (pointer and strides)", op);
+  if (((uintptr_t)a->seg_p | (uintptr_t)a->seg_ws) & 15) return fail(-9, "%s: seg_p and seg_ws must be 16-byte aligned", op);
   return 0;
 }
 

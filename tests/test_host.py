@@ -126,6 +126,10 @@ def test_chunk_count_and_row_alignment_are_checked_before_any_launch():
                 _lib.Tensor4(fake, 130 * 64 + 4, 64, 64), _lib.Tensor4(fake, 130 * 64, 64, 60)):
         for name in ("q", "k", "v", "o"):
             assert lib.lmoe_chunk_simple_gla_fwd(C.byref(args(**{name: bad})), None) == -9, name
+    for name in ("seg_p", "seg_ws"):
+        for off in (4, 8):
+            assert lib.lmoe_chunk_simple_gla_fwd(C.byref(args(**{name: fake + off})), None) == -9, name
+            assert b"seg_ws must be 16-byte aligned" in lib.lmoe_last_error()
     f32 = args(dtype=_lib.LMOE_F32, v=_lib.Tensor4(fake, 130 * 64, 68, 64))            # 4 elements are 16 bytes
     assert lib.lmoe_chunk_simple_gla_bwd(C.byref(f32), None) == -11                     # (passes on to the next check)
 
