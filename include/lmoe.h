@@ -149,7 +149,9 @@ typedef struct lmoe_args {
   int32_t dbeta_bf16;  /* element type of dbeta: 0 fp32, 1 bf16 (rounded once, on its way to memory) */
 } lmoe_args;
 
-/* Library version (major*10000 + minor*100 + patch). */
+/* Library version (major*10000 + minor*100 + patch).  lmoe_args grows at its end from one version to the next, and the
+ * library reads all of it: a caller checks that lmoe_version() is the LMOE_VERSION it was built with. */
+#define LMOE_VERSION 103
 int lmoe_version(void);
 /* Text of the last error on the calling thread ("" if none). */
 const char* lmoe_last_error(void);

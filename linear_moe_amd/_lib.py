@@ -14,6 +14,7 @@ LIB_PATH = os.path.join(_HERE, "liblmoe_hip.so")
 LMOE_BF16, LMOE_F32 = 0, 1
 GATE_NONE, GATE_SCALAR, GATE_VECTOR = 0, 1, 2
 CHUNK = 64
+VERSION = 103          # LMOE_VERSION of include/lmoe.h, whose lmoe_args the class Args below mirrors
 
 
 class Tensor4(C.Structure):
@@ -76,6 +77,9 @@ def load() -> C.CDLL:
             "(or __graft_entry__.build()).  This package has no fallback path.")
     lib = C.CDLL(LIB_PATH)
     lib.lmoe_version.restype = C.c_int
+    if lib.lmoe_version() != VERSION:
+        raise RuntimeError(f"{LIB_PATH} is version {lib.lmoe_version()}, this package needs {VERSION}: build it again with "
+                           f"`make -C {os.path.join(_HERE, 'csrc')}`")
     lib.lmoe_last_error.restype = C.c_char_p
     for name in ENTRY_POINTS[2:8]:
         fn = getattr(lib, name)

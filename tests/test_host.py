@@ -31,6 +31,20 @@ def test_library_exports_every_declared_symbol():
     assert lib.lmoe_version() >= 100
 
 
+def test_the_argument_block_of_another_version_is_refused(monkeypatch):
+    """The library reads the whole of lmoe_args: its length belongs to a version, which the header, the library and the
+    binding name alike, and a library of another version is not loaded."""
+    from linear_moe_amd import _lib
+    declared = int(re.search(r"#define\s+LMOE_VERSION\s+(\d+)", open(HEADER).read()).group(1))
+    assert _lib.load().lmoe_version() == _lib.VERSION == declared
+    # (a field more or less without a new version: raise LMOE_VERSION and _lib.VERSION with these numbers)
+    assert (declared, C.sizeof(_lib.Args), _lib.Args._fields_[-1][0]) == (103, 888, "dbeta_bf16")
+    monkeypatch.setattr(_lib, "VERSION", declared - 1)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match="is version 103"):
+        _lib.load()
+
+
 def test_ctypes_struct_matches_c_layout():
     from linear_moe_amd import _lib
     fields = [f[0] for f in _lib.Args._fields_]
