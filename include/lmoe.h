@@ -167,7 +167,7 @@ int64_t lmoe_workspace_bytes(int32_t op, int32_t dtype, int32_t part, int32_t B,
                              int32_t V, int32_t NT);
 
 /* Numbers (fp32) seg_p (part 0) and seg_ws (part 1) of this call need; 0 for both where the call is not cut.  Reads
- * dtype, B, T, H, K, V, N, NT, normalize and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op or
+ * dtype, gate, B, T, H, K, V, N, NT, normalize and cu_seqlens (NULL or not) of the argument block.  Negative for an invalid op or
  * part and for sizes the op itself refuses.  What is cut depends on T, N, H, K, V, the type, normalize and whether the input
  * is packed, not on where the offsets of packed input lie. */
 int64_t lmoe_split_floats(const lmoe_args* a, int32_t op, int32_t part);

@@ -8,6 +8,11 @@
 // P is handed on as D 1 + R with D = the product of the chunk decays in fp32 and R in the 2-byte type, and applied as
 // S <- D S + R S + Q with S rounded for the product R S only: what a chunk of the ordinary pass does to the state (the
 // carry in fp32, the update through 2-byte operands).
+// TWO (calls without a gate): nothing fades, and these two roundings per segment show beside those of the chunks: against
+// float64 o, dq and dk were off by 1.04 times as much as behind the pass over whole sequences, the final state by up to
+// 1.25 times where v falls to a hundredth half way.  R and the rounded S are then carried as two 2-byte terms each (hi hi +
+// hi lo + lo hi): 0.94 to 1.00 of the whole pass's error.  16 heads, 3001 tokens, K = V = 128: 61 -> 66 us (whole 92).
+// Gated calls stay at one term: 1.00 with the decays of a mixer (A in 1 .. 16), 0.96 at a decay of 0.002 per token.
 //
 // One work-group carries all columns of a segment: k, Tinv (q, the intra-chunk P) are fetched once per chunk for up to
 // V + K (V) columns, where the slices of the ordinary pass fetch them once per 32.  Every wave owns all K rows of 32
@@ -155,9 +160,12 @@ __device__ __forceinline__ void tile_times_state(f32x4 (&X)[4][NCB], const bf16*
 // M[16 rb + r][32 ks + 8 g ..+7] at frag_slot + 8 l: every load of a wave is 1 KB in one piece.
 template <int K> __host__ __device__ constexpr int frag_slot(int rb, int ks) { return (rb * (K / 32) + ks) * 512; }
 
+// 2-byte terms a number of R is carried in
+template <bool TWO> constexpr int split_terms = TWO ? 2 : 1;
+
 constexpr int SEG_FWD_THREADS = 512;      // waves 0 .. 3: up to 128 columns of Q, waves 4 .. 7: of P; all eight load
 // the part of one wave of fine segment s1 of head h: 32 of the W columns of Q (TRANS = false, W = V) or of P (W = K)
-template <int K, int V, bool TRANS>
+template <int K, int V, bool TRANS, bool TWO>
 __device__ __forceinline__ void seg_fwd_columns(const lmoe_args& a, const Split& sp, int s1, int h, const SegInfo& sg,
                                                 const SeqInfo& sq, bool busy, bool in_last3, char* s_mem, float (&s_g)[2][4 * CH]) {
   constexpr int NT = SEG_FWD_THREADS, LDK = seg_ld<K>, LDC = CH + LPAD, LDV = V + LPAD, NCB = 2;
@@ -281,7 +289,7 @@ __device__ __forceinline__ void seg_fwd_columns(const lmoe_args& a, const Split&
   } else {
     // R in the order in which the combination reads it as an operand (frag_slot): R^T as it lies in the accumulators,
     // R through LDS ([column][row], transposing reads)
-    constexpr int LDP = K + LPAD;
+    constexpr int LDP = K + LPAD, RK = split_terms<TWO> * K * K;
     bf16* const s_r = (bf16*)s_mem;
     if (busy) {
 #pragma unroll
@@ -294,8 +302,17 @@ __device__ __forceinline__ void seg_fwd_columns(const lmoe_args& a, const Split&
             for (int i = 0; i < 4; ++i)
               if (acc_row4(2 * ks + e, g) + i == col0 + 16 * cb + fr) S[2 * ks + e][cb][i] -= D;
           const bf16x8 x = frag_of_blocks(S[2 * ks][cb], S[2 * ks + 1][cb]);
-          if (sp.PT) *(bf16x8*)(sp.PT + slot * K * K + frag_slot<K>((col0 >> 4) + cb, ks) + 8 * l) = x;
-          *(bf16x8*)(s_r + (col0 + 16 * cb + fr) * LDP + 32 * ks + 8 * g) = x;
+          bf16* const pt = sp.PT + slot * RK + frag_slot<K>((col0 >> 4) + cb, ks) + 8 * l;
+          bf16* const r = s_r + (col0 + 16 * cb + fr) * LDP + 32 * ks + 8 * g;
+          if (sp.PT) *(bf16x8*)pt = x;
+          *(bf16x8*)r = x;
+          if constexpr (TWO) {
+            bf16x8 y;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = (bf16)(S[2 * ks + (e >> 2)][cb][e & 3] - (float)x[e]);
+            if (sp.PT) *(bf16x8*)(pt + K * K) = y;
+            *(bf16x8*)(r + K * LDP) = y;
+          }
         }
       if (wv == 0 && l == 0) {
         if (sp.PT) sp.DT[slot] = D;
@@ -306,17 +323,19 @@ __device__ __forceinline__ void seg_fwd_columns(const lmoe_args& a, const Split&
     lds_barrier();
     for (int u = wv; u < (K / 16) * KS; u += 4) {
       const int rb = u / KS, ks = u % KS;
-      *(bf16x8*)(sp.P + slot * K * K + frag_slot<K>(rb, ks) + 8 * l) = ET<bf16>::load_frag_t(s_r, LDP, 32 * ks, 16 * rb, l);
+      bf16* const p = sp.P + slot * RK + frag_slot<K>(rb, ks) + 8 * l;
+      *(bf16x8*)p = ET<bf16>::load_frag_t(s_r, LDP, 32 * ks, 16 * rb, l);
+      if constexpr (TWO) *(bf16x8*)(p + K * K) = ET<bf16>::load_frag_t(s_r + K * LDP, LDP, 32 * ks, 16 * rb, l);
     }
   }
 }
 
 // grid: (fine segment, head)
-template <int K, int V>
+template <int K, int V, bool TWO>
 __global__ __launch_bounds__(SEG_FWD_THREADS) void k_gdn_seg_fwd(const lmoe_args a, const Split sp) {
   static_assert(V <= 128 && K <= 128, "a wave per 32 columns");
   constexpr int LDK = seg_ld<K>, LDC = CH + LPAD, LDV = V + LPAD;
-  constexpr int TILES = 2 * (CH * LDK + CH * LDC + CH * LDV) * 2, RBYTES = K * (K + LPAD) * 2;
+  constexpr int TILES = 2 * (CH * LDK + CH * LDC + CH * LDV) * 2, RBYTES = split_terms<TWO> * K * (K + LPAD) * 2;
   __shared__ __attribute__((aligned(16))) char s_mem[TILES > RBYTES ? TILES : RBYTES];
   __shared__ __attribute__((aligned(16))) float s_g[2][4 * CH];   // e^b, e^{b_C - b}, beta, beta e^b
   const int h = blockIdx.x % a.H, s1 = blockIdx.x / a.H;
@@ -329,8 +348,8 @@ __global__ __launch_bounds__(SEG_FWD_THREADS) void k_gdn_seg_fwd(const lmoe_args
   if (in_last3 && (whole.nchunks <= sp.len3 || !sp.PT)) return;
   const SeqInfo sq = seg_cut(whole, sg.j, sp.len1);
   const int wv = wave_id();
-  if (wv >= 4) seg_fwd_columns<K, V, true>(a, sp, s1, h, sg, sq, sg.j > 0 && 32 * (wv - 4) < K, in_last3, s_mem, s_g);
-  else seg_fwd_columns<K, V, false>(a, sp, s1, h, sg, sq, !in_last3 && 32 * wv < V, in_last3, s_mem, s_g);
+  if (wv >= 4) seg_fwd_columns<K, V, true, TWO>(a, sp, s1, h, sg, sq, sg.j > 0 && 32 * (wv - 4) < K, in_last3, s_mem, s_g);
+  else seg_fwd_columns<K, V, false, TWO>(a, sp, s1, h, sg, sq, !in_last3 && 32 * wv < V, in_last3, s_mem, s_g);
 }
 
 constexpr int SEG_BWD_THREADS = 512;      // 16 of the V columns per wave
@@ -478,10 +497,10 @@ __global__ __launch_bounds__(SEG_BWD_THREADS) void k_gdn_seg_bwd(const lmoe_args
 // (backward: R_s^T, from the end); wave w holds the rows 32 w ..  The operands of the next segment are requested before
 // the products of this one.  Leaves the state every coarse segment starts from.  Bound by what a CU gets of R per step
 // (K = 128: 32 KB in 0.9 us).
-template <int K, bool BWD>
+template <int K, bool BWD, bool TWO>
 __global__ __launch_bounds__(2 * K) void k_split_combine(const lmoe_args a, const Split sp) {
-  constexpr int LD = K + LPAD, KS = K / 32;
-  __shared__ __attribute__((aligned(16))) bf16 s_S[2][16 * LD];
+  constexpr int LD = K + LPAD, KS = K / 32, TERMS = split_terms<TWO>;
+  __shared__ __attribute__((aligned(16))) bf16 s_S[2][TERMS][16 * LD];
   const int V = a.V, ncb = V / 16;
   // the column blocks of a pair on one XCD: they read the same P at the same time
   const int jj = blockIdx.x >> 3, cb = jj % ncb, pair = jj / ncb * 8 + (blockIdx.x & 7), h = pair % a.H, n = pair / a.H;
@@ -503,7 +522,7 @@ __global__ __launch_bounds__(2 * K) void k_split_combine(const lmoe_args a, cons
   if (nc < 2) return;
   const int base1 = seg_base(a, sp.len1, n), base3 = seg_base(a, sp.len3, n);
   const int first = BWD ? nf - 1 : 0, steps = BWD ? nf - 1 - f : (nc - 1) * f - 1;      // products that follow the first segment
-  struct Pre { bf16x8 A[2][KS]; f32x4 q[2]; float D; };
+  struct Pre { bf16x8 A[TERMS][2][KS]; f32x4 q[2]; float D; };
   Pre pre[2];
   auto load_q = [&](f32x4 (&q)[2], int s) {
     const float* p = sp.Q + ((int64_t)(base1 + s) * a.H + h) * plane + col;
@@ -517,12 +536,14 @@ __global__ __launch_bounds__(2 * K) void k_split_combine(const lmoe_args a, cons
     const int s = BWD ? first - t : t;
     load_q(x.q, s);
     const int64_t slot = (int64_t)(base1 + s) * a.H + h;
-    const bf16* R = (BWD ? sp.PT : sp.P) + slot * K * K + 8 * l;
+    const bf16* R = (BWD ? sp.PT : sp.P) + slot * TERMS * K * K + 8 * l;
     x.D = (BWD ? sp.DT : sp.D)[slot];
 #pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
+    for (int u = 0; u < TERMS; ++u)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) x.A[mi][ks] = *(const bf16x8*)(R + frag_slot<K>(row0 / 16 + mi, ks));
+      for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) x.A[u][mi][ks] = *(const bf16x8*)(R + u * K * K + frag_slot<K>(row0 / 16 + mi, ks));
   };
   f32x4 acc[2];
   load_q(acc, first);
@@ -543,21 +564,33 @@ __global__ __launch_bounds__(2 * K) void k_split_combine(const lmoe_args a, cons
     issue(pre[1 - cur], t0 + 2);
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) {
-      bf16x4 x;
+      f32x4 rest = acc[mi];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = (bf16)acc[mi][i];
-      *(bf16x4*)&s_S[cur][fr * LD + row0 + 16 * mi + 4 * g] = x;
+      for (int u = 0; u < TERMS; ++u) {
+        bf16x4 x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { x[i] = (bf16)rest[i]; rest[i] -= (float)x[i]; }
+        *(bf16x4*)&s_S[cur][u][fr * LD + row0 + 16 * mi + 4 * g] = x;
+      }
     }
     lds_barrier();
-    bf16x8 b[KS];
+    bf16x8 b[TERMS][KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) b[ks] = row_frag(&s_S[cur][fr * LD], ks, g);
+    for (int u = 0; u < TERMS; ++u)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) b[u][ks] = row_frag(&s_S[cur][u][fr * LD], ks, g);
 #pragma unroll
     for (int mi = 0; mi < 2; ++mi) acc[mi] = acc[mi] * pre[cur].D + pre[cur].q[mi];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-      for (int mi = 0; mi < 2; ++mi) ET<bf16>::mma(acc[mi], pre[cur].A[mi][ks], b[ks]);
+      for (int mi = 0; mi < 2; ++mi) {
+        ET<bf16>::mma(acc[mi], pre[cur].A[0][mi][ks], b[0][ks]);
+        if constexpr (TWO) {
+          ET<bf16>::mma(acc[mi], pre[cur].A[0][mi][ks], b[1][ks]);
+          ET<bf16>::mma(acc[mi], pre[cur].A[1][mi][ks], b[0][ks]);
+        }
+      }
     emit(t0 + 1);
   });
 }

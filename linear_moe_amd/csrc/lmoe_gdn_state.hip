@@ -15,27 +15,34 @@ template <typename T, int V> inline bool wide_slices(const lmoe_args& a) {
   constexpr int BW = GdnStateCfg<T>::BV_WIDE;
   return BW <= V && BW != GdnStateCfg<T>::BV && (int64_t)a.N * a.H * (V / BW) >= cu_count();
 }
+// The transitions of a call without a gate are carried in two terms (lmoe_gdn_split.hpp).
+inline bool two_terms(const lmoe_args& a) { return a.gate == LMOE_GATE_NONE; }
 // How the sequences of a call are cut: not at all without a workspace for it.
 inline Split gdn_split(const lmoe_args& a, bool bwd) {
   Split sp = {};
   if (!a.seg_ws || ((bwd || a.hs) && !a.seg_p)) return sp;
   sp = gdn_split_plan(a);
   if (!sp.len1) return sp;
-  const int64_t n1 = (int64_t)sp.n1 * a.H, n3 = (int64_t)sp.n3 * a.H;
+  const int64_t n1 = (int64_t)sp.n1 * a.H, n3 = (int64_t)sp.n3 * a.H, terms = two_terms(a) ? 2 : 1;
   sp.Q = a.seg_ws;
   sp.S = sp.Q + n1 * a.K * a.V;
   sp.P = (bf16*)(sp.S + n3 * a.K * a.V);
-  sp.D = (float*)(sp.P + n1 * a.K * a.K);
+  sp.D = (float*)(sp.P + n1 * terms * a.K * a.K);
   if (bwd || a.hs) {
     sp.PT = (bf16*)a.seg_p;
-    sp.DT = (float*)(sp.PT + n1 * a.K * a.K);
+    sp.DT = (float*)(sp.PT + n1 * terms * a.K * a.K);
   }
   return sp;
 }
 template <int K, int V> void combine(const lmoe_args& a, const Split& sp, bool bwd, hipStream_t st) {
   const dim3 grid((a.N * a.H + 7) / 8 * 8 * (V / 16)), block(2 * K);
-  if (bwd) hipLaunchKernelGGL((k_split_combine<K, true>), grid, block, 0, st, a, sp);
-  else hipLaunchKernelGGL((k_split_combine<K, false>), grid, block, 0, st, a, sp);
+  if (two_terms(a)) {
+    if (bwd) hipLaunchKernelGGL((k_split_combine<K, true, true>), grid, block, 0, st, a, sp);
+    else hipLaunchKernelGGL((k_split_combine<K, false, true>), grid, block, 0, st, a, sp);
+  } else {
+    if (bwd) hipLaunchKernelGGL((k_split_combine<K, true, false>), grid, block, 0, st, a, sp);
+    else hipLaunchKernelGGL((k_split_combine<K, false, false>), grid, block, 0, st, a, sp);
+  }
 }
 template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, hipStream_t st) {
   const int grid = ((a.N * a.H + 7) / 8) * 8 * (V / BV);
@@ -47,7 +54,8 @@ template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, 
       if constexpr (V <= 128) {
         const Split sp = gdn_split(a, false);
         if (sp.len1) {
-          hipLaunchKernelGGL((k_gdn_seg_fwd<K, V>), dim3(sp.n1 * a.H), dim3(SEG_FWD_THREADS), 0, st, a, sp);
+          if (two_terms(a)) hipLaunchKernelGGL((k_gdn_seg_fwd<K, V, true>), dim3(sp.n1 * a.H), dim3(SEG_FWD_THREADS), 0, st, a, sp);
+          else hipLaunchKernelGGL((k_gdn_seg_fwd<K, V, false>), dim3(sp.n1 * a.H), dim3(SEG_FWD_THREADS), 0, st, a, sp);
           combine<K, V>(a, sp, false, st);
           const int items = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
           if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true, false, true>), dim3(items), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
@@ -119,7 +127,8 @@ int64_t split_floats(const lmoe_args& a, int op, int part) {
   if (op == LMOE_OP_GLA && part == 1) return gla_split_floats(a);
   if (op != LMOE_OP_GATED_DELTA_RULE) return 0;
   const Split sp = gdn_split_plan(a);
-  const int64_t trans = (int64_t)sp.n1 * a.H * (a.K * a.K / 2 + 1);      // a 2-byte matrix and a decay per fine segment
+  // a matrix of one or two 2-byte terms and a decay per fine segment
+  const int64_t trans = (int64_t)sp.n1 * a.H * (a.K * a.K / (two_terms(a) ? 1 : 2) + 1);
   return part == 0 ? trans : (int64_t)(sp.n1 + sp.n3) * a.H * a.K * a.V + trans;
 }
 void launch_gdn_state_bwd(const lmoe_args& a, hipStream_t st) { dispatch_gdn<GdnStateBwd>(a, st); }

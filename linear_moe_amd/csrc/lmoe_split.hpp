@@ -18,7 +18,8 @@ struct Split {
   int32_t len1;          // chunks per fine segment
   int32_t len3;          // chunks per coarse segment (a multiple of len1)
   int32_t n1, n3;        // segments of all sequences (packed input: upper bounds; a segment beyond the true count ends at once)
-  bf16 *P, *PT;          // [n1][H][K][K]  transitions of the fine segments less their decay (delta rule), in operand order, and
+  bf16 *P, *PT;          // [n1][H][K][K]  transitions of the fine segments less their decay (delta rule; without a gate two
+                         // such matrices, hi and lo), in operand order, and
                          // the same transposed (kept for the backward; NULL in a call that keeps nothing)
   float *D, *DT;         // [n1][H]        decays of the fine segments (beside P, PT); chunk_gla: [n1][H][K]
   float* Q;              // [n1][H][K][V]  their contributions

@@ -160,3 +160,62 @@ def test_calls_without_heads_are_refused(cuda, dtype):
                lambda: chunk_gla(x, x, x, x.float(), head_first=False)):
         with pytest.raises(ValueError, match="dimension"):
             fn()
+
+
+def lengths(op, B, T, H, K, V, N=None, dtype=torch.bfloat16):
+    """Chunks per fine and per coarse segment."""
+    import ctypes as C
+    from linear_moe_amd import _lib
+    a = _lib.Args()
+    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N = _lib.LMOE_BF16 if dtype == torch.bfloat16 else _lib.LMOE_F32, B, T, H, K, V, N or B
+    a.NT = B * ((T + 63) // 64) + (N if N else 0)
+    a.cu_seqlens = 16 if N else None               # (only asked whether it is there)
+    fine, coarse = C.c_int32(), C.c_int32()
+    assert _lib.load().lmoe_split_lengths(C.byref(a), op, C.byref(fine), C.byref(coarse)) == 0
+    return fine.value, coarse.value
+
+
+def delta_inputs(seed, B, T, H, K, V, N, gated=True):
+    bf = lambda x: x.bfloat16()
+    ins = dict(q=bf(F.normalize(gen(seed, B, T, H, K), dim=-1)), k=bf(F.normalize(gen(seed + 1, B, T, H, K), dim=-1)),
+               v=bf(gen(seed + 2, B, T, H, V)), g=-F.softplus(gen(seed + 3, B, T, H)) * 0.003,
+               beta=bf(torch.sigmoid(gen(seed + 4, B, T, H))), h0=gen(seed + 5, N, H, K, V) * 0.3)
+    if not gated:
+        del ins["g"]
+    return ins, bf(gen(seed + 6, B, T, H, V)), gen(seed + 7, N, H, K, V)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_error_of_the_cut_behind_a_drop_of_v(cuda, monkeypatch, gated):
+    """A state that outlives many segments and a v that falls to a hundredth half way (the late chunks see what the early
+    ones left): against float64 the cut call is as exact as the whole one.  Without a gate transitions and states are
+    carried in two terms and the cut adds no rounding of its own: 1.05 for the scatter of two sums of as many roundings.
+    Gated: the whole pass rounds the state for one product per chunk, the cut adds one product per fine segment with two
+    rounded operands: with len1 >= 2 at most twice the variance, a factor sqrt(2) on the norm of the error."""
+    from linear_moe_amd import chunk_delta_rule, chunk_gated_delta_rule
+    from linear_moe_amd.gated_delta_rule import GDNCall
+    T, H, D = 3001, 2, 128
+    assert lengths(2, 1, T, H, D, D)[0] >= 2
+    ins, _, _ = delta_inputs(8100, 1, T, H, D, D, 1, gated)
+    ins["v"][:, T // 2:] *= 0.01
+    d = {n: x.double() for n, x in ins.items()}
+    g = d["g"] if gated else torch.zeros_like(d["beta"])
+    ref, ref_ht = naive.naive_recurrent_gated_delta_rule(d["q"], d["k"], d["v"], g, d["beta"], None, d["h0"], True, None, False)
+    x = [ins[n].to(cuda) for n in ("q", "k", "v") + (("g",) if gated else ()) + ("beta",)]
+    h0, fn = ins["h0"].to(cuda), chunk_gated_delta_rule if gated else chunk_delta_rule
+
+    def errors():
+        with torch.no_grad():
+            o, ht = fn(*x, initial_state=h0, output_final_state=True, head_first=False)
+        diff = lambda a, r: (a.cpu().double() - r)
+        n = T // 64 * 64
+        per_chunk = lambda t: t[:, :n].reshape(n // 64, -1).norm(dim=1)
+        return (per_chunk(diff(o, ref)) / per_chunk(ref)).max().item(), diff(o, ref).norm().item(), diff(ht, ref_ht).norm().item()
+
+    cut = errors()
+    monkeypatch.setattr(GDNCall, "_cut", lambda self, *a, **kw: setattr(self, "seg_ws", None))
+    whole = errors()
+    print(gated, "worst chunk, o, ht: cut", cut, "whole", whole)
+    assert cut[0] < TOL[torch.bfloat16]
+    bound = 2 ** 0.5 if gated else 1.05
+    assert cut[1] < bound * whole[1] and cut[2] < bound * whole[2]
