@@ -177,3 +177,37 @@ def test_routing_to_result_captures_into_a_graph_and_follows_new_routing_at_repl
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, refs[i]), i
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scaled_gather_and_row_product_are_the_backward_of_combine(cuda, dtype):
+    """lmoe_mom_gather with a scale and lmoe_mom_rowdot, the two passes that lmoe_mom_combine_bwd joins, against it and
+    against the products written out (float64)."""
+    from linear_moe_amd import _lib
+    from linear_moe_amd._host import stream_ptr
+    from linear_moe_amd.mom import mom_plan
+    lib = _lib.load()
+    B, S, topk, E, D = 2, 77, 2, 4, 72
+    sel = torch.topk(torch.rand(B, S, E, generator=torch.Generator().manual_seed(3), device="cpu"), topk, dim=-1).indices
+    plan = mom_plan(sel.to(cuda), E, 0.4)                       # a capacity: choices without a row (row_of = -1)
+    n, ntok = plan.T_total, B * S
+    assert (plan.row_of < 0).any()
+    y, g, w = (gen(8200 + i, *s, dtype=dtype).to(cuda) for i, s in enumerate(((n, D), (ntok, D), (ntok, topk))))
+    dt = _lib.LMOE_F32 if dtype == torch.float32 else _lib.LMOE_BF16
+    scale = w.reshape(-1)[plan.src_choice.long()].contiguous()
+    dy, dw, dy2, dw2 = torch.empty_like(y), torch.empty_like(w), torch.empty_like(y), torch.empty_like(w)
+    p = lambda t: t.data_ptr()
+    _lib.check(lib.lmoe_mom_gather(p(g), p(plan.src_token), p(scale), p(dy), n, D, dt, stream_ptr()), "gather")
+    _lib.check(lib.lmoe_mom_rowdot(p(y), p(plan.row_of), p(g), p(dw), ntok, topk, D, dt, stream_ptr()), "rowdot")
+    _lib.check(lib.lmoe_mom_combine_bwd(p(y), p(plan.row_of), p(plan.src_choice), p(w), p(g), p(dy2), p(dw2), ntok, n, topk,
+                                        D, dt, stream_ptr()), "combine_bwd")
+    torch.cuda.synchronize()
+    assert torch.equal(dy, dy2)                                 # one product, rounded once
+    rows = plan.row_of.cpu().long()
+    want_dy = g.cpu().double()[plan.src_token.cpu().long()] * scale.cpu().double()[:, None]
+    terms = g.cpu().double()[:, None] * y.cpu().double()[rows.clamp_min(0)] * (rows >= 0)[..., None]
+    # rounding to the element type is off by at most 2^-p of the value (p = 24, 8 bits of significand); sums are fp32
+    eps = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -8
+    assert ((dy.cpu().double() - want_dy).abs() <= eps * want_dy.abs()).all()
+    for x in (dw, dw2):
+        assert ((x.cpu().double() - terms.sum(-1)).abs() <= eps * terms.sum(-1).abs() + D * 2.0 ** -23 * terms.abs().sum(-1)).all()

@@ -175,6 +175,25 @@ def lengths(op, B, T, H, K, V, N=None, dtype=torch.bfloat16):
     return fine.value, coarse.value
 
 
+def check_part(fn_ref, fn, ins, do, dht, cuda, b, h, dtype=torch.bfloat16):
+    """As check, the whole call against the oracle on batch row b and head h alone (rows and heads do not mix).
+    Tensors [B, T, H, ...] and states [N, H, K, V]; b = None: packed input, all sequences."""
+    cut = lambda x, state: (x if b is None else x[b:b + 1])[(slice(None),) * (1 if state else 2) + (slice(h, h + 1),)]
+    ref_o, ref_ht, ref = oracle_grads(fn_ref, {n: cut(x, n == "h0") for n, x in ins.items()}, cut(do, False), cut(dht, True))
+    dev = {n: x.to(cuda).requires_grad_(True) for n, x in ins.items()}
+    o, ht = fn(**dev)
+    grads = torch.autograd.grad([o, ht], list(dev.values()), [do.to(cuda), dht.to(cuda)])
+    with torch.no_grad():
+        of, hf = fn(**dev)
+    torch.cuda.synchronize()
+    for x, y in ((o, of), (ht, hf)):
+        assert torch.equal(x.detach(), y)          # the forward-only instance is cut the same way
+    assert max_abs_rel(cut(o.detach(), False).cpu(), ref_o) < TOL[dtype]
+    assert max_abs_rel(cut(ht.detach(), True).cpu(), ref_ht) < TOL[dtype]
+    for (n, r), x in zip(ref.items(), grads):
+        assert max_abs_rel(cut(x, n == "h0").cpu(), r) < TOL[dtype], n
+
+
 def delta_inputs(seed, B, T, H, K, V, N, gated=True):
     bf = lambda x: x.bfloat16()
     ins = dict(q=bf(F.normalize(gen(seed, B, T, H, K), dim=-1)), k=bf(F.normalize(gen(seed + 1, B, T, H, K), dim=-1)),
@@ -183,6 +202,153 @@ def delta_inputs(seed, B, T, H, K, V, N, gated=True):
     if not gated:
         del ins["g"]
     return ins, bf(gen(seed + 6, B, T, H, V)), gen(seed + 7, N, H, K, V)
+
+
+@pytest.mark.parametrize("B,T,H,K,V,lens,cut", [
+    (1, 3001, 16, 128, 128, None, (3, 12)),        # four coarse segments, the last one of 11 chunks
+    (1, 6000, 4, 64, 128, None, (3, 6)),           # the last one of two fine segments, the second of one chunk
+    (1, 4096, 4, 128, 128, [2000, 2096], (2, 6)),
+    (1, 6000, 4, 128, 128, [5300, 0, 700], (2, 8)),
+    (1, 8000, 4, 64, 64, [64, 7935, 1], (3, 6)),
+])
+def test_gated_delta_rule_of_several_fine_segments(cuda, B, T, H, K, V, lens, cut):
+    """Coarse segments of more than one fine segment: transitions alone in the last coarse segment, states handed on
+    from every len3 / len1-th combination only, the first coarse segment left out of the backward's first step."""
+    from linear_moe_amd import chunk_gated_delta_rule
+    N = B if lens is None else len(lens)
+    assert lengths(2, B, T, H, K, V, None if lens is None else N) == cut
+    ins, do, dht = delta_inputs(7500, B, T, H, K, V, N)
+    cu = None if lens is None else torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    cud = None if cu is None else cu.to(cuda)
+    check_part(lambda q, k, v, g, beta, h0: naive.naive_recurrent_gated_delta_rule(q, k, v, g, beta, None, h0, True, cu, False),
+               lambda q, k, v, g, beta, h0: chunk_gated_delta_rule(q, k, v, g, beta, None, h0, True, cud, False),
+               ins, do, dht, cuda, None if lens else B - 1, H - 1)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+def test_delta_rule_cut_along_t_in_both_layouts(cuda, gated):
+    """Head-first views of the tensors of a time-first call: the same bits; without a gate (chunk_delta_rule) too."""
+    from linear_moe_amd import chunk_delta_rule, chunk_gated_delta_rule
+    B, T, H, K, V = 1, 1601, 2, 128, 128
+    assert lengths(2, B, T, H, K, V)[0] > 0
+    ins, do, dht = delta_inputs(7600, B, T, H, K, V, B, gated)
+    fn = chunk_gated_delta_rule if gated else chunk_delta_rule
+    tr = lambda x: x.transpose(1, 2)
+    order = ("q", "k", "v") + (("g",) if gated else ()) + ("beta",)
+
+    def ours(head_first):
+        def call(h0, **x):
+            o, ht = fn(*(tr(x[n]) if head_first else x[n] for n in order), initial_state=h0, output_final_state=True,
+                       head_first=head_first)
+            return (tr(o) if head_first else o), ht
+        return call
+    check_part(lambda q, k, v, beta, h0, g=None: naive.naive_recurrent_gated_delta_rule(
+        q, k, v, torch.zeros_like(beta) if g is None else g, beta, None, h0, True, None, False), ours(False), ins, do, dht, cuda, 0, 1)
+    dev = {n: x.to(cuda).requires_grad_(True) for n, x in ins.items()}
+    res = []
+    for head_first in (False, True):
+        o, ht = ours(head_first)(**dev)
+        res.append((o.detach(), ht.detach()) + torch.autograd.grad([o, ht], list(dev.values()), [do.to(cuda), dht.to(cuda)]))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,B,T,H,K,V,cut", [
+    (torch.bfloat16, 2, 1500, 8, 128, 128, (3, 6)),
+    (torch.bfloat16, 2, 2049, 8, 128, 128, (3, 9)),        # the last coarse segment of two fine ones, one token in the last chunk
+    (torch.float32, 2, 1000, 8, 128, 128, (2, 8)),
+    (torch.float32, 1, 1281, 8, 64, 64, (1, 3)),
+])
+@pytest.mark.parametrize("head_first", [True, False])
+def test_simple_gla_of_several_fine_segments(cuda, dtype, B, T, H, K, V, cut, head_first):
+    from linear_moe_amd import chunk_simple_gla
+    assert lengths(0, B, T, H, K, V, dtype=dtype) == cut
+    tr = lambda x: x.transpose(1, 2) if head_first else x
+    ins = dict(q=gen(7700, B, T, H, K).to(dtype), k=(gen(7701, B, T, H, K) * K ** -0.5).to(dtype),
+               v=gen(7702, B, T, H, V).to(dtype), g=-F.softplus(gen(7703, B, T, H)) * 0.003, h0=gen(7705, B, H, K, V) * 0.3)
+    do, dht = gen(7706, B, T, H, V).to(dtype), gen(7707, B, H, K, V)
+
+    def ours(q, k, v, g, h0):
+        o, ht = chunk_simple_gla(tr(q), tr(k), tr(v), tr(g), None, h0, True, None, head_first)
+        return tr(o), ht
+    check_part(lambda q, k, v, g, h0: naive.naive_recurrent_simple_gla(q, k, v, g, None, h0, True, None, False), ours,
+               ins, do, dht, cuda, B - 1, H - 1, dtype)
+
+
+@pytest.mark.parametrize("B,T,H,K,V,cut", [(2, 3000, 8, 128, 128, (4, 12)), (2, 4000, 8, 64, 64, (4, 8))])
+def test_gla_of_several_fine_segments(cuda, B, T, H, K, V, cut):
+    from linear_moe_amd import chunk_gla
+    assert lengths(1, B, T, H, K, V) == cut
+    ins = dict(q=gen(7800, B, T, H, K).bfloat16(), k=(gen(7801, B, T, H, K) * K ** -0.5).bfloat16(),
+               v=gen(7802, B, T, H, V).bfloat16(), g=F.logsigmoid(gen(7803, B, T, H, K)) * 0.01, h0=gen(7805, B, H, K, V) * 0.3)
+    do, dht = gen(7806, B, T, H, V).bfloat16(), gen(7807, B, H, K, V)
+    check_part(lambda q, k, v, g, h0: naive.naive_recurrent_gla(q, k, v, g, None, h0, True, None, False),
+               lambda q, k, v, g, h0: chunk_gla(q, k, v, g, None, h0, True, None, False), ins, do, dht, cuda, B - 1, H - 1)
+
+
+@pytest.mark.parametrize("D,T,B,H", [(128, 1601, 1, 2), (64, 2000, 2, 1)])
+def test_mixer_core_cut_along_t(cuda, D, T, B, H):
+    """v as a block of the projection, SiLU applied while the segments stage it: the bits of the op on silu(v)."""
+    import linear_moe_amd as L
+    assert lengths(2, B, T, H, D, D)[0] > 0
+    qkv, do = gen(7900, T, B, H * 3 * D).bfloat16().to(cuda), gen(7903, B, T, H, D).bfloat16().to(cuda)
+    g = -F.softplus(gen(7901, B, T, H)).to(cuda) * 0.003
+    beta = torch.sigmoid(gen(7902, B, T, H)).bfloat16().to(cuda)
+    res = []
+    for core in (True, False):
+        leaves = [t.clone().requires_grad_(True) for t in (qkv, g, beta)]
+        if core:
+            o = L.gdn_mixer_core(*leaves, H, D)
+        else:
+            q, k, v = L.gdn_qkv_prologue(leaves[0], H, D)
+            o, _ = L.chunk_gated_delta_rule(q, k, v, leaves[1], leaves[2], head_first=False)
+        res.append((o.detach(),) + torch.autograd.grad(o, leaves, do))
+    torch.cuda.synchronize()
+    (o1, dx1, dg1, db1), (o2, dx2, dg2, db2) = res
+    assert torch.equal(o1, o2) and torch.equal(dg1, dg2) and torch.equal(db1, db2)
+    d1, d2 = (x.view(T, B, H, 3 * D) for x in (dx1, dx2))
+    assert torch.equal(d1[..., :2 * D], d2[..., :2 * D])
+    assert max_abs_rel(d1[..., 2 * D:].float().cpu(), d2[..., 2 * D:].float().cpu()) < 1e-2   # dv: rounded once, not twice
+
+
+def test_a_captured_packed_step_that_is_cut_follows_the_offsets_it_finds_at_replay(cuda):
+    """The segments of packed sequences are found on the device: new offsets in the captured buffer (other lengths, a
+    sequence of one chunk, an empty one, another number of chunks) give what an eager call on them gives."""
+    from linear_moe_amd.gated_delta_rule import GDNCall
+    T, H, D = 8000, 4, 128
+    assert lengths(2, 1, T, H, D, D, 3) == (3, 12)
+    x, do, dht = delta_inputs(8000, 1, T, H, D, D, 3)
+    q, k, v, g, beta, h0 = (t.to(cuda) for t in x.values())
+    do, dht = do.to(cuda), dht.to(cuda)
+    offsets = [[0, 2600, 5300, 8000], [0, 1, 7000, 8000], [0, 8000, 8000, 8000], [0, 64, 128, 7990]]
+
+    def step(call, cu):
+        o, ht = call.forward(q, k, v, g, beta, None, h0, True, cu, False)
+        return [o, ht] + [t for t in call.backward(do, dht) if t is not None]
+
+    refs = [[t.clone() for t in step(GDNCall(keep=True), torch.tensor(c, dtype=torch.int32, device=cuda))] for c in offsets]
+    cu = torch.tensor(offsets[0], dtype=torch.int32, device=cuda)
+    call = GDNCall(keep=True)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(call, cu)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step(call, cu)
+    for i in (0, 1, 2, 3, 1, 0):
+        cu.copy_(torch.tensor(offsets[i], dtype=torch.int32))
+        for t in outs:
+            t.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        n = offsets[i][-1]                         # (rows behind the last sequence are nobody's)
+        for j, (a, b) in enumerate(zip(outs, refs[i])):
+            if a.shape[0] == 1:
+                a, b = a[:, :n], b[:, :n]
+            assert torch.equal(a, b), (i, j)
 
 
 @pytest.mark.parametrize("gated", [True, False])
