@@ -120,7 +120,9 @@ def stage_model(stage, K, V, s=2):
 
 
 def time_stages(call, lib, reps):
-    """Average duration (seconds) of every kernel, measured with events on the launch stream."""
+    """Average duration (seconds) of every kernel, measured with events on the launch stream.  (A stage is one kernel
+    here: 64 pairs of 4 V slices fill the CUs.  In a call cut along T the state passes bring their segment kernels.)"""
+    assert not call.fwd_args.seg_ws and not call.bwd_args.seg_ws
     import torch
     from linear_moe_amd import _lib
     st = C.c_void_p(torch.cuda.current_stream().cuda_stream)

@@ -362,8 +362,10 @@ int lmoe_mom_plan(const void* sel, int32_t is64, int32_t B, int32_t per_row, int
 int lmoe_seq_tables(const void* offsets, int32_t is64, int32_t N, int32_t nt_max, int32_t* cu, int32_t* chunk_map,
                     int32_t* seq_chunk0, int32_t* nt_dev, int32_t* seq_order, void* stream);
 
-/* Launch ONE kernel of an op's pipeline (profiling support: lets a harness time each kernel
- * with events on its own stream).  `a` must be the fully populated argument block of the
+/* Launch one step of an op's pipeline, a single kernel unless said otherwise (profiling support: lets a harness time each
+ * with events on its own stream).  A call cut along T (seg_ws given and lmoe_split_lengths not 0): the state passes,
+ * stages 1 and 4, are the pass over the coarse segments and, in front of it, what gives these their initial states: one
+ * more kernel, for the gated delta rule two.  `a` must be the fully populated argument block of the
  * op's fwd (stages 0-2, 7) or bwd (stages 3-5) entry point, with the intermediates of the
  * earlier stages already in place.  Stages: 0 gated-delta-rule WY preparation, 1 forward state
  * pass (scalar gates, and chunk_gla with 2-byte elements: the output o as well, so that the forward entry point
@@ -381,7 +383,8 @@ int lmoe_launch_stage(const lmoe_args* a, int32_t op, int32_t stage, void* strea
 /* Per-phase timing of the forward sequential pass of the gated delta rule (profiling support; no counterpart in the
  * reference).  Runs the pass once for the problem `a` (the fully populated argument block of
  * lmoe_chunk_gated_delta_rule_fwd, after its WY preparation has run: lmoe_launch_stage stage 0) with the instance
- * that records the shader clock in work-group `work_group`, and leaves in `trace` (device memory,
+ * that records the shader clock in work-group `work_group` (over whole sequences, whatever seg_ws: where the entry point
+ * cuts the call along T, its results differ from these by rounding), and leaves in `trace` (device memory,
  * int64 [4 slots][128 chunks][8 marks], zero where nothing was recorded; sequences longer than 128 chunks are traced
  * for their first 128) the cycle counter at these points of every chunk:
  *   slot 0, the consumer wave (carries the state):  0 arrives at barrier 1, 1 leaves it, 5 k S formed, 2 arrives at
@@ -393,7 +396,8 @@ int lmoe_launch_stage(const lmoe_args* a, int32_t op, int32_t stage, void* strea
  * Instance available for LMOE_BF16, K = V = 128, with tinv and hs given (-24 otherwise). */
 int lmoe_trace_gdn_state_fwd(const lmoe_args* a, int64_t* trace, int32_t work_group, void* stream);
 
-/* The same for the forward pass of chunk_simple_gla on 2-byte elements (k_state_fwd_b, one barrier per chunk):
+/* The same for the forward pass of chunk_simple_gla on 2-byte elements (k_state_fwd_b, one barrier per chunk; whole
+ * sequences here too):
  * trace = 3 x 24 x 8 int64 device words, trace[slot][chunk][mark] (chunks beyond 24 are not recorded), stamps of one
  * wave per team of work-group `work_group`.  Marks: 0 arrives at the barrier of the chunk, 1 leaves it, and
  *   slot 0, consumers: 5 state updated, 6 state copied to LDS, 2 their blocks of P of the next chunk formed, 3 the

@@ -27,9 +27,10 @@ struct Split {
   float* Z;              // [n1][H][K]     contributions to the normaliser's column (chunk_simple_gla)
 };
 
-// Sequences of fewer chunks gain nothing (three kernels in place of one).  Longer ones than 32 768 tokens are left whole
-// although they would gain: there a sequence gives the same bits alone and inside a large packed batch, whose other
-// sequences fill the CUs (tests/test_gpu_large.py holds the ops to it).
+// Sequences of fewer chunks gain nothing (three kernels in place of one).  Above 32 768 tokens (packed: on average) they
+// are left whole although they would gain (65 536 tokens, 16 heads, by the model of plan_split: 794 us in place of 1741):
+// there a sequence gives the same bits alone and inside a packed batch that fills the CUs, which the ops are held to.
+// Between the two limits it does not: what is cut depends on how many pairs a call has, and results differ by rounding.
 constexpr int SPLIT_MIN_CHUNKS = 24, SPLIT_MAX_CHUNKS = 512;
 
 __host__ __device__ inline int seg_count(int nchunks, int len) { return (nchunks + len - 1) / len; }

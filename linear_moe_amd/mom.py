@@ -62,7 +62,9 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
     by tensor operations), as the reference builds its tables (mom_linear_attention.py:28-66).  Without a capacity nothing is read
     back to the host: every routed token is kept, ``T_total = B * S * topk`` is known up front, and pack -> op ->
     combine can run inside a HIP graph capture with the plan in it.  With a capacity the number of surviving rows is
-    the one device-to-host read of the call.  ``check`` validates the memory indices (two more reads)."""
+    the one device-to-host read of the call.  ``check`` validates the memory indices (two more reads).  Unchecked indices
+    outside [0, num_memories) are a mistake of the caller: the kernels drop such a choice (``row_of`` -1; the rows behind
+    ``cu_seqlens[-1]`` then belong to nobody and hold ``src_token`` -1), the tensor operations are undefined for it."""
     if selected_memories.dim() != 3:
         raise ValueError("selected_memories must be [B, S, topk]")
     B, S, topk = selected_memories.shape
