@@ -208,7 +208,7 @@ def delta_inputs(seed, B, T, H, K, V, N, gated=True):
     (1, 3001, 16, 128, 128, None, (3, 12)),        # four coarse segments, the last one of 11 chunks
     (1, 6000, 4, 64, 128, None, (3, 6)),           # the last one of two fine segments, the second of one chunk
     (1, 4096, 4, 128, 128, [2000, 2096], (2, 6)),
-    (1, 6000, 4, 128, 128, [5300, 0, 700], (2, 8)),
+    (1, 6000, 4, 128, 128, [5300, 0, 700], (3, 9)),
     (1, 8000, 4, 64, 64, [64, 7935, 1], (3, 6)),
 ])
 def test_gated_delta_rule_of_several_fine_segments(cuda, B, T, H, K, V, lens, cut):

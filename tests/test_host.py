@@ -178,14 +178,14 @@ def test_the_cut_along_t_refuses_the_sizes_the_op_refuses():
 
 def test_the_cut_along_t_of_packed_input_follows_from_t_and_n():
     """NT is the chunk count where the offsets lie on the host and a bound of it where they lie on the device: the batch
-    is cut the same way.  One packed sequence is cut as a dense one of its length."""
+    is cut the same way."""
     from linear_moe_amd import _lib
     lib = _lib.load()
 
-    def lengths(T, H, D, N, NT, packed=True):
+    def lengths(T, H, D, N, NT):
         a = _lib.Args()
         a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_BF16, 1, T, H, D, D, N, NT
-        a.cu_seqlens = 0x1000 if packed else None  # (only asked whether it is there)
+        a.cu_seqlens = 0x1000                      # (only asked whether it is there)
         fine, coarse = C.c_int32(), C.c_int32()
         assert lib.lmoe_split_lengths(C.byref(a), 2, C.byref(fine), C.byref(coarse)) == 0
         parts = [lib.lmoe_split_floats(C.byref(a), 2, part) for part in (0, 1)]
@@ -199,8 +199,6 @@ def test_the_cut_along_t_of_packed_input_follows_from_t_and_n():
                 for D in (64, 128):
                     ch = -(-T // 64)
                     got = {lengths(T, H, D, N, nt) for nt in range(ch, ch + N + 1)}
-                    if N == 1:
-                        got.add(lengths(T, H, D, 1, ch, packed=False))
                     assert len(got) == 1, (T, N, H, D, got)
                     cut += got != {(0, 0)}
     assert cut > 100
