@@ -38,18 +38,18 @@ STAGE_NAMES = {0: "k_gdn_wy_fwd", 1: "k_gdn_state_fwd_reg", 4: "k_gdn_state_bwd"
 # sources (kernel_sources_sha16()) at that time, and a build whose sources differ reports traffic = null
 # rather than a stale number.
 CALIB_COPY_BYTES = 256 << 20
-MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237262329, "k_gdn_state_fwd_reg": 1120445959, "k_gdn_state_bwd": 946040654,
-                    "k_gdn_bwd_chunk": 1819604917}
-TRAFFIC_SOURCES_SHA16 = "dc1049acbfc894a8"
+MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237263293, "k_gdn_state_fwd_reg": 1117158774, "k_gdn_state_bwd": 946040007,
+                    "k_gdn_bwd_chunk": 1818253639}
+TRAFFIC_SOURCES_SHA16 = "63c5721e0d66b1b6"
 TRAFFIC_SOURCES = ("lmoe_common.hpp", "lmoe_seq.hpp", "lmoe_gdn_wy.hpp", "lmoe_gdn_state.hpp", "lmoe_gdn_state_reg.hpp", "lmoe_gdn_bwd_chunk.hpp",
                    "lmoe_split.hpp", "lmoe_gdn_split.hpp", "lmoe_gdn_fwd.hip", "lmoe_gdn_state.hip", "lmoe_gdn_bwd.hip")
 
 
 # HBM bytes per call of the other contract configurations (bench.py --other-configs), same counters and scaling,
 # summed over the kernels of the call; key = configuration number
-OTHER_TRAFFIC = {"1": 5115605, "2": 272953557, "3": 1281114784, "5": 16629827200, "6": 1445053504, "7": 6572810176,
-                 "8": 1510828587}
-OTHER_TRAFFIC_SHA16 = "14774007b9019ff2"
+OTHER_TRAFFIC = {"1": 5115520, "2": 272947584, "3": 1280976107, "5": 16620092864, "6": 1445203328, "7": 6568638293,
+                 "8": 1510926219}
+OTHER_TRAFFIC_SHA16 = "4e598dd83620abfa"
 
 
 def all_sources_sha16():
