@@ -289,9 +289,9 @@ def neighbours(lib, rows, D, dev, reps):
 def trace_state_fwd(lib, x, dims, work_group=16):
     """Per-phase breakdown of one chunk period of the forward sequential pass (k_gdn_state_fwd_reg) on the headline
     workload: the traced instance of the kernel records the shader clock where each team of the traced work-group
-    arrives at and leaves the two barriers of a chunk and at a few points in between
-    (lmoe_trace_gdn_state_fwd, include/lmoe.h).  Returns averages over the middle chunks of the sequence, in cycles
-    after the release of barrier 1 of the same chunk (negative: before it, i.e. in the previous chunk's phase 2)."""
+    enters the window of a chunk, arrives at and leaves the barrier at its end and at a few points in between
+    (lmoe_trace_gdn_state_fwd, include/lmoe.h).  Returns averages over the middle of the recorded chunks, in cycles
+    after the consumer wave has entered the window."""
     import torch
     from linear_moe_amd import _lib
     from linear_moe_amd.gated_delta_rule import GDNCall
@@ -310,27 +310,22 @@ def trace_state_fwd(lib, x, dims, work_group=16):
     e1.synchronize()
     traced_us = e0.elapsed_time(e1) * 1e3
     t = tr.cpu().view(slots, chunks, marks).double()
-    nch = min(chunks, (T + CH - 1) // CH)
+    nch = min(48, (T + CH - 1) // CH)                             # (the chunks the instance records)
     c0, c1 = nch // 4, nch - nch // 4
-    ref = t[0, c0:c1, 1]                                          # the consumer leaves barrier 1
-    period = float((t[0, c0 + 1:c1 + 1, 1] - t[0, c0:c1, 1]).mean())
-    names = {0: {0: "arrives_b1", 1: "leaves_b1", 5: "kS_formed", 2: "arrives_b2_vnew_written", 3: "leaves_b2",
-                 6: "state_updated", 4: "state_written"},
-             1: {0: "arrives_b1", 1: "leaves_b1", 2: "arrives_b2_qS_formed", 3: "leaves_b2", 4: "o_written"},
-             2: {0: "arrives_b1", 1: "leaves_b1", 6: "k_staged", 2: "arrives_b2_P_formed", 3: "leaves_b2",
-                 4: "stores_issued", 5: "loads_issued"},
-             3: {0: "arrives_b1", 1: "leaves_b1", 2: "arrives_b2_loads_issued", 3: "leaves_b2", 4: "tiles_staged"}}
+    ref = t[0, c0:c1, 0]                                          # the consumer enters the window of the chunk
+    period = float((t[0, c0 + 1:c1 + 1, 0] - t[0, c0:c1, 0]).mean())
+    names = {0: {0: "enters", 1: "kS_formed", 5: "v_new_formed", 6: "state_updated", 2: "arrives_state_written", 3: "leaves"},
+             1: {0: "enters", 1: "o_of_last_chunk_written", 2: "arrives_qS_and_P_formed", 3: "leaves"},
+             2: {0: "enters", 1: "stores_issued", 4: "k_staged", 2: "arrives_loads_issued", 3: "leaves"},
+             3: {0: "enters", 1: "stores_issued", 4: "tiles_staged", 2: "arrives_loads_issued", 3: "leaves"}}
     teams = {0: "consumer_wave", 1: "helper_wave", 2: "loader_team_1", 3: "loader_team_2"}
     out = {}
     for s_, nm in teams.items():
         out[nm] = {}
         for m, label in names[s_].items():
             d = float((t[s_, c0:c1, m] - ref).mean())
-            if m == 0:
-                d += period                                      # arrival at barrier 1 of the NEXT chunk
-                label = "arrives_next_b1"
             out[nm][label] = round(d)
-    return {"metric": "k_gdn_state_fwd_reg: shader-clock cycles after barrier 1 of a chunk, per team (traced build)",
+    return {"metric": "k_gdn_state_fwd_reg: shader-clock cycles inside the window of a chunk, per team (traced build)",
             "unit": "cycles", "work_group": work_group, "chunks_averaged": [c0, c1], "period_cycles": round(period),
             "traced_kernel_us": round(traced_us, 1), "cycles_per_us": round(period * nch / traced_us, 1),
             "teams": out}

@@ -385,14 +385,13 @@ int lmoe_launch_stage(const lmoe_args* a, int32_t op, int32_t stage, void* strea
  * lmoe_chunk_gated_delta_rule_fwd, after its WY preparation has run: lmoe_launch_stage stage 0) with the instance
  * that records the shader clock in work-group `work_group` (over whole sequences, whatever seg_ws: where the entry point
  * cuts the call along T, its results differ from these by rounding), and leaves in `trace` (device memory,
- * int64 [4 slots][128 chunks][8 marks], zero where nothing was recorded; sequences longer than 128 chunks are traced
- * for their first 128) the cycle counter at these points of every chunk:
- *   slot 0, the consumer wave (carries the state):  0 arrives at barrier 1, 1 leaves it, 5 k S formed, 2 arrives at
- *           barrier 2 (v_new written), 3 leaves it, 6 state updated, 4 state written for the next chunk
- *   slot 1, the helper wave (forms the output):     0, 1, 2 (q S formed), 3 as above, 4 o written
- *   slot 2, loader team 1 (k, P; all stores):       0, 1, 2 (tiles staged, results lifted), 3, 4 stores issued,
- *           5 loads issued
- *   slot 3, loader team 2 (q, Tinv, v, gates):      0, 1, 2 loads issued, 3, 4 tiles staged
+ * int64 [4 slots][128 chunks][8 marks], zero where nothing was recorded: the first 48 chunks of a sequence are) the cycle
+ * counter at these points of every chunk's window (there is one barrier per chunk, at the end of its window):
+ *   every slot: 0 enters the window, 2 arrives at the barrier, 3 leaves it
+ *   slot 0, the consumer wave (carries the state):  1 k S formed, 5 v_new formed, 6 state updated
+ *   slot 1, the helper wave (output, P):            1 output of the chunk before formed
+ *   slot 2, loader team 1 (k; stores v_new, P, o):  1 stores issued, 4 k of the next chunk staged
+ *   slot 3, loader team 2 (q, Tinv, v, gates; stores the state): 1 stores issued, 4 tiles of the next chunk staged
  * Instance available for LMOE_BF16, K = V = 128, with tinv and hs given (-24 otherwise). */
 int lmoe_trace_gdn_state_fwd(const lmoe_args* a, int64_t* trace, int32_t work_group, void* stream);
 

@@ -13,21 +13,27 @@
 //     it in.  For that to fit plain 16-byte row reads of the other operand, accumulator rows are NUMBERED accordingly:
 //     block pair (2 s, 2 s + 1), lane group g, element i  <->  index 32 s + 8 g + 4 e + i  (e = block parity).  The row an A
 //     operand lane reads (k, Tinv rows) and the columns a transposing read addresses (k^T) follow that numbering;
-//     nothing is ever permuted in memory.
+//     nothing is ever permuted in memory.  The same registers are 8 consecutive rows of a column: S^T and v_new^T go to
+//     LDS as 16-byte writes.
 //   * w and u are never formed: v_new = Tinv Z costs 6 products (Tinv is lower triangular) on top of X = k S.
-//   * Helper wave j (waves 2, 3) forms the output of the same 16 columns from what the consumers leave in LDS anyway
-//     (S^T at chunk start, which is the checkpoint the loaders store, and v_new): q S in phase 1, P v_new in phase 2,
-//     transposed so that a lane holds four consecutive columns of one token (8-byte writes of o).  
-//   * Loader teams as in k_gdn_state_fwd: team 1 stages k(c+1) in phase 1 and carries all stores; team 2
-//     stages q, Tinv, v, gates of chunk c+1 in phase 2.
-//   * The intra-chunk matrix P = (q k^T) . Gamma is formed here, by the four waves of team 1 in phase 1 (behind their
-//     staging of k, where they would otherwise wait for the consumers): the ten 16 x 16 blocks of the lower
-//     triangle, three or two per wave, from the q and k tiles and the gate table's b row into the P tile that the
-//     helpers read in phase 2.  The WY preparation then reads no q and writes no P, this pass reads none (8 KB per
-//     chunk and work-group less through the CU's memory pipe, which bounds it), and a forward-only call never has P
-//     in memory.  A call that saves for the backward writes P once: every V-slice work-group stores its share of
-//     the rows.  (Formed on the helper waves instead, as registers that feed (P v_new)^T directly, the pass was 45 us
-//     slower at T = 8192: 48 more products per chunk on a wave that shares a phase with the consumers.)
+//   * ONE barrier per chunk.  Every tile exists twice (156 KB of LDS at K = 128) and a window reads only what the window
+//     before it completed, so no team waits for another inside a window:
+//       consumers, window c:   v_new(c), S at the start of chunk c + 1
+//       helpers, window c:     the output of chunk c - 1 (its q S is in their registers, v_new and P of it in LDS), then
+//                              q S and P of chunk c
+//       team 1, window c:      stores v_new(c - 1), P(c - 1), o(c - 2); stages k(c + 1) and requests the next
+//       team 2, window c:      stores S at the start of chunk c; stages q, Tinv, v, gates of c + 1 and requests the next
+//     (Two barriers per chunk, P formed by team 1 in front of the second one, which the consumers waited for: a window was 4600
+//     cycles, of which the consumers worked 3700; now 3500, and 3300 of them are the consumers' reads.  B=2 H=16 T=2048 K=V=128
+//     saving: 58 -> 49 us; forward-only B=4 T=8192: 232 -> 191; the saving call of that size 268 -> 255, now bound by
+//     the 600 MB it writes.)
+//   * Helper wave j (waves 2, 3) forms the output of the columns 16 j .. from S^T and v_new^T in LDS, transposed so that
+//     a lane holds four consecutive columns of one token, and five of the ten blocks of the lower triangle of
+//     P = (q k^T) . Gamma over the q rows it reads for q S anyway (two rows of k blocks are all that P adds to its reads; on the
+//     loader waves P took 80 KB of reads per chunk).  P never passes through memory on its way to the output; a call
+//     that saves for the backward stores it once: every V-slice work-group its share of the rows.
+//   * The loaders' stores lie behind no branch (the first two windows are peeled off), so that a wait for a load never waits
+//     for stores behind it.
 #pragma once
 #include <type_traits>
 #include "lmoe_gdn_state.hpp"
@@ -40,7 +46,7 @@ namespace lmoe {
 // stall the traced wave at the issue); the traced work-group copies them out when it ends.  Slots: 0 consumer wave,
 // 1 helper wave, 2 loader team 1, 3 loader team 2; marks per (slot, chunk): see lmoe_trace_gdn_state_fwd in
 // include/lmoe.h.  Chunks beyond TRACE_CHUNKS are not recorded.
-constexpr int TRACE_CHUNKS = 128, TRACE_MARKS = 8, TRACE_SLOTS = 4;
+constexpr int TRACE_CHUNKS = 128, TRACE_MARKS = 8, TRACE_SLOTS = 4, TRACE_LDS_CHUNKS = 48;
 
 // A fragment of k^T for the state block mi (see the numbering above): contraction = tokens k0 + 8 g .. + 7 (rows of
 // the tile), lane fr <-> state row  32 (mi / 2) + 8 (fr / 4) + 4 (mi % 2) + fr % 4  (columns of the tile)
@@ -54,36 +60,45 @@ __device__ __forceinline__ bf16x8 load_frag_t_state(const bf16* tile, int ld, in
 }
 // (frag_of_blocks, lmoe_common.hpp: two accumulator blocks -> the 8 contraction elements of an operand)
 
+// f(number, ti, tj) for the blocks (ti >= tj) of the lower triangle of a 4 x 4 arrangement with tj = TA or tj = TB = 3 - TA
+template <int TA, int TB, int X = 0, int TI = TA, int TJ = TA, typename F>
+__device__ __forceinline__ void static_for_blocks(F&& f) {
+  if constexpr (TI < 4) {
+    f(std::integral_constant<int, X>(), std::integral_constant<int, TI>(), std::integral_constant<int, TJ>());
+    static_for_blocks<TA, TB, X + 1, TI + 1, TJ>(f);
+  } else if constexpr (TJ == TA) {
+    static_for_blocks<TA, TB, X, TB, TB>(f);
+  }
+}
+
 template <int K, int V, bool SAVE, bool TRACE = false, bool CUT = false>
 __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   typedef bf16 T;
   constexpr int BV = 32;
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int KT = K / 16, KS = K / 32;
-  // register sets per prefetch ring (deeper rings were measured: 3 and 4 sets for either team change nothing, the pass
-  // is bound by what the memory system delivers for its traffic, not by the lead of its requests)
-  constexpr int LPA = GdnStateCfg<T>::LPF, LPB = GdnStateCfg<T>::LPF;
-  __shared__ __attribute__((aligned(16))) T s_k[2 * CH * LDK];      // k [64][K] of chunks c, c + 1
-  __shared__ __attribute__((aligned(16))) T s_q[CH * LDK];          // q [64][K]
-  __shared__ __attribute__((aligned(16))) T s_ti[CH * LDC];         // Tinv [64][64]
-  __shared__ __attribute__((aligned(16))) T s_p[CH * LDC];          // P [64][64]
-  __shared__ __attribute__((aligned(16))) T s_v[CH * LDU];          // v [64][BV]
-  __shared__ __attribute__((aligned(16))) T s_hT[BV * LDK];         // S^T [BV][K] at chunk start
-  __shared__ __attribute__((aligned(16))) T s_vn[CH * LDU];         // v_new [64][BV]
-  __shared__ __attribute__((aligned(16))) T s_o[CH * LDU];          // o [64][BV]
-  __shared__ __attribute__((aligned(16))) float s_f[64], s_be[64];  // beta e^{b}, beta
-  __shared__ __attribute__((aligned(16))) float s_b[64];            // cumulative log-decay b
-  __shared__ __attribute__((aligned(16))) float s_eb[2][64], s_ed[2][64];
-  __shared__ float s_dec[2];                                        // e^{b_C}; buffer c & 1
-  __shared__ long long s_tr[TRACE ? TRACE_SLOTS * TRACE_CHUNKS * TRACE_MARKS : 1];
+  constexpr int LPA = GdnStateCfg<T>::LPF, LPB = GdnStateCfg<T>::LPF;       // register sets per prefetch ring (3: no change)
+  // every tile twice: buffer c & 1 belongs to chunk c (s_hT: the state at its start)
+  __shared__ __attribute__((aligned(16))) T s_k[2][CH * LDK];       // k [64][K]
+  __shared__ __attribute__((aligned(16))) T s_q[2][CH * LDK];       // q [64][K]
+  __shared__ __attribute__((aligned(16))) T s_ti[2][CH * LDC];      // Tinv [64][64]
+  __shared__ __attribute__((aligned(16))) T s_p[2][CH * LDC];       // P [64][64]
+  __shared__ __attribute__((aligned(16))) T s_v[2][CH * LDU];       // v [64][BV]
+  __shared__ __attribute__((aligned(16))) T s_hT[2][BV * LDK];      // S^T [BV][K]
+  __shared__ __attribute__((aligned(16))) T s_vT[2][BV * LDC];      // v_new^T [BV][64]
+  __shared__ __attribute__((aligned(16))) T s_o[2][CH * LDU];       // o [64][BV]
+  __shared__ __attribute__((aligned(16))) float s_gt[2][GATE_ROWS][CH];     // e^b, e^{b_C - b}, beta, beta e^b, b
+  __shared__ uint32_t s_tr[TRACE ? TRACE_SLOTS * TRACE_LDS_CHUNKS * TRACE_MARKS : 1];
+  __shared__ long long s_tr0;
   auto TR = [&](int slot, int c, int mark) {
     if constexpr (TRACE) {
-      if ((int)blockIdx.x == traced_wg && (threadIdx.x & 63) == 0 && c < TRACE_CHUNKS)
-        s_tr[(slot * TRACE_CHUNKS + c) * TRACE_MARKS + mark] = __builtin_readcyclecounter();
+      if ((int)blockIdx.x == traced_wg && (threadIdx.x & 63) == 0 && c < TRACE_LDS_CHUNKS)
+        s_tr[(slot * TRACE_LDS_CHUNKS + c) * TRACE_MARKS + mark] = (uint32_t)__builtin_readcyclecounter();
     }
   };
   if constexpr (TRACE) {
-    for (int i = threadIdx.x; i < TRACE_SLOTS * TRACE_CHUNKS * TRACE_MARKS; i += 3 * NTHR) s_tr[i] = 0;
+    for (int i = threadIdx.x; i < TRACE_SLOTS * TRACE_LDS_CHUNKS * TRACE_MARKS; i += 3 * NTHR) s_tr[i] = 0;
+    if (threadIdx.x == 0) s_tr0 = __builtin_readcyclecounter();
     __syncthreads();
   }
 
@@ -113,8 +128,14 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
   typedef TileIO<T, CH, CH> IOP;
   typedef TileIO<T, BV, K> IOHT;
 
+  auto store_state = [&](int c) {             // hs(c) <- S^T at the start of chunk c
+    typename IOHT::Regs rh;
+    IOHT::load_lds(rh, s_hT[c & 1], LDK);
+    IOHT::template store_global<true>(rh, (T*)a.hs + (((int64_t)(sq.chunk0 + c) * a.H + h) * V + v0) * K, K, BV);
+  };
+
   if (team == 1) {
-    // ------------------------- loaders, ring A (k, P) and all stores ----------------------
+    // ------------------------- loaders, ring A (k) and all stores -------------------------
     struct PreA { typename IOK::Regs rk; int len; };
     PreA pa[LPA];
     auto issue_a = [&](PreA& P, int c) {      // always issued, chunk index clamped (see k_gdn_state_fwd)
@@ -123,135 +144,88 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
       P.len = min(CH, sq.len - c * CH);
       IOK::load_nomask(P.rk, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, P.len);
     };
-    auto stage_k = [&](PreA& P, int c) {
+    auto stage_a = [&](PreA& P, int c) {
       IOK::mask(P.rk, P.len);
-      IOK::store_lds(P.rk, s_k + (c & 1) * CH * LDK, LDK);
+      IOK::store_lds(P.rk, s_k[c & 1], LDK);
     };
-    // this work-group's share of the rows of P (formed below, the whole matrix in s_p): 64 / NVS rows, every
-    // thread stores (threads beyond the share repeat a row with the same bytes: no store sits behind a branch)
-    constexpr int PROWS = CH / NVS;
-    const int pidx = (threadIdx.x & (NTHR - 1)) % (PROWS * 8);
-    const int prow = vsl * PROWS + pidx / 8, pcol = (pidx % 8) * 8;
-    auto store_result = [&](const typename IOV::Regs& r, const lmoe_tensor& dst, int c) {
+    // this work-group's share of the rows of P (formed by the helpers, the whole matrix in s_p): 64 / NVS rows, the same
+    // number of bytes from every thread (128 threads with 16 bytes each and 128 that repeated them, so that no store sat
+    // behind a branch, wrote P twice: 51 MB more of 603 at B=4 T=8192 H=16, and the writes bound a saving call)
+    constexpr int PROWS = CH / NVS, PVEC = CH * PROWS / NTHR;
+    typedef T pvec __attribute__((ext_vector_type(PVEC)));
+    const int pidx = threadIdx.x & (NTHR - 1);
+    const int prow = vsl * PROWS + pidx * PVEC / CH, pcol = pidx * PVEC % CH;
+    const int wt = wave_id() - 4;
+    auto store_saved = [&](int c) {           // v_new(c) (back in [token][column] through transposing reads) and P(c)
+      const pvec pv = *(const pvec*)(s_p[c & 1] + prow * LDC + pcol);
+      const typename ET<T>::frag x = ET<T>::load_frag_t(s_vT[c & 1], LDC, 0, 16 * wt, l);
+      __builtin_nontemporal_store(pv, (pvec*)((T*)a.pmat + (((int64_t)(sq.chunk0 + c) * a.H + h) * CH + prow) * CH + pcol));
+      // (all 64 rows: those past the end of a partial chunk are zero)
+      __builtin_nontemporal_store(x, (typename ET<T>::vec*)(slice_ptr<T>(a.vnew, sq.chunk0 + c, h, a.H, V, v0) + (16 * wt + (l & 15)) * SLICE_COLS + 8 * (l >> 4)));
+    };
+    auto store_out = [&](int c) {
       const int tok = sq.tok0 + c * CH;
       const int len = min(CH, sq.len - c * CH);
-      IOV::template store_global<true>(r, row_ptr<T>(dst, sq.b, tok, h) + v0, dst.st, len);
+      typename IOV::Regs ro;
+      IOV::load_lds_clamped(ro, s_o[c & 1], LDU, len);
+      IOV::template store_global_clamped<false>(ro, row_ptr<T>(a.o, sq.b, tok, h) + v0, a.o.st, len);
     };
-    // P = (q k^T) . Gamma of the chunk in the tiles, Gamma_ij = e^{b_i - b_j} for i >= j (rows past the end of a
-    // partial chunk: 0; its columns are zero through k): block number x = wave, wave + 4, wave + 8 of the ten blocks
-    // (ti, tj <= ti) of the lower triangle, formed transposed (k rows as the A operand) so that a lane holds four
-    // consecutive columns of one row (8-byte writes).  The six blocks above the diagonal are cleared once.
-    const int wt = wave_id() - 4;
-    auto form_p = [&](int c) {
-      const int fr = l & 15, g = l >> 4;
-      const T* s_kc = s_k + (c & 1) * CH * LDK;
-      const int len = min(CH, sq.len - c * CH);
-      int ti[3], tj[3];
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        const int idx = min(wt + 4 * x, 9);
-        ti[x] = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-        tj[x] = idx - ti[x] * (ti[x] + 1) / 2;
-      }
-      const int nx = wt < 2 ? 3 : 2;        // wave-uniform
-      f32x4 pc[3];
-#pragma unroll
-      for (int x = 0; x < 3; ++x) pc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
-      typename ET<T>::frag fq[2][3], fk[2][3];
-      auto fetch = [&](int ks, int buf) {
-#pragma unroll
-        for (int x = 0; x < 3; ++x) {
-          fq[buf][x] = ET<T>::load_frag(s_q + (16 * ti[x] + fr) * LDK + 32 * ks + 8 * g);
-          fk[buf][x] = ET<T>::load_frag(s_kc + (16 * tj[x] + fr) * LDK + 32 * ks + 8 * g);
-        }
-      };
-      fetch(0, 0);
-      // the decay factors (masked) while the first fragments are on their way: behind the products only a multiply,
-      // a conversion and the write are left
-      f32x4 gm[3];
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        const int i = 16 * ti[x] + fr, j0 = 16 * tj[x] + 4 * g;
-        const float bi = s_b[i];
-        const f32x4 bj = *(const f32x4*)&s_b[j0];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) gm[x][e] = (i >= j0 + e && i < len) ? texp<T>(bi - bj[e]) : 0.f;
-      }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) fetch(ks + 1, (ks + 1) & 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int x = 0; x < 3; ++x)
-          if (x < nx) ET<T>::mma(pc[x], fk[ks & 1][x], fq[ks & 1][x]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int x = 0; x < 3; ++x) {
-        if (x < nx) {
-          const int i = 16 * ti[x] + fr, j0 = 16 * tj[x] + 4 * g;
-          bf16x4 y;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = (bf16)(pc[x][e] * gm[x][e]);
-          *(bf16x4*)(s_p + i * LDC + j0) = y;
-        }
-      }
-    };
+    // the blocks of P above the diagonal, which no helper writes, are cleared once
     {
       const int t = threadIdx.x & (NTHR - 1), r = t >> 4, cc = t & 15;
 #pragma unroll
       for (int I = 0; I < 3; ++I)
 #pragma unroll
-        for (int J = I + 1; J < 4; ++J) s_p[(16 * I + r) * LDC + 16 * J + cc] = (T)0.f;
+        for (int J = I + 1; J < 4; ++J) s_p[0][(16 * I + r) * LDC + 16 * J + cc] = s_p[1][(16 * I + r) * LDC + 16 * J + cc] = (T)0.f;
     }
 #pragma unroll
     for (int j = 0; j < LPA; ++j) issue_a(pa[j], j);
     wait_all_loads();
-    stage_k(pa[0], 0);
-    lds_barrier();                                                                       // B0
-    typename IOHT::Regs rh;
-    typename IOV::Regs rvn, ro;
-    ring_loop<LPA>(sq.nchunks, [&](auto slot, const int c) {
-      constexpr int j = decltype(slot)::value, jn = (j + 1) % LPA;
+    stage_a(pa[0], 0);
+    issue_a(pa[0], LPA);
+    lds_barrier();
+    auto window = [&](auto slot, const int c, auto stores) {
+      constexpr int jn = (decltype(slot)::value + 1) % LPA;
       if (wave_id() == 4) TR(2, c, 0);
-      lds_barrier();                                                                     // B1
+      stores(c);
       if (wave_id() == 4) TR(2, c, 1);
-      stage_k(pa[jn], c + 1);               // (past the last chunk: a clamped copy of it, never used)
-      if constexpr (SAVE) IOHT::load_lds(rh, s_hT, LDK);
-      IOV::load_lds(ro, s_o, LDU);
-      if (wave_id() == 4) TR(2, c, 6);
-      // behind the staging: the first thousand cycles after the barrier every wave of the work-group reads LDS and
-      // a read of this team's takes that long to come back (measured: formed first, P was ready 250 cycles later
-      // and k staged 600 cycles later than in this order)
-      form_p(c);
-      if (wave_id() == 4) TR(2, c, 2);
-      lds_barrier();                                                                     // B2
-      if (wave_id() == 4) TR(2, c, 3);
-      if constexpr (SAVE) {
-        IOV::load_lds(rvn, s_vn, LDU);
-        const typename ET<T>::vec pv = *(const typename ET<T>::vec*)(s_p + prow * LDC + pcol);
-        IOHT::template store_global<true>(rh, (T*)a.hs + (((int64_t)(sq.chunk0 + c) * a.H + h) * V + v0) * K, K, BV);
-        __builtin_nontemporal_store(pv, (typename ET<T>::vec*)((T*)a.pmat + (((int64_t)(sq.chunk0 + c) * a.H + h) * CH + prow) * CH + pcol));
-      }
-      if (c > 0) store_result(ro, a.o, c - 1);
-      if constexpr (SAVE) IOV::template store_global<true>(rvn, slice_ptr<T>(a.vnew, sq.chunk0 + c, h, a.H, V, v0), SLICE_COLS, min(CH, sq.len - c * CH));
+      stage_a(pa[jn], c + 1);               // (past the last chunk: a clamped copy of it, never used)
       if (wave_id() == 4) TR(2, c, 4);
-      issue_a(pa[j], c + LPA);
-      if (wave_id() == 4) TR(2, c, 5);
-    });
+      issue_a(pa[jn], c + 1 + LPA);
+      if (wave_id() == 4) TR(2, c, 2);
+      lds_barrier();
+      if (wave_id() == 4) TR(2, c, 3);
+    };
+    // the first two windows have fewer results to store: outside of the loop, whose stores then lie behind no branch
+    window(std::integral_constant<int, 0>(), 0, [](int) {});
+    if (sq.nchunks > 1) {
+      window(std::integral_constant<int, 1 % LPA>(), 1, [&](int c) { if constexpr (SAVE) store_saved(c - 1); });
+      ring_loop<LPA>(sq.nchunks - 2, [&](auto slot, const int c2) {
+        window(std::integral_constant<int, (decltype(slot)::value + 2) % LPA>(), c2 + 2, [&](int c) {
+          if constexpr (SAVE) store_saved(c - 1);
+          store_out(c - 2);
+        });
+      });
+    }
+    if constexpr (SAVE) store_saved(sq.nchunks - 1);
+    if (sq.nchunks > 1) store_out(sq.nchunks - 2);
     lds_barrier();                                                                       // o of the last chunk
-    IOV::load_lds(ro, s_o, LDU);
-    store_result(ro, a.o, sq.nchunks - 1);
+    store_out(sq.nchunks - 1);
     if constexpr (TRACE) {
       if ((int)blockIdx.x == traced_wg)
-        for (int i = threadIdx.x & (NTHR - 1); i < TRACE_SLOTS * TRACE_CHUNKS * TRACE_MARKS; i += NTHR) tr[i] = s_tr[i];
+        for (int i = threadIdx.x & (NTHR - 1); i < TRACE_SLOTS * TRACE_CHUNKS * TRACE_MARKS; i += NTHR) {
+          const int c = i / TRACE_MARKS % TRACE_CHUNKS, slot = i / (TRACE_MARKS * TRACE_CHUNKS);
+          const uint32_t x = c < TRACE_LDS_CHUNKS ? s_tr[(slot * TRACE_LDS_CHUNKS + c) * TRACE_MARKS + i % TRACE_MARKS] : 0u;
+          tr[i] = x ? s_tr0 + (long long)(uint32_t)(x - (uint32_t)s_tr0) : 0;
+        }
     }
     return;
   }
   if (team == 2) {
     // ------------------------- loaders, ring B (q, Tinv, v, gates) ------------------------
-    struct PreB { typename IOK::Regs rq; typename IOP::Regs rt; typename IOV::Regs rv; float eb, ed, be, f, bb; int len; };
+    struct PreB { typename IOK::Regs rq; typename IOP::Regs rt; typename IOV::Regs rv; float gt, b; int len; };
     PreB pb[LPB];
+    const int wt = wave_id() - 8;            // each wave carries one row of the gate table; b: the last row, every wave
     auto issue_b = [&](PreB& P, int c) {
       c = min(c, sq.nchunks - 1);
       const int tok = sq.tok0 + c * CH;
@@ -260,15 +234,13 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
       IOP::load_nomask(P.rt, (const T*)a.tinv + ((int64_t)(sq.chunk0 + c) * a.H + h) * CH * CH, CH, CH);
       IOV::load_nomask(P.rv, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, P.len);
       const float* gc = a.gcum + ((int64_t)(sq.chunk0 + c) * a.H + h) * GATE_ROWS * CH;
-      P.eb = gc[l];
-      P.ed = gc[CH + l];
-      P.be = gc[2 * CH + l];
-      P.f = gc[3 * CH + l];
-      P.bb = gc[4 * CH + l];
+      P.gt = gc[wt * CH + l];
+      P.b = gc[4 * CH + l];
     };
     auto stage_b = [&](PreB& P, int buf) {
-      IOK::store_lds(P.rq, s_q, LDK);       // rows past the end only reach output rows that are not stored
-      IOP::store_lds(P.rt, s_ti, LDC);
+      IOK::mask(P.rq, P.len);                // (rows past the end: P is zero there as the backward expects it)
+      IOK::store_lds(P.rq, s_q[buf], LDK);
+      IOP::store_lds(P.rt, s_ti[buf], LDC);
       if (a.v_act) {                         // v = silu(v as given): the activation in front of the op, applied here
 #pragma unroll
         for (int p = 0; p < IOV::PASSES; ++p)
@@ -276,32 +248,27 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
           for (int i = 0; i < IOV::VEC; ++i) P.rv.v[p][i] = ET<T>::from_f(silu_of(ET<T>::to_f(P.rv.v[p][i])));
       }
       IOV::mask(P.rv, P.len);
-      IOV::store_lds(P.rv, s_v, LDU);
-      if (wave_id() == 8) {
-        s_be[l] = P.be;
-        s_f[l] = P.f;
-        s_b[l] = P.bb;
-        s_eb[buf][l] = P.eb;
-        s_ed[buf][l] = P.ed;
-        if (l == 63) s_dec[buf] = P.eb;
-      }
+      IOV::store_lds(P.rv, s_v[buf], LDU);
+      s_gt[buf][wt][l] = P.gt;
+      s_gt[buf][4][l] = P.b;                 // (the same from all four)
     };
 #pragma unroll
     for (int j = 0; j < LPB; ++j) issue_b(pb[j], j);
     wait_all_loads();
     stage_b(pb[0], 0);
-    lds_barrier();                                                                       // B0
+    issue_b(pb[0], LPB);
+    lds_barrier();
     ring_loop<LPB>(sq.nchunks, [&](auto slot, const int c) {
-      constexpr int j = decltype(slot)::value, jn = (j + 1) % LPB;
+      constexpr int jn = (decltype(slot)::value + 1) % LPB;
       if (wave_id() == 8) TR(3, c, 0);
-      lds_barrier();                                                                     // B1
+      if constexpr (SAVE) store_state(c);
       if (wave_id() == 8) TR(3, c, 1);
-      issue_b(pb[j], c + LPB);              // chunk c was staged before this barrier: refill its set
-      if (wave_id() == 8) TR(3, c, 2);
-      lds_barrier();                                                                     // B2
-      if (wave_id() == 8) TR(3, c, 3);
-      if (c + 1 < sq.nchunks) stage_b(pb[jn], (c + 1) & 1);
+      stage_b(pb[jn], (c + 1) & 1);         // (past the last chunk: a clamped copy of it, never used)
       if (wave_id() == 8) TR(3, c, 4);
+      issue_b(pb[jn], c + 1 + LPB);
+      if (wave_id() == 8) TR(3, c, 2);
+      lds_barrier();
+      if (wave_id() == 8) TR(3, c, 3);
     });
     lds_barrier();
     return;
@@ -311,69 +278,114 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
   const int fr = l & 15, g = l >> 4;
   const float scale = a.scale;
   if (wv >= 2) {
-    // ------------------------------ helpers: the output ----------------------------------
-    const int j = wv - 2;
-    lds_barrier();                                                                       // B0
-    for (int c = 0; c < sq.nchunks; ++c) {
-      const int cur = c & 1;
-      if (wv == 2) TR(1, c, 0);
-      lds_barrier();                                                                     // B1
-      if (wv == 2) TR(1, c, 1);
-      // (q S)^T: rows = columns of the slice (S^T as the A operand, read from the checkpoint tile), columns = tokens
-      f32x4 oa[4];
+    // --------------------- helpers: P of the chunk and the output of its columns ---------------------
+    __builtin_amdgcn_s_setprio(2);
+    // helper J: output columns 16 J .. of the slice; blocks (ti, tj) of P with tj = J and tj = 3 - J (five each)
+    auto help = [&](auto which) {
+      constexpr int J = decltype(which)::value;
+      constexpr int TA = J, TB = 3 - J;          // its two rows of k blocks
+      f32x4 oa[4];                               // (q S)^T of a chunk: columns of the slice x tokens 16 t ..
+      typename ET<T>::frag fv[2], fp[6];
+      // o(c) = scale (e^b q S + P v_new), in the window behind the one that formed q S, P and v_new
+      auto finish_fetch = [&](int c) {
+        const T* s_pc = s_p[c & 1];
+        const T* s_vc = s_vT[c & 1];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) oa[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-      {
-        typename ET<T>::frag fs[KS], fq[2][4];
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) fs[ks] = ET<T>::load_frag(s_hT + (16 * j + fr) * LDK + 32 * ks + 8 * g);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) fq[0][t] = ET<T>::load_frag(s_q + (16 * t + fr) * LDK + 8 * g);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          if (ks + 1 < KS) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) fq[(ks + 1) & 1][t] = ET<T>::load_frag(s_q + (16 * t + fr) * LDK + 32 * (ks + 1) + 8 * g);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int t = 0; t < 4; ++t) ET<T>::mma(oa[t], fs[ks], fq[ks & 1][t]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) oa[t] *= s_eb[cur][16 * t + fr];
-      if (wv == 2) TR(1, c, 2);
-      lds_barrier();                                                                     // B2
-      if (wv == 2) TR(1, c, 3);
-      {
-        // + (P v_new)^T: v_new^T through transposing reads of the tile the consumers wrote; P is lower triangular
-        typename ET<T>::frag fv[2], fp[6];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) fv[s] = ET<T>::load_frag_t(s_vn, LDU, 32 * s, 16 * j, l);
-        fp[0] = ET<T>::load_frag(s_p + (0 + fr) * LDC + 8 * g);
-        fp[1] = ET<T>::load_frag(s_p + (16 + fr) * LDC + 8 * g);
-        fp[2] = ET<T>::load_frag(s_p + (32 + fr) * LDC + 8 * g);
-        fp[3] = ET<T>::load_frag(s_p + (48 + fr) * LDC + 8 * g);
-        fp[4] = ET<T>::load_frag(s_p + (32 + fr) * LDC + 32 + 8 * g);
-        fp[5] = ET<T>::load_frag(s_p + (48 + fr) * LDC + 32 + 8 * g);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int s = 0; s < 2; ++s) fv[s] = ET<T>::load_frag(s_vc + (16 * J + fr) * LDC + 32 * s + 8 * g);
+        fp[0] = ET<T>::load_frag(s_pc + (0 + fr) * LDC + 8 * g);
+        fp[1] = ET<T>::load_frag(s_pc + (16 + fr) * LDC + 8 * g);
+        fp[2] = ET<T>::load_frag(s_pc + (32 + fr) * LDC + 8 * g);
+        fp[3] = ET<T>::load_frag(s_pc + (48 + fr) * LDC + 8 * g);
+        fp[4] = ET<T>::load_frag(s_pc + (32 + fr) * LDC + 32 + 8 * g);
+        fp[5] = ET<T>::load_frag(s_pc + (48 + fr) * LDC + 32 + 8 * g);
+      };
+      auto finish = [&](int c) {
         ET<T>::mma(oa[0], fv[0], fp[0]);
         ET<T>::mma(oa[1], fv[0], fp[1]);
         ET<T>::mma(oa[2], fv[0], fp[2]);
         ET<T>::mma(oa[3], fv[0], fp[3]);
         ET<T>::mma(oa[2], fv[1], fp[4]);
         ET<T>::mma(oa[3], fv[1], fp[5]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        oa[t] *= scale;
-        acc_to_lds_t<T>(oa[t], s_o, LDU, 16 * j, 16 * t, l);                             // o [token][column]: 8-byte writes
+        for (int t = 0; t < 4; ++t) {
+          oa[t] *= scale;
+          acc_to_lds_t<T>(oa[t], s_o[c & 1], LDU, 16 * J, 16 * t, l);                    // o [token][column]: 8-byte writes
+        }
+      };
+      lds_barrier();
+      for (int c = 0; c < sq.nchunks; ++c) {
+        const int cur = c & 1;
+        if (J == 0) TR(1, c, 0);
+        const T *s_kc = s_k[cur], *s_qc = s_q[cur], *s_hc = s_hT[cur];
+        typename ET<T>::frag fs[2], fq[2][4], fk[2][2];
+        auto fetch = [&](int ks, int buf) {
+          fs[buf] = ET<T>::load_frag(s_hc + (16 * J + fr) * LDK + 32 * ks + 8 * g);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) fq[buf][t] = ET<T>::load_frag(s_qc + (16 * t + fr) * LDK + 32 * ks + 8 * g);
+          fk[buf][0] = ET<T>::load_frag(s_kc + (16 * TA + fr) * LDK + 32 * ks + 8 * g);
+          fk[buf][1] = ET<T>::load_frag(s_kc + (16 * TB + fr) * LDK + 32 * ks + 8 * g);
+        };
+        if (c > 0) finish_fetch(c - 1);
+        f32x4 bj[2];
+        float bi[4], eb[4];
+        bj[0] = *(const f32x4*)&s_gt[cur][4][16 * TA + 4 * g];
+        bj[1] = *(const f32x4*)&s_gt[cur][4][16 * TB + 4 * g];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) { bi[t] = s_gt[cur][4][16 * t + fr]; eb[t] = s_gt[cur][0][16 * t + fr]; }
+        fetch(0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c > 0) finish(c - 1);
+        if (J == 0) TR(1, c, 1);
+        // the decay factors of P, Gamma_ij = e^{b_i - b_j} for i >= j, while the fragments are on their way (rows past
+        // the end of a partial chunk: q is zero there)
+        f32x4 gm[5];
+        static_for_blocks<TA, TB>([&](auto x, auto ti, auto tj) {
+          constexpr int X = decltype(x)::value, TI = decltype(ti)::value, TJ = decltype(tj)::value;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float y = texp<T>(bi[TI] - bj[TJ == TA ? 0 : 1][e]);
+            gm[X][e] = (TI > TJ || fr >= 4 * g + e) ? y : 0.f;
+          }
+        });
+        // (q S)^T and, over the same q rows, its blocks of P = (q k^T) . Gamma, formed transposed (k rows as the A
+        // operand) so that a lane holds four consecutive columns of one row (8-byte writes)
+        f32x4 pc[5];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) oa[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < 5; ++x) pc[x] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int bf = ks & 1;
+          if (ks + 1 < KS) fetch(ks + 1, bf ^ 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) ET<T>::mma(oa[t], fs[bf], fq[bf][t]);
+          static_for_blocks<TA, TB>([&](auto x, auto ti, auto tj) {
+            constexpr int X = decltype(x)::value, TI = decltype(ti)::value, TJ = decltype(tj)::value;
+            ET<T>::mma(pc[X], fk[bf][TJ == TA ? 0 : 1], fq[bf][TI]);
+          });
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        static_for_blocks<TA, TB>([&](auto x, auto ti, auto tj) {
+          constexpr int X = decltype(x)::value, TI = decltype(ti)::value, TJ = decltype(tj)::value;
+          bf16x4 y;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = (bf16)(pc[X][e] * gm[X][e]);
+          *(bf16x4*)(s_p[cur] + (16 * TI + fr) * LDC + 16 * TJ + 4 * g) = y;
+        });
+#pragma unroll
+        for (int t = 0; t < 4; ++t) oa[t] *= eb[t];
+        if (J == 0) TR(1, c, 2);
+        lds_barrier();
+        if (J == 0) TR(1, c, 3);
       }
-      if (wv == 2) TR(1, c, 4);
-    }
-    lds_barrier();
+      finish_fetch(sq.nchunks - 1);
+      finish(sq.nchunks - 1);
+      lds_barrier();
+    };
+    if (wv == 2) help(std::integral_constant<int, 0>());
+    else help(std::integral_constant<int, 1>());
     return;
   }
 
@@ -395,62 +407,81 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[mi][i] = h0[(int64_t)idx_of(mi, i) * V + vc];
   }
-  auto put_state = [&]() {                           // S^T [column][K]: four consecutive rows per lane and block
+  // the state as the operand of the next chunk and, the same registers, as S^T [column][K]: 8 consecutive rows per lane
+  typename ET<T>::frag bS[KS];
+  auto put_state = [&](int buf) {
 #pragma unroll
-    for (int mi = 0; mi < KT; ++mi) {
-      bf16x4 x;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = (bf16)S[mi][i];
-      *(bf16x4*)(s_hT + (16 * j + fr) * LDK + idx_of(mi, 0)) = x;
+    for (int ks = 0; ks < KS; ++ks) {
+      bS[ks] = frag_of_blocks(S[2 * ks], S[2 * ks + 1]);
+      *(bf16x8*)(s_hT[buf] + (16 * j + fr) * LDK + 32 * ks + 8 * g) = bS[ks];
     }
   };
-  put_state();
-  lds_barrier();                                                                         // B0
+  put_state(0);
+  lds_barrier();
   for (int c = 0; c < sq.nchunks; ++c) {
     const int cur = c & 1;
-    const T* s_kc = s_k + cur * CH * LDK;
-    typename ET<T>::frag bS[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) bS[ks] = frag_of_blocks(S[2 * ks], S[2 * ks + 1]);
+    const T* s_kc = s_k[cur];
     if (wv == 0) TR(0, c, 0);
-    lds_barrier();                                                                       // B1
-    if (wv == 0) TR(0, c, 1);
-    // X = k S
+    // X = k S; beside it, off the chain, what does not depend on it: e^{b_C} S, beta v
     f32x4 X[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) X[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    typename ET<T>::frag fv[2], fti[6];
-    f32x4 be[2][2], ff[2][2];
+    typename ET<T>::frag fti[6];
+    f32x4 bv[2][2], ff[2][2];
     {
-      typename ET<T>::frag fk[2][4];
+      typename ET<T>::frag fk[2][4], fv[2];
+      f32x4 be[2][2];
 #pragma unroll
       for (int t = 0; t < 4; ++t) fk[0][t] = ET<T>::load_frag(s_kc + arow_of(t) * LDK + 8 * g);
+      const float dec = s_gt[cur][0][CH - 1];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         if (ks + 1 < KS) {
 #pragma unroll
           for (int t = 0; t < 4; ++t) fk[(ks + 1) & 1][t] = ET<T>::load_frag(s_kc + arow_of(t) * LDK + 32 * (ks + 1) + 8 * g);
-        } else {
-          // what follows the product, requested while it runs: v^T, beta, beta e^{b}, and the six Tinv fragments
+        }
+        if (ks == KS - 2) {
 #pragma unroll
           for (int s = 0; s < 2; ++s) {
-            fv[s] = ET<T>::load_frag_t(s_v, LDU, 32 * s, 16 * j, l);
-            be[s][0] = *(const f32x4*)&s_be[32 * s + 8 * g]; be[s][1] = *(const f32x4*)&s_be[32 * s + 8 * g + 4];
-            ff[s][0] = *(const f32x4*)&s_f[32 * s + 8 * g]; ff[s][1] = *(const f32x4*)&s_f[32 * s + 8 * g + 4];
+            fv[s] = ET<T>::load_frag_t(s_v[cur], LDU, 32 * s, 16 * j, l);
+            be[s][0] = *(const f32x4*)&s_gt[cur][2][32 * s + 8 * g]; be[s][1] = *(const f32x4*)&s_gt[cur][2][32 * s + 8 * g + 4];
           }
+        }
+        if (ks == KS - 1) {
 #pragma unroll
-          for (int t = 0; t < 4; ++t) fti[t] = ET<T>::load_frag(s_ti + arow_of(t) * LDC + 8 * g);
-          fti[4] = ET<T>::load_frag(s_ti + arow_of(2) * LDC + 32 + 8 * g);
-          fti[5] = ET<T>::load_frag(s_ti + arow_of(3) * LDC + 32 + 8 * g);
+          for (int s = 0; s < 2; ++s) { ff[s][0] = *(const f32x4*)&s_gt[cur][3][32 * s + 8 * g]; ff[s][1] = *(const f32x4*)&s_gt[cur][3][32 * s + 8 * g + 4]; }
+#pragma unroll
+          for (int t = 0; t < 4; ++t) fti[t] = ET<T>::load_frag(s_ti[cur] + arow_of(t) * LDC + 8 * g);
+          fti[4] = ET<T>::load_frag(s_ti[cur] + arow_of(2) * LDC + 32 + 8 * g);
+          fti[5] = ET<T>::load_frag(s_ti[cur] + arow_of(3) * LDC + 32 + 8 * g);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 4; ++t) ET<T>::mma(X[t], fk[ks & 1][t], bS[ks]);
+        if (ks == 0) {
+#pragma unroll
+          for (int mi = 0; mi < KT; ++mi) S[mi] *= dec;
+        }
+        if (ks == KS - 1) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) bv[s][e][i] = be[s][e][i] * (float)fv[s][4 * e + i];
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (wv == 0) TR(0, c, 5);
+    if (wv == 0) TR(0, c, 1);
+    // the k^T fragments of the first half of the update
+    typename ET<T>::frag fkt[2][KT];
+#pragma unroll
+    for (int mi = 0; mi < KT; ++mi) fkt[0][mi] = load_frag_t_state(s_kc, LDK, 0, mi, l);
     // Z = beta v - (beta e^{b}) X  (8 tokens of this lane's column per 32-token step), then v_new = Tinv Z
+    f32x4 vn[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) vn[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     typename ET<T>::frag Z[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -458,72 +489,47 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
       for (int e = 0; e < 2; ++e)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          Z[s][4 * e + i] = (bf16)(be[s][e][i] * (float)fv[s][4 * e + i] - ff[s][e][i] * X[2 * s + e][i]);
-    f32x4 vn[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) vn[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+          Z[s][4 * e + i] = (bf16)__builtin_fmaf(-ff[s][e][i], X[2 * s + e][i], bv[s][e][i]);
     ET<T>::mma(vn[0], fti[0], Z[0]);
     ET<T>::mma(vn[1], fti[1], Z[0]);
     ET<T>::mma(vn[2], fti[2], Z[0]);
     ET<T>::mma(vn[3], fti[3], Z[0]);
     ET<T>::mma(vn[2], fti[4], Z[1]);
     ET<T>::mma(vn[3], fti[5], Z[1]);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      uint32_t xb[4], nb[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // v_new rounded once to the storage type: the state update, the output and the backward see the same values
-        const bf16 x = (bf16)vn[t][i];
-        vn[t][i] = (float)x;
-        xb[i] = (uint32_t)__builtin_bit_cast(uint16_t, x);
-      }
-      // v_new [token][column] for the helpers and the loaders: neighbouring lanes hold neighbouring columns of the same
-      // four tokens; they swap (quad permutation 1 0 3 2), the even lane writes tokens 0, 1 and the odd lane tokens
-      // 2, 3 of the pair of columns as whole 32-bit words
-#pragma unroll
-      for (int i = 0; i < 4; ++i) nb[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)xb[i], 0xB1, 0xf, 0xf, false);
-      const bool odd = fr & 1;
-      const uint32_t w0 = odd ? (nb[2] | (xb[2] << 16)) : (xb[0] | (nb[0] << 16));
-      const uint32_t w1 = odd ? (nb[3] | (xb[3] << 16)) : (xb[1] | (nb[1] << 16));
-      uint32_t* dst = (uint32_t*)(s_vn + idx_of(t, odd ? 2 : 0) * LDU + 16 * j + (fr & ~1));
-      dst[0] = w0;
-      dst[LDU / 2] = w1;
-    }
-    const float dec = s_dec[cur];
-    // the k^T fragments of the first half of the update do not depend on this chunk's results
-    typename ET<T>::frag fkt[KT];
-#pragma unroll
-    for (int mi = 0; mi < KT; ++mi) fkt[mi] = load_frag_t_state(s_kc, LDK, 0, mi, l);
+    __builtin_amdgcn_sched_barrier(0);
+    // (its factors and the fragments of the second half: Tinv's registers are free)
     f32x4 ed[2][2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) { ed[s][0] = *(const f32x4*)&s_ed[cur][32 * s + 8 * g]; ed[s][1] = *(const f32x4*)&s_ed[cur][32 * s + 8 * g + 4]; }
-    if (wv == 0) TR(0, c, 2);
-    lds_barrier();                                                                       // B2
-    if (wv == 0) TR(0, c, 3);
+    for (int s = 0; s < 2; ++s) { ed[s][0] = *(const f32x4*)&s_gt[cur][1][32 * s + 8 * g]; ed[s][1] = *(const f32x4*)&s_gt[cur][1][32 * s + 8 * g + 4]; }
 #pragma unroll
-    for (int mi = 0; mi < KT; ++mi) S[mi] *= dec;
+    for (int mi = 0; mi < KT; ++mi) fkt[1][mi] = load_frag_t_state(s_kc, LDK, 32, mi, l);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wv == 0) TR(0, c, 5);
+    // v_new rounded once to the storage type: the state update, the output and the backward see the same values
+    typename ET<T>::frag vb[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
+      vb[s] = frag_of_blocks(vn[2 * s], vn[2 * s + 1]);
       typename ET<T>::frag bvd;
 #pragma unroll
       for (int e = 0; e < 2; ++e)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) bvd[4 * e + i] = (bf16)(vn[2 * s + e][i] * ed[s][e][i]);
+        for (int i = 0; i < 4; ++i) bvd[4 * e + i] = (bf16)((float)vb[s][4 * e + i] * ed[s][e][i]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int mi = 0; mi < KT; ++mi) ET<T>::mma(S[mi], fkt[mi], bvd);
+      for (int mi = 0; mi < KT; ++mi) ET<T>::mma(S[mi], fkt[s][mi], bvd);
       __builtin_amdgcn_sched_barrier(0);
-      if (s == 0) {
-#pragma unroll
-        for (int mi = 0; mi < KT; ++mi) fkt[mi] = load_frag_t_state(s_kc, LDK, 32, mi, l);
-      }
     }
+    // v_new^T [column][64]: 8 consecutive tokens per lane
+#pragma unroll
+    for (int s = 0; s < 2; ++s) *(bf16x8*)(s_vT[cur] + (16 * j + fr) * LDC + 32 * s + 8 * g) = vb[s];
     if (wv == 0) TR(0, c, 6);
-    put_state();                                      // the state at the start of the next chunk
-    if (wv == 0) TR(0, c, 4);
+    put_state(cur ^ 1);                               // the state at the start of the next chunk
+    if (wv == 0) TR(0, c, 2);
+    lds_barrier();
+    if (wv == 0) TR(0, c, 3);
   }
-  lds_barrier();                                                                         // results of the last chunk
+  lds_barrier();
   if (a.ht && item.last) {
     float* ht = a.ht + ((int64_t)n * a.H + h) * K * V;
 #pragma unroll
