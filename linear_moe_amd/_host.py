@@ -195,6 +195,11 @@ class SeqPlan:
         if self.N > 1 and int(nch.max()) != int(nch.min()):
             self.seq_order = torch.argsort(nch, descending=True, stable=True).to(torch.int32).to(device)
 
+    @property
+    def tables(self):
+        """What the native launch path takes."""
+        return (self.N, self.NT, self.cu, self.chunk_map, self.seq_chunk0, self.seq_order, self.nt_dev)
+
     def _build_on_device(self, T: int, cu_seqlens: torch.Tensor):
         dev = cu_seqlens.device
         N = cu_seqlens.numel() - 1
@@ -344,6 +349,20 @@ def stream_ptr() -> int:
     """The current stream of the current device, as the library takes it.  (The raw handle: building the stream object
     of ``torch.cuda.current_stream()`` for it takes longer than all the other arguments of a small call.)"""
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+# The steps of a call (checks, argument block, allocations, the call of the library) in native code, for the calls that
+# need no conversion, copy or refusal: csrc/lmoe_native.cpp.  It returns None for any other call, which then takes the
+# steps in Python.  (Host time of a call, small sizes on one machine: one token 20 -> 8 us; forward 23 -> 15; forward and
+# backward of the gated delta rule 143 -> 90, of which autograd itself is 27 to 60.)
+def native(fn: str, what: str, op: int, q, *args):
+    """``forward``, ``backward`` or ``recurrent`` of the native path: its results, or None (not a call for it)."""
+    if not q.is_cuda:
+        return None
+    r = getattr(_lib.native(), fn)(op, q, *args, stream_ptr())
+    if type(r) is int:
+        _lib.check(r, what)
+    return r
 
 
 def ptr(x: Optional[torch.Tensor]):

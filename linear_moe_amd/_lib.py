@@ -168,6 +168,25 @@ def load() -> C.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The launch path in native code (``csrc/lmoe_native.cpp``), bound to the library."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as m
+        except ImportError as e:
+            raise RuntimeError(f"the native launch path does not load ({e}): build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
+        if m.bind(LIB_PATH) != VERSION:
+            raise RuntimeError(f"the native launch path was built for another version than {VERSION}: build it again with "
+                               f"`make -C {os.path.join(_HERE, 'csrc')}`")
+        _native = m
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = load().lmoe_last_error().decode()

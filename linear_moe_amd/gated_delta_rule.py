@@ -17,7 +17,7 @@ import torch
 from . import _lib
 from .l2norm import l2_norm
 from ._host import (HEAD_DIMS, WIDE_V, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    no_tokens, ptr, stash, stream_ptr, unstash)
+                    native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 def _scalar_dt(x: torch.Tensor) -> int:
@@ -44,10 +44,25 @@ class GDNCall:
         read v, and ``backward`` returns the gradient with respect to that argument."""
         ctx = self
         lib = _lib.load()
+        plan = None
+        if cu_seqlens is not None:
+            B, T = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)[:2]
+            plan = seq_plan(B, T, cu_seqlens, q.device)
+        if not self.keep:
+            tables = None if plan is None else plan.tables
+            r = native("forward", "chunk_gated_delta_rule forward", self.OP, q, k, v, g, beta, initial_state, tables,
+                       scale, output_final_state, head_first, save, 0, 0.0, v_act)
+            if r is not None:
+                o, ht, *kept = r
+                ctx.saved = (q, k, v, g, beta, initial_state, *kept)
+                ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, None, head_first, scale
+                ctx.has_h0, ctx.v_act, self.seg_ws = initial_state is not None, bool(v_act), None
+                return o, ht
         dims = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)
         B, T, H, K, V = dims
         q, k, v = _aligned(q), _aligned(k), _aligned(v)
-        plan = seq_plan(B, T, cu_seqlens, q.device)
+        if plan is None:
+            plan = seq_plan(B, T, None, q.device)
         want = (B, H, T) if head_first else (B, T, H)
         if beta is None or tuple(beta.shape) != want:
             raise ValueError(f"beta must have shape {want}")
@@ -117,8 +132,18 @@ class GDNCall:
         ctx = self
         lib = _lib.load()
         q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew, seg_p = ctx.saved
-        plan, dims, head_first = ctx.plan, ctx.dims, ctx.head_first
+        head_first = ctx.head_first
+        if not self.keep:
+            raw = (None, None) if qk_raw is None else qk_raw
+            r = native("backward", "chunk_gated_delta_rule backward", self.OP, q, k, v, g, beta, h0, ctx.plan and
+                       ctx.plan.tables, ctx.scale, do, dht, head_first, (hs, tinv, pmat, gcum, vnew, seg_p), (ctx.v_act,
+                       dq_out, dk_out, dv_out, *raw, float(qk_eps)))
+            if r is not None:
+                dq, dk, dv, dg, dbeta, dh0 = r
+                return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dbeta, dh0
+        dims = ctx.dims or _check_inputs(q, k, v, head_first, None, wide_v=True)
         B, T, H, K, V = dims
+        plan = ctx.plan or seq_plan(B, T, None, q.device)
         do = _aligned(do)
         a = base_args(q, k, v, head_first, ctx.scale, plan, dims)
         a.gate = _lib.GATE_NONE if g is None else _lib.GATE_SCALAR

@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    cut_workspace, no_tokens, ptr, stash, stream_ptr, unstash)
+                    cut_workspace, native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class GLACall:
@@ -35,6 +35,21 @@ class GLACall:
         """save=False: a forward-only call (nothing requires a gradient): the per-chunk states are not written where
         the state pass forms the output itself (bf16); the fp32 path's output kernel reads them."""
         lib = _lib.load()
+        plan = None
+        if cu_seqlens is not None:
+            B, T = _check_inputs(q, k, v, head_first, cu_seqlens)[:2]
+            if g is not None and g.shape == q.shape:
+                plan = seq_plan(B, T, cu_seqlens, q.device)
+        if not self.keep:
+            tables = None if plan is None else plan.tables
+            r = native("forward", "chunk_gla forward", self.OP, q, k, v, g, None, initial_state, tables, scale,
+                       output_final_state, head_first, save, 0, 0.0, False)
+            if r is not None:
+                o, ht, *kept = r
+                self.saved = (q, k, v, g, initial_state, *kept)
+                self.plan, self.dims, self.head_first, self.scale = plan, None, head_first, scale
+                self.has_h0 = initial_state is not None
+                return o, ht
         dims = _check_inputs(q, k, v, head_first, cu_seqlens)
         B, T, H, K, V = dims
         if g is None or tuple(g.shape) != tuple(q.shape):
@@ -43,7 +58,8 @@ class GLACall:
         if q.dtype == torch.float32 or g.dtype not in (torch.float32, torch.bfloat16):
             g = g.float()
         q, k, v, g = _aligned(q), _aligned(k), _aligned(v), _aligned(g)
-        plan = seq_plan(B, T, cu_seqlens, q.device)
+        if plan is None:
+            plan = seq_plan(B, T, cu_seqlens, q.device)
         h0 = _state_check(initial_state, plan.N, H, K, V, "initial_state")
         a = base_args(q, k, v, head_first, scale, plan, dims)
         self._gate(a, g, head_first)
@@ -71,7 +87,15 @@ class GLACall:
     def backward(self, do, dht):
         lib = _lib.load()
         q, k, v, g, h0, hs, amat, qe, ke, gdec = self.saved
-        plan, dims, head_first = self.plan, self.dims, self.head_first
+        head_first = self.head_first
+        if not self.keep:
+            r = native("backward", "chunk_gla backward", self.OP, q, k, v, g, None, h0, self.plan and self.plan.tables,
+                       self.scale, do, dht, head_first, (hs, amat, qe, ke, gdec), None)
+            if r is not None:
+                dq, dk, dv, dg, _, dh0 = r
+                return dq, dk, dv, dg, dh0
+        dims = self.dims or _check_inputs(q, k, v, head_first, None)
+        plan = self.plan or seq_plan(dims[0], dims[1], None, q.device)
         do = _aligned(do)
         a = base_args(q, k, v, head_first, self.scale, plan, dims)
         self._gate(a, g, head_first)

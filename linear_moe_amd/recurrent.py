@@ -15,7 +15,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from ._host import seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, ptr, stream_ptr
+from ._host import seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, native, ptr, stream_ptr
 from .delta_rule import chunk_delta_rule
 from .gated_delta_rule import chunk_gated_delta_rule
 from .gla import chunk_gla
@@ -35,6 +35,11 @@ def _sdt(x: torch.Tensor) -> int:
 def _recurrent(op, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first, qk_eps=0.0):
     """qk_eps > 0 (delta rule): q and k are L2-normalised by the kernel, qk_eps inside the root."""
     lib = _lib.load()
+    if cu_seqlens is None:
+        r = native("recurrent", "fused_recurrent forward", op, q, k, v, g, beta, initial_state, None, scale, output_final_state,
+                   head_first, qk_eps)
+        if r is not None:
+            return r
     dims = _check_inputs(q, k, v, head_first, cu_seqlens)
     B, T, H, K, V = dims
     q, k, v = _aligned(q.detach()), _aligned(k.detach()), _aligned(v.detach())

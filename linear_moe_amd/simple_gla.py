@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    cut_workspace, no_tokens, ptr, stash, stream_ptr, unstash)
+                    cut_workspace, native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class SimpleGLACall:
@@ -37,10 +37,27 @@ class SimpleGLACall:
         before dividing); ``backward`` then takes the gradient of den beside that of o."""
         ctx = self
         lib = _lib.load()
+        plan = None
+        if cu_seqlens is not None:
+            B, T = _check_inputs(q, k, v, head_first, cu_seqlens)[:2]
+            plan = seq_plan(B, T, cu_seqlens, q.device)
+        if not self.keep:
+            tables = None if plan is None else plan.tables
+            r = native("forward", "chunk_simple_gla forward", self.OP, q, k, v, g, None, initial_state, tables, scale,
+                       output_final_state, head_first, save, 2 if emit_den else 0 if norm_eps is None else 1, 0.0 if
+                       emit_den or norm_eps is None else norm_eps, False)
+            if r is not None:
+                o, ht, hs, den, zs = r
+                ctx.saved = (q, k, v, g, initial_state, hs, None if emit_den else den, zs)
+                ctx.norm_eps, ctx.emit_den, self.den = (0.0 if emit_den else norm_eps), emit_den, (den if emit_den else None)
+                ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, None, head_first, scale
+                ctx.has_h0 = initial_state is not None
+                return o, ht
         dims = _check_inputs(q, k, v, head_first, cu_seqlens)
         B, T, H, K, V = dims
         q, k, v = _aligned(q), _aligned(k), _aligned(v)
-        plan = seq_plan(B, T, cu_seqlens, q.device)
+        if plan is None:
+            plan = seq_plan(B, T, None, q.device)
         if g is not None:
             want = (B, H, T) if head_first else (B, T, H)
             if tuple(g.shape) != want:
@@ -87,8 +104,17 @@ class SimpleGLACall:
         ctx = self
         lib = _lib.load()
         q, k, v, g, h0, hs, den, zs = ctx.saved
-        plan, dims, head_first = ctx.plan, ctx.dims, ctx.head_first
+        head_first = ctx.head_first
+        if not self.keep:
+            extra = None if ctx.norm_eps is None else (2 if ctx.emit_den else 1, ctx.norm_eps, o, dden)
+            r = native("backward", "chunk_simple_gla backward", self.OP, q, k, v, g, None, h0, ctx.plan and
+                       ctx.plan.tables, ctx.scale, do, dht, head_first, (hs, den, zs), extra)
+            if r is not None:
+                dq, dk, dv, dg, _, dh0 = r
+                return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dh0
+        dims = ctx.dims or _check_inputs(q, k, v, head_first, None)
         B, T, H, K, V = dims
+        plan = ctx.plan or seq_plan(B, T, None, q.device)
         do = _aligned(do)
         a = base_args(q, k, v, head_first, ctx.scale, plan, dims)
         a.gate = _lib.GATE_NONE if g is None else _lib.GATE_SCALAR

@@ -1,0 +1,153 @@
+"""The launch path in native code (csrc/lmoe_native.cpp) against the same steps in Python: the same bits for every form
+of a call that it takes, and None, i.e. the Python steps, for the forms it does not."""
+import itertools
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(op, B, T, H, K, V, dtype, head_first, strided, gdt, cuda, seed=5):
+    gen = torch.Generator(device=cuda).manual_seed(seed)
+    rn = lambda *s: torch.randn(*s, generator=gen, device=cuda)
+
+    def rows(D, dt=dtype):
+        shape = (B, H, T, D) if head_first else (B, T, H, D)
+        if not strided:
+            return rn(*shape).to(dt)
+        # a view with swapped axes of a wider buffer: aligned rows, strides of its own
+        x = rn(B, shape[2], shape[1], D + 16).to(dt)
+        return x.transpose(1, 2)[..., :D]
+    norm = lambda x: x / x.float().norm(dim=-1, keepdim=True).to(x.dtype)
+    tok = (B, H, T) if head_first else (B, T, H)
+    q, k, v = norm(rows(K)), norm(rows(K)), rows(V)
+    if strided:
+        q = rows(K) * 0.1
+    g = {0: lambda: -rn(*tok).abs().to(gdt) * 0.1, 1: lambda: (-rn(*q.shape).abs() * 0.05).to(gdt), 2: lambda: -rn(*tok).abs().to(gdt)}[op]()
+    beta = torch.sigmoid(rn(*tok)).to(gdt) if op == 2 else None
+    return dict(q=q, k=k, v=v, g=g, beta=beta)
+
+
+def _call(op, keep):
+    from linear_moe_amd.gated_delta_rule import GDNCall
+    from linear_moe_amd.gla import GLACall
+    from linear_moe_amd.simple_gla import SimpleGLACall
+    return (SimpleGLACall, GLACall, GDNCall)[op](keep)
+
+
+def _both(op, x, h0, ofs, cu, hf, do, dht, monkeypatch, **kw):
+    """results of the two paths; ``kept`` forces the Python steps, the other one must not reach them"""
+    import linear_moe_amd._host as host
+    import linear_moe_amd.gated_delta_rule as gdr
+    import linear_moe_amd.gla as gla
+    import linear_moe_amd.simple_gla as sg
+    args = [x["q"], x["k"], x["v"], x["g"]] + ([x["beta"]] if op == 2 else []) + [None, h0, ofs, cu, hf]
+    out = []
+    for keep in (True, False):
+        c = _call(op, keep)
+        with monkeypatch.context() as m:
+            if not keep:
+                for mod in (sg, gla, gdr):
+                    m.setattr(mod, "base_args", None)          # (the Python steps would call it)
+            o, ht = c.forward(*args, **kw)
+            extra = (o,) if kw.get("norm_eps") is not None else ()
+            out.append([o, ht, *c.backward(do, dht if ofs else None, *extra)])
+    return out
+
+
+FORMS = list(itertools.product((0, 1, 2), (torch.bfloat16, torch.float32), (True, False), (False, True)))
+
+
+@pytest.mark.parametrize("op,dtype,head_first,strided", [f for f in FORMS if not (f[0] == 2 and f[1] == torch.float32)])
+@pytest.mark.parametrize("T,with_state,gdt", [(1, True, torch.float32), (200, False, torch.bfloat16), (1900, True, torch.float32)])
+def test_same_bits_as_the_python_steps(cuda, monkeypatch, op, dtype, head_first, strided, T, with_state, gdt):
+    if op == 1 and dtype == torch.float32:
+        gdt = torch.float32
+    B, H, K, V = 2, 3, 64, 128
+    x = _inputs(op, B, T, H, K, V, dtype, head_first, strided, gdt, cuda)
+    h0 = torch.randn(B, H, K, V, device=cuda) if with_state else None
+    do = torch.randn(x["v"].shape, device=cuda).to(dtype)
+    dht = torch.randn(B, H, K, V, device=cuda)
+    ref, got = _both(op, x, h0, with_state, None, head_first, do, dht, monkeypatch)
+    for a, b in zip(ref, got):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("host_offsets", [True, False])
+def test_same_bits_packed(cuda, monkeypatch, op, host_offsets):
+    cu = torch.tensor([0, 70, 70, 71, 500], dtype=torch.int32)
+    cu = cu if host_offsets else cu.to(cuda)
+    x = _inputs(op, 1, 500, 2, 128, 128, torch.bfloat16, False, False, torch.float32, cuda)
+    h0, dht = torch.randn(4, 2, 128, 128, device=cuda), torch.randn(4, 2, 128, 128, device=cuda)
+    do = torch.randn_like(x["v"])
+    ref, got = _both(op, x, h0, True, cu, False, do, dht, monkeypatch)
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(ref, got))
+
+
+@pytest.mark.parametrize("T", [1, 1000])
+def test_same_bits_normalized(cuda, monkeypatch, T):
+    x = _inputs(0, 2, T, 2, 64, 64, torch.bfloat16, True, False, torch.float32, cuda)
+    x["q"], x["k"], x["g"] = x["q"].abs(), x["k"].abs(), None
+    do = torch.randn_like(x["v"])
+    ref, got = _both(0, x, None, False, None, True, do, None, monkeypatch, norm_eps=1e-10)
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(ref, got))
+
+
+def test_ungated_delta_rule_same_bits(cuda, monkeypatch):
+    x = _inputs(2, 1, 2000, 2, 128, 64, torch.bfloat16, False, False, torch.bfloat16, cuda)
+    x["g"] = None
+    ref, got = _both(2, x, None, True, None, False, torch.randn_like(x["v"]), torch.randn(1, 2, 128, 64, device=cuda), monkeypatch)
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(ref, got))
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("head_first", [True, False])
+def test_recurrent_same_bits(cuda, monkeypatch, op, head_first):
+    import linear_moe_amd as L
+    import linear_moe_amd.recurrent as rec
+    x = _inputs(op, 3, 2, 2, 64, 128, torch.bfloat16, head_first, True, torch.float32, cuda)
+    h0 = torch.randn(3, 2, 64, 128, device=cuda)
+    f = (L.fused_recurrent_simple_gla, L.fused_recurrent_gla, L.fused_recurrent_gated_delta_rule)[op]
+    args = [x["q"], x["k"], x["v"], x["g"]] + ([x["beta"]] if op == 2 else [])
+    with monkeypatch.context() as m:
+        m.setattr(rec, "base_args", None)
+        got = f(*args, initial_state=h0, output_final_state=True, head_first=head_first)
+    with monkeypatch.context() as m:
+        m.setattr(rec, "native", lambda *a: None)
+        ref = f(*args, initial_state=h0, output_final_state=True, head_first=head_first)
+    assert torch.equal(ref[0], got[0]) and torch.equal(ref[1], got[1]) and ref[0].stride() == got[0].stride()
+
+
+def test_other_calls_take_the_python_steps(cuda):
+    """what the native path hands back: a subclass, a last dimension with a stride, misaligned rows, other types of gate
+    or state; and what is refused stays refused, in the words of the Python steps"""
+    import linear_moe_amd as L
+    from linear_moe_amd._host import native
+    x = _inputs(0, 2, 100, 2, 64, 64, torch.bfloat16, True, False, torch.float32, cuda)
+    q, k, v, g = x["q"], x["k"], x["v"], x["g"]
+    call = lambda q, k, v, g, h0=None: native("forward", "t", 0, q, k, v, g, None, h0, None, None, True, True, False, 0, 0.0, False)
+    ref = L.chunk_simple_gla(q, k, v, g)[0]
+    assert torch.equal(call(q, k, v, g)[0], ref)
+
+    class Sub(torch.Tensor):
+        pass
+
+    wide = torch.zeros(2, 2, 100, 65, device=cuda, dtype=torch.bfloat16)
+    wide[..., 1:] = q
+    for other in ((q.as_subclass(Sub), k, v, g), (q.transpose(2, 3).contiguous().transpose(2, 3), k, v, g),
+                  (wide[..., 1:], k, v, g), (q, k, v, g.half())):
+        assert call(*other) is None
+        assert (L.chunk_simple_gla(*other)[0].float() - ref.float()).abs().max() <= 1e-2 * ref.float().abs().max()
+    h0 = torch.randn(2, 2, 64, 64, device=cuda)
+    assert call(q, k, v, g, h0.bfloat16()) is None
+    for bad, err in (((q, k[:, :, :50], v, g), ValueError), ((q, k.float(), v, g), ValueError), ((q, k, v, g[:, :, :50]), ValueError),
+                     ((q, k.cpu(), v, g), RuntimeError)):
+        assert call(*bad) is None
+        with pytest.raises(err):
+            L.chunk_simple_gla(*bad)
+    with pytest.raises(ValueError):
+        L.chunk_simple_gla(q, k, v, g, initial_state=h0[:1])
