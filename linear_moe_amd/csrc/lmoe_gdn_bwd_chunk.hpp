@@ -37,7 +37,13 @@
 //     window w: the compute team works on slice w (buffer w % 3); the loaders stage slice w + 2, then q
 //     (window 2) and k (window 3), and slices 0, 1 of the next item during b .. d
 //   one slice buffer:  [R(0)] D(0) R(1) D(1) .. D(NS-1) | A | b c d | R(0) of the next item
+// What bounds it (8192 items, K = V = 128, 16 heads): with its loads served by the L2 and nothing stored 237 us, the compute
+// waves alone 167, the loader waves alone 174; with memory, the loaders alone 304 (5.8 TB/s).  So the loader waves: their
+// work between two requests was cut to dot-product instructions for <dZ, v> and <S, dS'>, one set of divisions
+// per item, and the compute waves' LDS traffic (reads and 2-byte accesses of stage 2) to a third.  370 -> 350 us; where
+// memory binds less 50 -> 43 (2048 x 2 tokens), 97 -> 78 (K = V = 64, 4096 x 4).
 #pragma once
+#include <type_traits>
 #include "lmoe_seq.hpp"
 
 namespace lmoe {
@@ -51,18 +57,6 @@ template <typename T, int K, int BVH, int NBUF> struct GdnBwdChunkLds {
   static constexpr int NREG = S_END + 2 * CH * LDK;               // ..; q, k
   static constexpr int BYTES = NREG * (int)sizeof(T) + (13 * 64 + 16) * 4;
 };
-
-// gemm with a scheduling fence after every 32-deep step: at most one step's fragments are in flight,
-// which keeps the register budget of a kernel with many live accumulators
-template <typename T, int MB, int NB, bool AT, bool BT>
-__device__ __forceinline__ void gemm_bounded(f32x4 (&acc)[MB][NB], const T* A, int lda, int a0,
-                                             const T* B, int ldb, int b0, int k0, int k1, int l) {
-#pragma unroll
-  for (int kk = k0; kk < k1; kk += 32) {
-    gemm<T, MB, NB, AT, BT>(acc, A, lda, a0, B, ldb, b0, kk, kk + 32, l);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-}
 
 // compile-time loop: f(IC<0>()), .., f(IC<N - 1>())
 template <int I> struct IC { static constexpr int value = I; };
@@ -140,28 +134,39 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     float dbv[PV];     // partial <dZ, v> of this thread's rows of that item
 #pragma unroll
     for (int p = 0; p < PV; ++p) dbv[p] = 0.f;
-    // unit u counted from the first unit of item it (u >= NU: units of the item after it)
-    auto issue = [&](auto uc, int it) {
-      constexpr int u = decltype(uc)::value, unit = u % NU;
-      Unit& R = U[u % DEPTH];
-      it = __builtin_amdgcn_readfirstlane(min(it + (u / NU) * stride, nitems - 1));
-      // with many slices per item the scalar addresses of all of them, formed at the top of the item, do not fit the
-      // scalar registers: the item index is made opaque per unit, so that each unit's addresses are formed where it
-      // is requested
-      if constexpr (NS > 4) asm volatile("" : "+s"(it));
-      const int cid = it / a.H, h = it % a.H;
+    // Where an item's rows lie: worked out once per item, for its six units, its stores and (as the item after this one) its
+    // first units.  (Per unit, the divisions by H and by the chunks of a sequence were a thousand scalar instructions
+    // per item on the waves whose requests bound the kernel.  The row pointers are formed where they are used: kept as
+    // well, they spill to vector lanes.)
+    struct Item { int it, h, b, tok, len; };
+    auto item_at = [&](int it) {
+      Item I;
+      I.it = __builtin_amdgcn_readfirstlane(min(it, nitems - 1));
+      const int cid = I.it / a.H;
+      I.h = I.it - cid * a.H;
       const ChunkInfo ci = chunk_info(a, cid);
-      R.len = ci.len;
+      I.b = ci.b; I.tok = ci.tok; I.len = ci.len;
+      return I;
+    };
+    auto rows = [&](const lmoe_tensor& x, const Item& I) { return row_ptr<T>(x, I.b, I.tok, I.h); };
+    // unit u counted from the first unit of the item cur (u >= NU: units of the item after it, nxt)
+    auto issue = [&](auto uc, const Item& cur, const Item& nxt) {
+      constexpr int u = decltype(uc)::value, unit = u % NU;
+      static_assert(u < 2 * NU, "units of this item and the next");
+      const Item& I = u < NU ? cur : nxt;
+      Unit& R = U[u % DEPTH];
+      R.len = I.len;
       if constexpr (unit < NS) {
         constexpr int vv = unit * BVH;
         static_assert(BVH == SLICE_COLS, "a slice of this kernel is one block of vnew / dvnew");
-        const lmoe_tensor* ts[4] = {&a.d_o, &a.vnew, &a.dvnew, &a.v};
+        // do, v: the caller's rows; vnew, dvnew (= dZ): one contiguous block per (chunk, head, slice)
+        const int64_t block = ((int64_t)I.it * NS + unit) * (CH * SLICE_COLS);
+        const T* ts[4] = {rows(a.d_o, I) + vv, (const T*)a.vnew.ptr + block, (const T*)a.dvnew.ptr + block, rows(a.v, I) + vv};
+        const int64_t st[4] = {a.d_o.st, SLICE_COLS, SLICE_COLS, a.v.st};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           typename IOV::Regs r;
-          // do, v: the caller's rows; vnew, dvnew (= dZ): one contiguous block per (chunk, head, slice)
-          if (t == 1 || t == 2) IOV::load_nomask(r, slice_ptr<T>(*ts[t], cid, h, a.H, V, vv), SLICE_COLS, ci.len, tid);
-          else IOV::load_nomask(r, row_ptr<T>(*ts[t], ci.b, ci.tok, h) + vv, ts[t]->st, ci.len, tid);
+          IOV::load_nomask(r, ts[t], st[t], I.len, tid);
 #pragma unroll
           for (int p = 0; p < PV; ++p) R.v[t * PV + p] = r.v[p];
         }
@@ -169,14 +174,14 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           typename IOH::Regs r;
-          IOH::load_nomask(r, hp[t] + ((int64_t)it * V + vv) * K, K, BVH, tid);         // it = cid * H + h
+          IOH::load_nomask(r, hp[t] + ((int64_t)I.it * V + vv) * K, K, BVH, tid);       // it = cid * H + h
 #pragma unroll
           for (int p = 0; p < PH; ++p) R.v[4 * PV + t * PH + p] = r.v[p];
         }
       } else {
-        const lmoe_tensor& x = unit == NS ? a.q : a.k;
         typename IOK::Regs r;
-        IOK::load_nomask(r, row_ptr<T>(x, ci.b, ci.tok, h), x.st, ci.len, tid);
+        const lmoe_tensor& x = unit == NS ? a.q : a.k;
+        IOK::load_nomask(r, rows(x, I), x.st, I.len, tid);
 #pragma unroll
         for (int p = 0; p < PK; ++p) R.v[p] = r.v[p];
       }
@@ -199,19 +204,19 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           const vec z = R.v[2 * PV + p], vv = R.v[3 * PV + p];
           vec o;
           float s = 0.f;
+          if (a.v_act) {
+            // v as given is the argument of a SiLU: the op runs on silu(v) (rounded to the element type, as the
+            // forward pass staged it) and dv is the gradient with respect to the argument
 #pragma unroll
-          for (int i = 0; i < IOV::VEC; ++i) {
-            const float zf = ET<T>::to_f(z[i]);
-            if (a.v_act) {
-              // v as given is the argument of a SiLU: the op runs on silu(v) (rounded to the element type, as the
-              // forward pass staged it) and dv is the gradient with respect to the argument
-              const float vr = ET<T>::to_f(vv[i]);
+            for (int i = 0; i < IOV::VEC; ++i) {
+              const float zf = ET<T>::to_f(z[i]), vr = ET<T>::to_f(vv[i]);
               o[i] = ET<T>::from_f(zf * bt * silu_grad(vr));
               s += zf * ET<T>::to_f(ET<T>::from_f(silu_of(vr)));
-            } else {
-              o[i] = ET<T>::from_f(zf * bt);
-              s += zf * ET<T>::to_f(vv[i]);
             }
+          } else {
+#pragma unroll
+            for (int i = 0; i < IOV::VEC; ++i) o[i] = ET<T>::from_f(ET<T>::to_f(z[i]) * bt);
+            s = dot_vec(z, vv, 0.f);
           }
           d.r.v[p] = o;
           s = group_sum<IOV::VPR>(s);                   // the VPR lanes that hold one row are neighbours
@@ -231,9 +236,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
 #pragma unroll
         for (int p = 0; p < PH; ++p) { rh.v[p] = R.v[4 * PV + p]; rdh.v[p] = R.v[4 * PV + PH + p]; }
 #pragma unroll
-        for (int p = 0; p < PH; ++p)
-#pragma unroll
-          for (int i = 0; i < IOH::VEC; ++i) hdh += ET<T>::to_f(rh.v[p][i]) * ET<T>::to_f(rdh.v[p][i]);
+        for (int p = 0; p < PH; ++p) hdh = dot_vec(rh.v[p], rdh.v[p], hdh);
         pin(hdh);                                         // here, not where the item is closed (the tiles would stay live)
         IOH::store_lds(rh, base + A_H, LDK, tid);
         IOH::store_lds(rdh, base + A_DH, LDK, tid);
@@ -245,16 +248,16 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
         IOK::store_lds(r, smem + (unit == NS ? B_Q : B_K), LDK, tid);
       }
     };
-    auto store_dv = [&](const DV& d, const ChunkInfo& ci, int h, int s) {
-      IOV::template store_global_clamped<true>(d.r, row_ptr<T>(a.dv, ci.b, ci.tok, h) + s * BVH, a.dv.st, ci.len, tid);
+    auto store_dv = [&](const DV& d, const Item& I, int s) {
+      IOV::template store_global_clamped<true>(d.r, rows(a.dv, I) + s * BVH, a.dv.st, I.len, tid);
     };
+    // an item and the request of its gates
     auto issue_gates = [&](int it) {
-      it = __builtin_amdgcn_readfirstlane(min(it, nitems - 1));
-      const int cid = it / a.H, h = it % a.H;
-      const ChunkInfo ci = chunk_info(a, cid);
-      glen = ci.len;
-      graw = gate_prefetch(a, ci.b, ci.tok, ci.len, h);
-      braw = load_scalar_raw(a.beta.ptr, a.beta_dtype, row_off(a.beta, ci.b, ci.tok + min(l, ci.len - 1), h));
+      const Item I = item_at(it);
+      glen = I.len;
+      graw = gate_prefetch(a, I.b, I.tok, I.len, I.h);
+      braw = load_scalar_raw(a.beta.ptr, a.beta_dtype, row_off(a.beta, I.b, I.tok + min(l, I.len - 1), I.h));
+      return I;
     };
     // gate cumsum and beta of an item into copy par
     auto stage_gates = [&](int par) {
@@ -278,12 +281,10 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     // with the sums of a row over the VPR neighbouring lanes that hold it (the arithmetic, step for step, of the row
     // kernel that does the same in front of the op: the results agree bit for bit)
     typename IOK::Regs XQ, XK;
-    auto issue_raw = [&](int it) __attribute__((always_inline)) {
+    auto issue_raw = [&](const Item& I) __attribute__((always_inline)) {
       if constexpr (QKACT) {
-        const int cid = it / a.H, h = it % a.H;
-        const ChunkInfo ci = chunk_info(a, cid);
-        IOK::load_nomask(XQ, row_ptr<T>(a.q_raw, ci.b, ci.tok, h), a.q_raw.st, ci.len, tid);
-        IOK::load_nomask(XK, row_ptr<T>(a.k_raw, ci.b, ci.tok, h), a.k_raw.st, ci.len, tid);
+        IOK::load_nomask(XQ, rows(a.q_raw, I), a.q_raw.st, I.len, tid);
+        IOK::load_nomask(XK, rows(a.k_raw, I), a.k_raw.st, I.len, tid);
       }
     };
     auto act_backward = [&](typename IOK::Regs& r, const typename IOK::Regs& X) __attribute__((always_inline)) {
@@ -313,35 +314,27 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     // item like every load past the end and skip the loop)
     const int it0 = min((int)blockIdx.x, nitems - 1);
     DV d0, d1;
-    issue_gates(it0);
-    static_for<DEPTH>([&](auto jc) { issue(jc, it0); });
+    Item cur = issue_gates(it0);
+    static_for<DEPTH>([&](auto jc) { issue(jc, cur, cur); });
     // the first loads may be ordered freely by the compiler; were they still pending at the loop
     // header, its wait-count analysis would carry that order into every iteration
     wait_all_loads();
     stage_gates(0);
-    issue_gates(it0 + stride);
+    Item nxt = issue_gates(it0 + stride);
     lds_barrier();                                                                       // beta of the first item staged
-    {
-      const ChunkInfo ci = chunk_info(a, it0 / a.H);
-      stage(IC<0>(), 0, 0, d0);
-      issue(IC<DEPTH>(), it0);
-      store_dv(d0, ci, it0 % a.H, 0);
-      if constexpr (NBUF == 3) {
-        stage(IC<1>(), 1, 0, d1);
-        issue(IC<1 + DEPTH>(), it0);
-        store_dv(d1, ci, it0 % a.H, 1);
-      }
+    stage(IC<0>(), 0, 0, d0);
+    issue(IC<DEPTH>(), cur, nxt);
+    store_dv(d0, cur, 0);
+    if constexpr (NBUF == 3) {
+      stage(IC<1>(), 1, 0, d1);
+      issue(IC<1 + DEPTH>(), cur, nxt);
+      store_dv(d1, cur, 1);
     }
     int par = 0;
     lds_barrier();                                                                       // first slice staged
     for (int it = blockIdx.x; it < nitems; it += stride) {
       tid = fresh_index(tid) & (NTHR - 1);
-      const int cid = it / a.H, h = it % a.H;
-      const ChunkInfo ci = chunk_info(a, cid);
-      // the item after this one (past the end: the last item once more, see issue)
-      const int itn = __builtin_amdgcn_readfirstlane(min(it + stride, nitems - 1));
-      const int hn = itn % a.H;
-      const ChunkInfo cin = chunk_info(a, itn / a.H);
+      Item aft;                                                                          // two items ahead
       if constexpr (NBUF == 3) {
         // window w: the compute team works on slice w.  Slice s lives in buffer s % 3 and is staged two
         // windows ahead; q and k follow in windows 2 and 3.
@@ -354,22 +347,22 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           stage(IC<u>(), u % 3, par, d0);
           if constexpr (w == NS - 1) close_item();
           lds_barrier();                                                                 // D(w); the last one is A
-          if constexpr (u < NS) store_dv(d0, ci, h, u);
-          if constexpr (w < NS - 1) issue(IC<u + DEPTH>(), it);                          // q, k, slice 0 of the next item
+          if constexpr (u < NS) store_dv(d0, cur, u);
+          if constexpr (w < NS - 1) issue(IC<u + DEPTH>(), cur, nxt);                       // q, k, slice 0 of the next item
         });
-        issue_raw(it);                                                                   // (QKACT) used behind d
-        issue(IC<NS + 1 + DEPTH>(), it);                                                 // slice 1 of the next item
+        issue_raw(cur);                                                                  // (QKACT) used behind d
+        issue(IC<NS + 1 + DEPTH>(), cur, nxt);                                           // slice 1 of the next item
         stage_gates(par ^ 1);                                  // the next item's; its copy is idle since d of the last item
-        issue_gates(it + 2 * stride);
+        aft = issue_gates(it + 2 * stride);
         lds_barrier();                                                                   // b
         stage(IC<NU>(), 0, par ^ 1, d0);                       // slice 0 of the next item (buffer 0: slice 3 is done)
         lds_barrier();                                                                   // c
-        store_dv(d0, cin, hn, 0);
-        issue(IC<NU + DEPTH>(), it);                                                     // slice 2 of the next item
+        store_dv(d0, nxt, 0);
+        issue(IC<NU + DEPTH>(), cur, nxt);                                               // slice 2 of the next item
         stage(IC<NU + 1>(), 1, par ^ 1, d1);                   // slice 1 of the next item
         lds_barrier();                                                                   // d: dq, dk lie in the q, k tiles
-        store_dv(d1, cin, hn, 1);
-        issue(IC<NU + 1 + DEPTH>(), it);                                                 // slice 3 of the next item
+        store_dv(d1, nxt, 1);
+        issue(IC<NU + 1 + DEPTH>(), cur, nxt);                                           // slice 3 of the next item
       } else {
         static_for<NS>([&](auto sc) {
           constexpr int s = decltype(sc)::value;
@@ -377,38 +370,40 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           lds_barrier();                                                                 // D(s)
           if constexpr (s + 1 < NS) {
             stage(IC<s + 1>(), 0, par, d0);
-            issue(IC<s + 1 + DEPTH>(), it);
-            store_dv(d0, ci, h, s + 1);
+            issue(IC<s + 1 + DEPTH>(), cur, nxt);
+            store_dv(d0, cur, s + 1);
           }
         });
         stage(IC<NS>(), 0, par, d0);                                                     // q
-        issue(IC<NS + DEPTH>(), it);
+        issue(IC<NS + DEPTH>(), cur, nxt);
         stage(IC<NS + 1>(), 0, par, d0);                                                 // k
-        issue(IC<NS + 1 + DEPTH>(), it);
+        issue(IC<NS + 1 + DEPTH>(), cur, nxt);
         close_item();
         lds_barrier();                                                                   // A
         stage_gates(par ^ 1);
-        issue_gates(it + 2 * stride);
+        aft = issue_gates(it + 2 * stride);
         lds_barrier();                                                                   // b
         lds_barrier();                                                                   // c
         lds_barrier();                                                                   // d
       }
       {
         typename IOK::Regs r;
-        IOK::load_lds_clamped(r, smem + B_Q, LDK, ci.len, tid);
+        IOK::load_lds_clamped(r, smem + B_Q, LDK, cur.len, tid);
         act_backward(r, XQ);
-        IOK::template store_global_clamped<true>(r, row_ptr<T>(a.dq, ci.b, ci.tok, h), a.dq.st, ci.len, tid);
-        IOK::load_lds_clamped(r, smem + B_K, LDK, ci.len, tid);
+        IOK::template store_global_clamped<true>(r, rows(a.dq, cur), a.dq.st, cur.len, tid);
+        IOK::load_lds_clamped(r, smem + B_K, LDK, cur.len, tid);
         act_backward(r, XK);
-        IOK::template store_global_clamped<true>(r, row_ptr<T>(a.dk, ci.b, ci.tok, h), a.dk.st, ci.len, tid);
+        IOK::template store_global_clamped<true>(r, rows(a.dk, cur), a.dk.st, cur.len, tid);
       }
       if constexpr (NBUF == 1) {
         stage(IC<NU>(), 0, par ^ 1, d0);                       // slice 0 of the next item
-        issue(IC<NU + DEPTH>(), it);
-        store_dv(d0, cin, hn, 0);
+        issue(IC<NU + DEPTH>(), cur, nxt);
+        store_dv(d0, nxt, 0);
         lds_barrier();                                                                   // R(0) of the next item
       }
       par ^= 1;
+      cur = nxt;
+      nxt = aft;
     }
     return;
   }
@@ -431,9 +426,15 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     // the iteration instead of living in registers for the whole kernel
     const int l = fresh_index(lane_id()) & 63;
     const int fr = l & 15, fg = 8 * (l >> 4);
-    const int rb = r0 + 4 * (l >> 4);      // accumulator element i is row rb + i, column (tile) + fr
-    f32x4 dP[1][2], dLf[1][2], dqi[1][NBK], dkd[1][NBK], dkbg[1][NBK];
-    acc_zero(dP); acc_zero(dLf); acc_zero(dqi); acc_zero(dkd); acc_zero(dkbg);
+    const int rb = r0 + 4 * (l >> 4);      // chunk x chunk products: element i is row rb + i, column (tile) + fr
+    // K-wide products are formed transposed (the state, k or q as the A operand): element i is K column kc + 16 ni + i of
+    // token r0 + fr, so that q, k are read and dq, dk written four columns (8 bytes) at a time and the factors of a token
+    // are one value per lane.  (Token by row, the same accesses were 96 2-byte ones per wave and item.)
+    const int tk = r0 + fr, kc = k0 + 4 * (l >> 4);
+    f32x4 dP[1][2], dLf[1][2], dqi[NBK], dkd[NBK], dkbg[NBK];
+    acc_zero(dP); acc_zero(dLf);
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni) dqi[ni] = dkd[ni] = dkbg[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
     // ---- stage 1 ----
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -457,9 +458,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
 #pragma unroll
         for (int ni = 0; ni < NBK; ++ni) {
           const typename ET<T>::frag bH = ET<T>::load_frag_t(HT, LDK, kk, k0 + 16 * ni, l);
-          ET<T>::mma(dqi[0][ni], aDO, bH);
-          ET<T>::mma(dkbg[0][ni], aDZ, bH);                                              // + dZ S^T: dk_bg is its negative
-          ET<T>::mma(dkd[0][ni], aVN, ET<T>::load_frag_t(DHT, LDK, kk, k0 + 16 * ni, l));
+          ET<T>::mma(dqi[ni], bH, aDO);
+          ET<T>::mma(dkbg[ni], bH, aDZ);                                                 // + dZ S^T: dk_bg is its negative
+          ET<T>::mma(dkd[ni], ET<T>::load_frag_t(DHT, LDK, kk, k0 + 16 * ni, l), aVN);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -468,6 +469,18 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     if constexpr (NBUF == 1) lds_barrier();                                              // A: q, k staged
     // ---- stage 2 ----
     T* Qt = smem + B_Q; T* Kt = smem + B_K; T* T0 = smem + B_T0; T* T1 = smem + B_T1; T* T2 = smem + B_T2;
+    typedef typename ET<T>::vec4 vec4;
+    typedef typename ET<T>::frag frag;
+    constexpr int CS = CH / 32;
+    // The k^T fragments serve three of the four products and are requested while G and dM are formed; the rows of q and k
+    // that the sums need are read once.  (Every product with fragments of its own, each step waited for: 80 transposing
+    // reads per wave and item where these are 32, and the LDS round trips of 8 steps behind barrier b.)
+    frag ft[CS][NBK];
+    vec4 k4[NBK], q4[NBK];
+#pragma unroll
+    for (int ks = 0; ks < CS; ++ks)
+#pragma unroll
+      for (int ni = 0; ni < NBK; ++ni) ft[ks][ni] = ET<T>::load_frag_t(Kt, LDK, 32 * ks, k0 + 16 * ni, l);
 #pragma unroll
     for (int nj = 0; nj < 2; ++nj) {
       f32x4 g, m, mb;
@@ -484,95 +497,101 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
       acc_to_lds_t<T>(mb, T2, LDC, r0, c0 + 16 * nj, l);                                 // (diag(beta) dM)^T [j][i]
     }
     lds_barrier();                                                                       // b
-    float dbp[4] = {0.f, 0.f, 0.f, 0.f};      // db of rows rb + i (partial over lanes and column halves)
-    float dbt[4] = {0.f, 0.f, 0.f, 0.f};      // dbeta of rows rb + i, the part through k_b
+    float dbp[4] = {0.f, 0.f, 0.f, 0.f};      // db of token tk (partial over elements, lanes and column halves)
+    float dbt[4] = {0.f, 0.f, 0.f, 0.f};      // dbeta of token tk, the part through k_b
     float kk = 0.f;
-    f32x4 dq[1][NBK], dk[1][NBK];
-    acc_zero(dq);
-    gemm_bounded<T, 1, NBK, true, true>(dq, T0, LDC, r0, Kt, LDK, k0, 0, CH, l);         // G k
+    // acc += (tile^T's rows r0 .., or the tile's rows) times what ft holds.  The tiles are triangular: rows of the first
+    // half have no entries in the second half of the contraction, and the other way round for the transposed tile
+    auto products = [&](f32x4 (&acc)[NBK], const T* tile, auto transposed) {
+      constexpr bool TR = decltype(transposed)::value;
+      frag fb[CS];
+#pragma unroll
+      for (int ks = 0; ks < CS; ++ks)
+        fb[ks] = TR ? ET<T>::load_frag_t(tile, LDC, 32 * ks, r0, l) : ET<T>::load_frag(tile + tk * LDC + 32 * ks + fg);
+#pragma unroll
+      for (int ni = 0; ni < NBK; ++ni) acc[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < CS; ++ks) {
+        if (TR ? (ks == 0 || r0 >= 32) : (ks == 1 || r0 < 32)) {
+#pragma unroll
+          for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(acc[ni], ft[ks][ni], fb[ks]);
+        }
+      }
+    };
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni) {
+      q4[ni] = *(const vec4*)(Qt + tk * LDK + kc + 16 * ni);
+      k4[ni] = *(const vec4*)(Kt + tk * LDK + kc + 16 * ni);
+    }
+    const float ebt = s_eb[tk], edt = s_ed[tk], bt = s_beta[tk];
+    f32x4 dq[NBK], dk[NBK], m[NBK];
+    products(dq, T0, std::true_type());                                                  // (G k)^T
+    products(m, T1, std::true_type());                                                   // (dM k)^T: closes dk_b
 #pragma unroll
     for (int ni = 0; ni < NBK; ++ni)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = rb + i, cc = k0 + 16 * ni + fr;
-        const float dqv = scale * s_eb[r] * dqi[0][ni][i] + dq[0][ni][i];
-        dbp[i] += ET<T>::to_f(Qt[r * LDK + cc]) * dqv;
-        dq[0][ni][i] = dqv;                                                              // final dq
+        const float dqv = scale * ebt * dqi[ni][i] + dq[ni][i];
+        dbp[i] += ET<T>::to_f(q4[ni][i]) * dqv;
+        dq[ni][i] = dqv;                                                                 // final dq
       }
     pin(dbp);
-    __builtin_amdgcn_sched_barrier(0);
-    acc_zero(dk);
-    gemm_bounded<T, 1, NBK, false, true>(dk, T0, LDC, r0, Qt, LDK, k0, 0, CH, l);        // G^T q
 #pragma unroll
     for (int ni = 0; ni < NBK; ++ni)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = rb + i, cc = k0 + 16 * ni + fr;
-        const float kv = ET<T>::to_f(Kt[r * LDK + cc]);
-        const float dkdv = s_ed[r] * dkd[0][ni][i];
-        const float dkv = dkdv + dk[0][ni][i];
+        const float kv = ET<T>::to_f(k4[ni][i]);
+        const float kbv = kv * bt;
+        const float dkbgv = -dkbg[ni][i];
+        const float dkb = m[ni][i] + dkbgv * ebt;
+        dbt[i] += dkb * kv;
+        dbp[i] += kbv * m[ni][i] + dkbgv * kbv * ebt;
+        dk[ni][i] = dkb * bt;
+      }
+    pin(dbp);
+    pin(dbt);
+    products(m, T2, std::false_type());                                                  // (dM^T k_b)^T
+    // k^T is done with: q^T for the last product
+#pragma unroll
+    for (int ks = 0; ks < CS; ++ks)
+#pragma unroll
+      for (int ni = 0; ni < NBK; ++ni) ft[ks][ni] = ET<T>::load_frag_t(Qt, LDK, 32 * ks, k0 + 16 * ni, l);
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dbp[i] -= ET<T>::to_f(k4[ni][i]) * m[ni][i];
+        dk[ni][i] += m[ni][i];
+      }
+    pin(dbp);
+    products(m, T0, std::false_type());                                                  // (G^T q)^T
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float kv = ET<T>::to_f(k4[ni][i]);
+        const float dkdv = edt * dkd[ni][i];
+        const float dkv = dkdv + m[ni][i];                                               // the part of dk that does not pass through the WY form
         dbp[i] -= kv * dkv;
         kk += kv * dkdv;
-        dk[0][ni][i] = dkv;                                                              // first part of dk
+        dk[ni][i] += dkv;                                                                // final dk
       }
-    pin(dbp);
-    pin(kk);
-    __builtin_amdgcn_sched_barrier(0);
-    {
-      // dM k first: it closes dk_b (dbeta, the k_b.(dM k) term); then dM^T k_b
-      // (k is re-read from LDS through an offset the compiler cannot see through: it would otherwise
-      // keep the values read for the first part of dk in registers)
-      const T* Kr = Kt + fresh_index(0);
-      f32x4 m[1][NBK];
-      acc_zero(m);
-      gemm_bounded<T, 1, NBK, true, true>(m, T1, LDC, r0, Kt, LDK, k0, 0, CH, l);
-#pragma unroll
-      for (int ni = 0; ni < NBK; ++ni)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = rb + i, cc = k0 + 16 * ni + fr;
-          const float kv = ET<T>::to_f(Kr[r * LDK + cc]);
-          const float bt = s_beta[r], eb = s_eb[r];
-          const float kbv = kv * bt;
-          const float dkbgv = -dkbg[0][ni][i];
-          const float dkb = m[0][ni][i] + dkbgv * eb;
-          dbt[i] += dkb * kv;
-          dbp[i] += kbv * m[0][ni][i] + dkbgv * kbv * eb;
-          dk[0][ni][i] += dkb * bt;
-        }
-      pin(dbp);
-      pin(dbt);
-      __builtin_amdgcn_sched_barrier(0);
-      const T* Kr2 = Kt + fresh_index(0);
-      acc_zero(m);
-      gemm_bounded<T, 1, NBK, false, true>(m, T2, LDC, r0, Kt, LDK, k0, 0, CH, l);
-#pragma unroll
-      for (int ni = 0; ni < NBK; ++ni)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = rb + i, cc = k0 + 16 * ni + fr;
-          dbp[i] -= ET<T>::to_f(Kr2[r * LDK + cc]) * m[0][ni][i];
-          dk[0][ni][i] += m[0][ni][i];                                                   // final dk
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      dbp[i] = group_sum<16>(dbp[i]);
-      dbt[i] = group_sum<16>(dbt[i]);
-    }
+    // over the elements and the four lanes that hold a token
+    float dbs = (dbp[0] + dbp[1]) + (dbp[2] + dbp[3]), dts = (dbt[0] + dbt[1]) + (dbt[2] + dbt[3]);
+    dbs += __shfl_xor(dbs, 16, 64);
+    dts += __shfl_xor(dts, 16, 64);
+    dbs += __shfl_xor(dbs, 32, 64);
+    dts += __shfl_xor(dts, 32, 64);
     kk = wave_sum(kk);
     lds_barrier();                                                                       // c: q, k, the chunk x chunk tiles read
 #pragma unroll
     for (int ni = 0; ni < NBK; ++ni) {
-      acc_to_lds<T>(dq[0][ni], Qt, LDK, r0, k0 + 16 * ni, l);                            // dq, dk on their way out
-      acc_to_lds<T>(dk[0][ni], Kt, LDK, r0, k0 + 16 * ni, l);
+      acc_to_lds_t<T>(dq[ni], Qt, LDK, k0 + 16 * ni, r0, l);                          // dq, dk on their way out
+      acc_to_lds_t<T>(dk[ni], Kt, LDK, k0 + 16 * ni, r0, l);
     }
-    if (fr == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        s_db[ch][rb + i] = dbp[i];
-        s_dbeta[ch][rb + i] = dbt[i];
-      }
+    if (l < 16) {
+      s_db[ch][tk] = dbs;
+      s_dbeta[ch][tk] = dts;
     }
     if (l == 0) s_red[4 + wv] = kk;
     lds_barrier();                                                                       // d
