@@ -18,16 +18,19 @@ namespace lmoe {
 // In-LDS inverse of the unit lower triangular matrix I + L (64 x 64, fp32).
 //   sL : strictly lower part L (upper part and diagonal must be 0), leading dimension ldl
 //   sX : receives (I + L)^-1, leading dimension ldx
-//   sY : scratch, one 16 x 17 fp32 block per wave (4 * 272 floats)
-// Block forward substitution with 16 x 16 blocks.  The four diagonal blocks are inverted by the
-// four waves on the vector ALU (one column per lane).  The off-diagonal blocks follow by block
-// distance d = I - J, one block per wave, on the matrix cores in fp32 (v_mfma_f32_16x16x4_f32):
-//   Y = sum_{M = J}^{I-1} L_IM X_MJ   (4 d instructions),   X_IJ = - X_II Y   (4 instructions),
-// with Y passed through the wave's own scratch block, so a round needs one work-group barrier.
+//   sY : scratch, four 16 x 17 fp32 blocks (4 * 272 floats)
+// 16 x 16 blocks.  The four diagonal blocks are inverted on the vector ALU by forward substitution, one column per
+// lane: all four by one wave.  The rest on the matrix cores in fp32 (v_mfma_f32_16x16x4_f32), by halves: first the
+// blocks (1, 0) and (3, 2),  X_10 = - X_11 (L_10 X_00),  which completes the inverses of the two 32 x 32 diagonal halves, then
+// the lower left half,  Y = L_21 X_11,  X_21 = - X_22 Y,  a block per wave with Y exchanged through LDS.
+// What bounds it is the SIMD with the most of it: three work-groups share a CU, and a wave's index decides its SIMD.  By block
+// distance (three rounds of 3, 2, 1 blocks) wave 0 had 36 of the 64 matrix instructions of an item in every work-group, and the
+// substitution ran on 16 lanes of all four waves; now no wave has more than 20 and 24 follow one another: 68 -> 62 us for
+// 8192 items, of which the inverse 28 -> 22 (and 60 with an item's place worked out once instead of three times).
 // Must be called by all 256 threads (l, tid: lane and thread index); sL must be complete and sX free
 // (barrier before the call).
 __device__ __forceinline__ void tri_inverse_64(const float* sL, int ldl, float* sX, int ldx, float* sY, int l, int tid) {
-  const int wv = wave_id();
+  const int share = wave_id();          // what this wave does
   // clear X (upper blocks stay zero)
   // the six blocks above the diagonal are zero; nothing else writes them, so no barrier before the rest
   {
@@ -37,11 +40,12 @@ __device__ __forceinline__ void tri_inverse_64(const float* sL, int ldl, float* 
 #pragma unroll
       for (int J = I + 1; J < 4; ++J) sX[(16 * I + r) * ldx + 16 * J + c] = 0.f;
   }
-  if (l < 16) {
-    // lane c solves column c by forward substitution; every lane reads the same coefficients (broadcast
+  if (share == 0) {
+    // lane 16 g + c solves column c of block g; the lanes of a block read the same coefficients (broadcast
     // reads of whole rows).  The rows are requested in three batches ahead of their use: reading each
     // coefficient where it is used cost one LDS round trip per row (1.3 us of an 11 us item)
-    const float* lb = sL + 16 * wv * ldl + 16 * wv;
+    const int g16 = l & 48, col = l & 15;
+    const float* lb = sL + g16 * ldl + g16;
     f32x4 c[16][4];
     auto rows = [&](auto i0, auto i1) {
 #pragma unroll
@@ -53,7 +57,7 @@ __device__ __forceinline__ void tri_inverse_64(const float* sL, int ldl, float* 
     auto solve = [&](auto i0, auto i1) {
 #pragma unroll
       for (int i = decltype(i0)::value; i < decltype(i1)::value; ++i) {
-        float s = (i == l) ? 1.f : 0.f;
+        float s = (i == col) ? 1.f : 0.f;
 #pragma unroll
         for (int m = 0; m < i; ++m) s -= c[i][m >> 2][m & 3] * x[m];
         x[i] = s;
@@ -75,48 +79,76 @@ __device__ __forceinline__ void tri_inverse_64(const float* sL, int ldl, float* 
     __builtin_amdgcn_sched_barrier(0);
     solve(I12(), I16());
 #pragma unroll
-    for (int i = 0; i < 16; ++i) sX[(16 * wv + i) * ldx + 16 * wv + l] = x[i];
+    for (int i = 0; i < 16; ++i) sX[(g16 + i) * ldx + g16 + col] = x[i];
   }
   lds_barrier();
   // operand layout of the 16 x 16 x 4 instruction: A[m = l % 16][k = l / 16], B[k = l / 16][n = l % 16],
   // result rows 4 (l / 16) + i of column l % 16
   const int r16 = l & 15, k4 = l >> 4;
-  float* yb = sY + wv * 272;
+  // blocks (1, 0) and (3, 2): Y = L_IJ X_JJ passes through a scratch block of the wave's own
+  if (share == 1 || share == 2) {
+    const int J = share == 1 ? 0 : 2, I = J + 1;
+    float* yb = sY + share * 272;
+    float la[4], xb[4], xd[4];
 #pragma unroll
-  for (int d = 1; d < 4; ++d) {
-    if (wv + d < 4) {                      // wave-uniform: block (I, J) = (wv + d, wv)
-      const int J = wv, I = wv + d;
-      // every operand of the round is requested before the first product (one LDS round trip instead of
-      // one per instruction)
-      float la[12], xb[12], xd[4];
+    for (int t = 0; t < 4; ++t) {
+      la[t] = sL[(16 * I + r16) * ldl + 16 * J + 4 * t + k4];
+      xb[t] = sX[(16 * J + 4 * t + k4) * ldx + 16 * J + r16];
+      xd[t] = sX[(16 * I + r16) * ldx + 16 * I + 4 * t + k4];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 y = {0.f, 0.f, 0.f, 0.f}, x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int t = 0; t < 4 * d; ++t) {
+    for (int t = 0; t < 4; ++t) y = __builtin_amdgcn_mfma_f32_16x16x4f32(la[t], xb[t], y, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) yb[(4 * k4 + i) * 17 + r16] = y[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float yv[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) yv[t] = yb[(4 * t + k4) * 17 + r16];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x = __builtin_amdgcn_mfma_f32_16x16x4f32(xd[t], yv[t], x, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sX[(16 * I + 4 * k4 + i) * ldx + 16 * J + r16] = -x[i];
+  }
+  lds_barrier();
+  {
+    // the lower left half, block (I, J): (3, 0), (2, 1), (2, 0), (3, 1) for the shares 0 .. 3.  Triangular: the first column
+    // of blocks takes both blocks of X_11, the second one; likewise X_22 and the rows
+    const int I = share == 1 || share == 2 ? 2 : 3, J = share & 1;
+    float la[8], xb[8], xd[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      if (t < 4 || J == 0) {
         la[t] = sL[(16 * I + r16) * ldl + 16 * J + 4 * t + k4];
         xb[t] = sX[(16 * J + 4 * t + k4) * ldx + 16 * J + r16];
       }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) xd[t] = sX[(16 * I + r16) * ldx + 16 * I + 4 * t + k4];
-      __builtin_amdgcn_sched_barrier(0);
-      f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < 4 * d; ++t) y = __builtin_amdgcn_mfma_f32_16x16x4f32(la[t], xb[t], y, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) yb[(4 * k4 + i) * 17 + r16] = y[i];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      float yv[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) yv[t] = yb[(4 * t + k4) * 17 + r16];
-      __builtin_amdgcn_sched_barrier(0);
-      f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int t = 0; t < 4; ++t) x = __builtin_amdgcn_mfma_f32_16x16x4f32(xd[t], yv[t], x, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) sX[(16 * I + 4 * k4 + i) * ldx + 16 * J + r16] = -x[i];
+      if (t < 4 || I == 3) xd[t] = sX[(16 * I + r16) * ldx + 32 + 4 * t + k4];
     }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 y = {0.f, 0.f, 0.f, 0.f}, x = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (t < 4 || J == 0) y = __builtin_amdgcn_mfma_f32_16x16x4f32(la[t], xb[t], y, 0, 0, 0);
+    float* yb = sY + (2 * (I - 2) + J) * 272;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) yb[(4 * k4 + i) * 17 + r16] = y[i];
     lds_barrier();
+    float yv[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (t < 4 || I == 3) yv[t] = sY[(2 * (t >> 2) + J) * 272 + (4 * (t & 3) + k4) * 17 + r16];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (t < 4 || I == 3) x = __builtin_amdgcn_mfma_f32_16x16x4f32(xd[t], yv[t], x, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sX[(16 * I + 4 * k4 + i) * ldx + 16 * J + r16] = -x[i];
   }
+  lds_barrier();
 }
 
 // SAVE = false (no Tinv buffer given): Tinv is not written.  With Tinv written and 2-byte elements the
@@ -158,35 +190,41 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
   typename IOV::Regs rv;
   RowFrags<T, K> fq;
   uint32_t graw, braw;
-  auto item_of = [&](int it, int& h) {
+  // an item's place: worked out once, when it is the next one
+  struct Item { int h; ChunkInfo ci; int64_t at; };          // at: its number
+  auto item_of = [&](int it) {
+    Item I;
     it = min(it, nitems - 1);
-    h = it % a.H;
-    return chunk_info(a, it / a.H);
+    const int cid = it / a.H;
+    I.h = it - cid * a.H;
+    I.ci = chunk_info(a, cid);
+    I.at = it;
+    return I;
   };
   // q enters only as the A operand of q k^T: each wave takes its 16 rows straight into fragments
-  auto issue_q = [&](int it) { if constexpr (LEAN) return; int h; const ChunkInfo ci = item_of(it, h); fq.load(row_ptr<T>(a.q, ci.b, ci.tok, h), a.q.st, 16 * wv, ci.len - 1); };
-  auto issue_k = [&](int it) { int h; const ChunkInfo ci = item_of(it, h); IOK::load_nomask(rk, row_ptr<T>(a.k, ci.b, ci.tok, h), a.k.st, ci.len); };
-  auto issue_v = [&](int it) {
-    if constexpr (!LEAN) { int h; const ChunkInfo ci = item_of(it, h); IOV::load_nomask(rv, row_ptr<T>(a.v, ci.b, ci.tok, h), a.v.st, ci.len); }
+  auto issue_q = [&](const Item& I) { if constexpr (!LEAN) fq.load(row_ptr<T>(a.q, I.ci.b, I.ci.tok, I.h), a.q.st, 16 * wv, I.ci.len - 1); };
+  auto issue_k = [&](const Item& I) { IOK::load_nomask(rk, row_ptr<T>(a.k, I.ci.b, I.ci.tok, I.h), a.k.st, I.ci.len); };
+  auto issue_v = [&](const Item& I) {
+    if constexpr (!LEAN) IOV::load_nomask(rv, row_ptr<T>(a.v, I.ci.b, I.ci.tok, I.h), a.v.st, I.ci.len);
   };
-  auto issue_gb = [&](int it) {
-    int h; const ChunkInfo ci = item_of(it, h);
-    graw = gate_prefetch(a, ci.b, ci.tok, ci.len, h);
-    braw = load_scalar_raw(a.beta.ptr, a.beta_dtype, row_off(a.beta, ci.b, ci.tok + min(l, ci.len - 1), h));
+  auto issue_gb = [&](const Item& I) {
+    graw = gate_prefetch(a, I.ci.b, I.ci.tok, I.ci.len, I.h);
+    braw = load_scalar_raw(a.beta.ptr, a.beta_dtype, row_off(a.beta, I.ci.b, I.ci.tok + min(l, I.ci.len - 1), I.h));
   };
-  issue_q(blockIdx.x);
-  issue_k(blockIdx.x);
-  issue_v(blockIdx.x);
-  issue_gb(blockIdx.x);
+  Item cur = item_of(blockIdx.x);
+  issue_q(cur);
+  issue_k(cur);
+  issue_v(cur);
+  issue_gb(cur);
   wait_all_loads();   // the first loads may be ordered freely; the loop's waits must not inherit that order
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
   // lane / thread index refreshed per item: the address arithmetic derived from them stays inside the
   // iteration instead of living in registers for the whole kernel
   const int l = fresh_index(lane_id()) & 63;
   const int tid = fresh_index((int)threadIdx.x) & (NTHR - 1);
-  const int cid = it / a.H, h = it % a.H;
-  const ChunkInfo ci = chunk_info(a, cid);
-  const int nxt = it + gridDim.x;
+  const Item nxt = item_of(it + gridDim.x);
+  const ChunkInfo ci = cur.ci;
+  const int h = cur.h;
   IOK::mask(rk, ci.len, tid);
   if constexpr (!LEAN) IOV::mask(rv, ci.len, tid);
   lds_barrier();      // the previous item has left every tile
@@ -209,7 +247,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
     // the wait for the next item's inputs a wait for this item's last stores as well
     // (rows 2, 3: beta and beta e^{b}, zero past the end of the chunk -- the sequential passes then read no beta,
     // whose run-time element type would put a load behind a branch in their prefetch loops)
-    float* gc = a.gcum + ((int64_t)cid * a.H + h) * GATE_ROWS * CH;
+    float* gc = a.gcum + cur.at * GATE_ROWS * CH;
     const int row = tid >> 6;
     gc[tid] = row == 0 ? eb : row == 1 ? ed : row == 2 ? bl : bl * eb;
     gc[4 * CH + l] = xb;       // (all four waves, the same bytes)
@@ -234,7 +272,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
     // zero and skipped (wave-uniform), and one exponential per element serves both.  P goes to global
     // memory, staged through the (still unused) X tile
     T* s_P = (T*)s_X;
-    T* pg = (T*)a.pmat + ((int64_t)cid * a.H + h) * CH * CH;
+    T* pg = (T*)a.pmat + cur.at * CH * CH;
     f32x4 m[4], pm[4];
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) { m[nj] = f32x4{0.f, 0.f, 0.f, 0.f}; pm[nj] = m[nj]; }
@@ -282,7 +320,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
   lds_barrier();   // L is complete, the P staging has been read: the inverse may overwrite X
   tri_inverse_64(s_L, LDC, s_X, LDC, s_Y, l, tid);       // barriers inside; s_L is dead afterwards
   {
-    T* tg = (T*)a.tinv + ((int64_t)cid * a.H + h) * CH * CH;
+    T* tg = (T*)a.tinv + cur.at * CH * CH;
 #pragma unroll
     for (int p = 0; p < CH * CH / 4 / NTHR; ++p) {      // fixed trip count: see the decay table above
       const int idx = p * NTHR + tid;
@@ -334,6 +372,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
     IOV::template store_global_clamped<true>(ou, row_ptr<T>(a.u, ci.b, ci.tok, h), a.u.st, ci.len, tid);
   }
   }
+  cur = nxt;
   }   // items
 }
 
