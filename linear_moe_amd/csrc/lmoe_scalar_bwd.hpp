@@ -614,7 +614,7 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqk(const lmoe_args a) {
 //               the next item, request those of the one after
 //     compute : P^T strip | products of slice s, dv stores | D, A | (dP . Gamma)^T -> LDS | b | products, combine |
 //               c | stores | E
-// Every sum is formed in the order of k_bwd_dv and k_bwd_dqk: the results are theirs bit for bit.
+// dv is formed in the order of k_bwd_dv, bit for bit.
 // ------------------------------------------------------------------------- //
 // NORM (see k_state_bwd): d_o is the gradient of the normalised output.  With rD = 1 / D, dd = scale dden (the sum of
 // the partial rows of norm_ws), z = the sum of the keys before the chunk (zs) and dz = the gradient of the column of
@@ -663,31 +663,39 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
     const int e_norm = min((int)(threadIdx.x & (NTHR - 1)), WS_ROW - 1);
     // Every prefetch is issued unconditionally (item index clamped to the last item): a load that
     // is skipped on some path would make the compiler drain all outstanding loads at every use.
-    auto issue_slice = [&](int it, int vv) {
-      it = min(it, nitems - 1);
-      const int cid = it / a.H, h = it % a.H;
-      const ChunkInfo ci = chunk_info(a, cid);
+    // (an item's place is worked out once per item, not per request)
+    struct Item { int it, h; ChunkInfo ci; };
+    auto item_at = [&](int it) {
+      Item I;
+      I.it = __builtin_amdgcn_readfirstlane(min(it, nitems - 1));
+      const int cid = I.it / a.H;
+      I.h = I.it - cid * a.H;
+      I.ci = chunk_info(a, cid);
+      return I;
+    };
+    auto issue_slice = [&](const Item& I, int vv) {
+      const ChunkInfo& ci = I.ci;
+      const int h = I.h;
       S.len = ci.len;
       IOV::load_nomask(S.rd, row_ptr<T>(a.d_o, ci.b, ci.tok, h) + vv, a.d_o.st, ci.len);
       IOV::load_nomask(S.rv, row_ptr<T>(a.v, ci.b, ci.tok, h) + vv, a.v.st, ci.len);
-      IOH::load_nomask(S.rh, (const T*)a.hs + (((int64_t)cid * a.H + h) * V + vv) * K, K, BVH);
-      IOH::load_nomask(S.rdh, (const T*)a.dhs + (((int64_t)cid * a.H + h) * V + vv) * K, K, BVH);
+      IOH::load_nomask(S.rh, (const T*)a.hs + ((int64_t)I.it * V + vv) * K, K, BVH);          // it = cid * H + h
+      IOH::load_nomask(S.rdh, (const T*)a.dhs + ((int64_t)I.it * V + vv) * K, K, BVH);
     };
-    auto issue_qk = [&](int it) {
-      it = min(it, nitems - 1);
-      const int cid = it / a.H, h = it % a.H;
-      const ChunkInfo ci = chunk_info(a, cid);
+    auto issue_qk = [&](const Item& I) {
+      const ChunkInfo& ci = I.ci;
+      const int h = I.h;
       Q.len = ci.len;
       IOK::load_nomask(Q.rq, row_ptr<T>(a.q, ci.b, ci.tok, h), a.q.st, ci.len);
       IOK::load_nomask(Q.rk, row_ptr<T>(a.k, ci.b, ci.tok, h), a.k.st, ci.len);
       Q.graw = gate_prefetch(a, ci.b, ci.tok, ci.len, h);
       if constexpr (NORM) {
-        const float* ws = a.norm_ws + (int64_t)it * WS_SLOTS * WS_ROW + e_norm;          // it = cid * H + h
+        const float* ws = a.norm_ws + (int64_t)I.it * WS_SLOTS * WS_ROW + e_norm;
 #pragma unroll
         for (int sl = 0; sl < WS_SLOTS; ++sl) Q.ws[sl] = ws[sl * WS_ROW];
         const lmoe_tensor& dt = NORM == 1 ? a.den : a.dden;               // (NORM = 2: read, not used, for rows)
         const float* den = (const float*)dt.ptr + row_off(dt, ci.b, ci.tok + min(e_norm, ci.len - 1), h);
-        const float* zc = a.zs + (int64_t)it * K + max(e_norm - CH, 0);
+        const float* zc = a.zs + (int64_t)I.it * K + max(e_norm - CH, 0);
         Q.x = *(e_norm < CH ? den : zc);
       }
     };
@@ -695,9 +703,7 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
     auto stage_slice = [&](int buf) {
       T* base = smem + buf * BUF1;
 #pragma unroll
-      for (int p = 0; p < IOH::PASSES; ++p)
-#pragma unroll
-        for (int i = 0; i < IOH::VEC; ++i) hdh += ET<T>::to_f(S.rh.v[p][i]) * ET<T>::to_f(S.rdh.v[p][i]);
+      for (int p = 0; p < IOH::PASSES; ++p) hdh = dot_vec(S.rh.v[p], S.rdh.v[p], hdh);
       IOV::mask(S.rd, S.len);
       IOV::mask(S.rv, S.len);
       IOV::store_lds(S.rd, base + A_DO, LDV);
@@ -725,29 +731,30 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
       IOK::store_lds(Q.rq, smem + B_Q, LDK);
       IOK::store_lds(Q.rk, smem + B_K, LDK);
     };
-    // the slice after slice s of item it
-    auto issue_next = [&](int it, int s) {
-      if (s + 1 < NS) issue_slice(it, (s + 1) * BVH); else issue_slice(it + stride, 0);
+    // the slice after slice s of an item
+    auto issue_next = [&](const Item& I, const Item& after, int s) {
+      if (s + 1 < NS) issue_slice(I, (s + 1) * BVH); else issue_slice(after, 0);
     };
-    const int it0 = blockIdx.x;
-    issue_slice(it0, 0);
-    issue_qk(it0);
+    Item cur = item_at(blockIdx.x), nxt = item_at(blockIdx.x + stride);
+    issue_slice(cur, 0);
+    issue_qk(cur);
     // the first loads may be ordered freely by the compiler; were they still pending at the loop
     // header, its wait-count analysis would carry that order into every iteration
     wait_all_loads();
     stage_slice(0);
     stage_qk(0);
-    issue_qk(it0 + stride);
-    issue_next(it0, 0);
+    issue_qk(nxt);
+    issue_next(cur, nxt, 0);
     lds_barrier();                                                                       // first item staged
     int par = 0;
-    for (int it = it0; it < nitems; it += stride, par ^= 1) {
+    for (int it = blockIdx.x; it < nitems; it += stride, par ^= 1) {
+      const Item aft = item_at(it + 2 * stride);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         if (s > 0) lds_barrier();                                                        // R(s)
         if (s + 1 < NS) {
           stage_slice((s + 1) & 1);        // its buffer was left when the compute team passed R(s) (s = 0: E)
-          issue_next(it, s + 1);
+          issue_next(cur, nxt, s + 1);
         }
       }
       lds_barrier();                                                                     // D
@@ -756,12 +763,14 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
       hdh = 0.f;
       lds_barrier();                                                                     // A
       stage_slice(0);                      // slice 0 of the next item (buffer 0 is idle in phase B)
-      issue_next(it + stride, 0);
+      issue_next(nxt, aft, 0);
       lds_barrier();                                                                     // b
       lds_barrier();                                                                     // c
       stage_qk(par ^ 1);                   // q, k of this item were read for the last time before c
-      issue_qk(it + 2 * stride);
+      issue_qk(aft);
       lds_barrier();                                                                     // E
+      cur = nxt;
+      nxt = aft;
     }
     return;
   }
@@ -810,8 +819,13 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
 #pragma unroll
     for (int kq = 0; kq < CS; ++kq) fpt[kq] = ET<T>::load_frag(PT + j * LDC + 32 * kq + fg);
 
-    f32x4 dP[1][4], dqi[1][NBK], dkd[1][NBK];
-    acc_zero(dP); acc_zero(dqi); acc_zero(dkd);
+    // K-wide products are formed transposed (the state, k or q as the A operand): element i is column 16 ni + 4 g + i of
+    // token j, so that q, k are read and dq, dk staged four columns at a time and a token's factors are one value
+    // per lane (token by row: 64 2-byte reads and 64 2-byte writes per wave and item)
+    f32x4 dP[1][4], dqi[NBK], dkd[NBK];
+    acc_zero(dP);
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni) dqi[ni] = dkd[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       if (s > 0) lds_barrier();                                                          // R(s)
@@ -829,8 +843,8 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
 #pragma unroll
         for (int ni = 0; ni < NBK; ++ni) {
           const typename ET<T>::frag bH = ET<T>::load_frag_t(HT, LDK, kk, 16 * ni, lf);
-          ET<T>::mma(dqi[0][ni], aDO, bH);
-          ET<T>::mma(dkd[0][ni], aVN, ET<T>::load_frag_t(DHT, LDK, kk, 16 * ni, lf));
+          ET<T>::mma(dqi[ni], bH, aDO);
+          ET<T>::mma(dkd[ni], ET<T>::load_frag_t(DHT, LDK, kk, 16 * ni, lf), aVN);
           if (ni % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -881,53 +895,70 @@ __global__ __launch_bounds__(2 * NTHR) void k_bwd_dqkv(const lmoe_args a) {
       acc_to_lds_t<T>(p, PT, LDC, 16 * wv, 16 * nj, lf);      // [j][i]
     }
     lds_barrier();                                                                       // b
-    f32x4 dq[1][NBK], dk[1][NBK];
-    acc_zero(dq); acc_zero(dk);
-    // dq_intra[i][c] = sum_j dPG[i][j] k[j][c] : A = dPG^T stored [j][i] (contraction along rows)
-    gemm<T, 1, NBK, true, true>(dq, PT, LDC, 16 * wv, KT, LDK, 0, 0, CH, lf);
+    f32x4 dq[NBK], dk[NBK];
+#pragma unroll
+    for (int ni = 0; ni < NBK; ++ni) dq[ni] = dk[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // (dP k)^T over rows of PT, then (dP^T q)^T; triangular: the first 32 tokens take the first half of the contraction
+    // of the one, the others the second half of the other
+#pragma unroll
+    for (int ks = 0; ks < CS; ++ks) {
+      if (ks == 0 || wv >= 2) {
+        const typename ET<T>::frag fb = ET<T>::load_frag_t(PT, LDC, 32 * ks, 16 * wv, lf);
+#pragma unroll
+        for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(dq[ni], ET<T>::load_frag_t(KT, LDK, 32 * ks, 16 * ni, lf), fb);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
-    // dk_intra[j][c] = sum_i dPG[i][j] q[i][c] : A = dPG^T rows j (contraction along columns)
-    gemm<T, 1, NBK, false, true>(dk, PT, LDC, 16 * wv, QT, LDK, 0, 0, CH, lf);
+#pragma unroll
+    for (int ks = 0; ks < CS; ++ks) {
+      if (ks == 1 || wv < 2) {
+        const typename ET<T>::frag fb = ET<T>::load_frag(PT + j * LDC + 32 * ks + fg);
+#pragma unroll
+        for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(dk[ni], ET<T>::load_frag_t(QT, LDK, 32 * ks, 16 * ni, lf), fb);
+      }
+    }
     __builtin_amdgcn_sched_barrier(0);
-    // combine and form db_i = q_i.dq_i - k_i.dk_i ; kk = sum_j (dk_d . k_d)_j
+    // combine and form db_j = q_j.dq_j - k_j.dk_j ; kk = sum_j (dk_d . k_d)_j
     float dbp[4] = {0.f, 0.f, 0.f, 0.f};
     float kk = 0.f;
+    const float fq_ = NORM ? s_rD[par][NORM ? j : 0] : s_eb[par][j], ddj = s_dd[NORM ? par : 0][NORM ? j : 0];
 #pragma unroll
-    for (int ni = 0; ni < NBK; ++ni)
+    for (int ni = 0; ni < NBK; ++ni) {
+      const int cc = 16 * ni + 4 * g;
+      const bf16x4 q4 = *(const bf16x4*)(QT + j * LDK + cc), k4 = *(const bf16x4*)(KT + j * LDK + cc);
+      f32x4 z4, dz4;
+      if constexpr (NORM) { z4 = *(const f32x4*)&s_z[par][cc]; dz4 = *(const f32x4*)&s_dz[par][cc]; }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wv + 4 * g + i, cc = 16 * ni + fr;
-        const float qv = ET<T>::to_f(QT[r * LDK + cc]);
-        const float kv = ET<T>::to_f(KT[r * LDK + cc]);
+        const float qv = (float)q4[i], kv = (float)k4[i];
         float dqv, dkdv;
         if constexpr (NORM) {
-          dqv = a.scale * s_rD[par][r] * dqi[0][ni][i] + s_dd[par][r] * s_z[par][cc] + dq[0][ni][i];
-          dkdv = dkd[0][ni][i] + s_dz[par][cc];
+          dqv = a.scale * fq_ * dqi[ni][i] + ddj * z4[i] + dq[ni][i];
+          dkdv = dkd[ni][i] + dz4[i];
         } else {
-          dqv = a.scale * s_eb[par][r] * dqi[0][ni][i] + dq[0][ni][i];
-          dkdv = s_ed[par][r] * dkd[0][ni][i];
+          dqv = a.scale * fq_ * dqi[ni][i] + dq[ni][i];
+          dkdv = edj * dkd[ni][i];
         }
-        const float dkv = dkdv + dk[0][ni][i];
+        const float dkv = dkdv + dk[ni][i];
         dbp[i] += qv * dqv - kv * dkv;
         kk += kv * dkdv;
-        dq[0][ni][i] = dqv;
-        dk[0][ni][i] = dkv;
+        dq[ni][i] = dqv;
+        dk[ni][i] = dkv;
       }
-    // reduce db over the 16 lanes that share a row group, kk over the whole team
-#pragma unroll
-    for (int i = 0; i < 4; ++i) dbp[i] = group_sum<16>(dbp[i]);
-    if (fr == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) s_db[16 * wv + 4 * g + i] = dbp[i];
     }
+    // db over the elements and the four lanes that hold a token, kk over the whole team
+    float dbs = (dbp[0] + dbp[1]) + (dbp[2] + dbp[3]);
+    dbs += __shfl_xor(dbs, 16, 64);
+    dbs += __shfl_xor(dbs, 32, 64);
+    if (g == 0) s_db[j] = dbs;
     kk = wave_sum(kk);
     if (lf == 0) s_red[4 + wv] = kk;
     lds_barrier();     // c: the q, k tiles go to the next item; the idle slice buffer is the store staging
     {
       T* stg = smem + BUF1 + wv * 16 * LDK;
-      store_strip<T, NBK>(dq, stg, row_ptr<T>(a.dq, ci.b, ci.tok + 16 * wv, h), a.dq.st, ci.len - 16 * wv, 1.0f, lf);
+      store_strip_t<T, NBK>(dq, stg, row_ptr<T>(a.dq, ci.b, ci.tok + 16 * wv, h), a.dq.st, ci.len - 16 * wv, 1.0f, lf);
       T* stg2 = smem + BUF1 + (4 + wv) * 16 * LDK;
-      store_strip<T, NBK>(dk, stg2, row_ptr<T>(a.dk, ci.b, ci.tok + 16 * wv, h), a.dk.st, ci.len - 16 * wv, 1.0f, lf);
+      store_strip_t<T, NBK>(dk, stg2, row_ptr<T>(a.dk, ci.b, ci.tok + 16 * wv, h), a.dk.st, ci.len - 16 * wv, 1.0f, lf);
     }
     if (threadIdx.x < 64) {
       const int t = threadIdx.x;
