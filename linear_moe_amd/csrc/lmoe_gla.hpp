@@ -935,7 +935,7 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   constexpr int B_BYTES = SUB ? S_BYTES : B_END * 4;
   constexpr int NBYTES = (A_END * (int)sizeof(T) > B_BYTES) ? A_END * (int)sizeof(T) : B_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char smem_raw[NBYTES];
-  __shared__ float s_hdh[K], s_kk[4 * K];
+  __shared__ __attribute__((aligned(16))) float s_hdh[K], s_kk[4 * K];
   T* smT = (T*)smem_raw;
   float* smF = (float*)smem_raw;
 
@@ -948,7 +948,9 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   typedef TileIO<T, CH, K, NW> IOK;
   typedef GlaGate<GT, K, NW> GG;
 
-  f32x4 dP[1][2], dqi[1][NBH], dkd[1][NBH];
+  // K-wide products are formed transposed (the state, q~ or k~ as the A operand): element i is column cc + 16 ni + i of token r,
+  // so that the epilogue reads q, k, gates and writes dq, dk, db four columns at a time
+  f32x4 dP[1][2], dqi[NBH][1], dkd[NBH][1];
   acc_zero(dP); acc_zero(dqi); acc_zero(dkd);
   float hdh[IOH::PASSES];
 #pragma unroll
@@ -990,9 +992,7 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
     IOV::mask(x.rd, ci.len);
     IOV::mask(x.rv, ci.len);
 #pragma unroll
-    for (int p = 0; p < IOH::PASSES; ++p)
-#pragma unroll
-      for (int i = 0; i < IOH::VEC; ++i) hdh[p] += ET<T>::to_f(x.rh.v[p][i]) * ET<T>::to_f(x.rdh.v[p][i]);
+    for (int p = 0; p < IOH::PASSES; ++p) hdh[p] = dot_vec(x.rh.v[p], x.rdh.v[p], hdh[p]);
     IOV::store_lds(x.rd, smT + A_DO, LDV);
     IOV::store_lds(x.rv, smT + A_V, LDV);
     IOH::store_lds(x.rh, smT + A_H, LDV);
@@ -1005,8 +1005,8 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
     }
     lds_barrier();      // LDS-only barriers: the loads requested above stay in flight
     gemm_nt<T, 1, 2, true>(dP, smT + A_DO, LDV, 16 * wv, smT + A_V, LDV, 32 * hf, 0, BVH);
-    gemm_nt<T, 1, NBH, true>(dqi, smT + A_DO, LDV, 16 * wv, smT + A_H, LDV, hf * (K / 2), 0, BVH);
-    gemm_nt<T, 1, NBH, true>(dkd, smT + A_V, LDV, 16 * wv, smT + A_DH, LDV, hf * (K / 2), 0, BVH);
+    gemm_nt<T, NBH, 1, true>(dqi, smT + A_H, LDV, hf * (K / 2), smT + A_DO, LDV, 16 * wv, 0, BVH);
+    gemm_nt<T, NBH, 1, true>(dkd, smT + A_DH, LDV, hf * (K / 2), smT + A_V, LDV, 16 * wv, 0, BVH);
     if constexpr (DV) {
       // dv^T of the slice = scale do^T A + dS'^T (k e^{b_C - b})^T, the products and the rounding of k_gla_bwd_dv
       // (same operands, same order): a lane holds four consecutive V columns of one token, 8-byte stores
@@ -1078,8 +1078,15 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   // those rows of the scaled operand are zero and the diagonal block takes the per-pair loops below.
   // Two rounds over one stacked LDS tile: sub-chunks {0, 3}, then {1, 2} (contraction ranges in multiples of 32
   // tokens: k~ of sub-chunk 0 / 1 / 2 / 3 holds 32 / 32 / 64 / 64 rows, q~ 64 / 64 / 32 / 32).
+  // factors of a sub-chunk's rows that depend on the column only: e^{ref_w} and e^{b_C - ref'_w}
+  __shared__ __attribute__((aligned(16))) float s_er[4 * K], s_ec[4 * K];
+  for (int idx = threadIdx.x; idx < 4 * K; idx += NW) {
+    const int w = idx / K, c = idx % K;
+    s_er[idx] = w == 0 ? 1.f : texp<T>(sB[(16 * w - 1) * LDB + c]);
+    s_ec[idx] = texp<T>(sB[63 * LDB + c] - sB[(16 * w + 15) * LDB + c]);
+  }
   int unsafe = 0;
-  f32x4 dqo[1][NBH], dko[1][NBH];
+  f32x4 dqo[NBH][1], dko[NBH][1];
   acc_zero(dqo); acc_zero(dko);
   if constexpr (SUB) {
     __shared__ int s_unsafe;
@@ -1149,29 +1156,37 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
       if (wv == wa || wv == wb) {
         const int sg = wv == wa ? 0 : 1;
         const int nk = wv < 2 ? 32 : 64;                                // tokens j < nk
-        gemm<T, 1, NBH, false, true>(dqo, tDA, LDC, 16 * wv, tKT + SEGROW[sg] * LDK, LDK, hf * (K / 2), 0, nk);
+        gemm<T, NBH, 1, true, false>(dqo, tKT + SEGROW[sg] * LDK, LDK, hf * (K / 2), tDA, LDC, 16 * wv, 0, nk);
         const int i0 = wv < 2 ? 0 : 32;                                 // tokens i >= i0
-        gemm<T, 1, NBH, true, true>(dko, tDA, LDC, 16 * wv, tKT + (SEGROW[2 + sg] - i0) * LDK, LDK, hf * (K / 2), i0, CH);
+        gemm<T, NBH, 1, true, true>(dko, tKT + (SEGROW[2 + sg] - i0) * LDK, LDK, hf * (K / 2), tDA, LDC, 16 * wv, i0, CH);
       }
       __syncthreads();
     }
+  } else {
+    __syncthreads();
   }
   const int jlo = SUB ? 16 * wv : 0, ihi = SUB ? 16 * wv + 16 : CH;   // range of the pairwise loops
   T* dqd = row_ptr<T>(a.dq, ci.b, ci.tok, h);
   T* dkd_g = row_ptr<T>(a.dk, ci.b, ci.tok, h);
-  const int ch = hf * (K / 2) + (l & 15);   // first column of this lane
+  typedef typename ET<T>::vec4 vec4;
+  const int r = 16 * wv + (l & 15);                    // token of this lane
+  const int ch = hf * (K / 2) + 4 * (l >> 4);          // first column of this lane
   constexpr int NG = NBH < 4 ? NBH : 4;
-  float kkp[NBH];                      // per column: sum over this lane's rows of (dk_d . k_d)
   float dbv[NBH][4];
   static_assert(NBH % NG == 0, "column tiles are taken NG at a time");
+  auto put4 = [&](T* p, const float (&x)[4]) {
+    vec4 y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = ET<T>::from_f(x[i]);
+    *(vec4*)p = y;
+  };
 #pragma unroll
   for (int nh = 0; nh < NBH; nh += NG) {
     // Diagonal block of this wave's sub-chunk, for NG column tiles at a time.  One pass over the 16 tokens
     // j of the sub-chunk serves both sums: dA is lower triangular (zero above the diagonal), so
     //   sq[r] += dA(r, j) k_j e,   sk[r] += dA(j, r) q_j e,   e = e^{-|b_r - b_j|}
     // (b decreases along the chunk: the exponent wanted is b_r - b_j for j <= r and b_j - b_r for j >= r;
-    // where it is not, the dA factor is zero).  k_j, q_j, b_j are read once per token and column and serve
-    // the lane's four rows; the dA values are read once per token and serve the NG column tiles.
+    // where it is not, the dA factor is zero).  The dA values are read once per token and serve all columns of the lane.
     float sqv[NG][4], skv[NG][4], brv[NG][4];
 #pragma unroll
     for (int n4 = 0; n4 < NG; ++n4)
@@ -1181,79 +1196,71 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
 #pragma unroll
       for (int n4 = 0; n4 < NG; ++n4)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sqv[n4][i] = skv[n4][i] = 0.f;
-          brv[n4][i] = sB[(16 * wv + 4 * (l >> 4) + i) * LDB + 16 * (nh + n4) + ch] * TEXP_PRESCALE<T>;
-        }
+        for (int i = 0; i < 4; ++i) brv[n4][i] = sB[r * LDB + 16 * (nh + n4) + ch + i] * TEXP_PRESCALE<T>;
       for (int jj = 0; jj < 16; ++jj) {
         const int j = 16 * wv + jj;
-        float pq[4], pk[4];
+        const float pq = Pm(r, j), pk = Pm(j, r);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 16 * wv + 4 * (l >> 4) + i;
-          pq[i] = Pm(r, j);
-          pk[i] = Pm(j, r);
-        }
-#pragma unroll
-        for (int n4 = 0; n4 < NG; ++n4) {
-          const int cc = 16 * (nh + n4) + ch;
-          const float kj = Km(j, cc), qj = Qm(j, cc), bj = sB[j * LDB + cc] * TEXP_PRESCALE<T>;
+        for (int n4 = 0; n4 < NG; ++n4)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float e = texp_scaled<T>(-fabsf(brv[n4][i] - bj));
-            sqv[n4][i] += pq[i] * kj * e;
-            skv[n4][i] += pk[i] * qj * e;
+            const int cc = 16 * (nh + n4) + ch + i;
+            const float e = texp_scaled<T>(-fabsf(brv[n4][i] - sB[j * LDB + cc] * TEXP_PRESCALE<T>));
+            sqv[n4][i] += pq * Km(j, cc) * e;
+            skv[n4][i] += pk * Qm(j, cc) * e;
           }
-        }
       }
     }
 #pragma unroll
     for (int n4 = 0; n4 < NG; ++n4) {
       const int ni = nh + n4;
       const int cc = 16 * ni + ch;
-      const float bC = sB[63 * LDB + cc];
       // Two exponentials per element, e^{b_r - ref_w} and e^{ref'_w - b_r} (both exponents <= 0); the other two
       // factors of a row follow from them through one factor per column: e^{b_r} = e^{ref_w} e^{b_r - ref_w},
       // e^{b_C - b_r} = e^{b_C - ref'_w} e^{ref'_w - b_r}
-      const float refq = wv == 0 ? 0.f : sB[(16 * wv - 1) * LDB + cc], refk = sB[(16 * wv + 15) * LDB + cc];
-      const float eref = texp<T>(refq), eC = texp<T>(bC - refk);
-      kkp[ni] = 0.f;
+      f32x4 refq = {0.f, 0.f, 0.f, 0.f};
+      if (wv > 0) refq = *(const f32x4*)&sB[(16 * wv - 1) * LDB + cc];
+      const f32x4 refk = *(const f32x4*)&sB[(16 * wv + 15) * LDB + cc], br4 = *(const f32x4*)&sB[r * LDB + cc];
+      const f32x4 er4 = *(const f32x4*)&s_er[wv * K + cc], ec4 = *(const f32x4*)&s_ec[wv * K + cc];
+      float qo[4], ko[4], kkp[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wv + 4 * (l >> 4) + i;
-        const float br = sB[r * LDB + cc];
-        const float e1 = texp<T>(br - refq), e2 = texp<T>(refk - br);
+        const float br = br4[i];
+        const float e1 = texp<T>(br - refq[i]), e2 = texp<T>(refk[i] - br);
         float sq_ = 0.f, sk_ = 0.f;
         if constexpr (SUB) {
           sq_ = sqv[n4][i];
           sk_ = skv[n4][i];
-          sq_ += dqo[0][ni][i] * e1;
-          sk_ += dko[0][ni][i] * e2;
+          sq_ += dqo[ni][0][i] * e1;
+          sk_ += dko[ni][0][i] * e2;
         } else {
-          for (int j = jlo; j <= r; ++j) sq_ += Pm(r, j) * Km(j, cc) * texp<T>(br - sB[j * LDB + cc]);
-          for (int ii = r; ii < ihi; ++ii) sk_ += Pm(ii, r) * Qm(ii, cc) * texp<T>(sB[ii * LDB + cc] - br);
+          for (int j = jlo; j <= r; ++j) sq_ += Pm(r, j) * Km(j, cc + i) * texp<T>(br - sB[j * LDB + cc + i]);
+          for (int ii = r; ii < ihi; ++ii) sk_ += Pm(ii, r) * Qm(ii, cc + i) * texp<T>(sB[ii * LDB + cc + i] - br);
         }
-        const float qv = Qm(r, cc), kv = Km(r, cc);
-        const float ed = eC * e2;
-        const float dqv = a.scale * (eref * e1) * dqi[0][ni][i] + sq_;
-        const float dkdv = dkd[0][ni][i] * ed;
+        const float qv = Qm(r, cc + i), kv = Km(r, cc + i);
+        const float ed = ec4[i] * e2;
+        const float dqv = a.scale * (er4[i] * e1) * dqi[ni][0][i] + sq_;
+        const float dkdv = dkd[ni][0][i] * ed;
         const float dkv = dkdv + sk_;
-        kkp[ni] += kv * dkdv;
+        kkp[i] = kv * dkdv;
         dbv[ni][i] = qv * dqv - kv * dkv;
-        if constexpr (SUB) {
-          // on their way out through the q, k tiles: this element of them is read by this lane only from here on
-          // (the per-pair loops above read other rows' elements of the columns of this group before this point)
-          tQ[r * LDK + cc] = ET<T>::from_f(dqv);
-          tK[r * LDK + cc] = ET<T>::from_f(dkv);
-        } else if (r < ci.len) {
-          dqd[(int64_t)r * a.dq.st + cc] = ET<T>::from_f(dqv);
-          dkd_g[(int64_t)r * a.dk.st + cc] = ET<T>::from_f(dkv);
-        }
+        qo[i] = dqv;
+        ko[i] = dkv;
       }
-      // sum over the 4 row groups of the wave
-      kkp[ni] += __shfl_xor(kkp[ni], 16, 64);
-      kkp[ni] += __shfl_xor(kkp[ni], 32, 64);
-      if (l < 16) s_kk[wv * K + cc] = kkp[ni];
+      if constexpr (SUB) {
+        // on their way out through the q, k tiles: these elements of them are read by this lane only from here on
+        // (the per-pair loops above read other rows' elements of the columns of this group before this point)
+        put4(tQ + r * LDK + cc, qo);
+        put4(tK + r * LDK + cc, ko);
+      } else if (r < ci.len) {
+        put4(dqd + (int64_t)r * a.dq.st + cc, qo);
+        put4(dkd_g + (int64_t)r * a.dk.st + cc, ko);
+      }
+      // per column: sum over the 16 tokens of the wave
+      f32x4 s4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s4[i] = group_sum<16>(kkp[i]);
+      if ((l & 15) == 0) *(f32x4*)&s_kk[wv * K + cc] = s4;
     }
   }
   __syncthreads();   // all reads of the q tile are done: reuse it for db
@@ -1263,12 +1270,7 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   }
   float* sDB = SUB ? (float*)tKT : smF + B_Q;
 #pragma unroll
-  for (int ni = 0; ni < NBH; ++ni)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = 16 * wv + 4 * (l >> 4) + i, cc = 16 * ni + ch;
-      sDB[r * LDB + cc] = dbv[ni][i];
-    }
+  for (int ni = 0; ni < NBH; ++ni) *(f32x4*)&sDB[r * LDB + 16 * ni + ch] = f32x4{dbv[ni][0], dbv[ni][1], dbv[ni][2], dbv[ni][3]};
   __syncthreads();
   // dg = reverse cumsum of db over the tokens (+ the last-row term): a thread takes one channel over a segment
   // of tokens, the segment totals go through LDS (rows past the end of a partial chunk have zero db)
