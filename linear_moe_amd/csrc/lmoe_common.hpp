@@ -457,6 +457,41 @@ template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
       r.v[p] = *(const vec*)(src + (int64_t)row * row_stride + col);
     }
   }
+  // load_nomask for a loop over tiles of one tensor: where a thread's rows lie relative to the tile's first is the same for
+  // every full tile and worked out again only where the row count changes (a uniform branch with no load in it).  Each row's
+  // product with its 64-bit stride and the clamp cost 50 cycles of the issuing wave per load (K = V = 128: k_state_bwd 76 -> 68 us at
+  // 64 pairs of 64 chunks, k_gdn_state_bwd 51 -> 49 at 32 pairs of 32, k_gdn_wy_fwd 60 -> 58.5; no change in the
+  // register-resident forward pass and the chunk-parallel backward kernels, which keep load_nomask).
+  struct Rows { int64_t at[PASSES]; int n; };
+  static __device__ __forceinline__ void load_rows(Regs& r, Rows& o, const T* __restrict__ src, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
+    if (nvalid != o.n) {
+      const int last = (nvalid < ROWS ? nvalid : ROWS) - 1;
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p) {
+        int row, col; coords(p, row, col, tid);
+        row = row < last ? row : last;
+        o.at[p] = ((int64_t)row * row_stride + col) * (int64_t)sizeof(T);
+      }
+      o.n = nvalid;
+    }
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) r.v[p] = *(const vec*)((const char*)src + o.at[p]);
+  }
+  // The same with one offset kept (first_row: that of the thread's row in the first pass) for loops without the registers for
+  // all: the passes of a full tile lie a scalar apart, a partial one takes load_nomask (k_state_fwd_b: 97 -> 90 us forward-only,
+  // 120 -> 109 saving, 64 pairs of 64 chunks).
+  static __device__ __forceinline__ int64_t first_row(int64_t row_stride, int tid = threadIdx.x & (NT - 1)) {
+    return ((int64_t)(tid / VPR) * row_stride + (tid % VPR) * VEC) * (int64_t)sizeof(T);
+  }
+  static __device__ __forceinline__ void load_from(Regs& r, int64_t first, const T* __restrict__ src, int64_t row_stride, int nvalid) {
+    static_assert(NT % VPR == 0 && PASSES * (NT / VPR) == ROWS, "whole rows per pass");
+    if (nvalid >= ROWS) {
+#pragma unroll
+      for (int p = 0; p < PASSES; ++p) r.v[p] = *(const vec*)((const char*)(src + (int64_t)(p * (NT / VPR)) * row_stride) + first);
+    } else {
+      load_nomask(r, src, row_stride, nvalid);
+    }
+  }
   static __device__ __forceinline__ void mask(Regs& r, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     if (nvalid >= ROWS) return;                 // uniform: full tiles (the common case) skip it
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

@@ -464,12 +464,13 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a, c
     // ------------------------- loaders, ring A (q), dZ and all stores ---------------------
     struct PreA { typename IOK::Regs rq; int len; };
     PreA pa[LPF];
+    typename IOK::Rows oq = {};
     // always issued, chunk index clamped (see k_gdn_state_fwd); `it` counts chunks from the end
     auto issue_a = [&](PreA& P, int it) {
       const int c = max(sq.nchunks - 1 - it, 0);
       const int tok = sq.tok0 + c * CH;
       P.len = min(CH, sq.len - c * CH);
-      IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, P.len);
+      IOK::load_rows(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, P.len);
     };
     auto stage_a = [&](PreA& P) {
       IOK::mask(P.rq, P.len);
@@ -535,15 +536,17 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_bwd(const lmoe_args a, c
     // staged during phase 2 of the step before the one that reads them in phase 1
     struct PreB { typename IOK::Regs rk; typename IOP::Regs rp, rt; typename IOV::Regs rd; float eb, ed, f; int len; };
     PreB pb[LPF];
+    typename IOK::Rows ok = {};
+    typename IOV::Rows od = {};
     const float scale = a.scale;
     auto issue_b = [&](PreB& P, int it) {
       const int c = max(sq.nchunks - 1 - it, 0);
       const int tok = sq.tok0 + c * CH;
       P.len = min(CH, sq.len - c * CH);
-      IOK::load_nomask(P.rk, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, P.len);
+      IOK::load_rows(P.rk, ok, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, P.len);
       IOP::load_nomask(P.rp, (const T*)a.pmat + ((int64_t)(sq.chunk0 + c) * a.H + h) * CH * CH, CH, CH);
       IOP::load_nomask(P.rt, (const T*)a.tinv + ((int64_t)(sq.chunk0 + c) * a.H + h) * CH * CH, CH, CH);
-      IOV::load_nomask(P.rd, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, P.len);
+      IOV::load_rows(P.rd, od, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, P.len);
       const float* gc = a.gcum + ((int64_t)(sq.chunk0 + c) * a.H + h) * GATE_ROWS * CH;
       P.eb = gc[l];
       P.ed = gc[CH + l];

@@ -170,12 +170,14 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const
     const void* gptr = gated ? a.g.ptr : a.k.ptr;
     const float scale = a.scale;
     // always issued, chunk index clamped (see k_state_fwd)
+    typename IOK::Rows oq = {};
+    typename IOV::Rows od = {};
     auto issue = [&](Pre& P, int c) {
       c = max(c, 0);
       const int tok = sq.tok0 + c * CH;
       const int len = min(CH, sq.len - c * CH);
-      IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
-      IOV::load_nomask(P.rd, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, len);
+      IOK::load_rows(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
+      IOV::load_rows(P.rd, od, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, len);
       P.len = len;
       P.graw = load_scalar_raw(gptr, a.g_dtype, gated ? row_off(a.g, sq.b, tok + min(l, len - 1), h) : 0);
       if constexpr (NORM == 1) {

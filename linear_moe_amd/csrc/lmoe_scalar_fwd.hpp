@@ -403,6 +403,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
     // --------------------------------- loaders -------------------------------------------
     struct Pre { typename IOK::Regs rk, rq; typename IOV::Regs ru; uint32_t graw; int len; };
     Pre pre[3];                                              // register set = chunk % 3
+    // (slices of 64 columns at K = 128: no registers left for the offsets)
+    constexpr bool KEPT = !(K == 128 && BV == 64);
+    const int64_t ok = KEPT ? IOK::first_row(a.k.st) : 0, oq = KEPT ? IOK::first_row(a.q.st) : 0, ou = KEPT ? IOV::first_row(a.v.st) : 0;
     const bool gated = a.gate != LMOE_GATE_NONE && a.g.ptr != nullptr;
     const void* gptr = gated ? a.g.ptr : a.k.ptr;
     // Always issued (chunk index clamped to the last chunk; the surplus loads at the end of a
@@ -412,9 +415,15 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
       c = min(c, sq.nchunks - 1);
       const int tok = sq.tok0 + c * CH;
       const int len = min(CH, sq.len - c * CH);
-      IOK::load_nomask(P.rk, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, len);
-      IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
-      IOV::load_nomask(P.ru, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
+      if constexpr (KEPT) {
+        IOK::load_from(P.rk, ok, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, len);
+        IOK::load_from(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
+        IOV::load_from(P.ru, ou, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
+      } else {
+        IOK::load_nomask(P.rk, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, len);
+        IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
+        IOV::load_nomask(P.ru, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
+      }
       P.len = len;
       P.graw = load_scalar_raw(gptr, a.g_dtype, gated ? row_off(a.g, sq.b, tok + min(l, len - 1), h) : 0);
     };
