@@ -38,18 +38,18 @@ STAGE_NAMES = {0: "k_gdn_wy_fwd", 1: "k_gdn_state_fwd_reg", 4: "k_gdn_state_bwd"
 # sources (kernel_sources_sha16()) at that time, and a build whose sources differ reports traffic = null
 # rather than a stale number.
 CALIB_COPY_BYTES = 256 << 20
-MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237263293, "k_gdn_state_fwd_reg": 1117158774, "k_gdn_state_bwd": 946040007,
-                    "k_gdn_bwd_chunk": 1818253639}
-TRAFFIC_SOURCES_SHA16 = "63c5721e0d66b1b6"
+MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237250398, "k_gdn_state_fwd_reg": 1084679821, "k_gdn_state_bwd": 946048818,
+                    "k_gdn_bwd_chunk": 1830472407}
+TRAFFIC_SOURCES_SHA16 = "7fa3342ec8380191"
 TRAFFIC_SOURCES = ("lmoe_common.hpp", "lmoe_seq.hpp", "lmoe_gdn_wy.hpp", "lmoe_gdn_state.hpp", "lmoe_gdn_state_reg.hpp", "lmoe_gdn_bwd_chunk.hpp",
                    "lmoe_split.hpp", "lmoe_gdn_split.hpp", "lmoe_gdn_fwd.hip", "lmoe_gdn_state.hip", "lmoe_gdn_bwd.hip")
 
 
 # HBM bytes per call of the other contract configurations (bench.py --other-configs), same counters and scaling,
 # summed over the kernels of the call; key = configuration number
-OTHER_TRAFFIC = {"1": 5115520, "2": 272947584, "3": 1280976107, "5": 16620092864, "6": 1445203328, "7": 6568638293,
-                 "8": 1510926219}
-OTHER_TRAFFIC_SHA16 = "4e598dd83620abfa"
+OTHER_TRAFFIC = {"1": 5098880, "2": 272971904, "3": 1280805355, "5": 16600773771, "6": 1445252128, "7": 6528872299,
+                 "8": 1510810965}
+OTHER_TRAFFIC_SHA16 = "47a9f38774c1bb3f"
 
 
 def all_sources_sha16():
@@ -327,7 +327,7 @@ def trace_state_fwd(lib, x, dims, work_group=16):
             out[nm][label] = round(d)
     return {"metric": "k_gdn_state_fwd_reg: shader-clock cycles inside the window of a chunk, per team (traced build)",
             "unit": "cycles", "work_group": work_group, "chunks_averaged": [c0, c1], "period_cycles": round(period),
-            "traced_kernel_us": round(traced_us, 1), "cycles_per_us": round(period * nch / traced_us, 1),
+            "traced_kernel_us": round(traced_us, 1), "cycles_per_us": round(period * ((T + CH - 1) // CH) / traced_us, 1),
             "teams": out}
 
 
