@@ -345,6 +345,30 @@ def unstash(ctx, call):
     return t[ctx.n_stashed:]
 
 
+def came_back(x: Optional[torch.Tensor], shape, dtype, device, name: str) -> torch.Tensor:
+    """A tensor that was saved for the backward, as the kernels may read it: a saved-tensor hook hands back what it likes
+    (another type, other strides, a view), and the kernels index the full extent of ``shape``.  ``dtype=None``: a gate
+    (float32 or bfloat16, any strides); else contiguous, on a 16-byte boundary."""
+    if x is None or tuple(x.shape) != tuple(shape) or x.device != device:
+        raise RuntimeError(f"{name}, saved for the backward with shape {tuple(shape)} on {device}, came back as "
+                           f"{None if x is None else (tuple(x.shape), str(x.device))}")
+    if dtype is None:
+        return x if x.dtype in _DT else x.float()
+    x = x.to(dtype).contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
+def inputs_came_back(q, k, v, do, head_first: bool, wide_v: bool = False):
+    """q, k, v as they come back from autograd (see ``came_back``) and the gradient of the output, which autograd gives
+    the shape and type of the output: checked against each other, in rows the kernels take.  Returns them and the
+    dimensions of the call."""
+    dims = _check_inputs(q, k, v, head_first, None, wide_v)
+    if do.shape != v.shape or do.dtype != v.dtype or do.device != v.device:
+        raise RuntimeError(f"the gradient of the output ({tuple(do.shape)}, {do.dtype}, {do.device}) does not fit v as it was "
+                           f"saved for the backward ({tuple(v.shape)}, {v.dtype}, {v.device})")
+    return (*(_aligned(x) for x in (q, k, v, do)), dims)
+
+
 def stream_ptr() -> int:
     """The current stream of the current device, as the library takes it.  (The raw handle: building the stream object
     of ``torch.cuda.current_stream()`` for it takes longer than all the other arguments of a small call.)"""

@@ -71,11 +71,13 @@ struct Call {
   int64_t B, T, H, K, V, N, NT;
   lmoe_args a = {};
   Tensor q, k, v, g, beta, h0;
-  Tensor chunked(std::initializer_list<int64_t> tail, at::ScalarType t) const {      // [NT, H, ...]
+  typedef std::initializer_list<int64_t> Tail;
+  c10::SmallVector<int64_t, 6> chunked_shape(Tail tail) const {                       // [NT, H, ...]
     c10::SmallVector<int64_t, 6> s = {std::max<int64_t>(NT, 1), H};
     s.append(tail.begin(), tail.end());
-    return at::empty(s, q.options().dtype(t).requires_grad(false));
+    return s;
   }
+  Tensor chunked(Tail tail, at::ScalarType t) const { return at::empty(chunked_shape(tail), q.options().dtype(t).requires_grad(false)); }
   Tensor states() const { return at::empty({N, H, K, V}, q.options().dtype(at::kFloat)); }
   c10::SmallVector<int64_t, 3> token_shape() const {
     return head_first ? c10::SmallVector<int64_t, 3>{B, H, T} : c10::SmallVector<int64_t, 3>{B, T, H};
@@ -261,10 +263,13 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
     PyObject* sv = o[12];
     need(PyTuple_Check(sv));
     auto saved = [&](Py_ssize_t i) { need(i < PyTuple_GET_SIZE(sv)); return plain_or_none(PyTuple_GET_ITEM(sv, i), c.dev); };
-    // (what was saved may have been through a hook: on its way back it must be what the kernels wrote)
-    auto kept = [&](Py_ssize_t i, at::ScalarType t) {
+    // What was saved may have been through a hook, which hands back what it likes; the kernels index the full extent: of the
+    // type and size that forward allocated, contiguous and on a 16-byte boundary.  (Anything else: the Python steps convert or
+    // refuse it, _host.came_back.)
+    auto kept = [&](Py_ssize_t i, at::ScalarType t, Call::Tail tail) {
       const Tensor x = saved(i);
-      need(x.defined() && x.is_contiguous() && x.scalar_type() == t && x.size(0) == std::max<int64_t>(c.NT, 1));
+      need(x.defined() && x.is_contiguous() && x.scalar_type() == t && x.sizes() == at::IntArrayRef(c.chunked_shape(tail)));
+      need((reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0);
       return x.data_ptr();
     };
     const auto dt = c.q.scalar_type();
@@ -274,8 +279,8 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
     Tensor dq, dk, dv, dg, dbeta, ws, norm_ws, den, ones;
     const Tensor dh0 = c.h0.defined() ? fresh(c.h0) : Tensor();
     c.a.dh0 = (float*)ptr(dh0);
-    c.a.hs = kept(0, dt);
-    const Tensor dhs = fresh(saved(0));
+    c.a.hs = kept(0, dt, {c.K, c.V});
+    const Tensor dhs = c.chunked({c.K, c.V}, dt);
     c.a.dhs = ptr(dhs);
     auto gradients = [&] {
       if (!dq.defined()) dq = fresh(c.q);
@@ -289,7 +294,7 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
       if (has_extra) {
         norm_ws = c.chunked({c.V / 32, 64 + c.K}, at::kFloat);
         c.a.normalize = (int)PyLong_AsLong(extra(0)); c.a.norm_eps = (float)PyFloat_AsDouble(extra(1));
-        c.a.zs = (float*)kept(2, at::kFloat); c.a.norm_ws = (float*)norm_ws.data_ptr();
+        c.a.zs = (float*)kept(2, at::kFloat, {c.K}); c.a.norm_ws = (float*)norm_ws.data_ptr();
         if (c.a.normalize == 2) {
           den = plain(extra(3), c.dev);
           need(f32(den) && den.is_contiguous() && den.sizes() == at::IntArrayRef(c.token_shape()));
@@ -305,13 +310,13 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
       ws = c.cut(op);
     } else if (op == OP_GLA) {
       gradients();
-      c.a.amat = kept(1, dt); c.a.qe = kept(2, dt); c.a.ke = kept(3, dt); c.a.gcum = (float*)kept(4, at::kFloat);
+      c.a.amat = kept(1, dt, {64, 64}); c.a.qe = kept(2, dt, {64, c.K}); c.a.ke = kept(3, dt, {64, c.K}); c.a.gcum = (float*)kept(4, at::kFloat, {c.K});
       dg = at::empty(c.g.sizes(), c.g.options());             // (in the type of g, by the kernel)
       c.a.dg = desc(dg, hf);
       ws = c.cut(op);
     } else {
-      c.a.tinv = kept(1, dt); c.a.pmat = kept(2, dt); c.a.gcum = (float*)kept(3, at::kFloat); c.a.vnew.ptr = kept(4, dt);
-      const Tensor dvnew = fresh(saved(4)), seg_p = saved(5);
+      c.a.tinv = kept(1, dt, {64, 64}); c.a.pmat = kept(2, dt, {64, 64}); c.a.gcum = (float*)kept(3, at::kFloat, {5, 64}); c.a.vnew.ptr = kept(4, dt, {c.V / 32, 64, 32});
+      const Tensor dvnew = c.chunked({c.V / 32, 64, 32}, dt), seg_p = saved(5);
       c.a.dvnew.ptr = dvnew.data_ptr();
       if (has_extra) {
         c.a.v_act = yes(extra(0));
@@ -322,6 +327,7 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
           if (given[i].defined()) need(given[i].sizes() == like[i]->sizes() && given[i].scalar_type() == dt && rows_aligned(given[i]));
         }
         dq = given[0]; dk = given[1]; dv = given[2];
+        need(given[3].defined() == given[4].defined());
         if (given[3].defined()) { c.a.q_raw = desc(given[3], hf); c.a.k_raw = desc(given[4], hf); c.a.qk_eps = (float)PyFloat_AsDouble(extra(6)); }
       }
       gradients();
@@ -330,7 +336,7 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
       c.a.dbeta_bf16 = bf16(dbeta);
       c.a.dg = desc(dg, hf); c.a.dbeta = desc(dbeta, hf);
       if (seg_p.defined()) {
-        need(f32(seg_p) && seg_p.is_contiguous());
+        need(f32(seg_p) && seg_p.is_contiguous() && (reinterpret_cast<uintptr_t>(seg_p.data_ptr()) & 15) == 0);
         ws = c.cut(op);
         need(!ws.defined() || seg_p.numel() == lib.split_floats(&c.a, op, 0));
         if (ws.defined()) c.a.seg_p = (float*)seg_p.data_ptr();

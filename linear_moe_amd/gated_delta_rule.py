@@ -17,7 +17,7 @@ import torch
 from . import _lib
 from .l2norm import l2_norm
 from ._host import (HEAD_DIMS, WIDE_V, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    native, no_tokens, ptr, stash, stream_ptr, unstash)
+                    came_back, inputs_came_back, native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 def _scalar_dt(x: torch.Tensor) -> int:
@@ -118,8 +118,11 @@ class GDNCall:
         n = lib.lmoe_split_floats(C.byref(a), self.OP, 1)
         if n <= 0:
             return None
+        n_p = lib.lmoe_split_floats(C.byref(a), self.OP, 0)
         if save:
-            seg_p = torch.empty(lib.lmoe_split_floats(C.byref(a), self.OP, 0), dtype=torch.float32, device=dev)
+            seg_p = torch.empty(n_p, dtype=torch.float32, device=dev)
+        elif seg_p is not None:
+            seg_p = came_back(seg_p, (n_p,), torch.float32, dev, "seg_p")
         self.seg_ws = torch.empty(n, dtype=torch.float32, device=dev)
         a.seg_p, a.seg_ws = ptr(seg_p), self.seg_ws.data_ptr()
         return seg_p
@@ -141,10 +144,17 @@ class GDNCall:
             if r is not None:
                 dq, dk, dv, dg, dbeta, dh0 = r
                 return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dbeta, dh0
-        dims = ctx.dims or _check_inputs(q, k, v, head_first, None, wide_v=True)
+        q, k, v, do, dims = inputs_came_back(q, k, v, do, head_first, wide_v=True)
         B, T, H, K, V = dims
         plan = ctx.plan or seq_plan(B, T, None, q.device)
-        do = _aligned(do)
+        dev, dt, tok, nt = q.device, q.dtype, ((B, H, T) if head_first else (B, T, H)), max(plan.NT, 1)
+        g = None if g is None else came_back(g, tok, None, dev, "g")
+        beta = came_back(beta, tok, None, dev, "beta")
+        if ctx.has_h0:
+            h0 = came_back(h0, (plan.N, H, K, V), torch.float32, dev, "initial_state")
+        hs, tinv = came_back(hs, (nt, H, K, V), dt, dev, "hs"), came_back(tinv, (nt, H, 64, 64), dt, dev, "tinv")
+        pmat, gcum = came_back(pmat, (nt, H, 64, 64), dt, dev, "pmat"), came_back(gcum, (nt, H, 5, 64), torch.float32, dev, "gcum")
+        vnew = came_back(vnew, (nt, H, V // 32, 64, 32), dt, dev, "vnew")
         a = base_args(q, k, v, head_first, ctx.scale, plan, dims)
         a.gate = _lib.GATE_NONE if g is None else _lib.GATE_SCALAR
         if g is not None:
@@ -156,7 +166,6 @@ class GDNCall:
         a.d_o = _desc(do, head_first)
         dht = None if dht is None else dht.float().contiguous()
         a.dht = ptr(dht)
-        dev, dt = q.device, q.dtype
         dq = torch.empty_like(q) if dq_out is None else dq_out
         dk = torch.empty_like(k) if dk_out is None else dk_out
         dv = torch.empty_like(v) if dv_out is None else dv_out

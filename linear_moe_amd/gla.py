@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    cut_workspace, native, no_tokens, ptr, stash, stream_ptr, unstash)
+                    came_back, cut_workspace, inputs_came_back, native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class GLACall:
@@ -94,9 +94,17 @@ class GLACall:
             if r is not None:
                 dq, dk, dv, dg, _, dh0 = r
                 return dq, dk, dv, dg, dh0
-        dims = self.dims or _check_inputs(q, k, v, head_first, None)
-        plan = self.plan or seq_plan(dims[0], dims[1], None, q.device)
-        do = _aligned(do)
+        q, k, v, do, dims = inputs_came_back(q, k, v, do, head_first)
+        B, T, H, K, V = dims
+        plan = self.plan or seq_plan(B, T, None, q.device)
+        dev, dt, nt = q.device, q.dtype, max(plan.NT, 1)
+        g = came_back(g, q.shape, None, dev, "g")
+        g = _aligned(g if dt == torch.bfloat16 else g.float())
+        if self.has_h0:
+            h0 = came_back(h0, (plan.N, H, K, V), torch.float32, dev, "initial_state")
+        hs, amat = came_back(hs, (nt, H, K, V), dt, dev, "hs"), came_back(amat, (nt, H, 64, 64), dt, dev, "amat")
+        qe, ke = came_back(qe, (nt, H, 64, K), dt, dev, "qe"), came_back(ke, (nt, H, 64, K), dt, dev, "ke")
+        gdec = came_back(gdec, (nt, H, K), torch.float32, dev, "gdec")
         a = base_args(q, k, v, head_first, self.scale, plan, dims)
         self._gate(a, g, head_first)
         a.h0, a.hs, a.amat = ptr(h0), hs.data_ptr(), amat.data_ptr()

@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    cut_workspace, native, no_tokens, ptr, stash, stream_ptr, unstash)
+                    came_back, cut_workspace, inputs_came_back, native, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class SimpleGLACall:
@@ -112,10 +112,20 @@ class SimpleGLACall:
             if r is not None:
                 dq, dk, dv, dg, _, dh0 = r
                 return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dh0
-        dims = ctx.dims or _check_inputs(q, k, v, head_first, None)
+        q, k, v, do, dims = inputs_came_back(q, k, v, do, head_first)
         B, T, H, K, V = dims
         plan = ctx.plan or seq_plan(B, T, None, q.device)
-        do = _aligned(do)
+        tok, nt = ((B, H, T) if head_first else (B, T, H)), max(plan.NT, 1)
+        dev = q.device
+        hs = came_back(hs, (nt, H, K, V), q.dtype, dev, "hs")
+        if g is not None:
+            g = came_back(g, tok, None, dev, "g")
+        if ctx.has_h0:
+            h0 = came_back(h0, (plan.N, H, K, V), torch.float32, dev, "initial_state")
+        if ctx.norm_eps is not None:
+            zs = came_back(zs, (nt, H, K), torch.float32, dev, "zs")
+            if not ctx.emit_den:
+                den, o = came_back(den, tok, torch.float32, dev, "den"), _aligned(came_back(o, v.shape, None, dev, "o").to(v.dtype))
         a = base_args(q, k, v, head_first, ctx.scale, plan, dims)
         a.gate = _lib.GATE_NONE if g is None else _lib.GATE_SCALAR
         if g is not None:
@@ -142,11 +152,9 @@ class SimpleGLACall:
             norm_ws = torch.empty(max(plan.NT, 1), H, V // 32, 64 + K, dtype=torch.float32, device=q.device)
             a.norm_eps, a.zs, a.norm_ws = norm_eps, zs.data_ptr(), norm_ws.data_ptr()
             if ctx.emit_den:
-                shape = (B, H, T) if head_first else (B, T, H)
-                dden = torch.zeros(shape, dtype=torch.float32, device=q.device) if dden is None else dden.float().contiguous()
+                dden = torch.zeros(tok, dtype=torch.float32, device=q.device) if dden is None else dden.float().contiguous()
                 a.normalize, a.dden = 2, _desc(dden, head_first)
             else:
-                o = _aligned(o)
                 a.normalize, a.den, a.o = 1, _desc(den, head_first), _desc(o, head_first)
         seg_ws = cut_workspace(lib, a, self.OP, q.device)
         _lib.check(lib.lmoe_chunk_simple_gla_bwd(C.byref(a), stream_ptr()), "chunk_simple_gla backward")

@@ -151,3 +151,66 @@ def test_other_calls_take_the_python_steps(cuda):
             L.chunk_simple_gla(*bad)
     with pytest.raises(ValueError):
         L.chunk_simple_gla(q, k, v, g, initial_state=h0[:1])
+
+
+# What is saved for the backward, in the order it is handed to autograd (see the ops' ``call.saved``): the buffers of the
+# forward pass behind q, k, v, gate(s); with norm_eps the output is the last one
+SAVED = {"simple": ("q", "k", "v", "g", "hs"), "normalized": ("q", "k", "v", "hs", "den", "zs", "o"),
+         "gla": ("q", "k", "v", "g", "hs", "amat", "qe", "ke", "gdec"),
+         "gdn": ("q", "k", "v", "g", "beta", "h0", "hs", "tinv", "pmat", "gcum", "vnew"),
+         "gdn_cut": ("q", "k", "v", "g", "beta", "h0", "hs", "tinv", "pmat", "gcum", "vnew", "seg_p")}
+
+
+def _through_hooks(kind, cuda, change):
+    """gradients of one call whose saved tensors come back as change(name, x)"""
+    import linear_moe_amd as L
+    op = 2 if kind.startswith("gdn") else 1 if kind == "gla" else 0
+    B, T = (1, 4000) if kind == "gdn_cut" else (2, 200)
+    x = _inputs(op, B, T, 2, 64, 64, torch.bfloat16, False, False, torch.float32, cuda)
+    if kind == "normalized":
+        x["q"], x["k"], x["g"] = x["q"].abs(), x["k"].abs(), None
+    leaves = [t.requires_grad_() for t in x.values() if t is not None]
+    names = SAVED[kind]
+    count = [0]
+
+    def pack(t):
+        count[0] += 1
+        return count[0] - 1, t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda p: change(names[p[0]], p[1])):
+        if kind == "simple":
+            o, _ = L.chunk_simple_gla(x["q"], x["k"], x["v"], x["g"], head_first=False)
+        elif kind == "normalized":
+            o, _ = L.chunk_linear_attn(x["q"], x["k"], x["v"], head_first=False)
+        elif kind == "gla":
+            o, _ = L.chunk_gla(x["q"], x["k"], x["v"], x["g"], head_first=False)
+        else:
+            h0 = torch.ones(B, 2, 64, 64, device=cuda, requires_grad=True)
+            leaves.append(h0)
+            o, _ = L.chunk_gated_delta_rule(x["q"], x["k"], x["v"], x["g"], x["beta"], initial_state=h0)
+    assert count[0] == len(names), (count[0], names)
+    do = torch.randn(o.shape, device=cuda, generator=torch.Generator(device=cuda).manual_seed(3)).to(o.dtype)
+    return torch.autograd.grad(o, leaves, do)
+
+
+def _misaligned(x):
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype, device=x.device)
+    flat[1:] = x.reshape(-1)
+    return flat[1:].view(x.shape)
+
+
+@pytest.mark.parametrize("kind", list(SAVED))
+def test_saved_tensors_that_come_back_changed(cuda, kind):
+    """the kernels index the full extent of what was saved: another type, other strides or another place in memory of a buffer
+    give the same gradients, a shorter buffer (or input) is refused before anything is launched"""
+    ref = _through_hooks(kind, cuda, lambda n, x: x)
+    buffers = [n for n in SAVED[kind] if n not in ("q", "k", "v", "g", "beta", "o")]
+    changes = [lambda x: x.double() if x.dtype == torch.float32 else x.float(),
+               lambda x: x.mT.contiguous().mT if x.dim() > 1 else x.double(), _misaligned]
+    for name, f in itertools.product(buffers, changes):
+        got = _through_hooks(kind, cuda, lambda n, x: f(x) if n == name else x)
+        assert all(torch.equal(a, b) for a, b in zip(ref, got)), name
+    for name in SAVED[kind]:
+        for cut in (lambda x: x[:, :1] if x.dim() > 1 else x[:-4], lambda x: x[..., :-4], lambda x: x.cpu()):
+            with pytest.raises((RuntimeError, ValueError)):
+                _through_hooks(kind, cuda, lambda n, x: cut(x) if n == name else x)

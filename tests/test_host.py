@@ -569,3 +569,21 @@ def test_ops_on_other_head_dims_are_the_op_on_padded_blocks(op, K, V):
     if op == "gdn":
         with pytest.raises(ValueError, match="one block"):
             by_head_dim_blocks(core, torch.zeros(1, 2, 1, 160), torch.zeros(1, 2, 1, 160), v[:1, :2, :1], None, None, False, False, op)
+
+
+def test_saved_tensors_come_back_as_they_were_saved():
+    """what a saved-tensor hook hands back is brought into the form the kernels index, or refused"""
+    from linear_moe_amd._host import came_back
+    dev = torch.device("cpu")
+    x = torch.randn(3, 2, 64, 128).bfloat16()
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype)
+    flat[1:] = x.reshape(-1)
+    for y in (x, x.float(), x.mT.contiguous().mT, flat[1:].view(x.shape)):
+        z = came_back(y, (3, 2, 64, 128), torch.bfloat16, dev, "hs")
+        assert torch.equal(z, x) and z.is_contiguous() and z.data_ptr() % 16 == 0
+    assert came_back(x, x.shape, torch.bfloat16, dev, "hs") is x
+    g = torch.randn(4, 6)[:, ::2]
+    assert came_back(g, (4, 3), None, dev, "g") is g and came_back(g.half(), (4, 3), None, dev, "g").dtype == torch.float32
+    for y in (None, x[:, :1], x[..., :-4], x.flatten(), x.to("meta")):
+        with pytest.raises(RuntimeError, match="hs, saved for the backward"):
+            came_back(y, (3, 2, 64, 128), torch.bfloat16, dev, "hs")
