@@ -5,9 +5,8 @@ The hot kernels of the gated delta rule and the forward pass and the fused backw
 steering: refreshed lane indices, pinned sums, fenced products).  A compiler or source change that makes one of them
 spill, or lowers the number of waves it runs with, costs a large factor in speed without failing any test.  This
 script reads the per-kernel resource reports that ``-Rpass-analysis=kernel-resource-usage`` wrote at compile time
-(``<unit>.remarks``) and fails the build when an instance for 2-byte elements (the performance path) of a guarded
-kernel uses scratch memory, spills vector registers, or falls below its minimum occupancy.  4-byte instances are the
-parity path and are only reported.
+(``<unit>.remarks``) and fails the build when an instance of a guarded kernel uses scratch memory or spills vector
+registers, or when one for 2-byte elements (the performance path) falls below its minimum occupancy.
 
 usage: check_resources.py unit.remarks [...]
 """
@@ -65,22 +64,20 @@ def main(paths):
                 line = (f"{kern:<18} {'bf16' if two_byte else 'fp32'} vgpr {r.get('vgpr', -1):3d} agpr {r.get('agpr', -1):3d} "
                         f"scratch {r.get('scratch', -1):4d} B  vgpr-spill {r.get('vspill', -1):3d}  waves/SIMD {r.get('occ', -1)}  "
                         f"lds {r.get('lds', -1)}  {name}")
-                if not two_byte:
-                    continue
                 seen[kern] += 1
-                if r.get("scratch", 1) != 0 or r.get("vspill", 1) != 0 or r.get("occ", 0) < min_occ:
+                if r.get("scratch", 1) != 0 or r.get("vspill", 1) != 0 or (two_byte and r.get("occ", 0) < min_occ):
                     bad.append(line)
     missing = [k for k, n in seen.items() if n == 0]
     if missing:
         print("check_resources: no resource report found for", ", ".join(missing), file=sys.stderr)
         return 1
     if bad:
-        print("check_resources: 2-byte instances of guarded kernels spill or lost occupancy "
-              "(needed: scratch 0, vgpr-spill 0, waves/SIMD >= " + str(GUARDED) + "):", file=sys.stderr)
+        print("check_resources: instances of guarded kernels spill or lost occupancy "
+              "(needed: scratch 0, vgpr-spill 0; 2-byte: waves/SIMD >= " + str(GUARDED) + "):", file=sys.stderr)
         for b in bad:
             print("  " + b, file=sys.stderr)
         return 1
-    print(f"check_resources: {sum(seen.values())} bf16 instances of {len(GUARDED)} guarded kernels: no scratch, no spills, "
+    print(f"check_resources: {sum(seen.values())} instances of {len(GUARDED)} guarded kernels: no scratch, no spills, "
           "occupancy as tuned")
     return 0
 

@@ -204,7 +204,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           const vec z = R.v[2 * PV + p], vv = R.v[3 * PV + p];
           vec o;
           float s = 0.f;
-          if (a.v_act) {
+          if (sizeof(T) == 2 && a.v_act) {
             // v as given is the argument of a SiLU: the op runs on silu(v) (rounded to the element type, as the
             // forward pass staged it) and dv is the gradient with respect to the argument
 #pragma unroll
@@ -391,6 +391,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
         IOK::load_lds_clamped(r, smem + B_Q, LDK, cur.len, tid);
         act_backward(r, XQ);
         IOK::template store_global_clamped<true>(r, rows(a.dq, cur), a.dq.st, cur.len, tid);
+        if constexpr (sizeof(T) == 4) tid = fresh_index(tid) & (NTHR - 1);       // (one tile's addresses at a time: both spill)
         IOK::load_lds_clamped(r, smem + B_K, LDK, cur.len, tid);
         act_backward(r, XK);
         IOK::template store_global_clamped<true>(r, rows(a.dk, cur), a.dk.st, cur.len, tid);
@@ -475,12 +476,25 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     // The k^T fragments serve three of the four products and are requested while G and dM are formed; the rows of q and k
     // that the sums need are read once.  (Every product with fragments of its own, each step waited for: 80 transposing
     // reads per wave and item where these are 32, and the LDS round trips of 8 steps behind barrier b.)
-    frag ft[CS][NBK];
+    // 2-byte elements only: a 4-byte fragment is eight registers, and kept they and the rows spill (81 registers at K = 128;
+    // 1024 items, K = V = 128: 197 us, and 156 without).  Those instances read each where it is used, a step at a time.
+    constexpr bool KEPT = sizeof(T) == 2;
+    frag ft[KEPT ? CS : 1][NBK];
     vec4 k4[NBK], q4[NBK];
+    auto keep = [&](const T* tile) {
+      if constexpr (KEPT) {
 #pragma unroll
-    for (int ks = 0; ks < CS; ++ks)
+        for (int ks = 0; ks < CS; ++ks)
 #pragma unroll
-      for (int ni = 0; ni < NBK; ++ni) ft[ks][ni] = ET<T>::load_frag_t(Kt, LDK, 32 * ks, k0 + 16 * ni, l);
+          for (int ni = 0; ni < NBK; ++ni) ft[ks][ni] = ET<T>::load_frag_t(tile, LDK, 32 * ks, k0 + 16 * ni, l);
+      }
+    };
+    // (4-byte: through an offset the compiler cannot see through, which would otherwise keep the values of the first reading)
+    auto row4 = [&](const vec4& kept, const T* tile, int ni) -> vec4 {
+      if constexpr (KEPT) return kept;
+      else return *(const vec4*)(tile + fresh_index(tk * LDK + kc + 16 * ni));
+    };
+    keep(Kt);
 #pragma unroll
     for (int nj = 0; nj < 2; ++nj) {
       f32x4 g, m, mb;
@@ -500,47 +514,66 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
     float dbp[4] = {0.f, 0.f, 0.f, 0.f};      // db of token tk (partial over elements, lanes and column halves)
     float dbt[4] = {0.f, 0.f, 0.f, 0.f};      // dbeta of token tk, the part through k_b
     float kk = 0.f;
-    // acc += (tile^T's rows r0 .., or the tile's rows) times what ft holds.  The tiles are triangular: rows of the first
-    // half have no entries in the second half of the contraction, and the other way round for the transposed tile
-    auto products = [&](f32x4 (&acc)[NBK], const T* tile, auto transposed) {
+    // acc += (tile^T's rows r0 .., or the tile's rows) times the operand x (q or k), which ft holds.  The tiles are triangular:
+    // rows of the first half have no entries in the second half of the contraction, and the other way round for the
+    // transposed tile
+    auto products = [&](f32x4 (&acc)[NBK], const T* tile, auto transposed, const T* x) {
       constexpr bool TR = decltype(transposed)::value;
-      frag fb[CS];
+      auto tile_frag = [&](int ks) {
+        return TR ? ET<T>::load_frag_t(tile, LDC, 32 * ks, r0, l) : ET<T>::load_frag(tile + tk * LDC + 32 * ks + fg);
+      };
+      frag fb[KEPT ? CS : 1];
+      if constexpr (!KEPT) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (KEPT) {
 #pragma unroll
-      for (int ks = 0; ks < CS; ++ks)
-        fb[ks] = TR ? ET<T>::load_frag_t(tile, LDC, 32 * ks, r0, l) : ET<T>::load_frag(tile + tk * LDC + 32 * ks + fg);
+        for (int ks = 0; ks < CS; ++ks) fb[ks] = tile_frag(ks);
+      }
 #pragma unroll
       for (int ni = 0; ni < NBK; ++ni) acc[ni] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < CS; ++ks) {
         if (TR ? (ks == 0 || r0 >= 32) : (ks == 1 || r0 < 32)) {
+          if constexpr (KEPT) {
 #pragma unroll
-          for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(acc[ni], ft[ks][ni], fb[ks]);
+            for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(acc[ni], ft[ks][ni], fb[ks]);
+          } else {
+            const frag y = tile_frag(ks);
+#pragma unroll
+            for (int ni = 0; ni < NBK; ++ni) ET<T>::mma(acc[ni], ET<T>::load_frag_t(x, LDK, 32 * ks, k0 + 16 * ni, l), y);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
       }
     };
+    if constexpr (KEPT) {
 #pragma unroll
-    for (int ni = 0; ni < NBK; ++ni) {
-      q4[ni] = *(const vec4*)(Qt + tk * LDK + kc + 16 * ni);
-      k4[ni] = *(const vec4*)(Kt + tk * LDK + kc + 16 * ni);
+      for (int ni = 0; ni < NBK; ++ni) {
+        q4[ni] = *(const vec4*)(Qt + tk * LDK + kc + 16 * ni);
+        k4[ni] = *(const vec4*)(Kt + tk * LDK + kc + 16 * ni);
+      }
     }
     const float ebt = s_eb[tk], edt = s_ed[tk], bt = s_beta[tk];
     f32x4 dq[NBK], dk[NBK], m[NBK];
-    products(dq, T0, std::true_type());                                                  // (G k)^T
-    products(m, T1, std::true_type());                                                   // (dM k)^T: closes dk_b
+    products(dq, T0, std::true_type(), Kt);                                              // (G k)^T
+    if constexpr (KEPT) products(m, T1, std::true_type(), Kt);                           // (dM k)^T: closes dk_b
 #pragma unroll
-    for (int ni = 0; ni < NBK; ++ni)
+    for (int ni = 0; ni < NBK; ++ni) {
+      const vec4 q_ = row4(q4[ni], Qt, ni);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float dqv = scale * ebt * dqi[ni][i] + dq[ni][i];
-        dbp[i] += ET<T>::to_f(q4[ni][i]) * dqv;
+        dbp[i] += ET<T>::to_f(q_[i]) * dqv;
         dq[ni][i] = dqv;                                                                 // final dq
       }
+    }
     pin(dbp);
+    if constexpr (!KEPT) products(m, T1, std::true_type(), Kt);
 #pragma unroll
-    for (int ni = 0; ni < NBK; ++ni)
+    for (int ni = 0; ni < NBK; ++ni) {
+      const vec4 k_ = row4(k4[ni], Kt, ni);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float kv = ET<T>::to_f(k4[ni][i]);
+        const float kv = ET<T>::to_f(k_[i]);
         const float kbv = kv * bt;
         const float dkbgv = -dkbg[ni][i];
         const float dkb = m[ni][i] + dkbgv * ebt;
@@ -548,34 +581,35 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
         dbp[i] += kbv * m[ni][i] + dkbgv * kbv * ebt;
         dk[ni][i] = dkb * bt;
       }
+    }
     pin(dbp);
     pin(dbt);
-    products(m, T2, std::false_type());                                                  // (dM^T k_b)^T
-    // k^T is done with: q^T for the last product
+    products(m, T2, std::false_type(), Kt);                                              // (dM^T k_b)^T
+    keep(Qt);                                              // k^T is done with: q^T for the last product
 #pragma unroll
-    for (int ks = 0; ks < CS; ++ks)
-#pragma unroll
-      for (int ni = 0; ni < NBK; ++ni) ft[ks][ni] = ET<T>::load_frag_t(Qt, LDK, 32 * ks, k0 + 16 * ni, l);
-#pragma unroll
-    for (int ni = 0; ni < NBK; ++ni)
+    for (int ni = 0; ni < NBK; ++ni) {
+      const vec4 k_ = row4(k4[ni], Kt, ni);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        dbp[i] -= ET<T>::to_f(k4[ni][i]) * m[ni][i];
+        dbp[i] -= ET<T>::to_f(k_[i]) * m[ni][i];
         dk[ni][i] += m[ni][i];
       }
+    }
     pin(dbp);
-    products(m, T0, std::false_type());                                                  // (G^T q)^T
+    products(m, T0, std::false_type(), Qt);                                              // (G^T q)^T
 #pragma unroll
-    for (int ni = 0; ni < NBK; ++ni)
+    for (int ni = 0; ni < NBK; ++ni) {
+      const vec4 k_ = row4(k4[ni], Kt, ni);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float kv = ET<T>::to_f(k4[ni][i]);
+        const float kv = ET<T>::to_f(k_[i]);
         const float dkdv = edt * dkd[ni][i];
         const float dkv = dkdv + m[ni][i];                                               // the part of dk that does not pass through the WY form
         dbp[i] -= kv * dkv;
         kk += kv * dkdv;
         dk[ni][i] += dkv;                                                                // final dk
       }
+    }
     // over the elements and the four lanes that hold a token
     float dbs = (dbp[0] + dbp[1]) + (dbp[2] + dbp[3]), dts = (dbt[0] + dbt[1]) + (dbt[2] + dbt[3]);
     dbs += __shfl_xor(dbs, 16, 64);
