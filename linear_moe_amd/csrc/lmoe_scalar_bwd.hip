@@ -35,13 +35,31 @@ template <typename T, int K, int V> struct StateBwd {
   }
   template <int BVX, bool CUT> static void launch(const lmoe_args& a, const Split& sp, hipStream_t st) {
     const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BVX)), block(2 * NTHR);
+    // Rows' places in registers (KEPT) are 12 to 17 of them at K = 128, and with 4-byte elements and in the wide slices of the
+    // normalised pass they cost a CU its second work-group.  That matters where the launch has one: more work-groups
+    // than CUs, without and with them (us): 4-byte, 64 pairs of 32 chunks 95 and 121, 24 pairs of 128 chunks cut 161 and
+    // 180; normalised, 256 pairs of 16 chunks 67 and 74.  With up to one per CU they gain, as they do elsewhere: 4-byte,
+    // 32 pairs of 128 chunks 242 and 228; normalised, 128 pairs of 32 chunks 76 and 72.
+    const bool second = grid.x > (unsigned)cu_count();
     if constexpr (sizeof(T) == 2) {        // the pass behind the normalised output exists for 2-byte elements
       if (a.normalize == 1) {
+        if constexpr (K == 128 && BVX == 64) {
+          if (second) {
+            hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 1, CUT, false>), grid, block, 0, st, a, sp);
+            return;
+          }
+        }
         hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 1, CUT>), grid, block, 0, st, a, sp);
         return;
       }
       if (a.normalize == 2) {
         hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 2, CUT>), grid, block, 0, st, a, sp);
+        return;
+      }
+    }
+    if constexpr (sizeof(T) == 4 && K == 128) {
+      if (second) {
+        hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 0, CUT, false>), grid, block, 0, st, a, sp);
         return;
       }
     }

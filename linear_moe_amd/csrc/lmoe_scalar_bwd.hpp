@@ -115,7 +115,8 @@ __global__ __launch_bounds__(NTHR) void k_bwd_dv(const lmoe_args a) {
 // before it divides): d_o is the gradient of o as it stands and dden comes in as a tensor; it enters once, in the first
 // V slice (the other slices carry zeros).
 constexpr int NORM_SLOT_COLS = 32;
-template <typename T, int K, int V, int BV, int NORM = 0, bool CUT = false>
+// KEPT: where a loader thread's rows lie is kept in registers (TileIO::load_rows).
+template <typename T, int K, int V, int BV, int NORM = 0, bool CUT = false, bool KEPT = true>
 __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const Split sp) {
   constexpr int LDK = K + LPAD, LDU = BV + LPAD;
   constexpr int MB = K / 64, NB = BV / 16;
@@ -176,8 +177,13 @@ __global__ __launch_bounds__(2 * NTHR) void k_state_bwd(const lmoe_args a, const
       c = max(c, 0);
       const int tok = sq.tok0 + c * CH;
       const int len = min(CH, sq.len - c * CH);
-      IOK::load_rows(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
-      IOV::load_rows(P.rd, od, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, len);
+      if constexpr (KEPT) {
+        IOK::load_rows(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
+        IOV::load_rows(P.rd, od, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, len);
+      } else {
+        IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
+        IOV::load_nomask(P.rd, row_ptr<T>(a.d_o, sq.b, tok, h) + v0, a.d_o.st, len);
+      }
       P.len = len;
       P.graw = load_scalar_raw(gptr, a.g_dtype, gated ? row_off(a.g, sq.b, tok + min(l, len - 1), h) : 0);
       if constexpr (NORM == 1) {
