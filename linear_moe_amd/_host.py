@@ -197,8 +197,8 @@ class SeqPlan:
 
     @property
     def tables(self):
-        """What the native launch path takes."""
-        return (self.N, self.NT, self.cu, self.chunk_map, self.seq_chunk0, self.seq_order, self.nt_dev)
+        """What the native launch path takes: None for a dense call."""
+        return None if self.cu is None else (self.N, self.NT, self.cu, self.chunk_map, self.seq_chunk0, self.seq_order, self.nt_dev)
 
     def _build_on_device(self, T: int, cu_seqlens: torch.Tensor):
         dev = cu_seqlens.device

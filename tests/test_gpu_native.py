@@ -214,3 +214,27 @@ def test_saved_tensors_that_come_back_changed(cuda, kind):
         for cut in (lambda x: x[:, :1] if x.dim() > 1 else x[:-4], lambda x: x[..., :-4], lambda x: x.cpu()):
             with pytest.raises((RuntimeError, ValueError)):
                 _through_hooks(kind, cuda, lambda n, x: cut(x) if n == name else x)
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("head_first", [True, False])
+@pytest.mark.parametrize("T", [200, 1900])
+def test_backward_is_native_where_only_the_forward_was_not(cuda, monkeypatch, op, head_first, T):
+    """a 2-byte gate of the other kind sends the forward to the Python steps, which convert it: the backward has nothing to
+    convert any more and takes the native path, with the same bits"""
+    import linear_moe_amd.gated_delta_rule as gdr
+    import linear_moe_amd.gla as gla
+    import linear_moe_amd.simple_gla as sg
+    x = _inputs(op, 2, T, 2, 64, 64, torch.bfloat16, head_first, False, torch.float16, cuda)
+    args = [x["q"], x["k"], x["v"], x["g"]] + ([x["beta"]] if op == 2 else []) + [None, None, False, None, head_first]
+    do = torch.randn_like(x["v"])
+    out = []
+    for keep in (True, False):
+        c = _call(op, keep)
+        o, _ = c.forward(*args)
+        with monkeypatch.context() as m:
+            if not keep:
+                for mod in (sg, gla, gdr):
+                    m.setattr(mod, "base_args", None)
+            out.append([o, *c.backward(do, None)])
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(*out))
