@@ -380,7 +380,7 @@ def stream_ptr() -> int:
 # steps in Python.  (Host time of a call, small sizes on one machine: one token 20 -> 8 us; forward 23 -> 15; forward and
 # backward of the gated delta rule 143 -> 90, of which autograd itself is 27 to 60.)
 def native(fn: str, what: str, op: int, q, *args):
-    """``forward``, ``backward`` or ``recurrent`` of the native path: its results, or None (not a call for it)."""
+    """``forward``, ``backward``, ``intact`` or ``recurrent`` of the native path: its results, or None (not a call for it)."""
     if not q.is_cuda:
         return None
     r = getattr(_lib.native(), fn)(op, q, *args, stream_ptr())

@@ -44,11 +44,12 @@ class GDNCall:
         read v, and ``backward`` returns the gradient with respect to that argument."""
         ctx = self
         lib = _lib.load()
-        plan = None
+        plan = dims = None
         if cu_seqlens is not None:
-            B, T = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)[:2]
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)
+            B, T = dims[:2]
             plan = seq_plan(B, T, cu_seqlens, q.device)
-        if not self.keep:
+        if not self.keep and q.dtype != torch.float32:           # (4-byte elements need w and u as well)
             tables = None if plan is None else plan.tables
             r = native("forward", "chunk_gated_delta_rule forward", self.OP, q, k, v, g, beta, initial_state, tables,
                        scale, output_final_state, head_first, save, 0, 0.0, v_act)
@@ -58,7 +59,8 @@ class GDNCall:
                 ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, None, head_first, scale
                 ctx.has_h0, ctx.v_act, self.seg_ws = initial_state is not None, bool(v_act), None
                 return o, ht
-        dims = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)
+        if dims is None:
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens, wide_v=True)
         B, T, H, K, V = dims
         q, k, v = _aligned(q), _aligned(k), _aligned(v)
         if plan is None:
@@ -136,25 +138,34 @@ class GDNCall:
         lib = _lib.load()
         q, k, v, g, beta, h0, hs, tinv, pmat, gcum, vnew, seg_p = ctx.saved
         head_first = ctx.head_first
+        dims = None
         if not self.keep:
-            raw = (None, None) if qk_raw is None else qk_raw
-            r = native("backward", "chunk_gated_delta_rule backward", self.OP, q, k, v, g, beta, h0, ctx.plan and
-                       ctx.plan.tables, ctx.scale, do, dht, head_first, (hs, tinv, pmat, gcum, vnew, seg_p), (ctx.v_act,
-                       dq_out, dk_out, dv_out, *raw, float(qk_eps)))
-            if r is not None:
-                dq, dk, dv, dg, dbeta, dh0 = r
-                return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dbeta, dh0
-        q, k, v, do, dims = inputs_came_back(q, k, v, do, head_first, wide_v=True)
+            raw, what = (None, None) if qk_raw is None else qk_raw, "chunk_gated_delta_rule backward"
+            args = (self.OP, q, k, v, g, beta, h0, ctx.plan and ctx.plan.tables, ctx.scale, do, dht, head_first, (hs, tinv, pmat, gcum,
+                    vnew, seg_p), (ctx.v_act, dq_out, dk_out, dv_out, *raw, float(qk_eps)))
+            if q.dtype != torch.float32:
+                r = native("backward", what, *args)
+                if r is not None:
+                    dq, dk, dv, dg, dbeta, dh0 = r
+                    return dq, dk, dv, (dg if dg is None or dg.dtype == g.dtype else dg.to(g.dtype)), dbeta, dh0
+            else:
+                dims = native("intact", what, *args)
+        intact = dims is not None
+        if not intact:
+            q, k, v, do, dims = inputs_came_back(q, k, v, do, head_first, wide_v=True)
         B, T, H, K, V = dims
         plan = ctx.plan or seq_plan(B, T, None, q.device)
-        dev, dt, tok, nt = q.device, q.dtype, ((B, H, T) if head_first else (B, T, H)), max(plan.NT, 1)
-        g = None if g is None else came_back(g, tok, None, dev, "g")
-        beta = came_back(beta, tok, None, dev, "beta")
-        if ctx.has_h0:
-            h0 = came_back(h0, (plan.N, H, K, V), torch.float32, dev, "initial_state")
-        hs, tinv = came_back(hs, (nt, H, K, V), dt, dev, "hs"), came_back(tinv, (nt, H, 64, 64), dt, dev, "tinv")
-        pmat, gcum = came_back(pmat, (nt, H, 64, 64), dt, dev, "pmat"), came_back(gcum, (nt, H, 5, 64), torch.float32, dev, "gcum")
-        vnew = came_back(vnew, (nt, H, V // 32, 64, 32), dt, dev, "vnew")
+        dev, dt = q.device, q.dtype
+        if not intact:
+            tok, nt = ((B, H, T) if head_first else (B, T, H)), max(plan.NT, 1)
+            g = None if g is None else came_back(g, tok, None, dev, "g")
+            beta = came_back(beta, tok, None, dev, "beta")
+            if ctx.has_h0:
+                h0 = came_back(h0, (plan.N, H, K, V), torch.float32, dev, "initial_state")
+            hs, tinv = came_back(hs, (nt, H, K, V), dt, dev, "hs"), came_back(tinv, (nt, H, 64, 64), dt, dev, "tinv")
+            pmat = came_back(pmat, (nt, H, 64, 64), dt, dev, "pmat")
+            gcum = came_back(gcum, (nt, H, 5, 64), torch.float32, dev, "gcum")
+            vnew = came_back(vnew, (nt, H, V // 32, 64, 32), dt, dev, "vnew")
         a = base_args(q, k, v, head_first, ctx.scale, plan, dims)
         a.gate = _lib.GATE_NONE if g is None else _lib.GATE_SCALAR
         if g is not None:

@@ -35,9 +35,10 @@ class GLACall:
         """save=False: a forward-only call (nothing requires a gradient): the per-chunk states are not written where
         the state pass forms the output itself (bf16); the fp32 path's output kernel reads them."""
         lib = _lib.load()
-        plan = None
+        plan = dims = None
         if cu_seqlens is not None:
-            B, T = _check_inputs(q, k, v, head_first, cu_seqlens)[:2]
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens)
+            B, T = dims[:2]
             if g is not None and g.shape == q.shape:
                 plan = seq_plan(B, T, cu_seqlens, q.device)
         if not self.keep:
@@ -50,7 +51,8 @@ class GLACall:
                 self.plan, self.dims, self.head_first, self.scale = plan, None, head_first, scale
                 self.has_h0 = initial_state is not None
                 return o, ht
-        dims = _check_inputs(q, k, v, head_first, cu_seqlens)
+        if dims is None:
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens)
         B, T, H, K, V = dims
         if g is None or tuple(g.shape) != tuple(q.shape):
             raise ValueError(f"g must have the shape of q {tuple(q.shape)}")

@@ -37,9 +37,10 @@ class SimpleGLACall:
         before dividing); ``backward`` then takes the gradient of den beside that of o."""
         ctx = self
         lib = _lib.load()
-        plan = None
+        plan = dims = None
         if cu_seqlens is not None:
-            B, T = _check_inputs(q, k, v, head_first, cu_seqlens)[:2]
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens)
+            B, T = dims[:2]
             plan = seq_plan(B, T, cu_seqlens, q.device)
         if not self.keep:
             tables = None if plan is None else plan.tables
@@ -53,7 +54,8 @@ class SimpleGLACall:
                 ctx.plan, ctx.dims, ctx.head_first, ctx.scale = plan, None, head_first, scale
                 ctx.has_h0 = initial_state is not None
                 return o, ht
-        dims = _check_inputs(q, k, v, head_first, cu_seqlens)
+        if dims is None:
+            dims = _check_inputs(q, k, v, head_first, cu_seqlens)
         B, T, H, K, V = dims
         q, k, v = _aligned(q), _aligned(k), _aligned(v)
         if plan is None:

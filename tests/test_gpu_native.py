@@ -216,6 +216,19 @@ def test_saved_tensors_that_come_back_changed(cuda, kind):
                 _through_hooks(kind, cuda, lambda n, x: cut(x) if n == name else x)
 
 
+def test_calls_handed_back_leave_no_error_behind(cuda):
+    """a call that is not for the native path gives None, whatever stopped it and at whichever check"""
+    from linear_moe_amd._host import native
+    x = _inputs(2, 2, 100, 2, 64, 64, torch.bfloat16, False, False, torch.float32, cuda)
+    f = lambda q, k, v, g, beta, scale=None, hf=False, eps=0.0: native("forward", "t", 2, q, k, v, g, beta, None, None, scale, False,
+                                                                      hf, True, 0, eps, False)
+    ok = (x["q"], x["k"], x["v"], x["g"], x["beta"])
+    assert type(f(*ok)) is tuple
+    assert f(*(t.float() for t in ok)) is None                                   # 4-byte delta rule
+    assert f(*ok[:3], ok[3].half(), ok[4]) is None and f(*ok[:4], ok[4].double()) is None and f(*ok[:4], None) is None
+    assert f(*ok, scale="x") is None and f(*ok, hf=torch.ones(2)) is None and f(*ok, eps="x") is None
+
+
 @pytest.mark.parametrize("op", [0, 1, 2])
 @pytest.mark.parametrize("head_first", [True, False])
 @pytest.mark.parametrize("T", [200, 1900])
