@@ -155,13 +155,12 @@ struct Call {
   }
 };
 
-template <typename F> int launch(F f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
-  return rc;
-}
+// Allocations and the launch run without the interpreter's lock, as torch's own allocating functions do: an allocation may wait
+// for the device (hipMalloc, or hipFree of cached blocks), and other threads go on meanwhile.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 PyObject* wrap(const Tensor& t) {
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
@@ -197,10 +196,16 @@ PyObject* recurrent(PyObject*, PyObject* const* o, Py_ssize_t n) {
   c.a.qk_eps = (float)PyFloat_AsDouble(o[11]);
   void* st = stream_of(o[12]);
   if (PyErr_Occurred()) return elsewhere();
-  const Tensor out = at::empty_like(c.v.detach());
-  const Tensor ht = final_state ? c.states() : Tensor();
-  c.a.o = desc(out, c.head_first); c.a.ht = (float*)ptr(ht);
-  return result(launch([&] { return lib.recurrent(&c.a, op, st); }), {out, ht});
+  Tensor out, ht;
+  int rc;
+  {
+    const Unlocked unlocked;
+    out = at::empty_like(c.v.detach());
+    if (final_state) ht = c.states();
+    c.a.o = desc(out, c.head_first); c.a.ht = (float*)ptr(ht);
+    rc = lib.recurrent(&c.a, op, st);
+  }
+  return result(rc, {out, ht});
   END_HANDLE_TH_ERRORS
 }
 
@@ -217,41 +222,39 @@ PyObject* forward(PyObject*, PyObject* const* o, Py_ssize_t n) {
   void* st = stream_of(o[15]);
   if ((normalize && (c.g.defined() || !two)) || PyErr_Occurred()) return elsewhere();
   const auto dt = c.q.scalar_type();
-  // (v_act: v is a block of a wider tensor; o is a tensor of its own)
-  const Tensor out = v_act ? at::empty(c.v.sizes(), c.v.options()) : at::empty_like(c.v);
-  const Tensor ht = final_state ? c.states() : Tensor();
-  c.a.o = desc(out, hf); c.a.ht = (float*)ptr(ht);
-  Tensor hs;
-  if (op == OP_SIMPLE) {
-    Tensor den, zs;
-    if (save) hs = c.chunked({c.K, c.V}, dt);
+  Tensor out, ht, hs, den, zs, amat, qe, ke, gcum, tinv, pmat, vnew, seg_p;
+  int rc;
+  {
+    const Unlocked unlocked;
+    // (v_act: v is a block of a wider tensor; o is a tensor of its own)
+    out = v_act ? at::empty(c.v.sizes(), c.v.options()) : at::empty_like(c.v);
+    if (final_state) ht = c.states();
+    c.a.o = desc(out, hf); c.a.ht = (float*)ptr(ht);
+    if (save || (op == OP_GLA && !two)) hs = c.chunked({c.K, c.V}, dt);
     c.a.hs = ptr(hs);
-    if (normalize) {
+    if (op == OP_SIMPLE && normalize) {
       den = at::empty(c.token_shape(), c.q.options().dtype(at::kFloat));
       if (save) zs = c.chunked({c.K}, at::kFloat);
       c.a.normalize = normalize; c.a.den = desc(den, hf); c.a.zs = (float*)ptr(zs);
+    } else if (op == OP_GLA) {
+      amat = c.chunked({64, 64}, dt); qe = c.chunked({64, c.K}, dt); ke = c.chunked({64, c.K}, dt); gcum = c.chunked({c.K}, at::kFloat);
+      c.a.amat = ptr(amat); c.a.qe = ptr(qe); c.a.ke = ptr(ke); c.a.gcum = (float*)ptr(gcum);
+    } else if (op == OP_GDN) {
+      if (save) { pmat = c.chunked({64, 64}, dt); vnew = c.chunked({c.V / 32, 64, 32}, dt); }
+      tinv = c.chunked({64, 64}, dt); gcum = c.chunked({5, 64}, at::kFloat);
+      c.a.tinv = ptr(tinv); c.a.pmat = ptr(pmat); c.a.gcum = (float*)ptr(gcum); c.a.vnew.ptr = ptr(vnew);
+      c.a.v_act = v_act;
     }
     const Tensor ws = c.cut(op);
-    return result(launch([&] { return lib.fwd[op](&c.a, st); }), {out, ht, hs, den, zs});
+    if (op == OP_GDN && ws.defined() && save) {
+      seg_p = at::empty({lib.split_floats(&c.a, op, 0)}, c.q.options().dtype(at::kFloat));
+      c.a.seg_p = (float*)seg_p.data_ptr();
+    }
+    rc = lib.fwd[op](&c.a, st);
   }
-  if (op == OP_GLA) {
-    if (save || !two) hs = c.chunked({c.K, c.V}, dt);
-    const Tensor amat = c.chunked({64, 64}, dt), qe = c.chunked({64, c.K}, dt), ke = c.chunked({64, c.K}, dt), gdec = c.chunked({c.K}, at::kFloat);
-    c.a.hs = ptr(hs); c.a.amat = ptr(amat); c.a.qe = ptr(qe); c.a.ke = ptr(ke); c.a.gcum = (float*)ptr(gdec);
-    const Tensor ws = c.cut(op);
-    return result(launch([&] { return lib.fwd[op](&c.a, st); }), {out, ht, hs, amat, qe, ke, gdec});
-  }
-  Tensor pmat, vnew, seg_p;
-  if (save) { hs = c.chunked({c.K, c.V}, dt); pmat = c.chunked({64, 64}, dt); vnew = c.chunked({c.V / 32, 64, 32}, dt); }
-  const Tensor tinv = c.chunked({64, 64}, dt), gcum = c.chunked({5, 64}, at::kFloat);
-  c.a.hs = ptr(hs); c.a.tinv = ptr(tinv); c.a.pmat = ptr(pmat); c.a.gcum = (float*)ptr(gcum); c.a.vnew.ptr = ptr(vnew);
-  c.a.v_act = v_act;
-  const Tensor ws = c.cut(op);
-  if (ws.defined() && save) {
-    seg_p = at::empty({lib.split_floats(&c.a, op, 0)}, c.q.options().dtype(at::kFloat));
-    c.a.seg_p = (float*)seg_p.data_ptr();
-  }
-  return result(launch([&] { return lib.fwd[op](&c.a, st); }), {out, ht, hs, tinv, pmat, gcum, vnew, seg_p});
+  if (op == OP_SIMPLE) return result(rc, {out, ht, hs, den, zs});
+  if (op == OP_GLA) return result(rc, {out, ht, hs, amat, qe, ke, gcum});
+  return result(rc, {out, ht, hs, tinv, pmat, gcum, vnew, seg_p});
   END_HANDLE_TH_ERRORS
 }
 
@@ -337,28 +340,35 @@ PyObject* backward(PyObject*, PyObject* const* o, Py_ssize_t n) {
   const auto dt = c.q.scalar_type();
   auto fresh = [&](const Tensor& x) { return at::empty_like(x.detach()); };
   auto or_fresh = [&](const Tensor& x, const Tensor& like) { return x.defined() ? x : fresh(like); };
-  const Tensor dq = or_fresh(c.given[0], c.q), dk = or_fresh(c.given[1], c.k), dv = or_fresh(c.given[2], c.v);
-  const Tensor dh0 = c.h0.defined() ? fresh(c.h0) : Tensor(), dhs = c.chunked({c.K, c.V}, dt);
-  c.a.dq = desc(dq, hf); c.a.dk = desc(dk, hf); c.a.dv = desc(dv, hf); c.a.dh0 = (float*)ptr(dh0); c.a.dhs = ptr(dhs);
-  Tensor dg, dbeta, dvnew, norm_ws, ws;
-  if (op == OP_GLA) {
-    dg = at::empty(c.g.sizes(), c.g.options());             // (in the type of g, by the kernel)
-  } else if (op == OP_GDN || c.g.defined()) {
-    const Tensor& like = op == OP_GDN ? c.beta : c.g;
-    dg = at::empty(like.sizes(), like.options().dtype(at::kFloat));
+  Tensor dq, dk, dv, dg, dbeta, dh0;
+  int rc;
+  {
+    const Unlocked unlocked;
+    dq = or_fresh(c.given[0], c.q); dk = or_fresh(c.given[1], c.k); dv = or_fresh(c.given[2], c.v);
+    if (c.h0.defined()) dh0 = fresh(c.h0);
+    const Tensor dhs = c.chunked({c.K, c.V}, dt);
+    c.a.dq = desc(dq, hf); c.a.dk = desc(dk, hf); c.a.dv = desc(dv, hf); c.a.dh0 = (float*)ptr(dh0); c.a.dhs = ptr(dhs);
+    Tensor dvnew, norm_ws, ws;
+    if (op == OP_GLA) {
+      dg = at::empty(c.g.sizes(), c.g.options());           // (in the type of g, by the kernel)
+    } else if (op == OP_GDN || c.g.defined()) {
+      const Tensor& like = op == OP_GDN ? c.beta : c.g;
+      dg = at::empty(like.sizes(), like.options().dtype(at::kFloat));
+    }
+    c.a.dg = desc(dg, hf);
+    if (c.a.normalize) {
+      norm_ws = c.chunked({c.V / 32, 64 + c.K}, at::kFloat);
+      c.a.norm_ws = (float*)norm_ws.data_ptr();
+    }
+    if (op == OP_GDN) {
+      dvnew = c.chunked({c.V / 32, 64, 32}, dt);
+      dbeta = at::empty(c.beta.sizes(), c.beta.options());
+      c.a.dvnew.ptr = ptr(dvnew); c.a.dbeta_bf16 = bf16(dbeta); c.a.dbeta = desc(dbeta, hf);
+    }
+    if (op != OP_GDN || c.a.seg_p) ws = c.cut(op);
+    rc = lib.bwd[op](&c.a, st);
   }
-  c.a.dg = desc(dg, hf);
-  if (c.a.normalize) {
-    norm_ws = c.chunked({c.V / 32, 64 + c.K}, at::kFloat);
-    c.a.norm_ws = (float*)norm_ws.data_ptr();
-  }
-  if (op == OP_GDN) {
-    dvnew = c.chunked({c.V / 32, 64, 32}, dt);
-    dbeta = at::empty(c.beta.sizes(), c.beta.options());
-    c.a.dvnew.ptr = ptr(dvnew); c.a.dbeta_bf16 = bf16(dbeta); c.a.dbeta = desc(dbeta, hf);
-  }
-  if (op != OP_GDN || c.a.seg_p) ws = c.cut(op);
-  return result(launch([&] { return lib.bwd[op](&c.a, st); }), {dq, dk, dv, c.g.defined() ? dg : Tensor(), dbeta, dh0});
+  return result(rc, {dq, dk, dv, c.g.defined() ? dg : Tensor(), dbeta, dh0});
   END_HANDLE_TH_ERRORS
 }
 

@@ -251,3 +251,42 @@ def test_backward_is_native_where_only_the_forward_was_not(cuda, monkeypatch, op
                     m.setattr(mod, "base_args", None)
             out.append([o, *c.backward(do, None)])
     assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_other_threads_run_while_a_call_allocates(cuda):
+    """the interpreter's lock is not held over the allocations: a call on an empty cache spends most of its time in them, and
+    another thread that only looks at the clock stands still for less than 0.4 of it (the middle of nine calls; 0.6 to 0.75 with
+    the lock held)"""
+    import sys
+    import threading
+    import time
+    import linear_moe_amd as L
+    x = _inputs(2, 4, 8192, 32, 128, 128, torch.bfloat16, False, False, torch.float32, cuda)
+    x["q"].requires_grad_()
+    interval, shares = sys.getswitchinterval(), []
+    sys.setswitchinterval(1e-4)
+    try:
+        for _ in range(10):
+            torch.cuda.synchronize()
+            torch.cuda.empty_cache()
+            worst, stop = [0.0], threading.Event()
+
+            def watch():
+                last = time.perf_counter()
+                while not stop.is_set():
+                    now = time.perf_counter()
+                    worst[0] = max(worst[0], now - last)
+                    last = now
+            th = threading.Thread(target=watch)
+            th.start()
+            time.sleep(0.01)
+            t = time.perf_counter()
+            o = L.chunk_gated_delta_rule(**x)[0]
+            t = time.perf_counter() - t
+            stop.set()
+            th.join()
+            shares.append(worst[0] / t)
+            del o
+    finally:
+        sys.setswitchinterval(interval)
+    assert sorted(shares[1:])[4] < 0.4, shares
