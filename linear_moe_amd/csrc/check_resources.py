@@ -26,13 +26,17 @@ GUARDED = {
     "k_gdn_seg_bwd": 2,
     "k_gdn_wy_fwd": 2,
     "k_gla_fwd_fused": 3,
-    "k_state_bwd": 4,         # two work-groups of 8 waves per CU; see KEPT
+    "k_state_bwd": 4,         # two work-groups of 8 waves per CU; see FLOORS
+    "k_gla_bwd_dqkg": 2,      # K = 64: two work-groups of 8 waves per CU, see FLOORS
     "k_bwd_dqkv": 2,          # one work-group of 8 waves per CU; its first version spilled loop-invariant lane arithmetic
 }
 ANY_TYPE = ("k_state_bwd",)
-# the instances of k_state_bwd whose kept places (last argument) cost the second work-group: launched where there is one
-# work-group per CU at most
-KEPT = re.compile(r"k_state_bwdI(DF16bLi128ELi\d+ELi64ELi1|fLi128ELi\d+ELi16ELi0)ELb[01]ELb1EE")
+# other minima of single instances
+FLOORS = (
+    # the instances whose kept places (last argument) cost the second work-group: launched where there is one per CU at most
+    (re.compile(r"k_state_bwdI(DF16bLi128ELi\d+ELi64ELi1|fLi128ELi\d+ELi16ELi0)ELb[01]ELb1EE"), 2),
+    (re.compile(r"k_gla_bwd_dqkgIDF16b(DF16b|f)Li64E"), 4),
+)
 FIELDS = {"ScratchSize [bytes/lane]": "scratch", "VGPRs Spill": "vspill", "Occupancy [waves/SIMD]": "occ",
           "VGPRs": "vgpr", "AGPRs": "agpr", "LDS Size [bytes/block]": "lds"}
 
@@ -70,8 +74,7 @@ def main(paths):
                         f"scratch {r.get('scratch', -1):4d} B  vgpr-spill {r.get('vspill', -1):3d}  waves/SIMD {r.get('occ', -1)}  "
                         f"lds {r.get('lds', -1)}  {name}")
                 seen[kern] += 1
-                if KEPT.search(name):
-                    min_occ = 2
+                min_occ = next((floor for pat, floor in FLOORS if pat.search(name)), min_occ)
                 if r.get("scratch", 1) != 0 or r.get("vspill", 1) != 0 or ((two_byte or kern in ANY_TYPE) and r.get("occ", 0) < min_occ):
                     bad.append(line)
     missing = [k for k, n in seen.items() if n == 0]

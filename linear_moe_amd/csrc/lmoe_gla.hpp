@@ -902,7 +902,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_bwd_dv(const lmoe_args a) {
 
 // ------------------------------------------------------------------------- //
 // dq, dk, dg (2-byte elements: dv as well), grid = (NT, H), 512 threads: wave w forms rows 16 (w % 4) .. of every product and
-// of its columns the half w / 4.  The kernel is a chain of short phases on LDS tiles (76 KB at K = 64, 135 KB at K = 128:
+// of its columns the half w / 4.  The kernel is a chain of short phases on LDS tiles (78 KB at K = 64, 138 KB at K = 128:
 // two, one work-groups per CU), so what hides its latencies is the number of waves per work-group.
 // ------------------------------------------------------------------------- //
 template <typename T, typename GT, int K, int V, int BVH>
@@ -930,10 +930,14 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   constexpr int S_B = 0, S_TBASE = CH * LDB * 4;
   constexpr int T_Q = 0, T_K = T_Q + CH * LDK, T_DA = T_K + CH * LDK, T_KT = T_DA + CH * LDC, T_END = T_KT + 192 * LDK;
   constexpr int S_BYTES = S_TBASE + T_END * (int)sizeof(T);
-  constexpr bool SUB = S_BYTES + 4096 <= 160 * 1024;
+  // beside it: s_hdh, s_kk, s_er, s_ec (13 K floats), the segment totals of the two cumulative sums (NW each), a flag
+  constexpr int BESIDE = (13 * K + 2 * NW) * 4 + 4;
+  constexpr bool SUB = S_BYTES + BESIDE <= 160 * 1024;
   static_assert(!SUB || 192 * LDK * (int)sizeof(T) >= CH * LDB * 4, "the db tile fits over the stacked k~, q~ tile");
   constexpr int B_BYTES = SUB ? S_BYTES : B_END * 4;
   constexpr int NBYTES = (A_END * (int)sizeof(T) > B_BYTES) ? A_END * (int)sizeof(T) : B_BYTES;
+  static_assert(NBYTES + BESIDE <= 160 * 1024, "the layout fits the LDS");
+  static_assert(K > 64 || sizeof(T) > 2 || 2 * (NBYTES + BESIDE) <= 160 * 1024, "two work-groups per CU, as the attribute assumes");
   __shared__ __attribute__((aligned(16))) unsigned char smem_raw[NBYTES];
   __shared__ __attribute__((aligned(16))) float s_hdh[K], s_kk[4 * K];
   T* smT = (T*)smem_raw;
