@@ -290,3 +290,91 @@ def test_other_threads_run_while_a_call_allocates(cuda):
     finally:
         sys.setswitchinterval(interval)
     assert sorted(shares[1:])[4] < 0.4, shares
+
+
+def _mods():
+    import linear_moe_amd.gated_delta_rule as gdr
+    import linear_moe_amd.gla as gla
+    import linear_moe_amd.simple_gla as sg
+    return sg, gla, gdr
+
+
+@pytest.mark.parametrize("op", [0, 1, 2])
+@pytest.mark.parametrize("form", ["dense", "head_first", "packed", "cut"])
+@pytest.mark.parametrize("what", ["expanded do", "misaligned do", "bfloat16 dht", "strided dht"])
+def test_backward_in_python_steps_behind_a_native_forward(cuda, monkeypatch, op, form, what):
+    """the forward was native (no plan of a dense call, no dimensions kept); a gradient that has to be converted sends the backward
+    to the Python steps, which give the bits of a call that took them throughout"""
+    mod, hf = _mods()[op], form == "head_first"
+    B, T, N = {"dense": (2, 200, 2), "head_first": (2, 200, 2), "packed": (1, 500, 4), "cut": (1, 4000, 1)}[form]
+    cu = torch.tensor([0, 70, 70, 71, 500], dtype=torch.int32, device=cuda) if form == "packed" else None
+    x = _inputs(op, B, T, 2, 64, 64, torch.bfloat16, hf, False, torch.float32, cuda)
+    h0, dht = torch.randn(N, 2, 64, 64, device=cuda), torch.randn(N, 2, 64, 64, device=cuda)
+    do = torch.randn_like(x["v"])
+    if what == "expanded do":
+        do = torch.ones((), device=cuda, dtype=torch.bfloat16).expand(x["v"].shape)
+    elif what == "misaligned do":
+        wide = torch.zeros(*do.shape[:3], 65, device=cuda, dtype=torch.bfloat16)
+        wide[..., 1:] = do
+        do = wide[..., 1:]
+    else:
+        dht = dht.bfloat16() if what == "bfloat16 dht" else dht.mT.contiguous().mT
+    args = [x["q"], x["k"], x["v"], x["g"]] + ([x["beta"]] if op == 2 else []) + [None, h0, True, cu, hf]
+    c = _call(op, True)
+    ref = [*c.forward(*args), *c.backward(do, dht)]
+    c = _call(op, False)
+    with monkeypatch.context() as m:
+        m.setattr(mod, "base_args", None)
+        got = list(c.forward(*args))
+    assert c.dims is None and (c.plan is None) == (cu is None) and (op != 2 or (c.saved[-1] is not None) == (form == "cut"))
+    answers, native = [], mod.native
+    with monkeypatch.context() as m:
+        m.setattr(mod, "native", lambda *a: answers.append(native(*a)) or answers[-1])
+        got += c.backward(do, dht)
+    assert answers == [None]
+    assert all((a is None and b is None) or torch.equal(a, b) for a, b in zip(ref, got))
+
+
+def _wide_v(cuda, T):
+    import linear_moe_amd as L
+    x = _inputs(2, 2, T, 3, 128, 256, torch.bfloat16, False, True, torch.bfloat16, cuda)
+    x["k"] = _inputs(2, 2, T, 3, 128, 64, torch.bfloat16, False, False, torch.float32, cuda)["k"]
+    ls = [t.requires_grad_() for t in x.values()]
+    o, ht = L.chunk_gated_delta_rule(*ls, output_final_state=True)
+    return [o, ht], ls
+
+
+def _mixer(cuda, T, D=64):
+    import linear_moe_amd as L
+    gen = torch.Generator(device=cuda).manual_seed(7)
+    rn = lambda *s: torch.randn(*s, generator=gen, device=cuda)
+    ls = [rn(T, 2, 3 * 3 * D).bfloat16(), -rn(2, T, 3).abs(), torch.sigmoid(rn(2, T, 3)).bfloat16()]
+    ls = [t.requires_grad_() for t in ls]
+    return [L.gdn_mixer_core(*ls, 3, D)], ls
+
+
+def _with_den(cuda, T):
+    from linear_moe_amd.simple_gla import chunk_simple_gla_with_den
+    x = _inputs(0, 2, T, 3, 128, 64, torch.bfloat16, True, True, torch.float32, cuda)
+    ls = [x["q"].abs(), x["k"].abs(), x["v"], torch.randn(2, 3, 128, 64, device=cuda, generator=torch.Generator(device=cuda).manual_seed(9))]
+    ls = [t.detach().requires_grad_() for t in ls]
+    o, den, ht = chunk_simple_gla_with_den(*ls[:3], None, ls[3], True)
+    return [o, den, ht], ls
+
+
+@pytest.mark.parametrize("form", [_wide_v, _mixer, lambda cuda, T: _mixer(cuda, T, 128), _with_den],
+                         ids=["V=256", "mixer D=64", "mixer D=128", "den"])
+@pytest.mark.parametrize("T", [1, 190, 4100])
+def test_other_forms_same_bits(cuda, monkeypatch, form, T):
+    """V = 256; silu(v), gradients written into the blocks of the projection's and the raw q, k of the mixer; den and its gradient"""
+    out = []
+    for python in (True, False):
+        with monkeypatch.context() as m:
+            for mod in _mods():
+                m.setattr(mod, "native", lambda *a: None) if python else m.setattr(mod, "base_args", None)
+            outs, ls = form(cuda, T)
+            gen = torch.Generator(device=cuda).manual_seed(11)
+            douts = [torch.randn(o.shape, generator=gen, device=cuda).to(o.dtype) for o in outs]
+            out.append([*outs, *torch.autograd.grad(outs, ls, douts)])
+    for a, b in zip(*out):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b) and b.abs().max() > 0
