@@ -368,8 +368,8 @@ template <typename T> __device__ __forceinline__ void scale_frag8(typename ET<T>
 }
 
 // c + <a, b> over the elements of a 16-byte vector.  2-byte elements: two products and their sum per instruction in place of two
-// conversions and a multiply-add each (products exact, fp32 sums; against float64 its error is 0.7 to 1.0 of the
-// multiply-add chain's, denormal operands included)
+// conversions and a multiply-add each (products exact, fp32 sums, denormals kept; against float64 its error is 0.96
+// to 0.97 of the multiply-add chain's for normal operands)
 __device__ __forceinline__ float dot_vec(const bf16x8& a, const bf16x8& b, float c) {
   typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
@@ -459,9 +459,9 @@ template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
   }
   // load_nomask for a loop over tiles of one tensor: where a thread's rows lie relative to the tile's first is the same for
   // every full tile and worked out again only where the row count changes (a uniform branch with no load in it).  Each row's
-  // product with its 64-bit stride and the clamp cost 50 cycles of the issuing wave per load (K = V = 128: k_state_bwd 76 -> 68 us at
-  // 64 pairs of 64 chunks, k_gdn_state_bwd 51 -> 49 at 32 pairs of 32, k_gdn_wy_fwd 60 -> 58.5; no change in the
-  // register-resident forward pass and the chunk-parallel backward kernels, which keep load_nomask).
+  // product with its 64-bit stride and the clamp cost 50 cycles of the issuing wave per load (K = V = 128: k_state_bwd 84 -> 77 us at
+  // 64 pairs of 64 chunks, k_gdn_state_bwd 53 -> 51 at 32 pairs of 32; no change in the register-resident forward pass, the
+  // WY preparation and the chunk-parallel backward kernels, which keep load_nomask).
   struct Rows { int64_t at[PASSES]; int n; };
   static __device__ __forceinline__ void load_rows(Regs& r, Rows& o, const T* __restrict__ src, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     if (nvalid != o.n) {
@@ -479,7 +479,7 @@ template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
   }
   // The same with one offset kept (first_row: that of the thread's row in the first pass) for loops without the registers for
   // all: the passes of a full tile lie a scalar apart, a partial one takes load_nomask (k_state_fwd_b: 97 -> 90 us forward-only,
-  // 120 -> 109 saving, 64 pairs of 64 chunks).
+  // 117 -> 112 saving, 64 pairs of 64 chunks).
   static __device__ __forceinline__ int64_t first_row(int64_t row_stride, int tid = threadIdx.x & (NT - 1)) {
     return ((int64_t)(tid / VPR) * row_stride + (tid % VPR) * VEC) * (int64_t)sizeof(T);
   }

@@ -38,7 +38,7 @@
 //     (window 2) and k (window 3), and slices 0, 1 of the next item during b .. d
 //   one slice buffer:  [R(0)] D(0) R(1) D(1) .. D(NS-1) | A | b c d | R(0) of the next item
 // What bounds it (8192 items, K = V = 128, 16 heads): with its loads served by the L2 and nothing stored 237 us, the compute
-// waves alone 167, the loader waves alone 174; with memory, the loaders alone 304 (5.8 TB/s).  So the loader waves: their
+// waves alone 167, the loader waves alone 174; with memory, the loaders alone 347, and 304 (5.8 TB/s) with their arithmetic out.  So the loader waves: their
 // work between two requests was cut to dot-product instructions for <dZ, v> and <S, dS'>, one set of divisions
 // per item, and the compute waves' LDS traffic (reads and 2-byte accesses of stage 2) to a third.  370 -> 350 us; where
 // memory binds less 50 -> 43 (2048 x 2 tokens), 97 -> 78 (K = V = 64, 4096 x 4).

@@ -42,10 +42,11 @@
 namespace lmoe {
 
 // Time stamps of the traced instance (TRACE = true): every team's leading wave notes the shader clock when it
-// arrives at and leaves the two barriers of a chunk and at a few points in between, into LDS (a global store would
-// stall the traced wave at the issue); the traced work-group copies them out when it ends.  Slots: 0 consumer wave,
-// 1 helper wave, 2 loader team 1, 3 loader team 2; marks per (slot, chunk): see lmoe_trace_gdn_state_fwd in
-// include/lmoe.h.  Chunks beyond TRACE_CHUNKS are not recorded.
+// enters the window of a chunk, when it arrives at and leaves the barrier at its end and at a few points in between, into LDS
+// (a global store would stall the traced wave at the issue); the traced work-group copies them out when it ends.
+// Slots: 0 consumer wave, 1 helper wave, 2 loader team 1, 3 loader team 2; marks per (slot, chunk): see
+// lmoe_trace_gdn_state_fwd in include/lmoe.h.  The first TRACE_LDS_CHUNKS chunks are recorded (what the LDS has room for beside
+// the tiles); the caller's buffer has TRACE_CHUNKS, zero where nothing was recorded.
 constexpr int TRACE_CHUNKS = 128, TRACE_MARKS = 8, TRACE_SLOTS = 4, TRACE_LDS_CHUNKS = 48;
 
 // A fragment of k^T for the state block mi (see the numbering above): contraction = tokens k0 + 8 g .. + 7 (rows of
@@ -150,7 +151,8 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
     };
     // this work-group's share of the rows of P (formed by the helpers, the whole matrix in s_p): 64 / NVS rows, the same
     // number of bytes from every thread (128 threads with 16 bytes each and 128 that repeated them, so that no store sat
-    // behind a branch, wrote P twice: 51 MB more of 603 at B=4 T=8192 H=16, and the writes bound a saving call)
+    // behind a branch, wrote part of P twice: 33 MB more of the 604 written at B=4 T=8192 H=16, by the counters, and the writes bound a
+    // saving call)
     constexpr int PROWS = CH / NVS, PVEC = CH * PROWS / NTHR;
     typedef T pvec __attribute__((ext_vector_type(PVEC)));
     const int pidx = threadIdx.x & (NTHR - 1);

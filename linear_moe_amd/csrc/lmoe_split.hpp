@@ -147,10 +147,11 @@ template <bool CUT> __device__ __forceinline__ PassItem pass_item_dense(const lm
 // were measured to take (us, K = V = 128, delta rule; half of it per chunk at K = V = 64):
 //   ordinary pass   1.7 per chunk up to 64 work-groups, 2.1 beyond, 2.2 on a full GPU
 //   step 1          7 + 3.3 per chunk        step 2   4 + 0.65 per fine segment       step 3   1 + 2.2 per chunk
-// These are the passes with two and three barriers per chunk the rule was fitted to.  The forward pass now takes 1.35 per
-// chunk (forward-only, up to 256 work-groups) to 1.6, and a cut it chooses still wins (whole -> cut, K = V = 128, one sequence,
-// forward / reverse): 4 heads 24 chunks 35 -> 29 / 36 -> 29; 16 heads 32 chunks 46 -> 39 / 47 -> 39, 47 chunks 65 -> 47 / 68 -> 48,
-// 128 chunks 169 -> 86 / 181 -> 93; with smaller constants 8 heads of 24 chunks (35 -> 29) would be left whole.
+// These are the passes with two and three barriers per chunk the rule was fitted to; the forward pass now takes 1.35 to 1.6 per
+// chunk.  Its cuts still win where the kernels count (one pass replayed as a graph, whole -> cut, K = V = 128: training 16 pairs
+// of 32 chunks 136 -> 124, 20 of 38 163 -> 162, 16 of 256 920 -> 615; forward 16 pairs of 47 chunks 80 -> 63, 8 of 24 46 -> 39;
+// all 324 calls of a sweep over pairs and lengths by a factor of 1.08 to 3.3).  A training call of up to 48 chunks that the
+// host issues one by one is bound by the host, and the cut's launches show (8 pairs of 24 chunks 125 -> 140).
 inline Split plan_split(const lmoe_args& a, int slices) {
   Split s = {};
   if (a.dtype != LMOE_BF16 || a.N < 1 || a.T < 1) return s;
