@@ -187,6 +187,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
   // stall at the issue (measured: 1.4 us of an 11 us item).  Always requested, item index clamped: a load
   // that is skipped on some path would make the compiler drain all outstanding loads at every use.
   typename IOK::Regs rk;
+  typename IOK::Rows ok = {};
   typename IOV::Regs rv;
   RowFrags<T, K> fq;
   uint32_t graw, braw;
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(NTHR, (sizeof(T) == 2 ? (SAVE ? 3 : 2) : 1)) void k
   };
   // q enters only as the A operand of q k^T: each wave takes its 16 rows straight into fragments
   auto issue_q = [&](const Item& I) { if constexpr (!LEAN) fq.load(row_ptr<T>(a.q, I.ci.b, I.ci.tok, I.h), a.q.st, 16 * wv, I.ci.len - 1); };
-  auto issue_k = [&](const Item& I) { IOK::load_nomask(rk, row_ptr<T>(a.k, I.ci.b, I.ci.tok, I.h), a.k.st, I.ci.len); };
+  auto issue_k = [&](const Item& I) { IOK::load_rows(rk, ok, row_ptr<T>(a.k, I.ci.b, I.ci.tok, I.h), a.k.st, I.ci.len); };
   auto issue_v = [&](const Item& I) {
     if constexpr (!LEAN) IOV::load_nomask(rv, row_ptr<T>(a.v, I.ci.b, I.ci.tok, I.h), a.v.st, I.ci.len);
   };
