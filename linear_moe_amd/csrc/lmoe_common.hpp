@@ -460,8 +460,8 @@ template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
   // load_nomask for a loop over tiles of one tensor: where a thread's rows lie relative to the tile's first is the same for
   // every full tile and worked out again only where the row count changes (a uniform branch with no load in it).  Each row's
   // product with its 64-bit stride and the clamp cost 50 cycles of the issuing wave per load (K = V = 128: k_state_bwd 84 -> 77 us at
-  // 64 pairs of 64 chunks, k_gdn_state_bwd 53 -> 51 at 32 pairs of 32; no change in the register-resident forward pass, the
-  // WY preparation and the chunk-parallel backward kernels, which keep load_nomask).
+  // 64 pairs of 64 chunks, k_gdn_state_bwd 53 -> 51 at 32 pairs of 32, k_gdn_wy_fwd 63.2 -> 62.5 for 8192 items, 238 -> 234 for
+  // 32768; no change in the register-resident forward pass and the chunk-parallel backward kernels, which keep load_nomask).
   struct Rows { int64_t at[PASSES]; int n; };
   static __device__ __forceinline__ void load_rows(Regs& r, Rows& o, const T* __restrict__ src, int64_t row_stride, int nvalid, int tid = threadIdx.x & (NT - 1)) {
     if (nvalid != o.n) {
