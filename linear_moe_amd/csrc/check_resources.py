@@ -35,6 +35,8 @@ ANY_TYPE = ("k_state_bwd",)
 FLOORS = (
     # the instances whose kept places (last argument) cost the second work-group: launched where there is one per CU at most
     (re.compile(r"k_state_bwdI(DF16bLi128ELi\d+ELi64ELi1|fLi128ELi\d+ELi16ELi0)ELb[01]ELb1EE"), 2),
+    # 4-byte elements at K = 64, without the kept places: three work-groups per CU
+    (re.compile(r"k_state_bwdIfLi64ELi\d+ELi16ELi0ELb[01]ELb0EE"), 6),
     (re.compile(r"k_gla_bwd_dqkgIDF16b(DF16b|f)Li64E"), 4),
 )
 FIELDS = {"ScratchSize [bytes/lane]": "scratch", "VGPRs Spill": "vspill", "Occupancy [waves/SIMD]": "occ",

@@ -35,16 +35,18 @@ template <typename T, int K, int V> struct StateBwd {
   }
   template <int BVX, bool CUT> static void launch(const lmoe_args& a, const Split& sp, hipStream_t st) {
     const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BVX)), block(2 * NTHR);
-    // Rows' places in registers (KEPT) are 12 to 17 of them at K = 128, and with 4-byte elements and in the wide slices of the
-    // normalised pass they cost a CU its second work-group.  That matters where the launch has one: more work-groups
-    // than CUs, without and with them (us): 4-byte, 64 pairs of 32 chunks 95 and 121, 24 pairs of 128 chunks cut 161 and
-    // 180; normalised, 256 pairs of 16 chunks 67 and 74.  With up to one per CU they gain, as they do elsewhere: 4-byte,
-    // 32 pairs of 128 chunks 242 and 228; normalised, 128 pairs of 32 chunks 76 and 72.
-    const bool second = grid.x > (unsigned)cu_count();
+    // Rows' places in registers (KEPT) are 10 to 17 of them, and with 4-byte elements and in the wide slices of the
+    // normalised pass (K = 128) they cost a CU its last work-group: the second at K = 128, the third at K = 64 with 4-byte elements.
+    // That matters where the launch has one, without and with them (us): K = 128, more work-groups than CUs: 4-byte, 64 pairs of
+    // 32 chunks 95 and 121, 24 pairs of 128 chunks cut 161 and 180; normalised, 256 pairs of 16 chunks 67 and 74.  K = 64, 4-byte,
+    // more than two per CU (whole backward): 96 pairs of 32 chunks, V = 128, 382 and 406, 384 of 16, V = 64, 459 and 466.
+    // With fewer they gain, as they do elsewhere: K = 128, 4-byte, 32 pairs of 128 chunks 242 and 228; normalised, 128 pairs
+    // of 32 chunks 76 and 72; K = 64, 4-byte, 128 pairs of 32 chunks, V = 64, 319 and 316.
+    const bool last = grid.x > (unsigned)(cu_count() * (K == 128 ? 1 : 2));
     if constexpr (sizeof(T) == 2) {        // the pass behind the normalised output exists for 2-byte elements
       if (a.normalize == 1) {
         if constexpr (K == 128 && BVX == 64) {
-          if (second) {
+          if (last) {
             hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 1, CUT, false>), grid, block, 0, st, a, sp);
             return;
           }
@@ -57,8 +59,8 @@ template <typename T, int K, int V> struct StateBwd {
         return;
       }
     }
-    if constexpr (sizeof(T) == 4 && K == 128) {
-      if (second) {
+    if constexpr (sizeof(T) == 4) {
+      if (last) {
         hipLaunchKernelGGL((k_state_bwd<T, K, V, BVX, 0, CUT, false>), grid, block, 0, st, a, sp);
         return;
       }

@@ -200,17 +200,17 @@ def test_dv_of_the_fused_backward_kernel_equals_the_kernel_of_its_own(cuda, B, H
 
 
 @pytest.mark.parametrize("V", [64, 128])
-@pytest.mark.parametrize("normalized", [False, True])
-def test_reverse_pass_on_both_sides_of_one_work_group_per_cu(cuda, V, normalized):
+@pytest.mark.parametrize("K,normalized", [(128, False), (128, True), (64, False)])
+def test_reverse_pass_on_both_sides_of_the_last_work_group_of_a_cu(cuda, V, K, normalized):
     """The reverse pass takes another instance from the first work-group beyond one per CU on (K = 128; 4-byte elements,
-    V slices of 16 columns, and the normalised pass with slices of 64): the same instructions on other registers, so the
-    heads that both launches hold get the same bits."""
+    V slices of 16 columns, and the normalised pass with slices of 64) or beyond two (K = 64, 4-byte): the same instructions
+    on other registers, so the heads that both launches hold get the same bits."""
     import linear_moe_amd as L
     cus = torch.cuda.get_device_properties(cuda).multi_processor_count
-    H1 = cus // (V // (64 if normalized else 16))           # heads of one work-group per CU
+    H1 = cus * (128 // K) // (V // (64 if normalized else 16))           # heads of as many work-groups
     dt = torch.bfloat16 if normalized else torch.float32
-    x = {n: (gen(80 + i, 1, H1 + 8, 130, D).abs() if normalized else gen(80 + i, 1, H1 + 8, 130, D)).to(cuda, dt)
-         for i, (n, D) in enumerate((("q", 128), ("k", 128), ("v", V), ("do", V)))}
+    x = {n: (gen(80 + i, 1, H1 + 8, 130, d).abs() if normalized else gen(80 + i, 1, H1 + 8, 130, d)).to(cuda, dt)
+         for i, (n, d) in enumerate((("q", K), ("k", K), ("v", V), ("do", V)))}
 
     def grads(H):
         ls = [x[n][:, :H].contiguous().requires_grad_() for n in ("q", "k", "v")]
