@@ -1072,8 +1072,10 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   const float* sB = sBw;
   // dA, q, k of the pairwise loops and the epilogue, from whichever tiles this layout keeps
   auto Pm = [&](int r, int j) { if constexpr (SUB) return ET<T>::to_f(tDA[r * LDC + j]); else return smF[B_DP + r * LDP + j]; };
-  auto Qm = [&](int r, int c) { if constexpr (SUB) return ET<T>::to_f(tQ[r * LDK + c]); else return smF[B_Q + r * LDB + c]; };
-  auto Km = [&](int r, int c) { if constexpr (SUB) return ET<T>::to_f(tK[r * LDK + c]); else return smF[B_K + r * LDB + c]; };
+  typedef typename ET<T>::vec4 vec4;
+  static_assert(SUB || sizeof(T) == 4, "the tiles of the other layout are 4-byte");
+  auto Qm4 = [&](int r, int c) { if constexpr (SUB) return *(const vec4*)(tQ + r * LDK + c); else return *(const vec4*)(smF + B_Q + r * LDB + c); };
+  auto Km4 = [&](int r, int c) { if constexpr (SUB) return *(const vec4*)(tK + r * LDK + c); else return *(const vec4*)(smF + B_K + r * LDB + c); };
   // Intra-chunk sums through reference gates (see k_gla_intra_fwd).  Wave w owns sub-chunk w:
   //   dq rows:  e^{b_i - ref_w}  [ dA(rows of w, j < 16 w + 16) (k_j e^{ref_w - b_j}) ],   ref_w  = b_{16 w - 1} (0 for w = 0)
   //   dk rows:  e^{ref'_w - b_j} [ dA^T(rows of w, i >= 16 w)   (q_i e^{b_i - ref'_w}) ],  ref'_w = b_{16 w + 15}
@@ -1169,10 +1171,8 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
   } else {
     __syncthreads();
   }
-  const int jlo = SUB ? 16 * wv : 0, ihi = SUB ? 16 * wv + 16 : CH;   // range of the pairwise loops
   T* dqd = row_ptr<T>(a.dq, ci.b, ci.tok, h);
   T* dkd_g = row_ptr<T>(a.dk, ci.b, ci.tok, h);
-  typedef typename ET<T>::vec4 vec4;
   const int r = 16 * wv + (l & 15);                    // token of this lane
   const int ch = hf * (K / 2) + 4 * (l >> 4);          // first column of this lane
   constexpr int NG = NBH < 4 ? NBH : 4;
@@ -1205,14 +1205,17 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
         const int j = 16 * wv + jj;
         const float pq = Pm(r, j), pk = Pm(j, r);
 #pragma unroll
-        for (int n4 = 0; n4 < NG; ++n4)
+        for (int n4 = 0; n4 < NG; ++n4) {
+          const int cc = 16 * (nh + n4) + ch;
+          const vec4 kj = Km4(j, cc), qj = Qm4(j, cc);
+          const f32x4 bj = *(const f32x4*)&sB[j * LDB + cc];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const int cc = 16 * (nh + n4) + ch + i;
-            const float e = texp_scaled<T>(-fabsf(brv[n4][i] - sB[j * LDB + cc] * TEXP_PRESCALE<T>));
-            sqv[n4][i] += pq * Km(j, cc) * e;
-            skv[n4][i] += pk * Qm(j, cc) * e;
+            const float e = texp_scaled<T>(-fabsf(brv[n4][i] - bj[i] * TEXP_PRESCALE<T>));
+            sqv[n4][i] += pq * ET<T>::to_f(kj[i]) * e;
+            skv[n4][i] += pk * ET<T>::to_f(qj[i]) * e;
           }
+        }
       }
     }
 #pragma unroll
@@ -1226,6 +1229,27 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
       if (wv > 0) refq = *(const f32x4*)&sB[(16 * wv - 1) * LDB + cc];
       const f32x4 refk = *(const f32x4*)&sB[(16 * wv + 15) * LDB + cc], br4 = *(const f32x4*)&sB[r * LDB + cc];
       const f32x4 er4 = *(const f32x4*)&s_er[wv * K + cc], ec4 = *(const f32x4*)&s_ec[wv * K + cc];
+      const vec4 q4 = Qm4(r, cc), k4 = Km4(r, cc);
+      f32x4 sqd = {0.f, 0.f, 0.f, 0.f}, skd = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (!SUB) {
+        // every pair of tokens (K = 128, 4-byte elements: no room for the stacked tile).  The exponentials bound it; one pass over
+        // the tokens serves the lane's four columns.  (Whole backward, B=2 T=2048 H=16 K=V=128, us: 517; with a pass per column,
+        // 4-byte reads and the lanes' 16 trip counts in each 683; that with the tokens along the accumulator's rows 617.)
+        for (int j = 0; j <= r; ++j) {
+          const float p = Pm(r, j);
+          const vec4 kj = Km4(j, cc);
+          const f32x4 bj = *(const f32x4*)&sB[j * LDB + cc];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sqd[i] += p * kj[i] * texp<T>(br4[i] - bj[i]);
+        }
+        for (int j = r; j < CH; ++j) {
+          const float p = Pm(j, r);
+          const vec4 qj = Qm4(j, cc);
+          const f32x4 bj = *(const f32x4*)&sB[j * LDB + cc];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) skd[i] += p * qj[i] * texp<T>(bj[i] - br4[i]);
+        }
+      }
       float qo[4], ko[4], kkp[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1238,10 +1262,10 @@ __global__ __launch_bounds__(2 * NTHR) __attribute__((amdgpu_waves_per_eu((K <= 
           sq_ += dqo[ni][0][i] * e1;
           sk_ += dko[ni][0][i] * e2;
         } else {
-          for (int j = jlo; j <= r; ++j) sq_ += Pm(r, j) * Km(j, cc + i) * texp<T>(br - sB[j * LDB + cc + i]);
-          for (int ii = r; ii < ihi; ++ii) sk_ += Pm(ii, r) * Qm(ii, cc + i) * texp<T>(sB[ii * LDB + cc + i] - br);
+          sq_ = sqd[i];
+          sk_ = skd[i];
         }
-        const float qv = Qm(r, cc + i), kv = Km(r, cc + i);
+        const float qv = ET<T>::to_f(q4[i]), kv = ET<T>::to_f(k4[i]);
         const float ed = ec4[i] * e2;
         const float dqv = a.scale * (er4[i] * e1) * dqi[ni][0][i] + sq_;
         const float dkdv = dkd[ni][0][i] * ed;
