@@ -479,7 +479,7 @@ template <typename T, int ROWS, int COLS, int NT = NTHR> struct TileIO {
   }
   // The same with one offset kept (first_row: that of the thread's row in the first pass) for loops without the registers for
   // all: the passes of a full tile lie a scalar apart, a partial one takes load_nomask (k_state_fwd_b: 97 -> 90 us forward-only,
-  // 117 -> 112 saving, 64 pairs of 64 chunks).
+  // 117 -> 112 saving, 64 pairs of 64 chunks, K = V = 128).
   static __device__ __forceinline__ int64_t first_row(int64_t row_stride, int tid = threadIdx.x & (NT - 1)) {
     return ((int64_t)(tid / VPR) * row_stride + (tid % VPR) * VEC) * (int64_t)sizeof(T);
   }

@@ -403,8 +403,11 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
     // --------------------------------- loaders -------------------------------------------
     struct Pre { typename IOK::Regs rk, rq; typename IOV::Regs ru; uint32_t graw; int len; };
     Pre pre[3];                                              // register set = chunk % 3
-    // (slices of 64 columns at K = 128: no registers left for the offsets)
-    constexpr bool KEPT = !(K == 128 && BV == 64);
+    // (slices of 64 columns at K = 128: no registers left for the offsets.  K = 64: half the passes per tile, so the branch on a
+    // partial tile costs more than it saves: without and with the offsets, V = 64, 64 pairs of 64 chunks 46.4 and 48.7 us, packed
+    // 8192 x 8 33.5 and 35.0, V = 128, 32 pairs of 32 chunks 33.2 and 35.3; only where a saving call writes more than the
+    // memory-side cache holds they gained, 73.5 and 70.4.  The normalised pass gains: 64 pairs of 64 chunks 64.9 and 60.0)
+    constexpr bool KEPT = K == 128 ? BV != 64 : NORM;
     const int64_t ok = KEPT ? IOK::first_row(a.k.st) : 0, oq = KEPT ? IOK::first_row(a.q.st) : 0, ou = KEPT ? IOV::first_row(a.v.st) : 0;
     const bool gated = a.gate != LMOE_GATE_NONE && a.g.ptr != nullptr;
     const void* gptr = gated ? a.g.ptr : a.k.ptr;
