@@ -1,4 +1,5 @@
 // Instantiation and launch of the forward kernel of chunk_simple_gla, plus the toolkit self-test.
+#include <type_traits>
 #include "lmoe_launch.hpp"
 #include "lmoe_scalar_split.hpp"
 
@@ -58,12 +59,34 @@ Split launch_scalar_seg(const lmoe_args& a, bool bwd, hipStream_t st) {
 template <typename T, int K, int V, int BV, bool CUT> void launch_fwd_b(const lmoe_args& a, const Split& sp, hipStream_t st) {
   const dim3 grid(((pass_items(a, sp) * a.H + 7) / 8) * 8 * (V / BV)), block(3 * NTHR);
   long long* const no_trace = nullptr;
+  // Which loads (KEPT).  Without and with the kept offset, us.  It needs registers, which slices of 64 columns at K = 128 have
+  // not, and gives a partial tile a path of its own, so it pays in the full ones:
+  //   K = 128: 64 pairs of 64 chunks 97 and 90, 60 pairs of 400 tokens 13.9 and 13.6; but 16 pairs of 100 tokens 7.5 and 7.8, of
+  //   30 tokens 6.3 and 6.8, of 64 5.9 and 5.7
+  //   K = 64, half the loads per tile: the plain pass loses (V = 64, 64 pairs of 64 chunks 46.4 and 48.7, packed 8192 x 8 33.5 and
+  //   35.0; only saving calls that write more than the memory-side cache holds gained, V = 128, 64 pairs of 64 chunks 73.5 and
+  //   70.4).  The normalised one: 64 pairs of 64 chunks 64.9 and 60.0, 60 pairs of 250 tokens 8.3 and 8.4, of 192 7.3 and 7.0;
+  //   saving 60 pairs of 1000 tokens 20.2 and 20.3, of 400 11.7 and 11.9, of 640 14.7 and 14.5
+  const bool tail = a.cu_seqlens || a.T % CH;
+  const int tokens = a.cu_seqlens ? a.T / max(a.N, 1) : a.T;                    // of a sequence, on average
+  auto go = [&](auto save, auto norm) {
+    constexpr bool SAVE = decltype(save)::value, NORM = decltype(norm)::value;
+    if constexpr (!CUT && fwd_may_keep<NORM, K, BV>()) {
+      if (tail && tokens < (K == 128 ? 128 : SAVE ? 1024 : 256)) {
+        hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, SAVE, false, NORM, CUT, false>), grid, block, 0, st, a, sp, no_trace, -1);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, SAVE, false, NORM, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
+  };
+  typedef std::true_type yes;
+  typedef std::false_type no;
   if (a.normalize) {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, true, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, true, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
+    if (a.hs) go(yes(), yes());
+    else go(no(), yes());
   } else {
-    if (a.hs) hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, true, false, false, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
-    else hipLaunchKernelGGL((k_state_fwd_b<T, K, V, BV, false, false, false, CUT>), grid, block, 0, st, a, sp, no_trace, -1);
+    if (a.hs) go(yes(), no());
+    else go(no(), no());
   }
 }
 template <typename T, int K, int V> struct StateFwd {

@@ -286,7 +286,10 @@ constexpr int SFWD_TRACE_CHUNKS = 24, SFWD_TRACE_MARKS = 8, SFWD_TRACE_SLOTS = 3
 // op with one more value column of ones, carried beside the state as one more accumulator column (z = the sum of the
 // keys of the chunks before, fp32 in LDS and, for the backward, in zs) and formed by every V slice for itself:
 // consumers z += k^T 1, output team q z and the row sums of P as two more products against a fragment of ones.
-template <typename T, int K, int V, int BV, bool SAVE, bool TRACE = false, bool NORM = false, bool CUT = false>
+//
+// KEPT: the loaders keep the offset of a thread's first row (TileIO::load_from; which calls take it: launch_fwd_b).
+template <bool NORM, int K, int BV> constexpr bool fwd_may_keep() { return K == 128 ? BV != 64 : NORM; }
+template <typename T, int K, int V, int BV, bool SAVE, bool TRACE = false, bool NORM = false, bool CUT = false, bool KEPT = fwd_may_keep<NORM, K, BV>()>
 __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   static_assert(sizeof(T) == 2, "2-byte elements");
   static_assert(!CUT || BV < 64, "wide slices fill the CUs: never cut along T");
@@ -403,11 +406,6 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
     // --------------------------------- loaders -------------------------------------------
     struct Pre { typename IOK::Regs rk, rq; typename IOV::Regs ru; uint32_t graw; int len; };
     Pre pre[3];                                              // register set = chunk % 3
-    // (slices of 64 columns at K = 128: no registers left for the offsets.  K = 64: half the passes per tile, so the branch on a
-    // partial tile costs more than it saves: without and with the offsets, V = 64, 64 pairs of 64 chunks 46.4 and 48.7 us, packed
-    // 8192 x 8 33.5 and 35.0, V = 128, 32 pairs of 32 chunks 33.2 and 35.3; only where a saving call writes more than the
-    // memory-side cache holds they gained, 73.5 and 70.4.  The normalised pass gains: 64 pairs of 64 chunks 64.9 and 60.0)
-    constexpr bool KEPT = K == 128 ? BV != 64 : NORM;
     const int64_t ok = KEPT ? IOK::first_row(a.k.st) : 0, oq = KEPT ? IOK::first_row(a.q.st) : 0, ou = KEPT ? IOV::first_row(a.v.st) : 0;
     const bool gated = a.gate != LMOE_GATE_NONE && a.g.ptr != nullptr;
     const void* gptr = gated ? a.g.ptr : a.k.ptr;

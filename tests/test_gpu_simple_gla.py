@@ -218,3 +218,21 @@ def test_reverse_pass_on_both_sides_of_the_last_work_group_of_a_cu(cuda, V, K, n
         return torch.autograd.grad(o, ls, x["do"][:, :H].contiguous())
     for a, b in zip(grads(H1), grads(H1 + 8)):
         assert torch.equal(a, b[:, :H1]) and a.abs().max() > 0
+
+
+@pytest.mark.parametrize("K,normalized,save,T", [(128, False, False, 128), (128, False, True, 128), (128, True, True, 128),
+                                                 (64, True, False, 256), (64, True, True, 1024)])
+@pytest.mark.parametrize("V", [64, 128])
+def test_forward_pass_on_both_sides_of_the_kept_offsets(cuda, V, K, normalized, save, T):
+    """Below T tokens and with a partial last chunk the pass of 2-byte elements takes the instance that works out every load's
+    place, from T on the one that keeps an offset: the same loads and products, so a token gets the same bits in both."""
+    import linear_moe_amd as L
+    x = {n: gen(90 + i, 1, 4, T, d) for i, (n, d) in enumerate((("q", K), ("k", K), ("v", V)))}
+    x = {n: (t.abs() if normalized else t).to(cuda, torch.bfloat16) for n, t in x.items()}
+
+    def out(n):
+        return L.chunk_linear_attn(*(t[:, :, :n].contiguous().requires_grad_(save) for t in x.values()), normalize=normalized)[0]
+    want = out(T)
+    for n in (T - 1, T - 30):
+        assert torch.equal(out(n), want[:, :, :n])
+    assert want.abs().max() > 0
