@@ -18,6 +18,7 @@ import sys
 # preparation two or three work-groups of 4 waves)
 GUARDED = {
     "k_state_fwd_b": 3,
+    "k_state_fwd_chunks": 3,  # K = 64: two work-groups of 12 waves per CU, see FLOORS
     "k_gdn_state_fwd": 3,
     "k_gdn_state_fwd_reg": 3,
     "k_gdn_state_bwd": 3,
@@ -30,13 +31,14 @@ GUARDED = {
     "k_gla_bwd_dqkg": 2,      # K = 64: two work-groups of 8 waves per CU, see FLOORS
     "k_bwd_dqkv": 2,          # one work-group of 8 waves per CU; its first version spilled loop-invariant lane arithmetic
 }
-ANY_TYPE = ("k_state_bwd",)
+ANY_TYPE = ("k_state_bwd", "k_state_fwd_chunks")
 # other minima of single instances
 FLOORS = (
     # the instances whose kept places (last argument) cost the second work-group: launched where there is one per CU at most
     (re.compile(r"k_state_bwdI(DF16bLi128ELi\d+ELi64ELi1|fLi128ELi\d+ELi16ELi0)ELb[01]ELb1EE"), 2),
     # 4-byte elements at K = 64, without the kept places: three work-groups per CU
     (re.compile(r"k_state_bwdIfLi64ELi\d+ELi16ELi0ELb[01]ELb0EE"), 6),
+    (re.compile(r"k_state_fwd_chunksILi64E"), 6),
     (re.compile(r"k_gla_bwd_dqkgIDF16b(DF16b|f)Li64E"), 4),
 )
 FIELDS = {"ScratchSize [bytes/lane]": "scratch", "VGPRs Spill": "vspill", "Occupancy [waves/SIMD]": "occ",

@@ -385,3 +385,29 @@ def test_error_of_the_cut_behind_a_drop_of_v(cuda, monkeypatch, gated):
     assert cut[0] < TOL[torch.bfloat16]
     bound = 2 ** 0.5 if gated else 1.05
     assert cut[1] < bound * whole[1] and cut[2] < bound * whole[2]
+
+
+@pytest.mark.parametrize("B,T,H,K,V", [
+    (1, 1, 1, 64, 64), (2, 63, 3, 128, 64), (1, 64, 8, 64, 128), (1, 65, 2, 128, 128),      # one chunk, and one token more
+    (2, 500, 4, 64, 64), (1, 512, 8, 128, 128),            # seven waves with a chunk in front each, or eight of them
+    (1, 513, 2, 64, 64), (32, 192, 4, 64, 64),             # beyond eight chunks, and more pairs than the CUs take: the pass
+])
+@pytest.mark.parametrize("gated", [False, True])
+def test_simple_gla_4_byte_chunk_by_chunk(cuda, B, T, H, K, V, gated):
+    """Short sequences in 4-byte elements: every chunk sums up the state it starts from.  Both layouts, a gate of 2-byte
+    elements; the states saved for the backward are those of the chunks."""
+    from linear_moe_amd import chunk_simple_gla
+    ins = dict(q=gen(7500, B, T, H, K), k=gen(7501, B, T, H, K) * K ** -0.5, v=gen(7502, B, T, H, V), h0=gen(7505, B, H, K, V) * 0.3)
+    if gated:                                               # (representable in either type)
+        ins["g"] = (-F.softplus(gen(7503, B, T, H)) * 0.01).bfloat16().float()
+    do, dht = gen(7506, B, T, H, V), gen(7507, B, H, K, V)
+    check(lambda q, k, v, h0, g=None: naive.naive_recurrent_simple_gla(q, k, v, g, None, h0, True, None, False),
+          lambda q, k, v, h0, g=None: chunk_simple_gla(q, k, v, g, None, h0, True, None, False),
+          ins, do, dht, cuda, torch.float32)
+    d = {n: x.to(cuda) for n, x in ins.items()}
+    hf = {n: x.transpose(1, 2).contiguous() if n != "h0" else x for n, x in d.items()}
+    o, _ = chunk_simple_gla(d["q"], d["k"], d["v"], d.get("g"), None, d["h0"], False, None, False)
+    of, _ = chunk_simple_gla(hf["q"], hf["k"], hf["v"], hf.get("g"), None, hf["h0"])
+    assert torch.equal(of.transpose(1, 2), o)
+    if gated:
+        assert torch.equal(chunk_simple_gla(d["q"], d["k"], d["v"], d["g"].bfloat16(), None, d["h0"], False, None, False)[0], o)
