@@ -12,6 +12,7 @@ import ctypes as C
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import Args, Tensor4, CHUNK
@@ -210,6 +211,10 @@ class SeqPlan:
                 offs = offs.to(torch.int64)
             offs = offs.contiguous()
             self.N, self.NT = N, nt_max
+            r = native_call("seq_tables", "chunk tables", offs, T, SEQ_TABLES_MAX)
+            if r is not None:
+                self.cu, self.chunk_map, self.seq_chunk0, self.seq_order, self.nt_dev = r
+                return
             tables = torch.empty(2 * nt_max + 3 * N + 3, dtype=torch.int32, device=dev)
             cmap, self.cu, self.seq_chunk0, self.nt_dev, order = tables.split([2 * nt_max, N + 1, N + 1, 1, N])
             self.chunk_map = cmap.view(nt_max, 2)
@@ -378,7 +383,9 @@ def stream_ptr() -> int:
 # The steps of a call (checks, argument block, allocations, the call of the library) in native code, for the calls that
 # need no conversion, copy or refusal: csrc/lmoe_native.cpp.  It returns None for any other call, which then takes the
 # steps in Python.  (Host time of a call, small sizes on one machine: one token 20 -> 8 us; forward 23 -> 15; forward and
-# backward of the gated delta rule 143 -> 90, of which autograd itself is 27 to 60.)
+# backward of the gated delta rule 143 -> 90, of which autograd itself is 27 to 60.  With the neighbours on it too: a mixer's
+# training step of gates, core and output gate 302 -> 229, one of a mixture of memories 336 -> 299; forward-only calls, which
+# need no node of the graph (no_node): chunk_linear_attn 14 -> 8, chunk_gated_delta_rule 19 -> 13.5.)
 def native(fn: str, what: str, op: int, q, *args):
     """``forward``, ``backward``, ``intact`` or ``recurrent`` of the native path: its results, or None (not a call for it)."""
     if not q.is_cuda:
@@ -387,6 +394,25 @@ def native(fn: str, what: str, op: int, q, *args):
     if type(r) is int:
         _lib.check(r, what)
     return r
+
+
+def native_call(fn: str, what: str, x, *args):
+    """The same for the functions of the neighbours (gates, prologue, output gate, routing), whose first argument is a tensor."""
+    if not x.is_cuda:
+        return None
+    r = getattr(_lib.native(), fn)(x, *args, stream_ptr())
+    if type(r) is int:
+        _lib.check(r, what)
+    return r
+
+
+def no_node(*xs) -> bool:
+    """Whether a call needs no node of the autograd graph: no gradient is wanted, and nothing is at work (a transform, forward-mode
+    differentiation) that has to see the op as a function of autograd and refuses it there.  Its steps then run without
+    one (5 us of a call that takes the GPU 9)."""
+    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in xs):
+        return False
+    return not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0
 
 
 def ptr(x: Optional[torch.Tensor]):

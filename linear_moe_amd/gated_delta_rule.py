@@ -17,7 +17,7 @@ import torch
 from . import _lib
 from .l2norm import l2_norm
 from ._host import (HEAD_DIMS, WIDE_V, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    came_back, inputs_came_back, native, no_tokens, ptr, stash, stream_ptr, unstash)
+                    came_back, inputs_came_back, native, no_node, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 def _scalar_dt(x: torch.Tensor) -> int:
@@ -113,6 +113,17 @@ class GDNCall:
         self.seg_ws = None
         return o, ht
 
+    def came_from_native(self, q, k, v, g, beta, scale, kept):
+        """What the native path keeps of a dense call on the v block of a projection (``lmoe_native.cpp``, mixer_forward)."""
+        self.saved = (q, k, v, g, beta, None, *kept)
+        self.plan, self.dims, self.head_first, self.scale = None, None, False, scale
+        self.has_h0, self.v_act, self.seg_ws = False, True, None
+
+    def backward_args(self, do, dht):
+        """The arguments of the native backward, but for the last (``extra``)."""
+        q, k, v, g, beta, h0, *kept = self.saved
+        return (self.OP, q, k, v, g, beta, h0, self.plan and self.plan.tables, self.scale, do, dht, self.head_first, tuple(kept))
+
     def _cut(self, lib, a, dev, save=False, seg_p=None):
         """The buffers of a call whose sequences are cut along T (``lmoe_args.seg_ws``; ``seg_p``, which a call that
         saves hands to its backward), or none."""
@@ -141,8 +152,7 @@ class GDNCall:
         dims = None
         if not self.keep:
             raw, what = (None, None) if qk_raw is None else qk_raw, "chunk_gated_delta_rule backward"
-            args = (self.OP, q, k, v, g, beta, h0, ctx.plan and ctx.plan.tables, ctx.scale, do, dht, head_first, (hs, tinv, pmat, gcum,
-                    vnew, seg_p), (ctx.v_act, dq_out, dk_out, dv_out, *raw, float(qk_eps)))
+            args = (*self.backward_args(do, dht), (ctx.v_act, dq_out, dk_out, dv_out, *raw, float(qk_eps)))
             if q.dtype != torch.float32:
                 r = native("backward", what, *args)
                 if r is not None:
@@ -271,5 +281,7 @@ def chunk_gated_delta_rule(
     r = no_tokens(q, k, v, head_first, cu_seqlens, initial_state, output_final_state, wide_v=True)
     if r is not None:
         return r
+    if no_node(q, k, v, g, beta, initial_state):
+        return GDNCall().forward(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, head_first, save=False)
     return _ChunkGatedDeltaRule.apply(q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                                       head_first)

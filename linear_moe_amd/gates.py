@@ -15,7 +15,7 @@ import math
 import torch
 
 from . import _lib
-from ._host import stream_ptr
+from ._host import native_call, stream_ptr
 
 
 def _dt(t):
@@ -27,6 +27,11 @@ def _dt(t):
 class _GdnGates(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, A_log, dt_bias):
+        ctx.pdt = (A_log.dtype, dt_bias.dtype)
+        r = native_call("gates_forward", "gdn_gates", a, b, A_log, dt_bias)
+        if r is not None:
+            ctx.save_for_backward(a, b, A_log, dt_bias)
+            return r
         if not a.is_cuda:
             raise RuntimeError("linear_moe_amd ops are GPU only (no CPU fallback)")
         if a.shape != b.shape or a.dtype != b.dtype:
@@ -43,12 +48,14 @@ class _GdnGates(torch.autograd.Function):
         _lib.check(lib.lmoe_gdn_gates_fwd(ac.data_ptr(), bc.data_ptr(), Af.data_ptr(), Bf.data_ptr(), g.data_ptr(),
                                           beta.data_ptr(), rows, H, _dt(a), stream_ptr()), "gdn_gates")
         ctx.save_for_backward(ac, bc, Af, Bf)
-        ctx.pdt = (A_log.dtype, dt_bias.dtype)
         return g, beta
 
     @staticmethod
     def backward(ctx, dg, dbeta):
         ac, bc, Af, Bf = ctx.saved_tensors
+        r = native_call("gates_backward", "gdn_gates backward", ac, bc, Af, Bf, dg, dbeta)
+        if r is not None:
+            return (*r[:2], r[2].to(ctx.pdt[0]), r[3].to(ctx.pdt[1]))
         lib = _lib.load()
         H = ac.shape[-1]
         rows = ac.numel() // H

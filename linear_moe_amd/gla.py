@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._host import (HEAD_DIMS, seq_plan, _aligned, _check_inputs, _desc, _state_check, base_args, by_head_dim_blocks,
-                    came_back, cut_workspace, inputs_came_back, native, no_tokens, ptr, stash, stream_ptr, unstash)
+                    came_back, cut_workspace, inputs_came_back, native, no_node, no_tokens, ptr, stash, stream_ptr, unstash)
 
 
 class GLACall:
@@ -172,4 +172,6 @@ def chunk_gla(
     r = no_tokens(q, k, v, head_first, cu_seqlens, initial_state, output_final_state)
     if r is not None:
         return r
+    if no_node(q, k, v, g, initial_state):
+        return GLACall().forward(q, k, v, g, scale, initial_state, output_final_state, cu_seqlens, head_first, save=False)
     return _ChunkGLA.apply(q, k, v, g, scale, initial_state, output_final_state, cu_seqlens, head_first)

@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._host import stash, stream_ptr, unstash
+from ._host import native_call, stash, stream_ptr, unstash
 
 
 def _dt(x):
@@ -71,18 +71,23 @@ class _GDNMixerCore(torch.autograd.Function):
             raise ValueError(f"gdn_mixer_core: {tuple(qkv.shape)} is not [T, B, {H} heads x 3 x {D}]")
         if D not in (64, 128):
             raise ValueError(f"gdn_mixer_core: head dimension {D} unsupported (64 or 128)")
+        call = GDNCall()
+        ctx.call, ctx.dims, ctx.eps, ctx.dt, ctx.shape = call, (T, B, H, D), eps, dt, qkv.shape
+        save = any(ctx.needs_input_grad[:3])
+        r = native_call("mixer_forward", "gdn_mixer_core", qkv, g, beta, H, D, eps, scale, save)
+        if r is not None:
+            o, q, k, v, *kept = r
+            call.came_from_native(q, k, v, g, beta, scale, kept)
+            stash(ctx, call, qkv)
+            return o
         lib = _lib.load()
         x = qkv.contiguous()
         q, k = (torch.empty(B, T, H, D, dtype=qkv.dtype, device=qkv.device) for _ in range(2))
         _lib.check(lib.lmoe_gdn_qkv_prologue_fwd(x.data_ptr(), q.data_ptr(), k.data_ptr(), None, T, B, H, D, dt, eps,
                                                  stream_ptr()), "gdn_mixer_core prologue")
         v = x.view(T, B, H, 3 * D)[..., 2 * D:].transpose(0, 1)            # [B, T, H, D], strided: the op reads it in place
-        call = GDNCall()
-        o, _ = call.forward(q, k, v, g, beta, scale, None, False, None, False,
-                            save=any(ctx.needs_input_grad[:3]), v_act=True)
-        ctx.call = call
+        o, _ = call.forward(q, k, v, g, beta, scale, None, False, None, False, save=save, v_act=True)
         stash(ctx, call, x)
-        ctx.dims, ctx.eps, ctx.dt, ctx.shape = (T, B, H, D), eps, dt, qkv.shape
         return o
 
     @staticmethod
@@ -92,11 +97,15 @@ class _GDNMixerCore(torch.autograd.Function):
         # the op writes all three blocks of the projection's gradient itself: dv as silu'(v) times its dv, dq and dk
         # through the backward of the L2 norm and of SiLU, applied to its dq, dk tiles on their way out, from the raw
         # rows of the projection
-        dx = torch.empty_like(x)
-        blocks = lambda t: [t.view(T, B, H, 3 * D)[..., i * D:(i + 1) * D].transpose(0, 1) for i in range(3)]
-        dxq, dxk, dxv = blocks(dx)
-        xq, xk, _ = blocks(x)
         try:
+            r = native_call("mixer_backward", "gdn_mixer_core backward", x, ctx.eps, *ctx.call.backward_args(do, None), None)
+            if r is not None:
+                (dx, dg, dbeta), g = r, ctx.call.saved[3]
+                return dx.view(ctx.shape), dg if dg is None else dg.to(g.dtype), dbeta, None, None, None, None
+            dx = torch.empty_like(x)
+            blocks = lambda t: [t.view(T, B, H, 3 * D)[..., i * D:(i + 1) * D].transpose(0, 1) for i in range(3)]
+            dxq, dxk, dxv = blocks(dx)
+            xq, xk, _ = blocks(x)
             _, _, _, dg, dbeta, _ = ctx.call.backward(do, None, dv_out=dxv, dq_out=dxq, dk_out=dxk, qk_raw=(xq, xk),
                                                       qk_eps=ctx.eps)
         finally:
@@ -124,6 +133,10 @@ def gdn_qkv_prologue(qkv: torch.Tensor, num_heads: int, head_dim: int, eps: floa
 class _SwishGateRelayout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, o, gate):
+        r = native_call("swish_forward", "swish_gate_relayout", o, gate)
+        if r is not None:
+            ctx.save_for_backward(o, gate)
+            return r[0]
         dt = _dt(o)
         if o.dim() != 4:
             raise ValueError("swish_gate_relayout: o must be [B, T, H, D]")
@@ -139,20 +152,22 @@ class _SwishGateRelayout(torch.autograd.Function):
         _lib.check(lib.lmoe_swish_gate_relayout_fwd(oc.data_ptr(), gc.data_ptr(), y.data_ptr(), T, B, W, dt, stream_ptr()),
                    "swish_gate_relayout")
         ctx.save_for_backward(oc, gc)
-        ctx.dims, ctx.dt, ctx.gshape = (T, B, W), dt, gate.shape
         return y
 
     @staticmethod
     def backward(ctx, dy):
         oc, gc = ctx.saved_tensors
-        T, B, W = ctx.dims
+        r = native_call("swish_backward", "swish_gate_relayout backward", oc, gc, dy)
+        if r is not None:
+            return r
+        B, T, W = oc.shape[0], oc.shape[1], oc.shape[2] * oc.shape[3]
         lib = _lib.load()
         dyc = dy.contiguous()
         do, dgate = torch.empty_like(oc), torch.empty_like(gc)
         _lib.check(lib.lmoe_swish_gate_relayout_bwd(oc.data_ptr(), gc.data_ptr(), dyc.data_ptr(), do.data_ptr(),
-                                                    dgate.data_ptr(), T, B, W, ctx.dt, stream_ptr()),
+                                                    dgate.data_ptr(), T, B, W, _dt(oc), stream_ptr()),
                    "swish_gate_relayout backward")
-        return do, dgate.view(ctx.gshape)
+        return do, dgate
 
 
 def swish_gate_relayout(o: torch.Tensor, o_gate: torch.Tensor) -> torch.Tensor:

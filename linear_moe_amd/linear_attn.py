@@ -12,6 +12,7 @@ from typing import Optional, Tuple
 
 import torch
 
+from ._host import HEAD_DIMS
 from .simple_gla import can_normalize, chunk_simple_gla, chunk_simple_gla_normalized, chunk_simple_gla_with_den
 
 
@@ -28,6 +29,9 @@ def chunk_linear_attn(
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """``_eps`` (not part of fla's signature): the epsilon of the normaliser, for the callers in this package whose
     reference functions carry their own (``based.py``)."""
+    if not normalize and type(q) is torch.Tensor and q.shape[-1] in HEAD_DIMS and (initial_state is None or
+                                                                                   initial_state.shape[-2] == q.shape[-1]):
+        return chunk_simple_gla(q, k, v, None, scale, initial_state, output_final_state, None, head_first)     # one block, as it is
     qb, kb = _key_blocks(q), _key_blocks(k)
     if [b.shape for b in qb] != [b.shape for b in kb]:
         raise ValueError("chunk_linear_attn: q and k must agree in shape")

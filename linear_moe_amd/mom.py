@@ -25,7 +25,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._host import stream_ptr
+from ._host import native_call, stream_ptr
 
 
 @dataclass
@@ -68,6 +68,10 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
     if selected_memories.dim() != 3:
         raise ValueError("selected_memories must be [B, S, topk]")
     B, S, topk = selected_memories.shape
+    if not check:
+        r = native_call("mom_plan", "mom_plan", selected_memories, num_memories, _cap(S, capacity))
+        if r is not None:
+            return _plan_of(r, B, S, topk, num_memories, capacity)
     dev = selected_memories.device
     sel = selected_memories.reshape(-1)                                        # flat (b, t, k)
     if check and sel.numel() and (int(sel.min()) < 0 or int(sel.max()) >= num_memories):
@@ -78,6 +82,20 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
         if plan is not None:
             return plan
     return _plan_by_sorting(sel.to(torch.int64), B, S, topk, num_memories, capacity)
+
+
+def _cap(S, capacity):
+    return -1 if capacity is None else max(0, min(math.ceil(S * capacity), 2 ** 31 - 1))
+
+
+def _plan_of(tables, B, S, topk, num_memories, capacity):
+    """The plan of the tables that the library's kernels have formed."""
+    cu, longest, offsets, src_token, src_choice, row_of = tables
+    T_total = B * S * topk
+    if capacity is not None:
+        T_total = int(cu[-1])                                                  # (the one read: how many survive)
+        src_token, src_choice = src_token[:T_total], src_choice[:T_total]
+    return MomPlan(B, S, topk, num_memories, T_total, src_token, src_choice, row_of, cu, longest, offsets)
 
 
 def _plan_native(sel, B, S, topk, num_memories, capacity):
@@ -94,16 +112,10 @@ def _plan_native(sel, B, S, topk, num_memories, capacity):
     wide = torch.empty(num_memories + 2, dtype=torch.int64, device=dev)
     counts, cu, src_token, src_choice, row_of = (torch.empty(k, dtype=torch.int32, device=dev)
                                                  for k in (ints, seqs + 1, n, n, n))
-    cap = -1 if capacity is None else max(0, min(math.ceil(S * capacity), 2 ** 31 - 1))
-    _lib.check(lib.lmoe_mom_plan(sel.data_ptr(), int(sel.dtype == torch.int64), B, S * topk, topk, num_memories, cap,
+    _lib.check(lib.lmoe_mom_plan(sel.data_ptr(), int(sel.dtype == torch.int64), B, S * topk, topk, num_memories, _cap(S, capacity),
                                  counts.data_ptr(), cu.data_ptr(), wide.data_ptr(), wide.data_ptr() + 8,
                                  src_token.data_ptr(), src_choice.data_ptr(), row_of.data_ptr(), stream_ptr()), "mom_plan")
-    T_total = n
-    if capacity is not None:
-        T_total = int(cu[-1])                                                  # (the one read: how many survive)
-        src_token, src_choice = src_token[:T_total], src_choice[:T_total]
-    return MomPlan(B, S, topk, num_memories, T_total, src_token, src_choice, row_of.view(B * S, topk), cu, wide[0],
-                   wide[1:])
+    return _plan_of((cu, wide[0], wide[1:], src_token, src_choice, row_of.view(B * S, topk)), B, S, topk, num_memories, capacity)
 
 
 def _plan_by_sorting(sel, B, S, topk, num_memories, capacity):
@@ -153,19 +165,25 @@ def _rows(x: torch.Tensor, n: int, what: str) -> torch.Tensor:
 class _Pack(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan):
+        ctx.plan, ctx.shape = plan, x.shape
+        r = native_call("mom_gather", "mom_pack", x, plan.B * plan.S, plan.src_token)
+        if r is not None:
+            return r[0]
         lib = _lib.load()
         x2 = _rows(x, plan.B * plan.S, "mom_pack")
         D = x2.shape[1]
         out = torch.empty(plan.T_total, D, dtype=x.dtype, device=x.device)
         _lib.check(lib.lmoe_mom_gather(x2.data_ptr(), plan.src_token.data_ptr(), None, out.data_ptr(), plan.T_total, D,
                                        _dt(x), stream_ptr()), "mom_pack")
-        ctx.plan, ctx.shape = plan, x.shape
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        lib = _lib.load()
         plan = ctx.plan
+        r = native_call("mom_combine", "mom_pack backward", dout, plan.T_total, plan.row_of, None, plan.B * plan.S, plan.topk)
+        if r is not None:
+            return r[0].view(ctx.shape), None
+        lib = _lib.load()
         d2 = dout.contiguous()
         D = d2.shape[1]
         dx = torch.empty(plan.B * plan.S, D, dtype=dout.dtype, device=dout.device)
@@ -177,6 +195,11 @@ class _Pack(torch.autograd.Function):
 class _Combine(torch.autograd.Function):
     @staticmethod
     def forward(ctx, y, w, plan):
+        ctx.plan, ctx.yshape, ctx.wshape, ctx.wdtype = plan, y.shape, w.shape, w.dtype
+        r = native_call("mom_combine", "mom_combine", y, plan.T_total, plan.row_of, w, plan.B * plan.S, plan.topk)
+        if r is not None:
+            ctx.save_for_backward(y, w)
+            return r[0].view((plan.B, plan.S) + tuple(y.shape[1:]))
         lib = _lib.load()
         y2 = _rows(y, plan.T_total, "mom_combine")
         D = y2.shape[1]
@@ -185,14 +208,18 @@ class _Combine(torch.autograd.Function):
         _lib.check(lib.lmoe_mom_combine(y2.data_ptr(), plan.row_of.data_ptr(), w2.data_ptr(), out.data_ptr(),
                                         plan.B * plan.S, plan.topk, D, _dt(y), stream_ptr()), "mom_combine")
         ctx.save_for_backward(y2, w2)
-        ctx.plan, ctx.yshape, ctx.wshape, ctx.wdtype = plan, y.shape, w.shape, w.dtype
         return out.view((plan.B, plan.S) + tuple(y.shape[1:]))
 
     @staticmethod
     def backward(ctx, dout):
-        lib = _lib.load()
         y2, w2 = ctx.saved_tensors
         plan = ctx.plan
+        r = native_call("mom_combine_backward", "mom_combine backward", y2, plan.T_total, plan.row_of, plan.src_choice, w2, dout,
+                        plan.B * plan.S, plan.topk)
+        if r is not None:
+            return r[0].view(ctx.yshape), r[1].view(ctx.wshape).to(ctx.wdtype), None
+        lib = _lib.load()
+        y2, w2 = y2.reshape(plan.T_total, -1), w2.reshape(plan.B * plan.S, plan.topk)
         D = y2.shape[1]
         g = dout.reshape(plan.B * plan.S, D).contiguous()
         # dy[row] = w[choice(row)] * dout[token(row)];  dw[t][k] = <dout[t], y[row_of[t][k]]>

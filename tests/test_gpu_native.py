@@ -378,3 +378,120 @@ def test_other_forms_same_bits(cuda, monkeypatch, form, T):
             out.append([*outs, *torch.autograd.grad(outs, ls, douts)])
     for a, b in zip(*out):
         assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b) and b.abs().max() > 0
+
+
+# ---- the neighbours of the ops ----
+def _neighbour_calls(cuda, B, T, H, D, dt):
+    """name -> (function of the leaves, leaves): the steps of a mixer around the op and of a mixture of memories"""
+    import linear_moe_amd as L
+    gen = torch.Generator(device=cuda).manual_seed(11)
+    rn = lambda *s: torch.randn(*s, generator=gen, device=cuda)
+    sel = torch.randint(0, 4, (B, T, 2), generator=gen, device=cuda)
+    plan = L.mom_plan(sel, 4)
+    calls = {"gates": (L.gdn_gates, (rn(B, T, H).to(dt), rn(B, T, H).to(dt), rn(H), rn(H))),
+             "swish": (L.swish_gate_relayout, (rn(B, T, H, D).to(dt), rn(T, B, H * D).to(dt))),
+             "pack": (lambda x: L.mom_pack(x, plan), (rn(B, T, H * D).to(dt),)),
+             "combine": (lambda y, w: L.mom_combine(y, plan, w), (rn(2 * B * T, H, D).to(dt), rn(B, T, 2).to(dt)))}
+    if dt == torch.bfloat16:
+        calls["mixer"] = (lambda x, g, beta: L.gdn_mixer_core(x, g, beta, H, D), (rn(T, B, H * 3 * D).to(dt), -rn(B, T, H).abs(), torch.sigmoid(rn(B, T, H)).to(dt)))
+        calls["mixer, no gate of its own type"] = (calls["mixer"][0], (rn(T, B, H, 3 * D).to(dt), -rn(B, T, H).abs().to(dt), torch.sigmoid(rn(B, T, H))))
+    return calls
+
+
+def _no_native(m):
+    import linear_moe_amd._host as host
+    import linear_moe_amd.gates as gates
+    import linear_moe_amd.layer_io as layer_io
+    import linear_moe_amd.mom as mom
+    for mod in (host, gates, layer_io, mom):
+        m.setattr(mod, "native_call", lambda *a: None)
+
+
+def _outputs(fn, leaves):
+    leaves = [x.detach().requires_grad_(True) for x in leaves]
+    outs = fn(*leaves)
+    outs = outs if isinstance(outs, tuple) else (outs,)
+    douts = [torch.randn(o.shape, generator=torch.Generator(device=o.device).manual_seed(3), device=o.device).to(o.dtype) for o in outs]
+    return [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, douts))
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,T,H,D", [(1, 1, 1, 64), (2, 130, 3, 128)])
+def test_neighbours_same_bits(cuda, monkeypatch, B, T, H, D, dt):
+    for name, (fn, leaves) in _neighbour_calls(cuda, B, T, H, D, dt).items():
+        with monkeypatch.context() as m:
+            _no_native(m)
+            ref = _outputs(fn, leaves)
+        with monkeypatch.context() as m:                   # (the Python steps would ask for it)
+            import linear_moe_amd._lib as _lib
+            m.setattr(_lib, "load", None)
+            got = _outputs(fn, leaves)
+        for a, b in zip(ref, got):
+            assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b), name
+
+
+def test_neighbours_in_other_forms(cuda, monkeypatch):
+    """Strided leaves, wider parameters: what the native path hands back runs as it did."""
+    B, T, H, D = 2, 70, 2, 64
+    for name, (fn, leaves) in _neighbour_calls(cuda, B, T, H, D, torch.bfloat16).items():
+        other = [x.transpose(-1, -2).contiguous().transpose(-1, -2) if x.dim() > 1 else x.double() for x in leaves]
+        with monkeypatch.context() as m:
+            _no_native(m)
+            ref = _outputs(fn, other)
+        for a, b in zip(ref, _outputs(fn, other)):
+            assert a.dtype == b.dtype and torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("is64", [True, False])
+@pytest.mark.parametrize("B,S,topk,E,capacity", [(1, 1, 1, 1, None), (2, 700, 2, 5, None), (3, 300, 2, 4, 0.4)])
+def test_routing_tables_same_bits(cuda, monkeypatch, is64, B, S, topk, E, capacity):
+    import linear_moe_amd as L
+    from linear_moe_amd._host import SeqPlan
+    sel = torch.randint(0, E, (B, S, topk), generator=torch.Generator().manual_seed(4)).to(torch.int64 if is64 else torch.int32).to(cuda)
+    with monkeypatch.context() as m:
+        _no_native(m)
+        ref = L.mom_plan(sel, E, capacity)
+        ref_seq = SeqPlan(1, max(ref.T_total, 1), ref.cu_seqlens, sel.device)
+    got = L.mom_plan(sel, E, capacity)
+    seq = SeqPlan(1, max(ref.T_total, 1), got.cu_seqlens, sel.device)
+    assert (got.T_total, got.B, got.S, got.topk) == (ref.T_total, B, S, topk)
+    for n in ("src_token", "src_choice", "row_of", "cu_seqlens", "max_len_dev", "mem_offsets_dev"):
+        a, b = getattr(ref, n), getattr(got, n)
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), n
+    nt = int(ref_seq.nt_dev)
+    assert (seq.N, seq.NT) == (ref_seq.N, ref_seq.NT) and torch.equal(seq.chunk_map[:nt], ref_seq.chunk_map[:nt])
+    for n in ("cu", "seq_chunk0", "nt_dev", "seq_order"):
+        a, b = getattr(ref_seq, n), getattr(seq, n)
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b)), n
+
+
+@pytest.mark.parametrize("name", ["gates", "swish", "combine", "mixer"])
+def test_neighbours_refuse_or_convert_what_hooks_hand_back(cuda, name):
+    """Another type of a saved tensor is not read as the type it had."""
+    fn, leaves = _neighbour_calls(cuda, 2, 70, 2, 64, torch.bfloat16)[name]
+    ref = _outputs(fn, leaves)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), lambda t: t):
+        for a, b in zip(ref, _outputs(fn, leaves)):
+            assert torch.equal(a, b)
+
+
+def test_calls_without_a_node_are_still_functions_of_autograd_for_transforms(cuda):
+    """Forward-only calls run without a node of the graph; what autograd refused it still refuses."""
+    import linear_moe_amd as L
+    from torch.autograd import forward_ad as fw
+    q, k, v = (torch.randn(1, 2, 70, 64, device=cuda).bfloat16() for _ in range(3))
+    ref = L.chunk_linear_attn(q, k, v, normalize=False)[0]
+    assert ref.grad_fn is None
+    with torch.no_grad():
+        o = L.chunk_linear_attn(q.requires_grad_(), k, v, normalize=False)[0]
+    assert torch.equal(o, ref) and not o.requires_grad
+    o = L.chunk_linear_attn(q, k, v, normalize=False)[0]
+    assert o.requires_grad and torch.equal(o, ref)
+    q = q.detach()
+    with fw.dual_level():
+        with pytest.raises((RuntimeError, NotImplementedError)):
+            L.chunk_simple_gla(fw.make_dual(q, q), k, v)
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda x: L.chunk_simple_gla(x, k, v)[0])(q.unsqueeze(0))
+    with pytest.raises(RuntimeError):                      # (nothing of the call is mapped over)
+        torch.func.vmap(lambda x: L.chunk_simple_gla(q, k, v)[0] + x)(torch.zeros(2, device=cuda))
