@@ -303,7 +303,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           for (int i = 0; i < IOK::VEC; ++i) { fv[i] = ET<T>::to_f(r.v[p][i]); c += fv[i] * sv[i]; }
           ss = group_sum<IOK::VPR>(ss);
           c = group_sum<IOK::VPR>(c);
-          const float rn = 1.0f / sqrtf(ss + a.qk_eps);
+          const float rn = rsqrt_fast(ss + a.qk_eps);
           c = c * rn * rn * rn;
 #pragma unroll
           for (int i = 0; i < IOK::VEC; ++i) r.v[p][i] = ET<T>::from_f((fv[i] * rn - c * sv[i]) * gv[i]);

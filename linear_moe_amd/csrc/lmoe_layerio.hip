@@ -71,7 +71,7 @@ __global__ __launch_bounds__(NTHR) void k_gdn_qkv_prologue(const T* __restrict__
       ssq += sq[i] * sq[i]; ssk += sk[i] * sk[i];
     }
     ssq = row_sum<LPR>(ssq); ssk = row_sum<LPR>(ssk);
-    const float rq = 1.0f / sqrtf(ssq + eps), rk = 1.0f / sqrtf(ssk + eps);
+    const float rq = rsqrt_fast(ssq + eps), rk = rsqrt_fast(ssk + eps);
     vec oq, ok;
     if constexpr (BWD) {
       const vec dqv = *(const vec*)(dq + r * D + lr * VEC), dkv = *(const vec*)(dk + r * D + lr * VEC);

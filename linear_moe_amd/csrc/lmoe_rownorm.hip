@@ -23,7 +23,7 @@ template <int LPR> __device__ __forceinline__ float lanes_sum(float x) {
   for (int d = 1; d < LPR; d <<= 1) x += __shfl_xor(x, d, 64);
   return x;
 }
-__device__ __forceinline__ float sigmoidf_(float z) { return 1.0f / (1.0f + __expf(-z)); }
+__device__ __forceinline__ float sigmoidf_(float z) { return sigmoid_fast(z); }
 
 // ------------------------------------------------------------------------- //
 // RMS norm (+ swish gate)
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(NTHR) void k_silu_l2norm(const T* __restrict__ x, c
       ss += sf[i] * sf[i];
     }
     ss = lanes_sum<LPR>(ss);
-    const float rstd = 1.0f / sqrtf(ss + eps);
+    const float rstd = rsqrt_fast(ss + eps);
     vec o;
     if constexpr (BWD) {
       const vec dv = *(const vec*)(dy + r * D + lr * VEC);
