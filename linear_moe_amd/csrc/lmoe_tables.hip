@@ -106,7 +106,7 @@ void launch_seq_tables(const void* offs, int is64, int N, int nt_max, int32_t* c
 
 // ------------------------------------------------------------------------- //
 // Routing tables of a mixture-of-memories layer: a stable counting sort of the choices (b, t, k) by (memory, batch row),
-// in three launches.  The choices of a batch row are one contiguous range, cut into segments; counts[(e B + b)
+// in three launches (few choices: one, k_mom_route below).  The choices of a batch row are one contiguous range, cut into segments; counts[(e B + b)
 // nseg + s] then lies in the order of the result, and its prefix sums are where every (memory, row, segment) begins.
 //   count: choices per memory of a segment
 //   scan:  prefix sums (one work-group), the capacity, offsets of the sequences; counts -> first row of a segment, less
@@ -232,6 +232,132 @@ __global__ __launch_bounds__(NTHR) void k_mom_place(const void* __restrict__ sel
   }
 }
 
+// The three steps in one launch, for few choices and up to 16 memories (mom_route_takes): every work-group counts the choices of
+// all segments for itself (out of the L2, a wave 64 at a time; lane e keeps the count of memory e from the ballots), its first
+// wave forms the prefix sums, and it places its own segment, a wave per 64 choices.  Nothing is handed from one launch to the next.
+// Bound by its launch, three round trips to memory and the counting, 64 choices in some 4 E + 16 instructions of a wave.
+// 2 x 2048 tokens, 4 memories, top 2: 13.4 us in three launches -> 7.7 (replayed as a graph; traced 3.2 + 7.1 + 4.6 -> 9.5; with
+// the prefix sums over the whole work-group, as in k_mom_scan, 12.0); 128 tokens, top 1: 12.0 -> 4.2.  Three launches take 13.4
+// to 14.2 whatever the sizes: 8192 choices of 16 memories 12.8 here, 16384 of 8 15.3, 32768 of 4 19.9 and of 16 40.
+constexpr int ROUTE_THR = 1024, ROUTE_SEG = 512, ROUTE_E = 16, ROUTE_MAX = 1024, ROUTE_WORK = 131072;
+static bool mom_route_takes(int64_t B, int64_t per_row, int64_t E) {
+  return E <= ROUTE_E && B * per_row * (E + 4) <= ROUTE_WORK && B * E * ((per_row + ROUTE_SEG - 1) / ROUTE_SEG) <= ROUTE_MAX;
+}
+// Exclusive prefix sums of x[0 .. n) in place, x[n] = total, by one wave: ROUTE_MAX / 64 consecutive entries per lane
+__device__ __forceinline__ void wave_exclusive_scan(int* x, int n, int lane) {
+  const int per = (n + 63) / 64, j0 = lane * per;
+  int sum = 0;
+  for (int i = j0; i < min(j0 + per, n); ++i) sum += x[i];
+  int incl = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += y;
+  }
+  int base = incl - sum;
+  for (int i = j0; i < min(j0 + per, n); ++i) {
+    const int y = x[i];
+    x[i] = base;
+    base += y;
+  }
+  if (lane == 63) x[n] = incl;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__global__ __launch_bounds__(ROUTE_THR) void k_mom_route(const void* __restrict__ sel, int is64, int per_row, int topk, int E, int cap,
+                                                         int32_t* __restrict__ cu, int64_t* __restrict__ max_len,
+                                                         int64_t* __restrict__ mem_offsets, int32_t* __restrict__ src_token,
+                                                         int32_t* __restrict__ src_choice, int32_t* __restrict__ row_of) {
+  constexpr int NW = ROUTE_THR / 64, GROUPS = ROUTE_SEG / 64, STEP = NW / GROUPS, AHEAD = 4;
+  __shared__ int s_ex[ROUTE_MAX + 1], s_cu[ROUTE_MAX + 1], s_grp[GROUPS][ROUTE_E], s_kept;
+  const int s = blockIdx.x, b = blockIdx.y, nseg = gridDim.x, B = gridDim.y;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), NS = E * B, M = NS * nseg;
+  // this wave's 64 choices of its own segment (waves beyond the segment's: none)
+  const int i_own = s * ROUTE_SEG + wv * 64 + lane;
+  const bool valid = wv < GROUPS && i_own < per_row;
+  const int64_t c = (int64_t)b * per_row + i_own;
+  const int e_own = valid ? memory_of(sel, is64, c, E) : E;
+  for (int i = t; i < M; i += ROUTE_THR) s_ex[i] = 0;
+  __syncthreads();
+  // 64 choices, number wv % GROUPS, of every STEP-th segment (segments of all rows in order); a few segments' loads at a time
+  int row = 0, seg = wv / GROUPS;
+  while (row < B) {
+    int key[AHEAD], at[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      while (seg >= nseg) { seg -= nseg; ++row; }
+      const int i = seg * ROUTE_SEG + (wv % GROUPS) * 64 + lane;
+      at[u] = row < B ? row * nseg + seg : -1;
+      key[u] = row < B && i < per_row ? memory_of(sel, is64, (int64_t)row * per_row + i, E) : E;
+      seg += STEP;
+    }
+    while (seg >= nseg) { seg -= nseg; ++row; }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      if (at[u] < 0) break;
+      int own = 0;
+      for (int e = 0; e < E; ++e) {
+        const int n = __popcll(__ballot(key[u] == e));
+        own = lane == e ? n : own;
+      }
+      if (lane < E) {
+        const int r = at[u] / nseg;
+        if (own) atomicAdd(&s_ex[(lane * B + r) * nseg + at[u] - r * nseg], own);
+        if (at[u] == b * nseg + s) s_grp[wv % GROUPS][lane] = own;
+      }
+    }
+  }
+  __syncthreads();
+  // prefix sums and the capacity, as in k_mom_scan
+  if (wv == 0) {
+    wave_exclusive_scan(s_ex, M, lane);
+    int kept = 0;
+    for (int i = lane; i < NS; i += 64) kept = max(kept, s_ex[(i + 1) * nseg] - s_ex[i * nseg]);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) kept = max(kept, __shfl_xor(kept, d, 64));
+    if (cap >= 0) kept = min(kept, cap);
+    for (int i = lane; i < NS; i += 64) s_cu[i] = min(s_ex[(i + 1) * nseg] - s_ex[i * nseg], kept);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_exclusive_scan(s_cu, NS, lane);
+    if (lane == 0) s_kept = kept;
+  }
+  __syncthreads();
+  if (s == 0 && b == 0) {
+    for (int i = t; i <= NS; i += ROUTE_THR) {
+      cu[i] = s_cu[i];
+      if (i % B == 0) mem_offsets[i / B] = s_cu[i];
+    }
+    if (t == 0) max_len[0] = s_kept;
+  }
+  if (wv < GROUPS) {
+    int bits = 1;
+    while ((E >> bits) != 0) ++bits;           // the keys are 0 .. E
+    const int rank = __popcll(same_key_lanes(e_own, bits) & ((1ull << lane) - 1));
+    int at = -1;
+    if (e_own < E) {
+      const int q = e_own * B + b, q0 = s_ex[q * nseg], len = s_ex[(q + 1) * nseg] - q0;
+      at = s_cu[q] + (s_ex[q * nseg + s] - q0) - (len - min(len, s_kept)) + rank;
+      for (int g = 0; g < wv; ++g) at += s_grp[g][e_own];
+      if (at < s_cu[q]) at = -1;               // (dropped by the capacity)
+    }
+    if (valid) {
+      row_of[c] = at;
+      if (at >= 0) {
+        src_choice[at] = (int32_t)c;
+        src_token[at] = (int32_t)c / topk;
+      }
+    }
+  }
+  const int64_t n = (int64_t)B * per_row, step = (int64_t)nseg * B * ROUTE_THR;
+  for (int64_t r = s_cu[NS] + ((int64_t)b * nseg + s) * ROUTE_THR + t; r < n; r += step) {
+    src_choice[r] = -1;
+    src_token[r] = -1;
+  }
+}
+
 static int64_t mom_segments(int64_t per_row, int seg) { return (per_row + seg - 1) / seg; }
 static int mom_seg(int64_t B, int64_t per_row, int64_t E) {
   return B * E * mom_segments(per_row, MOM_SEG_SHORT) <= MOM_SCAN_MAX ? MOM_SEG_SHORT : MOM_SEG_LONG;
@@ -247,6 +373,11 @@ int64_t mom_plan_ints(int64_t B, int64_t per_row, int64_t E) {
 void launch_mom_plan(const void* sel, int is64, int B, int per_row, int topk, int E, int cap, int32_t* counts, int32_t* cu,
                      int64_t* max_len, int64_t* mem_offsets, int32_t* src_token, int32_t* src_choice, int32_t* row_of,
                      hipStream_t st) {
+  if (mom_route_takes(B, per_row, E)) {
+    hipLaunchKernelGGL(k_mom_route, dim3((int)mom_segments(per_row, ROUTE_SEG), B), dim3(ROUTE_THR), 0, st, sel, is64, per_row, topk, E, cap,
+                       cu, max_len, mem_offsets, src_token, src_choice, row_of);
+    return;
+  }
   const int seg = mom_seg(B, per_row, E), nseg = (int)mom_segments(per_row, seg);
   int bits = 1;
   while ((E >> bits) != 0) ++bits;             // the keys are 0 .. E

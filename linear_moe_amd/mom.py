@@ -57,7 +57,7 @@ def mom_plan(selected_memories: torch.Tensor, num_memories: int, capacity: Optio
     """Index tables for ``selected_memories`` [B, S, topk] (as ``torch.topk`` returns them,
     mom_linear_attention.py:288).  ``capacity``: the reference's capacity factor; ``None`` keeps every token.
 
-    Built on the device (a stable counting sort by (memory, batch row) in three launches; what its kernels do not take
+    Built on the device (a stable counting sort by (memory, batch row) in one to three launches; what its kernels do not take
     -- more than 1024 memories, or more than 8192 counts of a memory in 2048 choices of a batch row --
     by tensor operations), as the reference builds its tables (mom_linear_attention.py:28-66).  Without a capacity nothing is read
     back to the host: every routed token is kept, ``T_total = B * S * topk`` is known up front, and pack -> op ->

@@ -74,3 +74,30 @@ def test_memories_out_of_range_are_dropped(cuda):
     mom_combine(y, plan, w).sum().backward()
     assert y.grad[:4].eq(1).all() and y.grad[4:].eq(0).all()
     assert torch.equal(w.grad.view(3, 2).ne(0).cpu(), torch.tensor([[True, False], [False, True], [True, True]]))
+
+
+@pytest.mark.parametrize("capacity", [None, 0.2])
+@pytest.mark.parametrize("B,S,topk,E", [(1, 63, 1, 16), (1, 65, 1, 17), (5, 511, 1, 2), (2, 513, 2, 16), (12, 512, 1, 16),
+                                        (64, 16, 1, 16), (65, 16, 1, 16), (1, 16384, 1, 4), (1, 16385, 1, 4)])
+def test_routing_tables_in_one_launch(cuda, B, S, topk, E, capacity):
+    """On both sides of what one launch takes: 16 memories, 1024 counts, 16384 choices of 4 memories; some choices out of range."""
+    from linear_moe_amd.mom import mom_plan
+    sel = torch.topk(torch.rand(B, S, E, generator=torch.Generator().manual_seed(B + S + E)), topk, dim=-1).indices
+    sel[:, ::7, -1] = E
+    sel[:, ::11, 0] = -1
+    # rows in order: by memory, batch row, time; the last max_len of every sequence
+    flat = sel.reshape(B, S * topk)
+    seqs = [[[b * S * topk + i for i in (flat[b] == e).nonzero()[:, 0].tolist()] for b in range(B)] for e in range(E)]
+    longest = max(len(x) for row in seqs for x in row)
+    keep = longest if capacity is None else min(longest, -int(-S * capacity // 1))
+    kept = [x[len(x) - min(len(x), keep):] for row in seqs for x in row]
+    choice = torch.tensor([c for x in kept for c in x], dtype=torch.int32)
+    cu = torch.tensor([0] + [len(x) for x in kept]).cumsum(0)
+    row_of = torch.full((B * S * topk,), -1, dtype=torch.int32)
+    row_of[choice.long()] = torch.arange(len(choice), dtype=torch.int32)
+    got = mom_plan(sel.to(cuda), E, capacity)
+    n = len(choice)
+    assert got.max_len == keep and torch.equal(got.cu_seqlens.cpu().long(), cu) and torch.equal(got.mem_offsets, cu[::B])
+    assert torch.equal(got.row_of.cpu().view(-1), row_of)
+    assert torch.equal(got.src_choice.cpu()[:n], choice) and torch.equal(got.src_token.cpu()[:n], choice // topk)
+    assert (got.src_choice[n:] == -1).all() and (got.src_token[n:] == -1).all()
