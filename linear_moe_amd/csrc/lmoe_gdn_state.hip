@@ -15,6 +15,8 @@ template <typename T, int V> inline bool wide_slices(const lmoe_args& a) {
   constexpr int BW = GdnStateCfg<T>::BV_WIDE;
   return BW <= V && BW != GdnStateCfg<T>::BV && (int64_t)a.N * a.H * (V / BW) >= cu_count();
 }
+// whether `slices` work-groups per (sequence, head) have a CU each
+inline bool pairs_on_cus(const lmoe_args& a, int slices) { return (int64_t)a.N * a.H * slices <= cu_count(); }
 // The transitions of a call without a gate are carried in two terms (lmoe_gdn_split.hpp).
 inline bool two_terms(const lmoe_args& a) { return a.gate == LMOE_GATE_NONE; }
 // How the sequences of a call are cut: not at all without a workspace for it.
@@ -60,6 +62,18 @@ template <typename T, int K, int V, int BV> void launch_fwd(const lmoe_args& a, 
           const int items = ((sp.n3 * a.H + 7) / 8) * 8 * (V / BV);
           if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true, false, true>), dim3(items), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
           else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false, false, true>), dim3(items), dim3(3 * NTHR), 0, st, a, sp, (long long*)nullptr, -1);
+          return;
+        }
+      }
+      // Slices of 16 columns where they all find a CU of their own: a chunk is a chain on one wave either way, and half the
+      // waves ask the LDS beside it.  us with the preparation in front, 32 and 16 columns: K = V = 128, 8 pairs of 16 chunks 31.4
+      // and 28.7, 32 of 32 62.1 and 58.6 (saving 64.5 and 62.9), K = V = 64, 32 of 32 46.0 and 42.7; but 48 pairs, K = V = 128,
+      // 67.9 and 99.9.  Same bits.
+      if constexpr (V <= 128) {
+        if (pairs_on_cus(a, V / 16)) {
+          const dim3 narrow(((a.N * a.H + 7) / 8) * 8 * (V / 16));
+          if (a.hs) hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, true, false, false, 16>), narrow, dim3(3 * NTHR), 0, st, a, Split{}, (long long*)nullptr, -1);
+          else hipLaunchKernelGGL((k_gdn_state_fwd_reg<K, V, false, false, false, 16>), narrow, dim3(3 * NTHR), 0, st, a, Split{}, (long long*)nullptr, -1);
           return;
         }
       }

@@ -32,6 +32,8 @@
 //     P = (q k^T) . Gamma over the q rows it reads for q S anyway (two rows of k blocks are all that P adds to its reads; on the
 //     loader waves P took 80 KB of reads per chunk).  P never passes through memory on its way to the output; a call
 //     that saves for the backward stores it once: every V-slice work-group its share of the rows.
+//   * Few (sequence, head) pairs (the rule: lmoe_gdn_state.hip) take slices of BV = 16 columns: one consumer wave, the
+//     columns' output split over the helpers by token blocks, the second consumer's wave gone.
 //   * The loaders' stores lie behind no branch (the first two windows are peeled off), so that a wait for a load never waits
 //     for stores behind it.
 #pragma once
@@ -72,10 +74,10 @@ __device__ __forceinline__ void static_for_blocks(F&& f) {
   }
 }
 
-template <int K, int V, bool SAVE, bool TRACE = false, bool CUT = false>
+template <int K, int V, bool SAVE, bool TRACE = false, bool CUT = false, int BV = 32>
 __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args a, const Split sp, long long* tr, int traced_wg) {
   typedef bf16 T;
-  constexpr int BV = 32;
+  static_assert(BV == 32 || BV == 16, "a consumer wave per 16 columns");
   constexpr int LDK = K + LPAD, LDC = CH + LPAD, LDU = BV + LPAD;
   constexpr int KT = K / 16, KS = K / 32;
   constexpr int LPA = GdnStateCfg<T>::LPF, LPB = GdnStateCfg<T>::LPF;       // register sets per prefetch ring (3: no change)
@@ -160,10 +162,12 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
     const int wt = wave_id() - 4;
     auto store_saved = [&](int c) {           // v_new(c) (back in [token][column] through transposing reads) and P(c)
       const pvec pv = *(const pvec*)(s_p[c & 1] + prow * LDC + pcol);
-      const typename ET<T>::frag x = ET<T>::load_frag_t(s_vT[c & 1], LDC, 0, 16 * wt, l);
+      // (BV = 16: a wave takes 32 tokens, waves 2, 3 the same again)
+      const int vl = BV == 32 ? l : (l & 31), vt = BV == 32 ? 16 * wt : 32 * (wt & 1) + 16 * (l >> 5);
+      const typename ET<T>::frag x = ET<T>::load_frag_t(s_vT[c & 1], LDC, 0, vt, vl);
       __builtin_nontemporal_store(pv, (pvec*)((T*)a.pmat + (((int64_t)(sq.chunk0 + c) * a.H + h) * CH + prow) * CH + pcol));
       // (all 64 rows: those past the end of a partial chunk are zero)
-      __builtin_nontemporal_store(x, (typename ET<T>::vec*)(slice_ptr<T>(a.vnew, sq.chunk0 + c, h, a.H, V, v0) + (16 * wt + (l & 15)) * SLICE_COLS + 8 * (l >> 4)));
+      __builtin_nontemporal_store(x, (typename ET<T>::vec*)(slice_ptr<T>(a.vnew, sq.chunk0 + c, h, a.H, V, v0) + (vt + (vl & 15)) * SLICE_COLS + 8 * (vl >> 4)));
     };
     auto store_out = [&](int c) {
       const int tok = sq.tok0 + c * CH;
@@ -286,32 +290,34 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
     auto help = [&](auto which) {
       constexpr int J = decltype(which)::value;
       constexpr int TA = J, TB = 3 - J;          // its two rows of k blocks
-      f32x4 oa[4];                               // (q S)^T of a chunk: columns of the slice x tokens 16 t ..
+      // (q S)^T of a chunk: columns of the slice x tokens 16 t ..  BV = 16: helper J takes the token blocks t = 2 J, 2 J + 1
+      constexpr int T0 = BV == 32 ? 0 : 2 * J, T1 = BV == 32 ? 4 : 2 * J + 2, C0 = BV == 32 ? 16 * J : 0;
+      f32x4 oa[4];
       typename ET<T>::frag fv[2], fp[6];
       // o(c) = scale (e^b q S + P v_new), in the window behind the one that formed q S, P and v_new
       auto finish_fetch = [&](int c) {
         const T* s_pc = s_p[c & 1];
         const T* s_vc = s_vT[c & 1];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) fv[s] = ET<T>::load_frag(s_vc + (16 * J + fr) * LDC + 32 * s + 8 * g);
-        fp[0] = ET<T>::load_frag(s_pc + (0 + fr) * LDC + 8 * g);
-        fp[1] = ET<T>::load_frag(s_pc + (16 + fr) * LDC + 8 * g);
-        fp[2] = ET<T>::load_frag(s_pc + (32 + fr) * LDC + 8 * g);
-        fp[3] = ET<T>::load_frag(s_pc + (48 + fr) * LDC + 8 * g);
-        fp[4] = ET<T>::load_frag(s_pc + (32 + fr) * LDC + 32 + 8 * g);
-        fp[5] = ET<T>::load_frag(s_pc + (48 + fr) * LDC + 32 + 8 * g);
+        for (int s = 0; s < 2; ++s) fv[s] = ET<T>::load_frag(s_vc + (C0 + fr) * LDC + 32 * s + 8 * g);
+#pragma unroll
+        for (int t = T0; t < T1; ++t) fp[t] = ET<T>::load_frag(s_pc + (16 * t + fr) * LDC + 8 * g);
+        if constexpr (T1 == 4) {
+          fp[4] = ET<T>::load_frag(s_pc + (32 + fr) * LDC + 32 + 8 * g);
+          fp[5] = ET<T>::load_frag(s_pc + (48 + fr) * LDC + 32 + 8 * g);
+        }
       };
       auto finish = [&](int c) {
-        ET<T>::mma(oa[0], fv[0], fp[0]);
-        ET<T>::mma(oa[1], fv[0], fp[1]);
-        ET<T>::mma(oa[2], fv[0], fp[2]);
-        ET<T>::mma(oa[3], fv[0], fp[3]);
-        ET<T>::mma(oa[2], fv[1], fp[4]);
-        ET<T>::mma(oa[3], fv[1], fp[5]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
+        for (int t = T0; t < T1; ++t) ET<T>::mma(oa[t], fv[0], fp[t]);
+        if constexpr (T1 == 4) {
+          ET<T>::mma(oa[2], fv[1], fp[4]);
+          ET<T>::mma(oa[3], fv[1], fp[5]);
+        }
+#pragma unroll
+        for (int t = T0; t < T1; ++t) {
           oa[t] *= scale;
-          acc_to_lds_t<T>(oa[t], s_o[c & 1], LDU, 16 * J, 16 * t, l);                    // o [token][column]: 8-byte writes
+          acc_to_lds_t<T>(oa[t], s_o[c & 1], LDU, C0, 16 * t, l);                    // o [token][column]: 8-byte writes
         }
       };
       lds_barrier();
@@ -321,7 +327,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
         const T *s_kc = s_k[cur], *s_qc = s_q[cur], *s_hc = s_hT[cur];
         typename ET<T>::frag fs[2], fq[2][4], fk[2][2];
         auto fetch = [&](int ks, int buf) {
-          fs[buf] = ET<T>::load_frag(s_hc + (16 * J + fr) * LDK + 32 * ks + 8 * g);
+          fs[buf] = ET<T>::load_frag(s_hc + (C0 + fr) * LDK + 32 * ks + 8 * g);
 #pragma unroll
           for (int t = 0; t < 4; ++t) fq[buf][t] = ET<T>::load_frag(s_qc + (16 * t + fr) * LDK + 32 * ks + 8 * g);
           fk[buf][0] = ET<T>::load_frag(s_kc + (16 * TA + fr) * LDK + 32 * ks + 8 * g);
@@ -362,7 +368,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
           if (ks + 1 < KS) fetch(ks + 1, bf ^ 1);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) ET<T>::mma(oa[t], fs[bf], fq[bf][t]);
+          for (int t = T0; t < T1; ++t) ET<T>::mma(oa[t], fs[bf], fq[bf][t]);
           static_for_blocks<TA, TB>([&](auto x, auto ti, auto tj) {
             constexpr int X = decltype(x)::value, TI = decltype(ti)::value, TJ = decltype(tj)::value;
             ET<T>::mma(pc[X], fk[bf][TJ == TA ? 0 : 1], fq[bf][TI]);
@@ -377,7 +383,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
           *(bf16x4*)(s_p[cur] + (16 * TI + fr) * LDC + 16 * TJ + 4 * g) = y;
         });
 #pragma unroll
-        for (int t = 0; t < 4; ++t) oa[t] *= eb[t];
+        for (int t = T0; t < T1; ++t) oa[t] *= eb[t];
         if (J == 0) TR(1, c, 2);
         lds_barrier();
         if (J == 0) TR(1, c, 3);
@@ -391,6 +397,7 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
     return;
   }
 
+  if (BV == 16 && wv == 1) return;                   // (a wave that has ended is not waited for at a barrier)
   // --------------------------------- consumers: the chain ---------------------------------
   __builtin_amdgcn_s_setprio(3);
   const int j = wv;

@@ -203,3 +203,29 @@ def test_forward_only_call_equals_the_saving_call(cuda):
     o2, ht2 = chunk_gated_delta_rule(q.clone().requires_grad_(True), k, v, g, beta, None, h0, True, None, False)
     torch.cuda.synchronize()
     assert torch.equal(o1, o2.detach()) and torch.equal(ht1, ht2.detach())
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("T", [1, 64, 65, 129, 700])
+def test_narrow_slices_of_the_forward_pass_same_bits(cuda, K, V, T):
+    """Few (sequence, head) pairs take V slices of half the width: outputs, final state and (through what the pass saves) every
+    gradient are those of the same rows in a batch with too many pairs for that."""
+    import torch.nn.functional as F
+    from linear_moe_amd import chunk_gated_delta_rule
+    H, B = 3, 30                                   # 3 pairs: narrow; 90: 32 columns
+    g_ = torch.Generator().manual_seed(K + V + T)
+    rn = lambda *s: torch.randn(*s, generator=g_)
+    x = dict(q=F.normalize(rn(1, T, H, K), dim=-1).bfloat16(), k=F.normalize(rn(1, T, H, K), dim=-1).bfloat16(), v=rn(1, T, H, V).bfloat16(),
+             g=-F.softplus(rn(1, T, H)) * 0.1, beta=torch.sigmoid(rn(1, T, H)).bfloat16(), h=rn(1, H, K, V))
+    do, dht = rn(1, T, H, V).bfloat16(), rn(1, H, K, V)
+    out = []
+    for n in (1, B):
+        rep = lambda t: t.to(cuda).expand(n, *t.shape[1:]).contiguous()
+        d = {k_: rep(t).requires_grad_(True) for k_, t in x.items()}
+        call = lambda: chunk_gated_delta_rule(d["q"], d["k"], d["v"], d["g"], d["beta"], None, d["h"], True)
+        o, ht = call()
+        grads = torch.autograd.grad([o, ht], list(d.values()), [rep(do), rep(dht)])
+        with torch.no_grad():
+            of, hf = call()
+        out.append([t[:1].detach() for t in (o, ht, of, hf, *grads)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
