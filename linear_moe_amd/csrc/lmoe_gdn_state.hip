@@ -103,6 +103,13 @@ template <typename T, int K, int V, int BV> void launch_bwd(const lmoe_args& a, 
       return;
     }
   }
+  if constexpr (sizeof(T) == 2 && V <= 128) {
+    // slices of 16 columns where they all find a CU of their own: 32 pairs of 32 chunks, K = V = 128, 50.9 -> 44.3 us; same bits
+    if (pairs_on_cus(a, V / 16)) {
+      hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, 16>), dim3(((a.N * a.H + 7) / 8) * 8 * (V / 16)), dim3(3 * NTHR), 0, st, a, Split{});
+      return;
+    }
+  }
   hipLaunchKernelGGL((k_gdn_state_bwd<T, K, V, BV>), dim3(((a.N * a.H + 7) / 8) * 8 * (V / BV)), dim3(3 * NTHR), 0, st, a, Split{});
 }
 template <typename T, int K, int V> struct GdnStateFwd {

@@ -208,7 +208,7 @@ def test_forward_only_call_equals_the_saving_call(cuda):
 @pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
 @pytest.mark.parametrize("T", [1, 64, 65, 129, 700])
 def test_narrow_slices_of_the_forward_pass_same_bits(cuda, K, V, T):
-    """Few (sequence, head) pairs take V slices of half the width: outputs, final state and (through what the pass saves) every
+    """Few (sequence, head) pairs take V slices of half the width in both passes: outputs, final state and (through what the pass saves) every
     gradient are those of the same rows in a batch with too many pairs for that."""
     import torch.nn.functional as F
     from linear_moe_amd import chunk_gated_delta_rule
