@@ -118,6 +118,10 @@ template <typename T, int K, int V> struct StateFwd {
       }
       const Split sp = launch_scalar_seg(a, false, st);
       if (sp.len1) launch_fwd_b<T, K, V, BV, true>(a, sp, st);
+      // slices of 16 columns where each finds a CU of its own (us, 32 and 16 columns; same bits): K = V = 128, 4 pairs of 8 chunks
+      // 14.1 and 13.1, 32 of 16 25.1 and 23.8, normalised 27.8 and 25.9, 32 of 32 51.3 and 44.5, saving 50.0 and 44.3; K = V = 64,
+      // 16 of 16 18.6 and 17.8; but 48 pairs of 16, K = V = 128, 26.0 and 42.8
+      else if ((int64_t)a.N * a.H * (V / 16) <= cu_count()) launch_fwd_b<T, K, V, 16, false>(a, sp, st);
       else launch_fwd_b<T, K, V, BV, false>(a, sp, st);
     } else {
       if (fwd_by_chunks(a)) {

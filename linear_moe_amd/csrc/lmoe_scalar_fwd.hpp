@@ -419,7 +419,8 @@ __global__ __launch_bounds__(3 * NTHR) void k_state_fwd_b(const lmoe_args a, con
       if constexpr (KEPT) {
         IOK::load_from(P.rk, ok, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, len);
         IOK::load_from(P.rq, oq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);
-        IOV::load_from(P.ru, ou, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
+        if constexpr (BV >= 32) IOV::load_from(P.ru, ou, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
+        else IOV::load_nomask(P.ru, row_ptr<T>(a.v, sq.b, tok, h) + v0, a.v.st, len);
       } else {
         IOK::load_nomask(P.rk, row_ptr<T>(a.k, sq.b, tok, h), a.k.st, len);
         IOK::load_nomask(P.rq, row_ptr<T>(a.q, sq.b, tok, h), a.q.st, len);

@@ -236,3 +236,33 @@ def test_forward_pass_on_both_sides_of_the_kept_offsets(cuda, V, K, normalized, 
     for n in (T - 1, T - 30):
         assert torch.equal(out(n), want[:, :, :n])
     assert want.abs().max() > 0
+
+
+@pytest.mark.parametrize("mode", ["plain", "gated", "normalized"])
+@pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("T", [1, 64, 128, 129, 260])
+def test_narrow_slices_same_bits(cuda, K, V, T, mode):
+    """Few (sequence, head) pairs take V slices of 16 columns in both passes: outputs, final state and gradients are those of the
+    same rows in a batch with too many pairs for that."""
+    from linear_moe_amd import chunk_linear_attn, chunk_simple_gla
+    H, B = 3, 30                                   # 3 pairs: 16 columns; 90: 32
+    x = {n: gen(110 + i, 1, H, T, d) for i, (n, d) in enumerate((("q", K), ("k", K), ("v", V)))}
+    x = {n: (t.abs() if mode == "normalized" else t).bfloat16() for n, t in x.items()}
+    x["h"] = gen(113, 1, H, K, V)
+    if mode == "gated":
+        x["g"] = F.logsigmoid(gen(114, 1, H, T)) / 4
+    do, dht = gen(115, 1, H, T, V).bfloat16(), gen(116, 1, H, K, V)
+    out = []
+    for n in (1, B):
+        rep = lambda t: t.to(cuda).expand(n, *t.shape[1:]).contiguous()
+        d = {k: rep(t).requires_grad_(True) for k, t in x.items()}
+        if mode == "gated":
+            call = lambda: chunk_simple_gla(d["q"], d["k"], d["v"], d["g"], None, d["h"], True)
+        else:
+            call = lambda: chunk_linear_attn(d["q"], d["k"], d["v"], None, d["h"], True, normalize=mode == "normalized")
+        o, ht = call()
+        grads = torch.autograd.grad([o, ht], list(d.values()), [rep(do), rep(dht)])
+        with torch.no_grad():
+            of, hf = call()
+        out.append([t[:1].detach() for t in (o, ht, of, hf, *grads)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
