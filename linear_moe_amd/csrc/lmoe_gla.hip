@@ -68,6 +68,15 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
           else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
           break;
         }
+        // slices of 16 columns where each finds a CU of its own: the step from chunk to chunk is a wave's serial chain over its
+        // columns (us, 32 and 16 columns, saving; same bits): K = V = 128, 4 pairs of 8 chunks 10.7 and 9.9, 16 of 16 19.3 and
+        // 17.8, 32 of 32 36.0 and 33.7; K = V = 64, 16 of 16 14.7 and 12.4.  With more work-groups than CUs k~ and q~ are read
+        // twice as often for nothing.
+        if ((int64_t)a.N * a.H * (V / 16) <= cu_count()) {
+          if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, 16, true>), dim3(pairs8 * (V / 16)), dim3(3 * NTHR), 0, st, a, sp);
+          else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, 16, false>), dim3(pairs8 * (V / 16)), dim3(3 * NTHR), 0, st, a, sp);
+          break;
+        }
         if (a.hs) hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, true>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
         else hipLaunchKernelGGL((k_gla_fwd_fused<T, K, V, Tl::BVS, false>), dim3(pairs8 * (V / Tl::BVS)), dim3(3 * NTHR), 0, st, a, sp);
         break;
@@ -86,6 +95,10 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
         const Split sp = launch_gla_seg<T, K, V, true>(a, st);
         if (sp.len1) {
           hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, Tl::BVS, true>), dim3((sp.n3 * a.H + 7) / 8 * 8 * (V / Tl::BVS)), block, 0, st, a, sp);
+          break;
+        }
+        if ((int64_t)a.N * a.H * (V / 16) <= cu_count()) {  // (as above: 9.8 and 7.9, 16.8 and 14.4, 30.4 and 27.6, 12.2 and 10.6)
+          hipLaunchKernelGGL((k_gla_state_bwd<T, GT, K, V, 16>), dim3((a.N * a.H + 7) / 8 * 8 * (V / 16)), block, 0, st, a, Split{});
           break;
         }
       }

@@ -480,14 +480,25 @@ __global__ __launch_bounds__(3 * NTHR) void k_gla_fwd_fused(const lmoe_args a, c
     auto save_state = [&](int c) {
       if constexpr (SAVE) {
         T* hs = (T*)a.hs + ((int64_t)(sq.chunk0 + c) * a.H + h) * K * V + v0;
+        if constexpr (BV >= 32) {
 #pragma unroll
-        for (int kb = 0; kb < K / 64; ++kb)
+          for (int kb = 0; kb < K / 64; ++kb)
 #pragma unroll
-          for (int vb = 0; vb < BV / 32; ++vb) {
-            const int k0 = 16 * (4 * kb + (wave - 4));
-            const typename ET<T>::frag x = ET<T>::load_frag_t(s_hT[c & 1], LDK, 32 * vb, k0, l);
-            *(typename ET<T>::vec*)(hs + (int64_t)(k0 + (l & 15)) * V + 32 * vb + 8 * (l >> 4)) = x;
+            for (int vb = 0; vb < BV / 32; ++vb) {
+              const int k0 = 16 * (4 * kb + (wave - 4));
+              const typename ET<T>::frag x = ET<T>::load_frag_t(s_hT[c & 1], LDK, 32 * vb, k0, l);
+              *(typename ET<T>::vec*)(hs + (int64_t)(k0 + (l & 15)) * V + 32 * vb + 8 * (l >> 4)) = x;
+            }
+        } else {
+          // 16 columns are two groups of 8: lanes of g >= 2 take the K rows 64 further on (K = 64: the same again, unstored)
+          const int up = (l >> 5) & 1;
+#pragma unroll
+          for (int kb = 0; kb < K / 64; kb += 2) {
+            const int k0 = 16 * (4 * (kb + (K > 64 ? up : 0)) + (wave - 4));
+            const typename ET<T>::frag x = ET<T>::load_frag_t(s_hT[c & 1], LDK, -16 * up, k0, l);
+            if (K > 64 || !up) *(typename ET<T>::vec*)(hs + (int64_t)(k0 + (l & 15)) * V + 8 * ((l >> 4) & 1)) = x;
           }
+        }
       }
     };
 #pragma unroll

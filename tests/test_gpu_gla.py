@@ -173,3 +173,26 @@ def test_gla_forward_only_call_equals_the_saving_call(cuda):
     o2, ht2 = chunk_gla(q.clone().requires_grad_(True), k, v, g, None, h0, True, None, False)
     torch.cuda.synchronize()
     assert torch.equal(o1, o2.detach()) and torch.equal(ht1, ht2.detach())
+
+
+@pytest.mark.parametrize("K,V", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("T", [1, 64, 65, 129, 260])
+def test_narrow_slices_same_bits(cuda, K, V, T):
+    """Few (sequence, head) pairs take V slices of 16 columns in both passes: outputs, final state and gradients (through the
+    states that the forward pass saves) are those of the same rows in a batch with too many pairs for that."""
+    from linear_moe_amd import chunk_gla
+    H, B = 3, 30                                   # 3 pairs: 16 columns; 90: 32
+    x = dict(q=gen(101, 1, H, T, K).bfloat16(), k=gen(102, 1, H, T, K).bfloat16(), v=gen(103, 1, H, T, V).bfloat16(),
+             g=F.logsigmoid(gen(104, 1, H, T, K)) / 16, h=gen(105, 1, H, K, V))
+    do, dht = gen(106, 1, H, T, V).bfloat16(), gen(107, 1, H, K, V)
+    out = []
+    for n in (1, B):
+        rep = lambda t: t.to(cuda).expand(n, *t.shape[1:]).contiguous()
+        d = {k: rep(t).requires_grad_(True) for k, t in x.items()}
+        call = lambda: chunk_gla(d["q"], d["k"], d["v"], d["g"], None, d["h"], True)
+        o, ht = call()
+        grads = torch.autograd.grad([o, ht], list(d.values()), [rep(do), rep(dht)])
+        with torch.no_grad():
+            of, hf = call()
+        out.append([t[:1].detach() for t in (o, ht, of, hf, *grads)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
