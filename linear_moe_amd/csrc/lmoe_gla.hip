@@ -42,7 +42,7 @@ static void launch_gla_t(const lmoe_args& a, int stage, hipStream_t st) {
   const bool wide = Tl::BVS_WIDE != Tl::BVS && (int64_t)a.N * a.H * (V / Tl::BVS_WIDE) >= cu_count();
   switch (stage) {
     case ST_GLA_INTRA_FWD:
-      hipLaunchKernelGGL((k_gla_intra_fwd<T, GT, K>), dim3(persistent_grid(a.NT * a.H, 2)), block, 0, st, a); break;
+      hipLaunchKernelGGL((k_gla_intra_fwd<T, GT, K>), dim3(persistent_grid(a.NT * a.H, 2)), dim3(GLA_INTRA_THREADS), 0, st, a); break;
     case ST_STATE_FWD:
       if constexpr (sizeof(T) == 2) {
         // 2-byte elements: the pass that holds the state also forms the output (k_gla_fwd_fused); hs == NULL: nothing

@@ -97,10 +97,16 @@ __device__ __forceinline__ void gla_gate_tile(const lmoe_args& a, int b, int tok
 //   factors through the cumulative gate at the last token before sub-chunk I, b* = b_{16 I - 1}:
 //     A_ij = sum_k (q_ik e^{b_ik - b*_k}) (k_jk e^{b*_k - b_jk}),   both exponents <= 0,
 //   which is a matrix product of two scaled tiles (MFMA).  Only the four diagonal blocks need the
-//   exponent per pair; they run on the vector ALU in fp32, one block per wave, four pairs per lane.
+//   exponent per pair; they run on the vector ALU in fp32, one block per two waves, two pairs per lane.
+//   LDS holds two (K = 64) or one (K = 128) of its work-groups per CU, each a chain of short phases, so what hides the latencies
+//   of LDS and exponentials is the waves of a work-group: eight in place of four, K = 128, 4096 items 125 -> 102 us, 4-byte
+//   K = 64, 512 items 25.3 -> 19.9, K = 128 88.5 -> 63.9; at K = 64, 2-byte, memory is near (4096 items 52 and 53, 256 9.4 -> 8.2).
 // ------------------------------------------------------------------------- //
+constexpr int GLA_INTRA_THREADS = 2 * NTHR;
+
 template <typename T, typename GT, int K>
-__global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
+__global__ __launch_bounds__(GLA_INTRA_THREADS) __attribute__((amdgpu_waves_per_eu((K <= 64 && sizeof(T) == 2) ? 4 : 2))) void k_gla_intra_fwd(const lmoe_args a) {
+  constexpr int NW = GLA_INTRA_THREADS;
   constexpr int LDB = K + 4, LDK = K + LPAD, LDC = CH + LPAD;
   __shared__ __attribute__((aligned(16))) float s_b[CH * LDB];
   __shared__ __attribute__((aligned(16))) T s_q[CH * LDK];        // q, k as loaded
@@ -111,10 +117,10 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
   __shared__ __attribute__((aligned(16))) T s_qt[(ONE_PASS ? CH : 16) * LDK];   // q~: rows scaled to the reference of their block row
   __shared__ __attribute__((aligned(16))) T s_kt[(ONE_PASS ? 160 : 48) * LDK];  // k~ of block rows 0..3: 16 + 32 + 48 + 64 rows
   __shared__ __attribute__((aligned(16))) T s_A[CH * LDC];
-  const int wv = wave_id(), l = lane_id();
-  typedef TileIO<T, CH, K> IOK;
-  typedef TileIO<T, CH, CH> IOA;
-  typedef GlaGate<GT, K> GG;
+  const int wv = wave_id(), l = lane_id();                         // 8 waves
+  typedef TileIO<T, CH, K, NW> IOK;
+  typedef TileIO<T, CH, CH, NW> IOA;
+  typedef GlaGate<GT, K, NW> GG;
   // persistent: item = (chunk, head); the next item's q, k, g are requested at the top of an item and stay in
   // flight behind its LDS-only barriers (item index clamped: every load is issued)
   const int nitems = num_chunks(a) * a.H;
@@ -145,7 +151,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
   {                                                                                        // blocks above the diagonal
     constexpr int VEC = ET<T>::VEC;
     static_assert((CH * LDC) % VEC == 0, "whole 16-byte pieces");
-    for (int idx = threadIdx.x; idx < CH * LDC / VEC; idx += NTHR) *(typename ET<T>::vec*)(s_A + idx * VEC) = ET<T>::zero();
+    for (int idx = threadIdx.x; idx < CH * LDC / VEC; idx += NW) *(typename ET<T>::vec*)(s_A + idx * VEC) = ET<T>::zero();
   }
   GG::template finish<LDB>(rg, ci.len, s_b, (float*)s_qt, TEXP_PRESCALE<T>);    // barriers inside; b in exp2 units
   // ---- gated operands for the other kernels: q e^{b}, k e^{b_C - b}, e^{b_C} ----
@@ -154,10 +160,10 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
     typedef typename ET<T>::vec vec;
     T* qe = (T*)a.qe + ((int64_t)cid * a.H + h) * CH * K;
     T* ke = (T*)a.ke + ((int64_t)cid * a.H + h) * CH * K;
-    static_assert(CH * K / VEC % NTHR == 0, "whole passes");
+    static_assert(CH * K / VEC % NW == 0, "whole passes");
 #pragma unroll
-    for (int ps = 0; ps < CH * K / VEC / NTHR; ++ps) {
-      const int e = ps * NTHR + threadIdx.x;
+    for (int ps = 0; ps < CH * K / VEC / NW; ++ps) {
+      const int e = ps * NW + threadIdx.x;
       const int r = e / (K / VEC), c0 = (e % (K / VEC)) * VEC;
       const vec qv = *(const vec*)(s_q + r * LDK + c0), kv = *(const vec*)(s_k + r * LDK + c0);
       vec qo, ko;
@@ -199,17 +205,17 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
   } else {
     unsafe = 15;
   }
-  // ---- diagonal blocks that cannot be factored: wave w owns block (w, w); lane -> row i, columns j0 .. j0 + 3 ----
-  if ((unsafe >> wv) & 1) {
-    const int i = 16 * wv + (l & 15), j0 = 16 * wv + 4 * (l >> 4);
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  // ---- diagonal blocks that cannot be factored: waves w and w + 4 own block (w, w); lane -> row i, columns j0, j0 + 1 ----
+  if ((unsafe >> (wv & 3)) & 1) {
+    const int i = 16 * (wv & 3) + (l & 15), j0 = 16 * (wv & 3) + 4 * (l >> 4) + 2 * (wv >> 2);
+    float acc[2] = {0.f, 0.f};
     for (int k4 = 0; k4 < K; k4 += 4) {
       const f32x4 bi = *(const f32x4*)(s_b + i * LDB + k4);
       float qi[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) qi[e] = ET<T>::to_f(s_q[i * LDK + k4 + e]);
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
+      for (int jj = 0; jj < 2; ++jj) {
         const int j = j0 + jj;
         const f32x4 bj = *(const f32x4*)(s_b + j * LDB + k4);
 #pragma unroll
@@ -218,7 +224,7 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
       }
     }
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) s_A[i * LDC + j0 + jj] = ET<T>::from_f(i >= j0 + jj ? acc[jj] : 0.f);
+    for (int jj = 0; jj < 2; ++jj) s_A[i * LDC + j0 + jj] = ET<T>::from_f(i >= j0 + jj ? acc[jj] : 0.f);
   }
   if constexpr (ONE_PASS) {
   // ---- scaled operands of all block rows at once: q~ (64 rows), k~ of block row I = rows 0 .. 16 I + 15 ----
@@ -227,11 +233,12 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
     typedef typename ET<T>::vec vec;
     // stacked rows 0 .. 63: q~; 64 .. 223: k~ of block rows 0 .. 3 (16-byte pieces).  Unrolled: a pass is a chain of
     // LDS reads, exponentials and a write, and seven (fourteen) of them one after the other cost a third of an item
-    constexpr int NPASS = (CH + 160) * (K / VEC) / NTHR;
-    static_assert((CH + 160) * (K / VEC) % NTHR == 0, "whole passes");
+    constexpr int NPC = (CH + 160) * (K / VEC), NPASS = (NPC + NW - 1) / NW;
+    static_assert(NPC % 64 == 0, "whole waves");
 #pragma unroll
     for (int ps = 0; ps < NPASS; ++ps) {
-      const int idx = ps * NTHR + threadIdx.x;
+      const int idx = ps * NW + threadIdx.x;
+      if (NPC % NW != 0 && ps == NPASS - 1 && wv >= NPC % NW / 64) break;
       const int sr = idx / (K / VEC), c0 = (idx % (K / VEC)) * VEC;
       const bool isq = sr < CH;
       const int kr = sr - CH;                                           // row of the stacked k~ tile
@@ -251,30 +258,31 @@ __global__ __launch_bounds__(NTHR) void k_gla_intra_fwd(const lmoe_args a) {
     }
   }
   lds_barrier();
-  // wave w: the blocks (I, w), I = w .. 3; the diagonal one masked to i >= j
-#pragma unroll
-  for (int I = 0; I < 4; ++I) {
-    if (wv > I || (wv == I && ((unsafe >> I) & 1))) continue;
+  // the ten blocks (I, J), J <= I, counted row by row from the last: wave w takes w and, of the first two, w + 8; the diagonal
+  // ones masked to i >= j
+  for (int nb = 9 - wv; nb >= 0; nb -= 8) {
+    const int I = nb < 1 ? 0 : nb < 3 ? 1 : nb < 6 ? 2 : 3, J = nb - I * (I + 1) / 2;
+    if (I == J && ((unsafe >> I) & 1)) continue;
     f32x4 t[1][1];
     acc_zero(t);
-    gemm<T, 1, 1, false, false, true>(t, s_qt, LDK, 16 * I, s_kt + KT_ROW0(I) * LDK, LDK, 16 * wv, 0, K);
-    if (wv == I) {
+    gemm<T, 1, 1, false, false, true>(t, s_qt, LDK, 16 * I, s_kt + KT_ROW0(I) * LDK, LDK, 16 * J, 0, K);
+    if (I == J) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         if (4 * (l >> 4) + e < (l & 15)) t[0][0][e] = 0.f;
     }
-    acc_to_lds<T>(t[0][0], s_A, LDC, 16 * I, 16 * wv);
+    acc_to_lds<T>(t[0][0], s_A, LDC, 16 * I, 16 * J);
   }
   lds_barrier();
   } else {
     // ---- blocks below the diagonal, one block row at a time ----
     for (int I = 1; I < 4; ++I) {
       const float* bs = s_b + (16 * I - 1) * LDB;                   // b* of this block row
-      for (int idx = threadIdx.x; idx < 16 * K; idx += NTHR) {
+      for (int idx = threadIdx.x; idx < 16 * K; idx += NW) {
         const int r = idx / K, c = idx % K, i = 16 * I + r;
         s_qt[r * LDK + c] = ET<T>::from_f(ET<T>::to_f(s_q[i * LDK + c]) * texp_scaled<T>(s_b[i * LDB + c] - bs[c]));
       }
-      for (int idx = threadIdx.x; idx < 16 * I * K; idx += NTHR) {
+      for (int idx = threadIdx.x; idx < 16 * I * K; idx += NW) {
         const int j = idx / K, c = idx % K;
         s_kt[j * LDK + c] = ET<T>::from_f(ET<T>::to_f(s_k[j * LDK + c]) * texp_scaled<T>(bs[c] - s_b[j * LDB + c]));
       }
