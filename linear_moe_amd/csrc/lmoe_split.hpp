@@ -142,15 +142,26 @@ template <bool CUT> __device__ __forceinline__ PassItem pass_item_dense(const lm
   p.last = j == nseg - 1;
   return p;
 }
+// What the rules below expect of a cut, as a part of the whole call by their figures: 0.9, less at K = V = 128 where the pass over whole
+// sequences takes slices of 16 columns (2-byte elements, a CU for each), which the figures do not know.  There (one call replayed as
+// a graph, us, cut : whole, forward; forward and backward) cuts lost at 0.90 of the delta rule's figures 50.0 : 47.4; 122 : 112 (16 pairs
+// of 28 chunks), of chunk_simple_gla's at 0.84 29.2 : 26.1; 83 : 71 (16 of 20), at 0.88 42.4 : 40.6; 114 : 106 (24 of 32), at 0.89 43.8 : 42.2;
+// 127 : 118 (32 of 32), and stay where the forward pass alone still wins: 0.80 57.3 : 62.1; 148 : 149 (16 of 40), 0.81 50.7 : 52.7; 126 : 122
+// (16 of 32), 0.83 22.2 : 22.9; 58 : 53 (8 of 17).  At K = V = 64 every cut up to 0.9 wins (by 1.08 to 2), and chunk_gla's do at
+// either.  Several packed sequences keep 0.9: the longest, which the average does not show, gains more.
+inline float cut_limit(const lmoe_args& a, float at128) {
+  const bool narrow = (!a.cu_seqlens || a.N == 1) && a.dtype == LMOE_BF16 && a.V <= 128 && (int64_t)a.N * a.H * (a.V / 16) <= cu_count();
+  return narrow ? 0.9f - (0.9f - at128) * fmaxf(0.f, (a.K + a.V) / 128.f - 1.f) : 0.9f;
+}
 // How a call is cut (pointers left open), or len1 = 0.  `slices` = work-groups of the ordinary pass per (sequence, head),
 // which hold a CU each; the work-groups of step 1 carry all columns and hold a CU each too.  Chosen by what the three steps
 // were measured to take (us, K = V = 128, delta rule; half of it per chunk at K = V = 64):
 //   ordinary pass   1.7 per chunk up to 64 work-groups, 2.1 beyond, 2.2 on a full GPU
 //   step 1          7 + 3.3 per chunk        step 2   4 + 0.65 per fine segment       step 3   1 + 2.2 per chunk
 // These are the passes with two and three barriers per chunk the rule was fitted to; the forward pass now takes 1.35 to 1.6 per
-// chunk.  Its cuts still win where the kernels count (one pass replayed as a graph, whole -> cut, K = V = 128: training 16 pairs
-// of 32 chunks 136 -> 124, 20 of 38 163 -> 162, 16 of 256 920 -> 615; forward 16 pairs of 47 chunks 80 -> 63, 8 of 24 46 -> 39;
-// all 324 calls of a sweep over pairs and lengths by a factor of 1.08 to 3.3).  A training call of up to 48 chunks that the
+// chunk, with slices of 16 columns less (cut_limit).  Where the kernels count (one pass replayed as a graph, whole -> cut, K = V = 128):
+// training 16 pairs of 48 chunks 170 -> 158, 16 of 256 920 -> 615; forward 16 pairs of 47 chunks 80 -> 63, 8 of 32 48 -> 43.  A
+// training call of up to 48 chunks that the
 // host issues one by one is bound by the host, and the cut's launches show (8 pairs of 24 chunks 125 -> 140).
 inline Split plan_split(const lmoe_args& a, int slices) {
   Split s = {};
@@ -171,7 +182,7 @@ inline Split plan_split(const lmoe_args& a, int slices) {
   const int rmax = packed && a.N > 1 ? (slots - a.N) / a.N : slots / a.N;
   if (chunks > seqs * SPLIT_MAX_CHUNKS) return s;
   for (int nch = packed ? seg_count(chunks + seqs, seqs) : least; nch >= least && nch >= SPLIT_MIN_CHUNKS && !s.len1; --nch) {
-    float best = 0.9f * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
+    float best = cut_limit(a, 0.85f) * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
     for (int r = 3; r <= rmax && r <= 32; ++r)
       for (int f = 1; f <= 4; ++f) {
         const int len3 = seg_count(nch, r), len1 = seg_count(len3, f), nf = seg_count(nch, len1);
@@ -190,7 +201,7 @@ inline Split plan_split(const lmoe_args& a, int slices) {
 // pass takes 2.5 to start, and `pre` per fine segment it starts from: work-groups in several rounds pay that every time.
 // Without these two terms 16 pairs of 49 chunks (K = V = 128, retention) were cut into 25 (1600 work-groups of two chunks,
 // 82 us for the pass that takes 64 in one piece), 28 pairs of 110 chunks into 16 (123 against 138).
-inline Split plan_cut(const lmoe_args& a, float c3, float b3, float c1, float pre, int64_t wg3, int64_t wg1) {
+inline Split plan_cut(const lmoe_args& a, float limit, float c3, float b3, float c1, float pre, int64_t wg3, int64_t wg1) {
   Split s = {};
   const int cus = cu_count(), nch = (a.T + CH - 1) / CH;
   const float w = (a.K + a.V) / 256.f;
@@ -199,7 +210,7 @@ inline Split plan_cut(const lmoe_args& a, float c3, float b3, float c1, float pr
     const int64_t full = wg / cus, rest = wg % cus;
     return 2.5f * rounds(wg, cus) + chunks * (full * (c3 + b3) + (rest ? c3 + b3 * rest / cus : 0.f));
   };
-  float best = 0.9f * pass(wg3, nch);
+  float best = limit * pass(wg3, nch);
   for (int r = 2; r <= 32 && r <= nch; ++r) {
     const int len3 = seg_count(nch, r);
     if (seg_count(nch, len3) != r) continue;
@@ -238,7 +249,7 @@ inline Split plan_split_scalar(const lmoe_args& a) {
   // forward and backward together, 384 of K = V = 128 759 -> 857)
   if (!f4 && a.normalize && 2 * wg3 >= cus) return s;
   const float c3 = f4 ? 1.9f + 4.1f * w : 0.45f + 0.85f * w, c1 = f4 ? 1.f + 2.f * w : 0.3f + 0.6f * w;
-  return plan_cut(a, c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
+  return plan_cut(a, cut_limit(a, 0.835f), c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
 }
 // The same for chunk_gla (2-byte elements, dense; a transition is one decay per state row).  The pass fetches q, k and the
 // intra-chunk matrix once per V slice of 32, so a chunk costs more the more CUs run one.  Measured, us per chunk with 64, 128,
@@ -251,7 +262,7 @@ inline Split plan_split_gla(const lmoe_args& a) {
   // wide slices fill the CUs; short and very long sequences are left whole, as above
   if ((int64_t)pairs * (a.V / 64) >= cu_count() || nch < 17 || nch > SPLIT_MAX_CHUNKS) return Split{};
   const float w = (a.K + a.V) / 256.f;
-  return plan_cut(a, 0.35f + 0.4f * w, 0.6f + 0.4f * w, 0.4f + 0.8f * w, 0.5f * w, (int64_t)pairs * (a.V / 32), pairs);
+  return plan_cut(a, 0.9f, 0.35f + 0.4f * w, 0.6f + 0.4f * w, 0.4f + 0.8f * w, 0.5f * w, (int64_t)pairs * (a.V / 32), pairs);
 }
 // S <- D S + Q over the n fine segments in front of a coarse one, in order (step = -1: behind it, from the last on).
 // q, d: Q (its column v0 + lane % 16, row krow0 + 4 (lane / 16)) and D of the first; four segments' loads at a time.

@@ -204,6 +204,28 @@ def delta_inputs(seed, B, T, H, K, V, N, gated=True):
     return ins, bf(gen(seed + 6, B, T, H, V)), gen(seed + 7, N, H, K, V)
 
 
+@pytest.mark.parametrize("op,H,T,D,cut", [(0, 16, 1280, 128, False), (0, 32, 2048, 128, False), (0, 16, 2048, 128, True), (0, 16, 1280, 64, True),
+                                          (2, 16, 1792, 128, False), (2, 16, 3008, 128, True), (2, 16, 2048, 64, True)])
+def test_calls_that_narrow_slices_outrun_are_left_whole(cuda, op, H, T, D, cut):
+    """On both sides of the line, dense and as one packed sequence; left whole, a call gives the bits that its rows have in a batch that fills the CUs."""
+    from linear_moe_amd import chunk_gated_delta_rule, chunk_simple_gla
+    assert (lengths(op, 1, T, H, D, D)[0] > 0) == cut
+    if op == 2:
+        assert (lengths(op, 1, T, H, D, D, 1)[0] > 0) == cut
+    x = [F.normalize(gen(7600, 1, T, H, D), dim=-1).bfloat16(), F.normalize(gen(7601, 1, T, H, D), dim=-1).bfloat16(),
+         gen(7602, 1, T, H, D).bfloat16(), -F.softplus(gen(7603, 1, T, H)) * 0.01, torch.sigmoid(gen(7604, 1, T, H)).bfloat16()]
+
+    def run(n):
+        d = [t.to(cuda).expand(n, *t.shape[1:]).contiguous().requires_grad_() for t in x[:5 if op == 2 else 4]]
+        f = chunk_gated_delta_rule if op == 2 else chunk_simple_gla
+        o, ht = f(*d, output_final_state=True, head_first=False)
+        return [t[:1].detach() for t in (o, ht, *torch.autograd.grad(o, d, torch.ones_like(o)))]
+    few, many = run(1), run(8)
+    for a, b in zip(few, many):
+        assert max_abs_rel(a, b) < TOL[torch.bfloat16]
+        assert cut or torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B,T,H,K,V,lens,cut", [
     (1, 3001, 16, 128, 128, None, (3, 12)),        # four coarse segments, the last one of 11 chunks
     (1, 6000, 4, 64, 128, None, (3, 6)),           # the last one of two fine segments, the second of one chunk
