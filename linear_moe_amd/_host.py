@@ -407,12 +407,14 @@ def native_call(fn: str, what: str, x, *args):
 
 
 def no_node(*xs) -> bool:
-    """Whether a call needs no node of the autograd graph: no gradient is wanted, and nothing is at work (a transform, forward-mode
-    differentiation) that has to see the op as a function of autograd and refuses it there.  Its steps then run without
-    one (5 us of a call that takes the GPU 9)."""
+    """Whether a call needs no node of the autograd graph: no gradient is wanted, and nothing is at work that has to see the op as a
+    function of autograd, to refuse it there (a transform, forward-mode differentiation) or to run it again (a trace being
+    recorded, which would hold the allocations of the steps alone).  Its steps then run without one (5 us of a call that
+    takes the GPU 9)."""
     if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in xs):
         return False
-    return not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0
+    return (not torch._C._are_functorch_transforms_active() and forward_ad._current_level < 0
+            and torch._C._get_tracing_state() is None)
 
 
 def ptr(x: Optional[torch.Tensor]):

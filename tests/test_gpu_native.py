@@ -495,3 +495,21 @@ def test_calls_without_a_node_are_still_functions_of_autograd_for_transforms(cud
         torch.func.vmap(lambda x: L.chunk_simple_gla(x, k, v)[0])(q.unsqueeze(0))
     with pytest.raises(RuntimeError):                      # (nothing of the call is mapped over)
         torch.func.vmap(lambda x: L.chunk_simple_gla(q, k, v)[0] + x)(torch.zeros(2, device=cuda))
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("op", ["simple_gla", "linear_attn", "linear_attn normalized", "gla", "gated_delta_rule"])
+def test_a_trace_replays_the_op_on_other_inputs(cuda, op):
+    import linear_moe_amd as L
+    f = {"simple_gla": lambda q, k, v: L.chunk_simple_gla(q, k, v, output_final_state=True),
+         "linear_attn": lambda q, k, v: L.chunk_linear_attn(q, k, v, normalize=False, output_final_state=True),
+         "linear_attn normalized": lambda q, k, v: L.chunk_linear_attn(q.abs(), k.abs(), v, output_final_state=True),
+         "gla": lambda q, k, v: L.chunk_gla(q, k, v, -k.abs(), output_final_state=True),
+         "gated_delta_rule": lambda q, k, v: L.chunk_gated_delta_rule(q, k, v, -q[..., 0].abs(), torch.sigmoid(k[..., 0]),
+                                                                      output_final_state=True)}[op]
+    gen = torch.Generator(device=cuda).manual_seed(2)
+    x, y = ([0.1 * torch.randn(1, 130, 2, 64, device=cuda, generator=gen).bfloat16() for _ in range(3)] for _ in range(2))
+    with torch.no_grad():
+        traced = torch.jit.trace(f, x, check_trace=False)
+        for a, b in zip(traced(*y), f(*y)):
+            assert torch.equal(a, b)

@@ -587,3 +587,35 @@ def test_saved_tensors_come_back_as_they_were_saved():
     for y in (None, x[:, :1], x[..., :-4], x.flatten(), x.to("meta")):
         with pytest.raises(RuntimeError, match="hs, saved for the backward"):
             came_back(y, (3, 2, 64, 128), torch.bfloat16, dev, "hs")
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("grad_mode", [True, False])
+@pytest.mark.parametrize("op", ["simple_gla", "normalized", "linear_attn", "gla", "gated_delta_rule"])
+def test_a_recorded_trace_runs_the_op(monkeypatch, op, grad_mode):
+    """A call whose inputs want no gradient runs without a node of the graph, but not while a trace is recorded: a trace holds the
+    node and runs it again on the inputs of the replay; of what the library does it would see the allocation alone.  (The
+    steps of the call are stood in for by a write that torch does not see, as the library's are.)"""
+    import linear_moe_amd as L
+    from linear_moe_amd.gated_delta_rule import GDNCall
+    from linear_moe_amd.gla import GLACall
+    from linear_moe_amd.simple_gla import SimpleGLACall, chunk_simple_gla_normalized
+
+    def steps(self, q, k, v, *args, **kw):
+        o = torch.empty_like(v)
+        C.memmove(o.data_ptr(), v.data_ptr(), v.numel() * v.element_size())
+        self.saved = ()
+        return o, None
+    for call in (SimpleGLACall, GLACall, GDNCall):
+        monkeypatch.setattr(call, "forward", steps)
+    dt = torch.bfloat16 if op == "normalized" else torch.float32
+    x = [torch.randn(1, 2, 5, 64, dtype=dt) for _ in range(3)]
+    f = {"simple_gla": lambda q, k, v: L.chunk_simple_gla(q, k, v)[0],
+         "normalized": lambda q, k, v: chunk_simple_gla_normalized(q, k, v)[0],
+         "linear_attn": lambda q, k, v: L.chunk_linear_attn(q, k, v, normalize=False)[0],
+         "gla": lambda q, k, v: L.chunk_gla(q, k, v, q)[0],
+         "gated_delta_rule": lambda q, k, v: L.chunk_gated_delta_rule(q, k, v, q[..., 0], k[..., 0])[0]}[op]
+    with torch.set_grad_enabled(grad_mode):
+        assert torch.equal(f(*x), x[2])
+        traced = torch.jit.trace(f, x, check_trace=False)
+        y = [torch.randn_like(t) for t in x]
+        assert torch.equal(traced(*y), y[2])
