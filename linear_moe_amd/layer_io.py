@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._host import native_call, stash, stream_ptr, unstash
+from ._host import came_back, native_call, stash, stream_ptr, unstash
 
 
 def _dt(x):
@@ -133,6 +133,7 @@ def gdn_qkv_prologue(qkv: torch.Tensor, num_heads: int, head_dim: int, eps: floa
 class _SwishGateRelayout(torch.autograd.Function):
     @staticmethod
     def forward(ctx, o, gate):
+        ctx.shapes, ctx.dtype = (o.shape, gate.shape), o.dtype
         r = native_call("swish_forward", "swish_gate_relayout", o, gate)
         if r is not None:
             ctx.save_for_backward(o, gate)
@@ -160,9 +161,11 @@ class _SwishGateRelayout(torch.autograd.Function):
         r = native_call("swish_backward", "swish_gate_relayout backward", oc, gc, dy)
         if r is not None:
             return r
-        B, T, W = oc.shape[0], oc.shape[1], oc.shape[2] * oc.shape[3]
+        (B, T, H, D), gshape = ctx.shapes
+        W = H * D
+        oc, gc = came_back(oc, (B, T, H, D), ctx.dtype, dy.device, "o"), came_back(gc, gshape, ctx.dtype, dy.device, "o_gate")
+        dyc = came_back(dy, (T, B, W), ctx.dtype, dy.device, "the gradient")
         lib = _lib.load()
-        dyc = dy.contiguous()
         do, dgate = torch.empty_like(oc), torch.empty_like(gc)
         _lib.check(lib.lmoe_swish_gate_relayout_bwd(oc.data_ptr(), gc.data_ptr(), dyc.data_ptr(), do.data_ptr(),
                                                     dgate.data_ptr(), T, B, W, _dt(oc), stream_ptr()),

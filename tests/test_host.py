@@ -619,3 +619,81 @@ def test_a_recorded_trace_runs_the_op(monkeypatch, op, grad_mode):
         traced = torch.jit.trace(f, x, check_trace=False)
         y = [torch.randn_like(t) for t in x]
         assert torch.equal(traced(*y), y[2])
+
+
+def _neighbours():
+    """name -> (call of the leaves, leaves, the library's backward function, place among its arguments of every saved tensor in the order
+    they are saved and of the gradients behind them)"""
+    import linear_moe_amd as L
+    rn = lambda *s: torch.randn(*s, generator=torch.Generator().manual_seed(3)).bfloat16()
+    return {"swish": (L.swish_gate_relayout, (rn(2, 5, 2, 64), rn(5, 2, 128)), "lmoe_swish_gate_relayout_bwd", (0, 1, 2))}
+
+
+def _misaligned(x):
+    flat = torch.empty(x.numel() + 1, dtype=x.dtype)
+    flat[1:] = x.reshape(-1)
+    return flat[1:].view(x.shape)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name", ["swish"])
+def test_the_neighbours_backward_reads_what_was_saved(monkeypatch, name, dt):
+    """A saved-tensor hook hands back what it likes: the library's backward gets the sizes and the type of the call and, at every
+    pointer, the rows that were saved (another type, strides or place in memory of what came back), or nothing is launched
+    (another shape).  On the CPU, with a stand-in for the library that keeps what it is handed."""
+    from linear_moe_amd import _lib, feature_map, gates, l2norm, layer_io, mom, rmsnorm
+    fn, leaves, bwd, inputs = _neighbours()[name]
+    leaves = [x.to(dt) if x.dtype == torch.bfloat16 else x for x in leaves]
+    for mod in (feature_map, gates, l2norm, layer_io, mom, rmsnorm):
+        monkeypatch.setattr(mod, "native_call", lambda *a: None, raising=False)
+        monkeypatch.setattr(mod, "stream_ptr", lambda: 0)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    real, calls, ref = _lib.load(), [], []
+
+    class Library:
+        def __getattr__(self, f):
+            if f != bwd:
+                return getattr(real, f) if f.endswith(("_partials", "_features")) else lambda *a: 0
+
+            def call(*a):
+                sizes = [x for x in a if not (isinstance(x, int) and x > 1 << 32) and x is not None]
+                assert not ref or sizes == ref[0][0], (sizes, ref[0][0])
+                calls.append((sizes, [C.string_at(a[i], n) for i, n in extents.items()]))
+                return 0
+            return call
+    monkeypatch.setattr(_lib, "load", Library)
+    extents = {}
+
+    def through(change):
+        ls, n = [x.detach().clone().requires_grad_(x.is_floating_point()) for x in leaves], [0]
+
+        def pack(t):
+            n[0] += 1
+            return n[0] - 1, t
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda p: change(*p)):
+            outs = fn(*ls)
+        outs = list(outs) if isinstance(outs, (tuple, list)) else [outs]
+        gen = torch.Generator().manual_seed(5)
+        douts = [torch.randn(o.shape, generator=gen).to(o.dtype) for o in outs]
+        grads = torch.autograd.grad(outs, [x for x in ls if x.requires_grad], douts, allow_unused=True)
+        assert all(g is None or (g.shape == x.shape and g.dtype == x.dtype) for g, x in zip(grads, ls))
+        return douts
+
+    saved = []
+    douts = through(lambda i, t: saved.append(t) or t)
+    for i, t in zip(inputs, [*saved, *douts]):
+        extents[i] = t.numel() * t.element_size()
+    calls.clear()
+    through(lambda i, t: t)
+    ref.append(calls.pop())
+    for i, t in enumerate(saved):
+        if t is None or not t.is_floating_point():
+            continue
+        for f in (lambda x: x.float() if x.dtype == torch.bfloat16 else x.double(), _misaligned,
+                  lambda x: x.mT.contiguous().mT if x.dim() > 1 else x.double()):
+            through(lambda j, x: f(x) if i == j else x)
+            assert calls.pop() == ref[0], i
+        for f in (lambda x: x[:-1], lambda x: x[..., :-8] if x.shape[-1] > 8 else x[..., :-1]):
+            with pytest.raises((RuntimeError, ValueError)):
+                through(lambda j, x: f(x) if i == j else x)
+    assert not calls
