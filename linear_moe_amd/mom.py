@@ -25,7 +25,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._host import native_call, stream_ptr
+from ._host import came_back, native_call, stream_ptr
 
 
 @dataclass
@@ -195,9 +195,10 @@ class _Pack(torch.autograd.Function):
 class _Combine(torch.autograd.Function):
     @staticmethod
     def forward(ctx, y, w, plan):
-        ctx.plan, ctx.yshape, ctx.wshape, ctx.wdtype = plan, y.shape, w.shape, w.dtype
+        ctx.plan, ctx.yshape, ctx.wshape, ctx.dtype, ctx.wdtype = plan, y.shape, w.shape, y.dtype, w.dtype
         r = native_call("mom_combine", "mom_combine", y, plan.T_total, plan.row_of, w, plan.B * plan.S, plan.topk)
         if r is not None:
+            ctx.saved_shapes = y.shape, w.shape
             ctx.save_for_backward(y, w)
             return r[0].view((plan.B, plan.S) + tuple(y.shape[1:]))
         lib = _lib.load()
@@ -207,6 +208,7 @@ class _Combine(torch.autograd.Function):
         out = torch.empty(plan.B * plan.S, D, dtype=y.dtype, device=y.device)
         _lib.check(lib.lmoe_mom_combine(y2.data_ptr(), plan.row_of.data_ptr(), w2.data_ptr(), out.data_ptr(),
                                         plan.B * plan.S, plan.topk, D, _dt(y), stream_ptr()), "mom_combine")
+        ctx.saved_shapes = y2.shape, w2.shape
         ctx.save_for_backward(y2, w2)
         return out.view((plan.B, plan.S) + tuple(y.shape[1:]))
 
@@ -219,9 +221,11 @@ class _Combine(torch.autograd.Function):
         if r is not None:
             return r[0].view(ctx.yshape), r[1].view(ctx.wshape).to(ctx.wdtype), None
         lib = _lib.load()
-        y2, w2 = y2.reshape(plan.T_total, -1), w2.reshape(plan.B * plan.S, plan.topk)
-        D = y2.shape[1]
-        g = dout.reshape(plan.B * plan.S, D).contiguous()
+        yshape, wshape = ctx.saved_shapes
+        D = yshape[1:].numel()
+        y2 = came_back(y2, yshape, ctx.dtype, dout.device, "y")
+        w2 = came_back(w2, wshape, ctx.dtype, dout.device, "routing_weights")
+        g = came_back(dout, (plan.B, plan.S, *ctx.yshape[1:]), ctx.dtype, dout.device, "the gradient")
         # dy[row] = w[choice(row)] * dout[token(row)];  dw[t][k] = <dout[t], y[row_of[t][k]]>
         dy, dw = torch.empty_like(y2), torch.empty_like(w2)
         _lib.check(lib.lmoe_mom_combine_bwd(y2.data_ptr(), plan.row_of.data_ptr(), plan.src_choice.data_ptr(),
