@@ -15,7 +15,7 @@ import math
 import torch
 
 from . import _lib
-from ._host import native_call, stream_ptr
+from ._host import came_back, native_call, stream_ptr
 
 
 def _dt(t):
@@ -28,6 +28,7 @@ class _GdnGates(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a, b, A_log, dt_bias):
         ctx.pdt = (A_log.dtype, dt_bias.dtype)
+        ctx.shape, ctx.dtype = a.shape, a.dtype
         r = native_call("gates_forward", "gdn_gates", a, b, A_log, dt_bias)
         if r is not None:
             ctx.save_for_backward(a, b, A_log, dt_bias)
@@ -56,8 +57,10 @@ class _GdnGates(torch.autograd.Function):
         r = native_call("gates_backward", "gdn_gates backward", ac, bc, Af, Bf, dg, dbeta)
         if r is not None:
             return (*r[:2], r[2].to(ctx.pdt[0]), r[3].to(ctx.pdt[1]))
+        dev, H = (dg if dbeta is None else dbeta).device, ctx.shape[-1]
+        ac, bc = came_back(ac, ctx.shape, ctx.dtype, dev, "a"), came_back(bc, ctx.shape, ctx.dtype, dev, "b")
+        Af, Bf = came_back(Af, (H,), torch.float32, dev, "A_log"), came_back(Bf, (H,), torch.float32, dev, "dt_bias")
         lib = _lib.load()
-        H = ac.shape[-1]
         rows = ac.numel() // H
         dgc = (torch.zeros_like(ac, dtype=torch.float32) if dg is None else dg.float().contiguous())
         dbc = (torch.zeros_like(bc) if dbeta is None else dbeta.to(bc.dtype).contiguous())

@@ -628,7 +628,8 @@ def _neighbours():
     rn = lambda *s: torch.randn(*s, generator=torch.Generator().manual_seed(3)).bfloat16()
     plan = L.mom_plan(torch.tensor([[[0, 2], [1, 2], [2, 0]]]), 3)
     return {"swish": (L.swish_gate_relayout, (rn(2, 5, 2, 64), rn(5, 2, 128)), "lmoe_swish_gate_relayout_bwd", (0, 1, 2)),
-            "combine": (lambda y, w: L.mom_combine(y, plan, w), (rn(6, 2, 64), rn(1, 3, 2)), "lmoe_mom_combine_bwd", (0, 3, 4))}
+            "combine": (lambda y, w: L.mom_combine(y, plan, w), (rn(6, 2, 64), rn(1, 3, 2)), "lmoe_mom_combine_bwd", (0, 3, 4)),
+            "gates": (L.gdn_gates, (rn(2, 5, 8), rn(2, 5, 8), rn(8).float(), rn(8).float()), "lmoe_gdn_gates_bwd", (0, 1, 2, 3, 4, 5))}
 
 
 def _misaligned(x):
@@ -638,7 +639,7 @@ def _misaligned(x):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("name", ["swish", "combine"])
+@pytest.mark.parametrize("name", ["swish", "combine", "gates"])
 def test_the_neighbours_backward_reads_what_was_saved(monkeypatch, name, dt):
     """A saved-tensor hook hands back what it likes: the library's backward gets the sizes and the type of the call and, at every
     pointer, the rows that were saved (another type, strides or place in memory of what came back), or nothing is launched
