@@ -16,7 +16,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._host import stream_ptr
+from ._host import came_back, stream_ptr
 
 
 class KeyBlocks(tuple):
@@ -62,7 +62,7 @@ class _QuadFeatureMap(torch.autograd.Function):
         _lib.check(lib.lmoe_quad_featmap_fwd(xc.data_ptr(), buf.data_ptr(), rows, D, Kp, c0, c1, cd, co, dt, stream_ptr()),
                    "quad_feature_map")
         ctx.save_for_backward(xc)
-        ctx.args = (D, Kp, c0, c1, cd, co, dt)
+        ctx.args, ctx.shape, ctx.dtype = (D, Kp, c0, c1, cd, co, dt), x.shape, x.dtype
         blocks, off = [], 0
         for w in _widths(Kp):
             blocks.append(buf[off:off + rows * w].view(*x.shape[:-1], w))
@@ -74,6 +74,7 @@ class _QuadFeatureMap(torch.autograd.Function):
     def backward(ctx, *dblocks):
         (xc,) = ctx.saved_tensors
         D, Kp, c0, c1, cd, co, dt = ctx.args
+        xc = came_back(xc, ctx.shape, ctx.dtype, next((d.device for d in dblocks if d is not None), xc.device), "x")
         lib = _lib.load()
         rows = xc.numel() // D
         dy = torch.empty(rows * Kp, dtype=xc.dtype, device=xc.device)

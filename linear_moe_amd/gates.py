@@ -95,14 +95,14 @@ class _GlaGate(torch.autograd.Function):
         _lib.check(lib.lmoe_gla_gate_fwd(xc.data_ptr(), y.data_ptr(), xc.numel(), _dt(x), float(normalizer), cm,
                                          stream_ptr()), "gla_gate")
         ctx.save_for_backward(xc)
-        ctx.args = (float(normalizer), cm)
+        ctx.args, ctx.shape, ctx.dtype = (float(normalizer), cm), x.shape, x.dtype
         return y
 
     @staticmethod
     def backward(ctx, dy):
         (xc,) = ctx.saved_tensors
+        xc, dyc = came_back(xc, ctx.shape, ctx.dtype, dy.device, "x"), came_back(dy, ctx.shape, ctx.dtype, dy.device, "the gradient")
         lib = _lib.load()
-        dyc = dy.contiguous()
         dx = torch.empty_like(xc)
         _lib.check(lib.lmoe_gla_gate_bwd(xc.data_ptr(), dyc.data_ptr(), dx.data_ptr(), xc.numel(), _dt(xc), ctx.args[0],
                                          ctx.args[1], stream_ptr()), "gla_gate backward")
@@ -134,11 +134,15 @@ class _Hgrn2Gates(torch.autograd.Function):
         _lib.check(lib.lmoe_hgrn2_gate_fwd(fc.data_ptr(), None if lb is None else lb.data_ptr(), k.data_ptr(), g.data_ptr(),
                                            fc.numel(), D, _dt(f), stream_ptr()), "hgrn2_gates")
         ctx.save_for_backward(fc, lb)
+        ctx.shape, ctx.dtype, ctx.bounded = f.shape, f.dtype, lb is not None
         return k, g
 
     @staticmethod
     def backward(ctx, dk, dg):
         fc, lb = ctx.saved_tensors
+        dev = (dk if dg is None else dg).device
+        fc = came_back(fc, ctx.shape, ctx.dtype, dev, "f")
+        lb = came_back(lb, ctx.shape[-1:], torch.float32, dev, "lower_bound") if ctx.bounded else None
         lib = _lib.load()
         dkc = torch.zeros_like(fc) if dk is None else dk.to(fc.dtype).contiguous()
         dgc = torch.zeros_like(fc, dtype=torch.float32) if dg is None else dg.float().contiguous()

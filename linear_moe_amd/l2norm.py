@@ -10,7 +10,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._host import stream_ptr
+from ._host import came_back, stream_ptr
 
 _DIMS = (64, 128, 256)
 
@@ -32,15 +32,15 @@ class _L2Norm(torch.autograd.Function):
         fwd = lib.lmoe_silu_l2norm_fwd if silu else lib.lmoe_l2norm_fwd
         _lib.check(fwd(xc.data_ptr(), y.data_ptr(), xc.numel() // D, D, dt, eps, stream_ptr()), "l2_norm")
         ctx.save_for_backward(xc)
-        ctx.eps, ctx.dt, ctx.silu = eps, dt, silu
+        ctx.shape, ctx.dtype, ctx.eps, ctx.dt, ctx.silu = x.shape, x.dtype, eps, dt, silu
         return y
 
     @staticmethod
     def backward(ctx, dy):
         (xc,) = ctx.saved_tensors
+        D = ctx.shape[-1]
+        xc, dyc = came_back(xc, ctx.shape, ctx.dtype, dy.device, "x"), came_back(dy, ctx.shape, ctx.dtype, dy.device, "the gradient")
         lib = _lib.load()
-        D = xc.shape[-1]
-        dyc = dy.contiguous()
         dx = torch.empty_like(xc)
         bwd = lib.lmoe_silu_l2norm_bwd if ctx.silu else lib.lmoe_l2norm_bwd
         _lib.check(bwd(xc.data_ptr(), dyc.data_ptr(), dx.data_ptr(), xc.numel() // D, D, ctx.dt, ctx.eps, stream_ptr()),

@@ -40,13 +40,15 @@ class _QKVPrologue(torch.autograd.Function):
         _lib.check(lib.lmoe_gdn_qkv_prologue_fwd(x.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), T, B, H, D, dt, eps,
                                                  stream_ptr()), "gdn_qkv_prologue")
         ctx.save_for_backward(x)
-        ctx.dims, ctx.eps, ctx.dt, ctx.shape = (T, B, H, D), eps, dt, qkv.shape
+        ctx.dims, ctx.eps, ctx.dt, ctx.shape, ctx.dtype = (T, B, H, D), eps, dt, qkv.shape, qkv.dtype
         return q, k, v
 
     @staticmethod
     def backward(ctx, dq, dk, dv):
         (x,) = ctx.saved_tensors
         T, B, H, D = ctx.dims
+        dev = next((g.device for g in (dq, dk, dv) if g is not None), x.device)
+        x = came_back(x, ctx.shape, ctx.dtype, dev, "qkv")
         lib = _lib.load()
         dq, dk, dv = (torch.zeros(B, T, H, D, dtype=x.dtype, device=x.device) if g is None else g.contiguous()
                       for g in (dq, dk, dv))
@@ -102,6 +104,7 @@ class _GDNMixerCore(torch.autograd.Function):
             if r is not None:
                 (dx, dg, dbeta), g = r, ctx.call.saved[3]
                 return dx.view(ctx.shape), dg if dg is None else dg.to(g.dtype), dbeta, None, None, None, None
+            x = came_back(x, ctx.shape, torch.bfloat16, do.device, "qkv")
             dx = torch.empty_like(x)
             blocks = lambda t: [t.view(T, B, H, 3 * D)[..., i * D:(i + 1) * D].transpose(0, 1) for i in range(3)]
             dxq, dxk, dxv = blocks(dx)

@@ -13,7 +13,7 @@ import torch
 from torch import nn
 
 from . import _lib
-from ._host import stream_ptr
+from ._host import came_back, stream_ptr
 
 _DIMS = (64, 128, 256)
 
@@ -44,16 +44,19 @@ class _RMSNorm(torch.autograd.Function):
                                             None if gc is None else gc.data_ptr(), y.data_ptr(), None, rows, D, dt, eps,
                                             stream_ptr()), "rms_norm")
         ctx.save_for_backward(xc, wc, gc)
-        ctx.eps, ctx.dt, ctx.wdtype = eps, dt, None if weight is None else weight.dtype
+        ctx.shape, ctx.dtype, ctx.eps, ctx.dt, ctx.wdtype = x.shape, x.dtype, eps, dt, None if weight is None else weight.dtype
+        ctx.gated = gate is not None
         return y
 
     @staticmethod
     def backward(ctx, dy):
         xc, wc, gc = ctx.saved_tensors
+        D = ctx.shape[-1]
+        xc, dyc = came_back(xc, ctx.shape, ctx.dtype, dy.device, "x"), came_back(dy, ctx.shape, ctx.dtype, dy.device, "the gradient")
+        wc = None if ctx.wdtype is None else came_back(wc, (D,), ctx.dtype, dy.device, "weight")
+        gc = came_back(gc, ctx.shape, ctx.dtype, dy.device, "gate") if ctx.gated else None
         lib = _lib.load()
-        D = xc.shape[-1]
         rows = xc.numel() // D
-        dyc = dy.contiguous()
         dx = torch.empty_like(xc)
         dgate = None if gc is None else torch.empty_like(gc)
         dw = None

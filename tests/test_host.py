@@ -629,7 +629,13 @@ def _neighbours():
     plan = L.mom_plan(torch.tensor([[[0, 2], [1, 2], [2, 0]]]), 3)
     return {"swish": (L.swish_gate_relayout, (rn(2, 5, 2, 64), rn(5, 2, 128)), "lmoe_swish_gate_relayout_bwd", (0, 1, 2)),
             "combine": (lambda y, w: L.mom_combine(y, plan, w), (rn(6, 2, 64), rn(1, 3, 2)), "lmoe_mom_combine_bwd", (0, 3, 4)),
-            "gates": (L.gdn_gates, (rn(2, 5, 8), rn(2, 5, 8), rn(8).float(), rn(8).float()), "lmoe_gdn_gates_bwd", (0, 1, 2, 3, 4, 5))}
+            "gates": (L.gdn_gates, (rn(2, 5, 8), rn(2, 5, 8), rn(8).float(), rn(8).float()), "lmoe_gdn_gates_bwd", (0, 1, 2, 3, 4, 5)),
+            "prologue": (lambda x: L.gdn_qkv_prologue(x, 2, 64), (rn(5, 2, 384),), "lmoe_gdn_qkv_prologue_bwd", (0, 1, 2, 3)),
+            "gla gate": (L.gla_gate, (rn(2, 5, 64),), "lmoe_gla_gate_bwd", (0, 1)),
+            "hgrn2 gates": (lambda f: L.hgrn2_gates(f, rn(64).float()), (rn(2, 5, 64),), "lmoe_hgrn2_gate_bwd", (0, 1, 2, 3)),
+            "rms norm": (lambda x, w, g: L.rms_norm_swish_gate(x, g, w), (rn(2, 5, 64), rn(64), rn(2, 5, 64)), "lmoe_rmsnorm_bwd", (0, 1, 2, 3)),
+            "l2 norm": (L.l2_norm, (rn(2, 5, 64),), "lmoe_l2norm_bwd", (0, 1)),
+            "feature map": (L.taylor_feature_map, (rn(2, 5, 16),), "lmoe_quad_featmap_bwd", (0,))}
 
 
 def _misaligned(x):
@@ -639,7 +645,7 @@ def _misaligned(x):
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("name", ["swish", "combine", "gates"])
+@pytest.mark.parametrize("name", ["swish", "combine", "gates", "prologue", "gla gate", "hgrn2 gates", "rms norm", "l2 norm", "feature map"])
 def test_the_neighbours_backward_reads_what_was_saved(monkeypatch, name, dt):
     """A saved-tensor hook hands back what it likes: the library's backward gets the sizes and the type of the call and, at every
     pointer, the rows that were saved (another type, strides or place in memory of what came back), or nothing is launched
