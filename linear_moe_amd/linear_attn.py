@@ -29,8 +29,8 @@ def chunk_linear_attn(
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """``_eps`` (not part of fla's signature): the epsilon of the normaliser, for the callers in this package whose
     reference functions carry their own (``based.py``)."""
-    if not normalize and type(q) is torch.Tensor and q.shape[-1] in HEAD_DIMS and (initial_state is None or
-                                                                                   initial_state.shape[-2] == q.shape[-1]):
+    if (not normalize and type(q) is type(k) is torch.Tensor and q.shape[-1] in HEAD_DIMS
+            and (initial_state is None or initial_state.shape[-2] == q.shape[-1])):
         return chunk_simple_gla(q, k, v, None, scale, initial_state, output_final_state, None, head_first)     # one block, as it is
     qb, kb = _key_blocks(q), _key_blocks(k)
     if [b.shape for b in qb] != [b.shape for b in kb]:

@@ -706,3 +706,18 @@ def test_the_neighbours_backward_reads_what_was_saved(monkeypatch, name, dt):
             with pytest.raises((RuntimeError, ValueError)):
                 through(lambda j, x: f(x) if i == j else x)
     assert not calls
+
+
+@pytest.mark.parametrize("T", [5, 0])
+def test_key_blocks_of_either_operand(monkeypatch, T):
+    """chunk_linear_attn takes q and k as tensors or as lists of key blocks, one as the one and one as the other too; tensors that
+    differ in shape are refused."""
+    import linear_moe_amd.linear_attn as la
+    q, k, v = (torch.randn(1, 2, T, 64) for _ in range(3))
+    for k_ in (k[:, :1], torch.randn(1, 2, T, 128), [k, k]):
+        with pytest.raises(ValueError):
+            la.chunk_linear_attn(q, k_, v, 1.0, normalize=False)
+    monkeypatch.setattr(la, "chunk_simple_gla", lambda q, k, v, *a: (q.sum(-1, keepdim=True) * k.sum(-1, keepdim=True) * v, None))
+    ref = la.chunk_linear_attn(q, k, v, 1.0, normalize=False)[0]
+    for q_, k_ in (([q], [k]), (q, [k]), ([q], k), (q, (k,))):
+        assert torch.equal(la.chunk_linear_attn(q_, k_, v, 1.0, normalize=False)[0], ref)
