@@ -713,6 +713,9 @@ def test_key_blocks_of_either_operand(monkeypatch, T):
     """chunk_linear_attn takes q and k as tensors or as lists of key blocks, one as the one and one as the other too; tensors that
     differ in shape are refused."""
     import linear_moe_amd.linear_attn as la
+    import linear_moe_amd.simple_gla as sg
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    monkeypatch.setattr(sg, "native", lambda *a: None)
     q, k, v = (torch.randn(1, 2, T, 64) for _ in range(3))
     for k_ in (k[:, :1], torch.randn(1, 2, T, 128), [k, k]):
         with pytest.raises(ValueError):
