@@ -180,3 +180,24 @@ def test_swish_gate_relayout_fwd_bwd(cuda, dtype):
     assert max_abs_rel(y.detach().cpu(), ref.detach()) < TOL[dtype]
     assert max_abs_rel(od.grad.cpu(), orf.grad) < TOL[dtype]
     assert max_abs_rel(gd.grad.cpu(), grf.grad) < TOL[dtype]
+
+
+def test_swish_of_gates_whose_sigmoid_is_denormal(cuda):
+    """sigmoid(z) below 2^-126 (z under -87.34) is a denormal float32 and z sigmoid(z) a normal one.  Bound: the exponential's argument
+    z log2(e), up to 128, rounded to 24 bits (128 ln 2 / 2^24 = 5.3e-6) and the spacing of the denormals (2^-149 / 2^-128)."""
+    from linear_moe_amd import swish_gate_relayout
+    z = torch.linspace(-88.7, -87.35, 512, dtype=torch.float32).view(8, 1, 64)
+    zr = z.double().requires_grad_(True)
+    ref = zr * torch.sigmoid(zr)
+    o, zd = torch.ones(1, 8, 1, 64, device=cuda).requires_grad_(True), z.to(cuda).requires_grad_(True)
+    y = swish_gate_relayout(o, zd)
+    do, dz = torch.autograd.grad(y, [o, zd], torch.ones_like(y))
+    rel = lambda a, b: ((a.detach().cpu().double().flatten() - b.flatten()) / b.flatten()).abs().max()
+    assert rel(y, ref.detach()) < 1e-5 and rel(do, ref.detach()) < 1e-5
+    assert rel(dz, torch.autograd.grad(ref.sum(), zr)[0]) < 1e-5
+    # the numbers beside such a gate keep their bits
+    z = torch.linspace(-87.0, 87.0, 4096).view(8, 1, 512)
+    o = torch.ones(1, 8, 8, 64, device=cuda)
+    ref, z[..., ::4] = swish_gate_relayout(o, z.to(cuda)), -88.0
+    y, keep = swish_gate_relayout(o, z.to(cuda)), torch.arange(512) % 4 != 0
+    assert torch.equal(y[..., keep], ref[..., keep])
