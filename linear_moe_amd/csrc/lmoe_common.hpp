@@ -121,49 +121,28 @@ template <> struct ET<float> {
   }
 };
 
-// The sigmoid of SiLU in the form every kernel that applies it shares (the results agree bit for bit between
+// SiLU and its derivative in the form every kernel that applies them shares (the results agree bit for bit between
 // the row kernels in front of the op and the op's own staging)
-// (The reciprocal from the hardware's, 1 ulp, and a Newton step in place of a division.  The hardware's has no denormals, and
-// 1 / (1 + e^-z) is one where z sigmoid(z) is not (z under -87.34): sigmoid_any forms it of (1 + e^-z) / 4, exactly, and
-// leaves the step out where y r is not a number; sigmoid_fast asks once for all numbers of a lane whether one of them needs that.
-// The arithmetic of these, not the bytes, bounds the loader waves of k_gdn_bwd_chunk behind the activations and the row kernels.
-// Traced, us, with divisions, with the step alone (zero in place of the denormals) and as here: k_gdn_bwd_chunk, 1024 items of
-// K = V = 128, 66.1, 64.4, 65.3; k_gdn_qkv_prologue, 65536 rows, 19.7, 15.8, 16.2; gradients of swish_gate_relayout, 4096 rows of 2048,
-// 17.4, 16.2, 16.1.  The reciprocal against float64, units of 2^-24, the division's and this: rms 0.40 and 0.40 on -3 .. 3, 0.34
-// and 0.34 on -20 .. 20, largest 1.0 and 1.0.)
-__device__ __forceinline__ float sigmoid_any(float z) {
+// (The reciprocal from the hardware's, 1 ulp, and a Newton step: 6 instructions behind the exponential in place of the 10 of a
+// division.  y = (1 + e^-z) / 4, exactly: the hardware's reciprocal has no denormals, and 1 / (1 + e^-z) is one where z sigmoid(z) is
+// not (z under -87.34).  In the step y is no infinity, so that it leaves r = 0 alone.  The arithmetic of these, not the bytes,
+// bounds the loader waves of k_gdn_bwd_chunk behind the activations and the row kernels.  Traced, us, with divisions and square
+// roots and now: k_gdn_bwd_chunk, 1024 items of K = V = 128, 66.2 -> 64.6; k_gdn_qkv_prologue, 65536 rows, 19.2 -> 15.9; gradients of
+// swish_gate_relayout, 4096 rows of 2048, 16.6 -> 16.2.  The step left out by a comparison and a selection, and the numbers of
+// a lane asked together whether one needs the scaling: 65.4 and 64.7, 16.2 and 15.9, 16.1 and 15.9.
+// The reciprocal against float64, units of 2^-24, the division's and this: rms 0.40 and 0.40 on -3 .. 3, 0.34 and 0.34 on
+// -20 .. 20, largest 1.0 and 1.0.)
+__device__ __forceinline__ float sigmoid_fast(float z) {
   const float y = __builtin_fmaf(0.25f, __expf(-z), 0.25f), r = __builtin_amdgcn_rcpf(y);
-  return 0.25f * (y < __builtin_inff() ? __builtin_fmaf(r, __builtin_fmaf(-y, r, 1.0f), r) : r);
-}
-template <int N> __device__ __forceinline__ void sigmoid_fast(const float (&z)[N], float (&s)[N]) {
-  float top = 0.f;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    const float y = 1.0f + __expf(-z[i]), r = __builtin_amdgcn_rcpf(y);
-    s[i] = __builtin_fmaf(r, __builtin_fmaf(-y, r, 1.0f), r);
-    top = fmaxf(top, y);
-  }
-  if (__builtin_expect(!(top < 0x1p126f), 0)) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) s[i] = sigmoid_any(z[i]);
-  }
+  return 0.25f * __builtin_fmaf(r, __builtin_fmaf(-fminf(y, 0x1.fffffep127f), r, 1.0f), r);
 }
 // 1 / sqrt(y), likewise
 __device__ __forceinline__ float rsqrt_fast(float y) {
   const float r = __builtin_amdgcn_rsqf(y);
   return y > 0x1p-126f && y < 0x1p126f ? r * __builtin_fmaf(-0.5f * y * r, r, 1.5f) : r;
 }
-// silu'(z) for a = sigmoid(z)
-__device__ __forceinline__ float silu_grad(float z, float a) { return a * (1.0f + z * (1.0f - a)); }
-// eight (four) elements in place
-template <typename T> __device__ __forceinline__ void silu_vec(typename ET<T>::vec& v) {
-  float z[ET<T>::VEC], s[ET<T>::VEC];
-#pragma unroll
-  for (int i = 0; i < ET<T>::VEC; ++i) z[i] = ET<T>::to_f(v[i]);
-  sigmoid_fast(z, s);
-#pragma unroll
-  for (int i = 0; i < ET<T>::VEC; ++i) v[i] = ET<T>::from_f(z[i] * s[i]);
-}
+__device__ __forceinline__ float silu_of(float z) { return z * sigmoid_fast(z); }
+__device__ __forceinline__ float silu_grad(float z) { const float a = sigmoid_fast(z); return a * (1.0f + z * (1.0f - a)); }
 
 // e^x for the pairwise decay factors: library expf on the fp32 path (keeps 1e-5 parity),
 // the hardware exp2 path for bf16 operands

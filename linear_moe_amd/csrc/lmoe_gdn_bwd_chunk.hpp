@@ -207,15 +207,11 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           if (sizeof(T) == 2 && a.v_act) {
             // v as given is the argument of a SiLU: the op runs on silu(v) (rounded to the element type, as the
             // forward pass staged it) and dv is the gradient with respect to the argument
-            float vr[IOV::VEC], sg[IOV::VEC];
-#pragma unroll
-            for (int i = 0; i < IOV::VEC; ++i) vr[i] = ET<T>::to_f(vv[i]);
-            sigmoid_fast(vr, sg);
 #pragma unroll
             for (int i = 0; i < IOV::VEC; ++i) {
-              const float zf = ET<T>::to_f(z[i]);
-              o[i] = ET<T>::from_f(zf * bt * silu_grad(vr[i], sg[i]));
-              s += zf * ET<T>::to_f(ET<T>::from_f(vr[i] * sg[i]));
+              const float zf = ET<T>::to_f(z[i]), vr = ET<T>::to_f(vv[i]);
+              o[i] = ET<T>::from_f(zf * bt * silu_grad(vr));
+              s += zf * ET<T>::to_f(ET<T>::from_f(silu_of(vr)));
             }
           } else {
 #pragma unroll
@@ -298,9 +294,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_bwd_chunk(const lmoe_args a) {
           float sv[IOK::VEC], gv[IOK::VEC], fv[IOK::VEC], ss = 0.f, c = 0.f;
 #pragma unroll
           for (int i = 0; i < IOK::VEC; ++i) {
-            const float x = ET<T>::to_f(X.v[p][i]), sg = sigmoid_any(x);     // (sigmoid_fast's registers spill here)
+            const float x = ET<T>::to_f(X.v[p][i]), sg = sigmoid_fast(x);
             sv[i] = x * sg;
-            gv[i] = silu_grad(x, sg);
+            gv[i] = sg * (1.0f + x * (1.0f - sg));
             ss += sv[i] * sv[i];
           }
 #pragma unroll

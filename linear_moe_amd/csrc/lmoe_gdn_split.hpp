@@ -46,7 +46,10 @@ template <int COLS, int NT> struct WideTile {
     for (int p = 0; p < PASSES; ++p) {
       int row, col; coords(p, row, col);
       if constexpr (SILU) {
-        if (act) silu_vec<bf16>(r.v[p]);
+        if (act) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) r.v[p][i] = (bf16)silu_of((float)r.v[p][i]);
+        }
       }
       if (len < CH) {                                             // uniform: only the last chunk of a sequence
         u32x4 w = __builtin_bit_cast(u32x4, r.v[p]);

@@ -249,7 +249,9 @@ __global__ __launch_bounds__(3 * NTHR) void k_gdn_state_fwd_reg(const lmoe_args 
       IOP::store_lds(P.rt, s_ti[buf], LDC);
       if (a.v_act) {                         // v = silu(v as given): the activation in front of the op, applied here
 #pragma unroll
-        for (int p = 0; p < IOV::PASSES; ++p) silu_vec<T>(P.rv.v[p]);
+        for (int p = 0; p < IOV::PASSES; ++p)
+#pragma unroll
+          for (int i = 0; i < IOV::VEC; ++i) P.rv.v[p][i] = ET<T>::from_f(silu_of(ET<T>::to_f(P.rv.v[p][i])));
       }
       IOV::mask(P.rv, P.len);
       IOV::store_lds(P.rv, s_v[buf], LDU);

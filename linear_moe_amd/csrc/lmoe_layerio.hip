@@ -17,6 +17,7 @@
 namespace lmoe {
 
 namespace {
+__device__ __forceinline__ float sigm(float z) { return sigmoid_fast(z); }
 // sum over the LPR neighbouring lanes that hold one row
 template <int LPR> __device__ __forceinline__ float row_sum(float x) {
   if constexpr (LPR <= 16) {
@@ -53,25 +54,20 @@ __global__ __launch_bounds__(NTHR) void k_gdn_qkv_prologue(const T* __restrict__
       const vec xv = *(const vec*)(src + 2 * D);
       vec dvv;
       if constexpr (BWD) dvv = *(const vec*)(dv + r * D + lr * VEC);
-      float z[VEC], s[VEC];
-#pragma unroll
-      for (int i = 0; i < VEC; ++i) z[i] = ET<T>::to_f(xv[i]);
-      sigmoid_fast(z, s);
 #pragma unroll
       for (int i = 0; i < VEC; ++i) {
-        if constexpr (BWD) ov[i] = ET<T>::from_f(ET<T>::to_f(dvv[i]) * s[i] * (1.0f + z[i] * (1.0f - s[i])));
-        else ov[i] = ET<T>::from_f(z[i] * s[i]);
+        const float zv = ET<T>::to_f(xv[i]), av = sigm(zv);
+        if constexpr (BWD) ov[i] = ET<T>::from_f(ET<T>::to_f(dvv[i]) * av * (1.0f + zv * (1.0f - av)));
+        else ov[i] = ET<T>::from_f(zv * av);
       }
     }
-    float z[2 * VEC], s[2 * VEC];                   // of q, of k
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) { z[i] = ET<T>::to_f(xq[i]); z[VEC + i] = ET<T>::to_f(xk[i]); }
-    sigmoid_fast(z, s);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      sq[i] = z[i] * s[i]; sk[i] = z[VEC + i] * s[VEC + i];
-      gq[i] = silu_grad(z[i], s[i]);
-      gk[i] = silu_grad(z[VEC + i], s[VEC + i]);
+      const float zq = ET<T>::to_f(xq[i]), zk = ET<T>::to_f(xk[i]);
+      const float aq = sigm(zq), ak = sigm(zk);
+      sq[i] = zq * aq; sk[i] = zk * ak;
+      gq[i] = aq * (1.0f + zq * (1.0f - aq));       // silu'(z)
+      gk[i] = ak * (1.0f + zk * (1.0f - ak));
       ssq += sq[i] * sq[i]; ssk += sk[i] * sk[i];
     }
     ssq = row_sum<LPR>(ssq); ssk = row_sum<LPR>(ssk);
@@ -123,13 +119,9 @@ __global__ __launch_bounds__(NTHR) void k_swish_gate_relayout(const T* __restric
     vec r0, r1;
     vec dv;
     if constexpr (BWD) dv = *(const vec*)(dy + ig);
-    float zs[VEC], sg[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) zs[j] = ET<T>::to_f(gv[j]);
-    sigmoid_fast(zs, sg);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
-      const float z = zs[j], s = sg[j], x = ET<T>::to_f(ov[j]);
+      const float z = ET<T>::to_f(gv[j]), s = sigm(z), x = ET<T>::to_f(ov[j]);
       if constexpr (BWD) {
         const float d = ET<T>::to_f(dv[j]);
         r0[j] = ET<T>::from_f(d * z * s);                                 // do

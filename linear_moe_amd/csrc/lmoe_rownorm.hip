@@ -23,12 +23,7 @@ template <int LPR> __device__ __forceinline__ float lanes_sum(float x) {
   for (int d = 1; d < LPR; d <<= 1) x += __shfl_xor(x, d, 64);
   return x;
 }
-// the sigmoids of a vector of gates
-template <typename T> __device__ __forceinline__ void gate_sigmoids(const typename ET<T>::vec& v, float (&z)[ET<T>::VEC], float (&s)[ET<T>::VEC]) {
-#pragma unroll
-  for (int i = 0; i < ET<T>::VEC; ++i) z[i] = ET<T>::to_f(v[i]);
-  sigmoid_fast(z, s);
-}
+__device__ __forceinline__ float sigmoidf_(float z) { return sigmoid_fast(z); }
 
 // ------------------------------------------------------------------------- //
 // RMS norm (+ swish gate)
@@ -53,12 +48,10 @@ __global__ __launch_bounds__(NTHR) void k_rmsnorm_fwd(const T* __restrict__ x, c
     ss = lanes_sum<LPR>(ss);
     const float rstd = 1.0f / sqrtf(ss * (1.0f / D) + eps);
     vec o;
-    float z[VEC], sg[VEC];
-    if constexpr (GATE) gate_sigmoids<T>(gv, z, sg);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       float v = xf[i] * rstd * wf[i];
-      if constexpr (GATE) v *= z[i] * sg[i];
+      if constexpr (GATE) { const float z = ET<T>::to_f(gv[i]); v *= z * sigmoidf_(z); }
       o[i] = ET<T>::from_f(v);
     }
     *(vec*)(y + r * D + lr * VEC) = o;
@@ -89,15 +82,15 @@ __global__ __launch_bounds__(NTHR) void k_rmsnorm_bwd(const T* __restrict__ x, c
     ss = lanes_sum<LPR>(ss);
     const float rstd = 1.0f / sqrtf(ss * (1.0f / D) + eps);
     vec og;
-    float c = 0.f, z[VEC], sg[VEC];
-    if constexpr (GATE) gate_sigmoids<T>(gv, z, sg);
+    float c = 0.f;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
       const float xh = xf[i] * rstd, d = ET<T>::to_f(dv[i]);
       float u = d;
       if constexpr (GATE) {
-        u = d * z[i] * sg[i];
-        og[i] = ET<T>::from_f(d * xh * wf[i] * sg[i] * (1.0f + z[i] * (1.0f - sg[i])));
+        const float z = ET<T>::to_f(gv[i]), sg = sigmoidf_(z);
+        u = d * z * sg;
+        og[i] = ET<T>::from_f(d * xh * wf[i] * sg * (1.0f + z * (1.0f - sg)));
       }
       dwacc[i] += u * xh;
       uf[i] = u * wf[i];
@@ -215,12 +208,12 @@ __global__ __launch_bounds__(NTHR) void k_silu_l2norm(const T* __restrict__ x, c
   const int lr = threadIdx.x % LPR, rb = threadIdx.x / LPR;
   for (int64_t r = (int64_t)blockIdx.x * RPB + rb; r < rows; r += (int64_t)gridDim.x * RPB) {
     const vec xv = *(const vec*)(x + r * D + lr * VEC);
-    float z[VEC], sg[VEC], sf[VEC], ds[VEC], ss = 0.f;
-    gate_sigmoids<T>(xv, z, sg);
+    float sf[VEC], ds[VEC], ss = 0.f;
 #pragma unroll
     for (int i = 0; i < VEC; ++i) {
-      sf[i] = z[i] * sg[i];
-      ds[i] = silu_grad(z[i], sg[i]);
+      const float z = ET<T>::to_f(xv[i]), sg = sigmoidf_(z);
+      sf[i] = z * sg;
+      ds[i] = sg * (1.0f + z * (1.0f - sg));       // silu'(z)
       ss += sf[i] * sf[i];
     }
     ss = lanes_sum<LPR>(ss);
