@@ -136,10 +136,14 @@ __device__ __forceinline__ float sigmoid_fast(float z) {
   const float y = __builtin_fmaf(0.25f, __expf(-z), 0.25f), r = __builtin_amdgcn_rcpf(y);
   return 0.25f * __builtin_fmaf(r, __builtin_fmaf(-fminf(y, 0x1.fffffep127f), r, 1.0f), r);
 }
-// 1 / sqrt(y), likewise
+// 1 / sqrt(y): the hardware's, 1 ulp, and a Newton step (for 0 infinity or NaN, for infinity 0).  The hardware's has no denormals
+// either: small arguments are scaled by a power of four.  Against float64, units of 2^-24, over 2^-126 .. 2^126, square root and
+// division and this: rms 0.60 and 0.47, largest 1.50 and 1.24 (the step as r (1.5 - 0.5 y r r): 0.55 and 2.56).
 __device__ __forceinline__ float rsqrt_fast(float y) {
-  const float r = __builtin_amdgcn_rsqf(y);
-  return y > 0x1p-126f && y < 0x1p126f ? r * __builtin_fmaf(-0.5f * y * r, r, 1.5f) : r;
+  const bool small = y < 0x1p-100f;
+  const float x = y * (small ? 0x1p64f : 1.0f), r = __builtin_amdgcn_rsqf(x);
+  const float z = __builtin_fmaf(0.5f * r, __builtin_fmaf(-fminf(x, 0x1.fffffep127f) * r, r, 1.0f), r);
+  return z * (small ? 0x1p32f : 1.0f);
 }
 __device__ __forceinline__ float silu_of(float z) { return z * sigmoid_fast(z); }
 __device__ __forceinline__ float silu_grad(float z) { const float a = sigmoid_fast(z); return a * (1.0f + z * (1.0f - a)); }

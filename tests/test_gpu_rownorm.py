@@ -201,3 +201,20 @@ def test_swish_of_gates_whose_sigmoid_is_denormal(cuda):
     ref, z[..., ::4] = swish_gate_relayout(o, z.to(cuda)), -88.0
     y, keep = swish_gate_relayout(o, z.to(cuda)), torch.arange(512) % 4 != 0
     assert torch.equal(y[..., keep], ref[..., keep])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_l2_norm_of_rows_whose_square_sum_is_denormal(cuda, D):
+    """eps = 0 and rows of some 1e-20: their squares add up to a denormal float32, their norm is an ordinary one.  Bound: every square is
+    rounded to the spacing of the denormals, 2^-149, which adds up to less than D 2^-150 / sum = 1e-5 in the sum."""
+    from linear_moe_amd import gdn_qkv_prologue, silu_l2_norm
+    x = gen(77, 6, 2, 3 * D) * (2e-20 * (64 / D) ** 0.5)
+    ref = torch.nn.functional.silu(x.double()).view(6, 2, 1, 3, D)
+    ref = ref / ref.norm(dim=-1, keepdim=True)
+    q, k, _ = gdn_qkv_prologue(x.to(cuda), 1, D, 0.0)
+    y = silu_l2_norm(x.view(6, 2, 3, D).to(cuda), 0.0)
+    assert max_abs_rel(y.cpu(), ref[:, :, 0]) < 1e-5
+    for i, z in enumerate((q, k)):
+        assert max_abs_rel(z.cpu(), ref[..., i, :].transpose(0, 1)) < 1e-5
+    zero = silu_l2_norm(torch.zeros(2, D, device=cuda), 1e-6)
+    assert torch.equal(zero, torch.zeros_like(zero))
