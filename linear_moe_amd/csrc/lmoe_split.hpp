@@ -142,16 +142,21 @@ template <bool CUT> __device__ __forceinline__ PassItem pass_item_dense(const lm
   p.last = j == nseg - 1;
   return p;
 }
-// What the rules below expect of a cut, as a part of the whole call by their figures: 0.9, less at K = V = 128 where the pass over whole
-// sequences takes slices of 16 columns (2-byte elements, a CU for each), which the figures do not know.  There (one call replayed as
-// a graph, us, cut : whole, forward; forward and backward) cuts lost at 0.90 of the delta rule's figures 50.0 : 47.4; 122 : 112 (16 pairs
-// of 28 chunks), of chunk_simple_gla's at 0.84 29.2 : 26.1; 83 : 71 (16 of 20), at 0.88 42.4 : 40.6; 114 : 106 (24 of 32), at 0.89 43.8 : 42.2;
-// 127 : 118 (32 of 32), and stay where the forward pass alone still wins: 0.80 57.3 : 62.1; 148 : 149 (16 of 40), 0.81 50.7 : 52.7; 126 : 122
-// (16 of 32), 0.83 22.2 : 22.9; 58 : 53 (8 of 17).  At K = V = 64 every cut up to 0.9 wins (by 1.08 to 2), and chunk_gla's do at
-// either.  Several packed sequences keep 0.9: the longest, which the average does not show, gains more.
-inline float cut_limit(const lmoe_args& a, float at128) {
-  const bool narrow = (!a.cu_seqlens || a.N == 1) && a.dtype == LMOE_BF16 && a.V <= 128 && (int64_t)a.N * a.H * (a.V / 16) <= cu_count();
-  return narrow ? 0.9f - (0.9f - at128) * fmaxf(0.f, (a.K + a.V) / 128.f - 1.f) : 0.9f;
+// What the rules below expect of a cut, as a part of the whole call by their figures: 0.9, less at V = 128 where the pass over whole
+// sequences takes slices of 16 columns (2-byte elements, a CU for each), which the figures do not know.  Every call that the lower
+// limits leave whole was timed both ways, one call replayed as a graph, time cut : whole.
+//   chunk_simple_gla, K = V = 128, 0.835: forward 0.99 to 1.29, forward and backward 1.05 to 1.29 (16 pairs of 20 chunks 28.6 : 25.0
+//     and 81 : 69 us, 32 of 43 61 : 51 and 177 : 149); with the normaliser 0.94 (16 of 21) to 1.23 and 1.02 to 1.27.  Below, cuts win:
+//     0.80 57.3 : 62.1 us forward (16 of 40), 0.83 22.2 : 22.9 (8 of 17; the training call of it loses, 58 : 53).
+//   chunk_simple_gla, K = 64, 0.868: 0.91 (8 of 17) to 1.29 and 0.95 (24 of 38) to 1.24; normalised 0.95 to 1.34 and 0.94 to 1.24
+//   delta rule, K = V = 128, 0.85: 0.98 (16 of 37) to 1.14 and 1.03 to 1.15
+// The same lower limits at the other sizes lost: delta rule K = 64, V = 128 0.92 to 1.07 and 0.95 to 1.05, K = 128, V = 64 0.88 to 1.01
+// and 0.94 to 1.05 (28 of 44 62 : 70 and 155 : 165 us), chunk_simple_gla K = 128, V = 64 0.79 to 1.06 and 0.94 to 1.07 (16 of 17 18.4 : 21.6
+// and 57 : 58).  At K = V = 64 every cut up to 0.9 wins (by 1.08 to 2), and chunk_gla's do there and at K = V = 128.  Several packed sequences
+// keep 0.9: the longest, which the average does not show, gains more.
+inline float cut_limit(const lmoe_args& a, float at128, float at64) {
+  const bool narrow = (!a.cu_seqlens || a.N == 1) && a.dtype == LMOE_BF16 && a.V == 128 && (int64_t)a.N * a.H * (a.V / 16) <= cu_count();
+  return !narrow ? 0.9f : a.K == 128 ? at128 : at64;
 }
 // How a call is cut (pointers left open), or len1 = 0.  `slices` = work-groups of the ordinary pass per (sequence, head),
 // which hold a CU each; the work-groups of step 1 carry all columns and hold a CU each too.  Chosen by what the three steps
@@ -182,7 +187,7 @@ inline Split plan_split(const lmoe_args& a, int slices) {
   const int rmax = packed && a.N > 1 ? (slots - a.N) / a.N : slots / a.N;
   if (chunks > seqs * SPLIT_MAX_CHUNKS) return s;
   for (int nch = packed ? seg_count(chunks + seqs, seqs) : least; nch >= least && nch >= SPLIT_MIN_CHUNKS && !s.len1; --nch) {
-    float best = cut_limit(a, 0.85f) * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
+    float best = cut_limit(a, 0.85f, 0.9f) * nch * w * (a.N * a.H * slices <= 64 ? 1.7f : 2.1f);
     for (int r = 3; r <= rmax && r <= 32; ++r)
       for (int f = 1; f <= 4; ++f) {
         const int len3 = seg_count(nch, r), len1 = seg_count(len3, f), nf = seg_count(nch, len1);
@@ -249,7 +254,7 @@ inline Split plan_split_scalar(const lmoe_args& a) {
   // forward and backward together, 384 of K = V = 128 759 -> 857)
   if (!f4 && a.normalize && 2 * wg3 >= cus) return s;
   const float c3 = f4 ? 1.9f + 4.1f * w : 0.45f + 0.85f * w, c1 = f4 ? 1.f + 2.f * w : 0.3f + 0.6f * w;
-  return plan_cut(a, cut_limit(a, 0.835f), c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
+  return plan_cut(a, cut_limit(a, 0.835f, 0.868f), c3, f4 ? 0.f : 0.3f * w, c1, (f4 ? 0.25f : 0.5f) * w, wg3, (int64_t)pairs * (f4 ? a.V / 32 : 1));
 }
 // The same for chunk_gla (2-byte elements, dense; a transition is one decay per state row).  The pass fetches q, k and the
 // intra-chunk matrix once per V slice of 32, so a chunk costs more the more CUs run one.  Measured, us per chunk with 64, 128,

@@ -209,6 +209,23 @@ def test_the_cut_along_t_of_packed_input_follows_from_t_and_n():
     assert lib.lmoe_split_lengths(C.byref(a), 3, None, None) == -21
 
 
+@pytest.mark.parametrize("op,K,V,pairs,chunks,cut", [
+    (0, 128, 128, 20, 32, False), (0, 128, 128, 16, 40, True), (0, 64, 128, 20, 31, False), (0, 64, 128, 16, 40, True),
+    (0, 128, 64, 16, 17, True), (0, 128, 64, 32, 23, True), (0, 64, 64, 16, 32, True),
+    (2, 128, 128, 20, 28, False), (2, 128, 128, 16, 47, True), (2, 64, 128, 16, 39, True), (2, 128, 64, 28, 44, True)])
+def test_which_calls_with_narrow_slices_are_cut(op, K, V, pairs, chunks, cut):
+    """The limit of a cut is lower where the pass over whole sequences is faster than the rule's figures, and only where both sides were
+    timed: V = 128, for the delta rule K = 128 too."""
+    from linear_moe_amd import _lib
+    a = _lib.Args()
+    H = 16 if pairs % 16 == 0 else pairs
+    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_BF16, pairs // H, chunks * 64, H, K, V, pairs // H, pairs // H * chunks
+    a.gate = _lib.GATE_SCALAR
+    fine, coarse = C.c_int32(), C.c_int32()
+    assert _lib.load().lmoe_split_lengths(C.byref(a), op, C.byref(fine), C.byref(coarse)) == 0
+    assert (fine.value > 0) == cut
+
+
 def test_options_outside_flas_signature_are_validated_before_any_launch():
     """V = 256 belongs to the gated delta rule alone (2-byte calls then need tinv); normalize belongs to ungated 2-byte
     calls of chunk_simple_gla and names the buffers it needs; v_act needs 2-byte elements and tinv.  Calls without
