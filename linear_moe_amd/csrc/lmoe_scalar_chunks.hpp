@@ -3,25 +3,26 @@
 // A pass over a sequence is a chain of chunks (4 us each at K = 64, 6 at K = 128) on few CUs, and cut into segments
 // (lmoe_scalar_split.hpp) two launches.  Here every work-group takes one (sequence, head, chunk, 16-column slice of V), sums up
 // the state its chunk starts from itself,  S = sum over the chunks in front of  (decay to their end)  k^T (e_d v),  and forms
-// the chunk's output: no chain, one launch.  The sums over the tokens in front are formed again by every chunk, which is
-// what bounds how long a sequence may be: fwd_by_chunks (lmoe_scalar_fwd.hip).
+// the chunk's output: no chain, one launch.  The sums over the tokens in front are formed again by every chunk, which with
+// the waves of a work-group bounds how long a sequence may be: fwd_by_chunks (lmoe_scalar_fwd.hip).
 #pragma once
 #include "lmoe_seq.hpp"
 
 namespace lmoe {
 
-constexpr int CHUNKS_PREFIX_WAVES = 8;
+constexpr int CHUNKS_PREFIX_WAVES = 8;      // at most so many chunks in front of a work-group's own (or behind the last)
 
-// Work-group of twelve waves.  Waves 0 .. 7 share the chunks in front of this one, each a run of consecutive ones, straight from
-// memory into matrix operands; their sums meet in LDS and are folded in order, S <- D S + Q.  Waves 8 .. 11 meanwhile form
+// Work-group of twelve waves.  Waves 0 .. 7 take one of the chunks in front of this one each, straight from memory into matrix
+// operands; their sums meet in LDS and are folded in order, S <- D S + Q.  Waves 8 .. 11 meanwhile form
 // (q k^T . Gamma) v  of 16 output rows each, also straight from memory, and add  e^b q S  when the state is there.  A matrix
 // step of four tokens is numbered so that the lanes' loads are 16-byte ones: a lane's four values of a k row are one row of
 // four blocks of the state, its four of a q row four steps of a contraction.  With a final state asked for, one more
 // work-group per sequence stands behind the last chunk.
 // Bound by its launch, the first loads and the matrix instructions of the last chunks' work-groups (a wave's share of a 64-token
-// chunk: 64 of 32 cycles at K = 64).  B=1 T=512 H=4 K=V=64: 12.3 us (segments and pass) -> 9.0; T = 256 (pass) 18.4 -> 7.8,
-// T = 64 7.0 -> 6.5; K = V = 128, T = 512 20.5 -> 14.2.  K = 64: loads of 8 steps in flight and 76 registers, for two
-// work-groups per CU (16 steps, 146 registers and one: 32 pairs of 8 chunks 28.5 -> 22.1); K = 128, where that spills: one, 148 registers.
+// chunk: 64 of 32 cycles at K = 64).  us, replayed as a graph, segments and pass (T = 256, 64: the pass) -> this, B = 1, H = 4:
+// K = V = 64, T = 512 12.4 -> 8.8, T = 256 18.4 -> 7.1, T = 64 7.05 -> 6.6; K = V = 128, T = 512 20.0 -> 13.8.  K = 64: loads of 8 steps
+// in flight and 76 registers, for two work-groups per CU (16 steps, 146 registers and one: 32 pairs of 8 chunks 28.5 -> 22.1);
+// K = 128, where that spills: one, 126 registers.  (A loop over a run of chunks per wave, for longer sequences: 148, K = V = 128 14.4.)
 template <int K, int V>
 __global__ __launch_bounds__(3 * NTHR, K == 64 ? 6 : 3) void k_state_fwd_chunks(const lmoe_args a) {
   constexpr int BV = 16, NVS = V / BV, NW = CHUNKS_PREFIX_WAVES, LD = K + 4, HB = K / 64, NK = K / 16, NS = K == 64 ? 4 : 8;
@@ -42,7 +43,6 @@ __global__ __launch_bounds__(3 * NTHR, K == 64 ? 6 : 3) void k_state_fwd_chunks(
   const int n = pair / a.H, h = pair % a.H, v0 = vsl * BV;
   const int l = lane_id(), fr = l & 15, g = l >> 4, wv = wave_id();
   const bool gated = a.gate != LMOE_GATE_NONE && a.g.ptr != nullptr;
-  const int run = (c + NW - 1) / NW;                                       // chunks of a prefix wave
   const float* const kp = row_ptr<float>(a.k, n, 0, h);
   const float* const vp = row_ptr<float>(a.v, n, 0, h) + v0 + fr;
   auto log_decay = [&](int tok, int len) {                                 // of this lane's token of a chunk
@@ -58,27 +58,19 @@ __global__ __launch_bounds__(3 * NTHR, K == 64 ? 6 : 3) void k_state_fwd_chunks(
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[i] = h0[i * V];
     }
-    f32x4 acc[HB][4];                        // [64-row group][m]: rows 64 hb + 16 g + 4 i + m of column fr
+    if (wv < c) {
+      f32x4 acc[HB][4];                      // [64-row group][m]: rows 64 hb + 16 g + 4 i + m of column fr
 #pragma unroll
-    for (int hb = 0; hb < HB; ++hb)
+      for (int hb = 0; hb < HB; ++hb)
 #pragma unroll
-      for (int m = 0; m < 4; ++m) acc[hb][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float dec = 1.f;
-    const int j0 = wv * run, j1 = min(j0 + run, c);
-    for (int j = j0; j < j1; ++j) {
-      const int tok = j * CH, len = min(CH, a.T - tok);
+        for (int m = 0; m < 4; ++m) acc[hb][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int tok = wv * CH, len = min(CH, a.T - tok);
       const float x = wave_incl_scan(log_decay(tok, len)), xl = __shfl(x, 63, 64);
       if (gated) {
         s_f[wv][l] = expf(xl - x);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const float d = expf(xl);
-#pragma unroll
-        for (int hb = 0; hb < HB; ++hb)
-#pragma unroll
-          for (int m = 0; m < 4; ++m) acc[hb][m] *= d;
-        dec *= d;
       }
       // token 16 g + s of step s (rows past the end of the sequence re-read the last one and count as zero)
 #pragma unroll 2
@@ -118,19 +110,16 @@ __global__ __launch_bounds__(3 * NTHR, K == 64 ? 6 : 3) void k_state_fwd_chunks(
 #pragma unroll
             for (int m = 0; m < 4; ++m) acc[hb][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[hb][s][m], vv[s], acc[hb][m], 0, 0, 0);
       }
-      __builtin_amdgcn_wave_barrier();
-    }
-    if (j0 < j1) {
 #pragma unroll
       for (int hb = 0; hb < HB; ++hb)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           *(f32x4*)&s_part[wv][fr * LD + 64 * hb + 16 * g + 4 * i] = f32x4{acc[hb][0][i], acc[hb][1][i], acc[hb][2][i], acc[hb][3][i]};
-      if (l == 0) s_dec[wv] = dec;
+      if (l == 0) s_dec[wv] = gated ? expf(xl) : 1.f;
     }
     lds_barrier();
     if (col < BV) {
-      for (int w = 0; w * run < c; ++w) S = S * s_dec[w] + *(const f32x4*)&s_part[w][col * LD + kr];
+      for (int w = 0; w < c; ++w) S = S * s_dec[w] + *(const f32x4*)&s_part[w][col * LD + kr];
       if (c < nch) {
         *(f32x4*)&s_S[col * LD + kr] = S;
         if (a.hs) *(f32x4*)((float*)a.hs + (((int64_t)(n * nch + c) * a.H + h) * V + v0 + col) * K + kr) = S;

@@ -24,15 +24,16 @@ inline Split scalar_split(const lmoe_args& a) {
   return sp;
 }
 // 4-byte elements: whether every chunk runs on its own (k_state_fwd_chunks).  Without and with it, us, K = V = 64 (two work-groups
-// to a CU): 32 pairs of 8 chunks 34 and 22, 64 of 4 19.5 and 18.5, 64 of 8 35 and 39, 4 of 16 13.9 and 12.6 but 16 of 16 26
-// and 28; K = V = 128 (one): 8 pairs of 8 chunks 26 and 22, 16 of 8 38 and 38, 16 of 4 29 and 18, 32 of 4 30 and 32.  Up to two
-// chunks there is next to nothing to form twice: 128 pairs of 2 21 and 16.5, K = V = 128 68 and 59; but with a final state,
-// one work-group more per sequence, 32 pairs of 1 12.9 and 14.8, 8 of 1 11.5 and 9.2.
+// to a CU): 32 pairs of 8 chunks 34 and 20, 64 of 4 19 and 17, 64 of 8 35 and 39; K = V = 128 (one): 8 pairs of 8 chunks 26
+// and 20, 16 of 8 38 and 38, 16 of 4 29 and 17, 32 of 4 30 and 32.  Up to two chunks there is next to nothing to form twice: 128
+// pairs of 2 21 and 16.5, K = V = 128 68 and 59; but with a final state, one work-group more per sequence, 32 pairs of 1 12.9
+// and 14.8, 8 of 1 11.5 and 9.2.  A chunk in front to a wave, eight at most: runs of two gave 4 pairs of 16 chunks 13.9 and
+// 12.6 but 16 of 16 26 and 28, and every other call their loop.
 inline bool fwd_by_chunks(const lmoe_args& a) {
   if (a.dtype == LMOE_BF16 || a.cu_seqlens) return false;
   const int nch = (a.T + CH - 1) / CH, per_cu = a.K == 64 ? 4 : 2;
   const int64_t wgs = (int64_t)a.N * a.H * (nch + (a.ht ? 1 : 0)) * (a.V / 16);
-  return nch <= 8 && wgs <= (int64_t)cu_count() * (a.ht ? min(nch, per_cu) : nch <= 2 ? 8 : per_cu);
+  return nch <= CHUNKS_PREFIX_WAVES && wgs <= (int64_t)cu_count() * (a.ht ? min(nch, per_cu) : nch <= 2 ? 8 : per_cu);
 }
 // (a forward call that runs by chunks needs no buffers; asked without either output, the larger of both directions)
 int64_t scalar_split_floats(const lmoe_args& a) {
