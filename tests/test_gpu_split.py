@@ -409,15 +409,34 @@ def test_error_of_the_cut_behind_a_drop_of_v(cuda, monkeypatch, gated):
     assert cut[1] < bound * whole[1] and cut[2] < bound * whole[2]
 
 
+def by_chunks(B, T, H, K, V, final_state):
+    """Whether a 4-byte call of chunk_simple_gla of three chunks and more runs chunk by chunk: it then asks for no workspace, while
+    the pass is cut."""
+    import ctypes as C
+    from linear_moe_amd import _lib
+    a = _lib.Args()
+    a.dtype, a.B, a.T, a.H, a.K, a.V, a.N, a.NT = _lib.LMOE_F32, B, T, H, K, V, B, B * ((T + 63) // 64)
+    assert _lib.load().lmoe_split_floats(C.byref(a), 0, 1) > 0
+    a.o, a.ht = _lib.Tensor4(16, 0, 0, 0), 16 if final_state else None     # (only asked whether they are there)
+    return _lib.load().lmoe_split_floats(C.byref(a), 0, 1) == 0
+
+
+def test_which_4_byte_calls_run_chunk_by_chunk(cuda):
+    for call, without, with_state in (((2, 500, 4, 64, 64), True, True), ((1, 512, 4, 128, 128), True, True), ((1, 511, 2, 128, 64), True, True),
+                                      ((1, 512, 8, 128, 128), True, False), ((1, 513, 2, 64, 64), False, False)):
+        assert (by_chunks(*call, False), by_chunks(*call, True)) == (without, with_state), call
+
+
 @pytest.mark.parametrize("B,T,H,K,V", [
     (1, 1, 1, 64, 64), (2, 63, 3, 128, 64), (1, 64, 8, 64, 128), (1, 65, 2, 128, 128),      # one chunk, and one token more
-    (2, 500, 4, 64, 64), (1, 512, 8, 128, 128),            # seven waves with a chunk in front each, or eight of them
+    (2, 500, 4, 64, 64), (1, 512, 4, 128, 128), (1, 511, 2, 128, 64),      # seven waves with a chunk in front each, or eight
+    (1, 512, 8, 128, 128),                                 # with a final state the pass
     (1, 513, 2, 64, 64), (32, 192, 4, 64, 64),             # beyond eight chunks, and more pairs than the CUs take: the pass
 ])
 @pytest.mark.parametrize("gated", [False, True])
 def test_simple_gla_4_byte_chunk_by_chunk(cuda, B, T, H, K, V, gated):
-    """Short sequences in 4-byte elements: every chunk sums up the state it starts from.  Both layouts, a gate of 2-byte
-    elements; the states saved for the backward are those of the chunks."""
+    """Short sequences in 4-byte elements: every chunk sums up the state it starts from.  With and without a final state, both
+    layouts, a gate of 2-byte elements; the states saved for the backward are those of the chunks."""
     from linear_moe_amd import chunk_simple_gla
     ins = dict(q=gen(7500, B, T, H, K), k=gen(7501, B, T, H, K) * K ** -0.5, v=gen(7502, B, T, H, V), h0=gen(7505, B, H, K, V) * 0.3)
     if gated:                                               # (representable in either type)
@@ -431,5 +450,7 @@ def test_simple_gla_4_byte_chunk_by_chunk(cuda, B, T, H, K, V, gated):
     o, _ = chunk_simple_gla(d["q"], d["k"], d["v"], d.get("g"), None, d["h0"], False, None, False)
     of, _ = chunk_simple_gla(hf["q"], hf["k"], hf["v"], hf.get("g"), None, hf["h0"])
     assert torch.equal(of.transpose(1, 2), o)
+    ref, _ = naive.naive_recurrent_simple_gla(*(ins[n].double() if n in ins else None for n in ("q", "k", "v", "g")), None, ins["h0"].double(), False, None, False)
+    assert max_abs_rel(o.cpu(), ref) < TOL[torch.float32]
     if gated:
         assert torch.equal(chunk_simple_gla(d["q"], d["k"], d["v"], d["g"].bfloat16(), None, d["h0"], False, None, False)[0], o)
