@@ -367,3 +367,46 @@ def test_saved_tensors_belong_to_autograd(cuda, op):
     work["k"].add_(1)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(o, [leaves[n] for n in names], do)
+
+
+# heads per sequence that give the passes over whole sequences V slices of 32 and of 64 columns (fewer pairs of a sequence and a head
+# take slices of 16): 8 packed sequences, or a batch of 2
+WIDER = {("packed", 128, 32): 6, ("packed", 128, 64): 17, ("packed", 64, 32): 10, ("packed", 64, 64): 34,
+         ("views", 128, 32): 20, ("views", 128, 64): 65, ("views", 64, 32): 35, ("views", 64, 64): 130}
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("K,V", [(64, 64), (128, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("form,columns", [("packed", 32), ("packed", 64), ("views", 32), ("views", 64)])
+def test_edges_of_the_passes_with_wider_slices(cuda, op, form, columns, K, V):
+    """Empty, one-token, whole and partial packed sequences, and head-first views of time-first tensors, with as many heads as the
+    wider V slices are launched for.  The first and the last head against the oracle (heads do not mix)."""
+    H, dtype = WIDER[form, V, columns], torch.bfloat16
+    lens = [0, 1, 63, 0, 64, 65, 70, 0] if form == "packed" else None
+    B, T, N = (1, sum(lens), len(lens)) if lens else (2, 150, 2)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32) if lens else None
+    pairs = N * H
+    assert (pairs * V // 16 > 256) and (pairs * V // 64 >= 256) == (columns == 64)
+    ins = _inputs(op, B * T, H, K, V, dtype, 3400)
+    ins = {n: x.reshape(B, T, *x.shape[2:]) for n, x in ins.items()}
+    h0, do, dht = gen(3410, N, H, K, V) * 0.5, gen(3411, B, T, H, V, dtype=dtype), gen(3412, N, H, K, V)
+    ends = [0, H - 1]
+    names = list(ins)
+    ref_in = {n: x[:, :, ends] for n, x in ins.items()}
+    ref_o, ref_ht, ref = oracle_grads(lambda **kw: _call(op, {n: kw[n] for n in names}, kw["h0"], cu, False), dict(ref_in, h0=h0[:, ends]),
+                                      do[:, :, ends], dht[:, ends])
+    dev = {n: x.to(cuda).requires_grad_(True) for n, x in dict(ins, h0=h0).items()}
+    if form == "packed":
+        o, ht = _call(op, dev, dev["h0"], cu.to(cuda), True)
+    else:
+        import linear_moe_amd as L
+        f = {"simple_gla": L.chunk_simple_gla, "gla": L.chunk_gla, "gdn": L.chunk_gated_delta_rule}[op]
+        o, ht = f(*(dev[n].transpose(1, 2) for n in names), initial_state=dev["h0"], output_final_state=True, head_first=True)
+        o = o.transpose(1, 2)
+    grads = dict(zip(dev, torch.autograd.grad([o, ht], list(dev.values()), [do.to(cuda), dht.to(cuda)])))
+    tol = TOL[dtype]
+    assert max_abs_rel(o.detach()[:, :, ends].cpu(), ref_o) < tol
+    assert max_abs_rel(ht.detach()[:, ends].cpu(), ref_ht) < tol
+    for n, r in ref.items():
+        x = grads[n][:, ends] if n == "h0" else grads[n][:, :, ends]
+        assert max_abs_rel(x.cpu(), r) < tol, n
