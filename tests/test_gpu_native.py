@@ -467,12 +467,36 @@ def test_routing_tables_same_bits(cuda, monkeypatch, is64, B, S, topk, E, capaci
 
 @pytest.mark.parametrize("name", ["gates", "swish", "combine", "mixer"])
 def test_neighbours_refuse_or_convert_what_hooks_hand_back(cuda, name):
-    """Another type of a saved tensor is not read as the type it had."""
+    """A saved tensor that comes back in another type, with other strides or at another place in memory is read as what was saved, or
+    refused; one of another shape or device is refused."""
     fn, leaves = _neighbour_calls(cuda, 2, 70, 2, 64, torch.bfloat16)[name]
-    ref = _outputs(fn, leaves)
-    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), lambda t: t):
-        for a, b in zip(ref, _outputs(fn, leaves)):
-            assert torch.equal(a, b)
+    ref, saved = _outputs(fn, leaves), []
+
+    def through(change):
+        count = [0]
+
+        def pack(t):
+            count[0] += 1
+            return count[0] - 1, t
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda p: change(*p)):
+            return _outputs(fn, leaves)
+
+    through(lambda i, t: saved.append(t) or t)
+    same = [lambda x: x.clone(), lambda x: x.float() if x.dtype == torch.bfloat16 else x.double(),
+            lambda x: x.mT.contiguous().mT if x.dim() > 1 else x.double(), _misaligned]
+    other = [lambda x: x[:1] if x.shape[0] > 1 else x[:, :1], lambda x: x[..., :-8] if x.shape[-1] > 8 else x[..., :-1], lambda x: x.cpu()]
+    converted = 0
+    for i, f in itertools.product(range(len(saved)), same):
+        try:
+            got = through(lambda j, x: f(x) if i == j else x)
+        except (RuntimeError, ValueError):
+            continue
+        converted += 1
+        assert all(torch.equal(a, b) for a, b in zip(ref, got)), i
+    assert converted >= (4 if name != "mixer" else 3) * len(saved)         # (q, k, v of another type than the call are refused)
+    for i, f in itertools.product(range(len(saved)), other):
+        with pytest.raises((RuntimeError, ValueError)):
+            through(lambda j, x: f(x) if i == j else x)
 
 
 def test_calls_without_a_node_are_still_functions_of_autograd_for_transforms(cuda):
