@@ -38,18 +38,18 @@ STAGE_NAMES = {0: "k_gdn_wy_fwd", 1: "k_gdn_state_fwd_reg", 4: "k_gdn_state_bwd"
 # sources (kernel_sources_sha16()) at that time, and a build whose sources differ reports traffic = null
 # rather than a stale number.
 CALIB_COPY_BYTES = 256 << 20
-MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237249132, "k_gdn_state_fwd_reg": 1084677352, "k_gdn_state_bwd": 946047680,
-                    "k_gdn_bwd_chunk": 1830561566}
-TRAFFIC_SOURCES_SHA16 = "f13bb9b8e366204e"
+MEASURED_TRAFFIC = {"k_gdn_wy_fwd": 237228907, "k_gdn_state_fwd_reg": 1084600621, "k_gdn_state_bwd": 945980338,
+                    "k_gdn_bwd_chunk": 1830352179}
+TRAFFIC_SOURCES_SHA16 = "a32943ea6b05ad13"
 TRAFFIC_SOURCES = ("lmoe_common.hpp", "lmoe_seq.hpp", "lmoe_gdn_wy.hpp", "lmoe_gdn_state.hpp", "lmoe_gdn_state_reg.hpp", "lmoe_gdn_bwd_chunk.hpp",
                    "lmoe_split.hpp", "lmoe_gdn_split.hpp", "lmoe_gdn_fwd.hip", "lmoe_gdn_state.hip", "lmoe_gdn_bwd.hip")
 
 
 # HBM bytes per call of the other contract configurations (bench.py --other-configs), same counters and scaling,
 # summed over the kernels of the call; key = configuration number
-OTHER_TRAFFIC = {"1": 5099051, "2": 272972288, "3": 1280737995, "5": 16599990389, "6": 1445063349, "7": 6530916672,
-                 "8": 1510800533}
-OTHER_TRAFFIC_SHA16 = "ff47752da92ac46d"
+OTHER_TRAFFIC = {"1": 5951818, "2": 272939182, "3": 1280113429, "5": 16606804540, "6": 1445133419, "7": 6523446926,
+                 "8": 1510695429}
+OTHER_TRAFFIC_SHA16 = "e6a18baeb1ea52ce"
 
 
 def all_sources_sha16():
